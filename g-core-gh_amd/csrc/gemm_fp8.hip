@@ -644,8 +644,7 @@ extern "C" int lp_gemm_fp8_grouped_nn(const void *Aq, const void *As, const void
     LP_REQUIRE(scale_dtype == LP_E8M0, "lp_gemm_fp8_grouped_nn: power-of-two (LP_E8M0) scales only");
     if (!gemm::grouped_nn_ok(As, Ws, scale_dtype, E, M_total, N, K))
         return fail(LP_ERR_UNSUPPORTED,
-                    "lp_gemm_fp8_grouped_nn: needs N %% 512 == 0, K %% 512 == 0, 4-byte aligned scale tables, at most 512 experts and "
-                    "operands below 4 GiB (got E=%d M=%lld N=%lld K=%lld): transpose the weights and call lp_gemm_fp8_grouped",
+                    "lp_gemm_fp8_grouped_nn: needs at most 512 experts and operands below 4 GiB (got E=%d M=%lld N=%lld K=%lld): transpose the weights and call lp_gemm_fp8_grouped",
                     E, (long long)M_total, (long long)N, (long long)K);
     return gemm::launch_grouped_nn(Aq, As, Wq, Ws, m_offsets, E, M_total, N, K, C, out_dtype, (hipStream_t)stream);
 }

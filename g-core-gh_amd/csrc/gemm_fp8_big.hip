@@ -223,6 +223,7 @@ typedef float f32x16v __attribute__((ext_vector_type(16)));
         "s44", "s45", "s46", "s47", "s48", "s49", "s50", "s51", "s52", "s53", "s54", "s55", "s56", "s57", "s58", "s59", "s60",   \
         "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", "s74", "s75", "s76", "s77",   \
         "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", "s87", "s88", "s98", "s99"
+#define LP_ASM_CLOBBERS_RAG "s93", "s94", "s95", "s96", "s97"
 #define LP_ASM_CLOBBERS_QUAD                                                                                              \
     "memory", "scc", "m0", "v72", "v73", "v74", "v75", "v76", "v77", "v78", "v79", "v80", "v81", "v82", "v83", "v84",     \
         "v85", "v86", "v87", "v88", "v89", "v90", "v91", "v92", "v93", "v94", "v95", "v96", "v97", "v98", "v99",          \
@@ -248,6 +249,7 @@ typedef float f32x16v __attribute__((ext_vector_type(16)));
         "a219", "a220", "a221", "a222", "a223", "a224", "a225", "a226", "a227", "a228", "a229", "a230", "a231",           \
         "a232", "a233", "a234", "a235", "a236", "a237", "a238", "a239", "a240", "a241", "a242", "a243", "a244",           \
         "a245", "a246", "a247", "a248", "a249", "a250", "a251", "a252", "a253", "a254", "a255"
+#define LP_ASM_INPUTS_RAG [klast] "s"(klast), [krem] "s"(krem), [swr] "v"(swr)
 #define LP_ASM_INPUTS_WIDE                                                                                                \
     [aoff0] "v"(aoff[0]), [aoff1] "v"(aoff[1]), [aoff2] "v"(aoff[2]), [aoff3] "v"(aoff[3]), [boff0] "v"(boff[0]),         \
         [soff] "v"(soff), [srd] "v"(srd), [ard0] "v"(ard0), [ard1] "v"(ard1), [brd0] "v"(brd0), [brd1] "v"(brd1),         \
@@ -322,6 +324,9 @@ struct AsmTile {
 // time is its chain of K steps rather than its arithmetic: the chain halves.
 // NST: LDS stages (2; 3 for the flat 128 x 256 tile, whose stage in use rotates through registers; 4 for the 128 x 128
 // tile with one K block per stage: three K steps in flight).
+// RAG: K is any multiple of 128 (the other loops: of 512: their scales move in aligned groups of four); a loop of its own,
+// since requesting scales that start at any address takes registers, a second write to LDS and a dozen scalar instructions
+// per trip (see gen_gemm_loop.py).
 // BROW: the weights carry an e8m0 scale per row and K block ([N, K/128] bytes) instead of per 128 rows; the matrix
 // instruction takes a scale per operand row anyway, so the loop only fetches them differently (hardware-scaled
 // 128 x 128 loop: waves 2 and 3 copy the weight-scale dwords of a group while waves 0 and 1 copy the activations').
@@ -339,13 +344,14 @@ struct AsmTile {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 template <int TM, int TN, int KSUB, bool HWS = false, bool DUAL = false, int NST = 2, bool BROW = false, bool STAGED = false, int WN = 2, bool NN = false,
-          bool BF16 = false>
+          bool BF16 = false, bool RAG = false>
 __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restrict__ Aq, const float *__restrict__ As,
                                          const uint8_t *__restrict__ Bq, const float *__restrict__ Bs, int64_t m0, int64_t M,
                                          int64_t n0, int64_t N, int64_t K, void *__restrict__ C, int64_t ldc, int out_dtype)
 {
     using T = AsmTile<TM, TN, KSUB, NST, WN>;
     constexpr int WAVES = T::WAVES, NBW = T::NBW;
+    static_assert(!RAG || (KSUB == 1 && !DUAL && !BROW && !BF16 && ((NST == 2 && TM == TN) || WN == 4)), "any K: the 128 x 128, 256 x 256 and flat tiles");
     static_assert(WN == 2 || (WN == 4 && TM == 128 && TN == 256 && KSUB == 1 && !DUAL && NST == 3 && !BROW), "four waves along N: the 128 x 256 tile, three stages");
     // NN: Bq is the weight as stored for C = A W, [K, N] row-major (row pitch N), Bs its [K / 128, N / 128] scale bytes:
     // the 256-row and the flat tile with e8m0 scales (the data gradient of the grouped linear)
@@ -366,7 +372,7 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
     const int wm = wave / WN, wn = wave % WN;
     const int l16 = lane & 15, lq = lane >> 4;
     const uint32_t kblocks = (uint32_t)(K / KB);
-    const uint32_t trips = (DUAL ? kblocks / 2 : kblocks) / 4;
+    const uint32_t trips = ((DUAL ? kblocks / 2 : kblocks) + (RAG ? 3 : 0)) / 4;
     constexpr int SS = HWS ? 1 : 4;                      // bytes per scale
     if (DUAL) {
         smem += kg * T::LDS_BYTES;
@@ -394,14 +400,18 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
         amask[i] = __ballot(m0 + row < M);
         // a lane whose row is past the end of the activations is switched off for the copy (amask): its offset only has to exist
         const int64_t m = m0 + row < M ? m0 + row : m0;
-        const int64_t n = n0 + row < N ? n0 + row : N - 1;          // i = 3 is unused when there are three copies
+        // Weight rows past the end feed results that are not stored.  In the second half of a 256-column tile they re-read the
+        // first half's rows, lines that are on their way already and different ones per lane, as the last row would not be
+        // (which is left for the unscaled GEMM, whose N is any multiple of 16).  i = 3 is unused when there are three copies.
+        const int64_t n = n0 + row < N ? n0 + row : (TN == 256 && row >= 128 && n0 + row - 128 < N ? n0 + row - 128 : N - 1);
         aoff[i] = (uint32_t)(m * K + swz(row, ld_slot) * 16);
         boff[i] = (uint32_t)(n * K + swz(row, ld_slot) * 16);
         if constexpr (NN) {
             // a copy moves 4 contraction rows of 256 bytes: lane -> row 4 (wave + WAVES i) + lane / 16 of the K step,
             // slot lane % 16, which holds chunk slot ^ nn_swz(row) of the row (columns n0 + 16 chunk ..)
             const int krow = 4 * (wave + WAVES * i) + (lane >> 4);
-            boff[i] = (uint32_t)((int64_t)krow * N + n0 + (((lane & 15) ^ nn_swz(krow)) << 4));
+            const int64_t ncol = n0 + (((lane & 15) ^ nn_swz(krow)) << 4);
+            boff[i] = (uint32_t)((int64_t)krow * N + (ncol < N ? ncol : ncol - 128));     // columns past the end: the tile's first half again
         }
     }
     (void)NBC;
@@ -473,11 +483,16 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
     // NN: the wave's weight scales are column (n0 + its first column) / 128 of the [K / 128, N / 128] byte table, one row per
     // K step: the loop loads the aligned dword around each byte (rows are a multiple of 4 bytes apart, checked on the
     // host, so the byte's place in the dword is the same for every step)
-    const uint64_t bsn_addr = (uint64_t)(uintptr_t)Bs + (uint64_t)(wcol0 >> 7);
-    const uint64_t bsn_u = uniform((const void *)(uintptr_t)(bsn_addr & ~(uint64_t)3));
+    const uint64_t bsn_addr = (uint64_t)(uintptr_t)Bs + (uint64_t)sblk;       // sblk: inside the table also for columns past N
+    const uint64_t bsn_u = uniform((const void *)(uintptr_t)(RAG ? bsn_addr : bsn_addr & ~(uint64_t)3));
     const uint32_t bsbfe = __builtin_amdgcn_readfirstlane((uint32_t)((bsn_addr & 3) * 8) | (8u << 16));
     const uint32_t bsstride = __builtin_amdgcn_readfirstlane((uint32_t)(N >> 7));
     const uint32_t bstep = __builtin_amdgcn_readfirstlane((uint32_t)(128 * N));
+    // RAG: bytes from the first to the last K block of an operand row, K blocks of the last trip (0: four), and where this
+    // lane writes the scales of the row it loads (see srd)
+    const uint32_t klast = __builtin_amdgcn_readfirstlane((kblocks - 1) * KB), krem = __builtin_amdgcn_readfirstlane(kblocks & 3);
+    const uint32_t swr = lds0 + T::S_LDS + wave * 1024 + lane * (HWS ? 4 : 16);
+    (void)klast; (void)krem; (void)swr;
     (void)bsn_u; (void)bsbfe; (void)bsstride; (void)bstep;
     // scale staging: 16 bytes per activation row (fp32, four K steps), or 4 bytes per row in 1 KB per copying wave (e8m0)
     const uint32_t srd = HWS ? lds0 + T::S_LDS + wm * 1024 + l16 * 4 : lds0 + T::S_LDS + arow_l * 16;
@@ -530,37 +545,70 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
         accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3; accs[4] = acc4; accs[5] = acc5; accs[6] = acc6;
     } else if constexpr (NN && WN == 4) {
         f32x16v acc0, acc1, acc2, acc3;
-        asm volatile(
+        if constexpr (RAG) {
+            asm volatile(
+#include "gemm_flat_hw_nn_rag_loop.inc"
+                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
+                : LP_ASM_INPUTS_NN, LP_ASM_INPUTS_RAG
+                : LP_ASM_CLOBBERS, LP_ASM_CLOBBERS_RAG, "s64", "s65", "s66", "s89", "s90", "s91", "s92");
+        } else {
+            asm volatile(
 #include "gemm_flat_hw_nn_loop.inc"
-            : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
-            : LP_ASM_INPUTS_NN
-            : LP_ASM_CLOBBERS, "s64", "s65", "s66", "s89", "s90", "s91", "s92");
+                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
+                : LP_ASM_INPUTS_NN
+                : LP_ASM_CLOBBERS, "s64", "s65", "s66", "s89", "s90", "s91", "s92");
+        }
         accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3;
     } else if constexpr (NN) {
         f32x16v acc0, acc1, acc2, acc3, acc4, acc5, acc6, acc7;
-        asm volatile(
+        if constexpr (RAG) {
+            asm volatile(
+#include "gemm_big_hw_nn_rag_loop.inc"
+                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3),
+                  "=&{v[192:207]}"(acc4), "=&{v[208:223]}"(acc5), "=&{v[224:239]}"(acc6), "=&{v[240:255]}"(acc7)
+                : LP_ASM_INPUTS_NN, LP_ASM_INPUTS_RAG, [brdn4] "v"(brdn[4]), [brdn5] "v"(brdn[5]), [brdn6] "v"(brdn[6]), [brdn7] "v"(brdn[7])
+                : LP_ASM_CLOBBERS, LP_ASM_CLOBBERS_RAG, "s64", "s65", "s66");
+        } else {
+            asm volatile(
 #include "gemm_big_hw_nn_loop.inc"
-            : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3),
-              "=&{v[192:207]}"(acc4), "=&{v[208:223]}"(acc5), "=&{v[224:239]}"(acc6), "=&{v[240:255]}"(acc7)
-            : LP_ASM_INPUTS_NN, [brdn4] "v"(brdn[4]), [brdn5] "v"(brdn[5]), [brdn6] "v"(brdn[6]), [brdn7] "v"(brdn[7])
-            : LP_ASM_CLOBBERS, "s64", "s65", "s66");
+                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3),
+                  "=&{v[192:207]}"(acc4), "=&{v[208:223]}"(acc5), "=&{v[224:239]}"(acc6), "=&{v[240:255]}"(acc7)
+                : LP_ASM_INPUTS_NN, [brdn4] "v"(brdn[4]), [brdn5] "v"(brdn[5]), [brdn6] "v"(brdn[6]), [brdn7] "v"(brdn[7])
+                : LP_ASM_CLOBBERS, "s64", "s65", "s66");
+        }
         accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3;
         accs[4] = acc4; accs[5] = acc5; accs[6] = acc6; accs[7] = acc7;
     } else if constexpr (WN == 4) {
         // the early hand-back of this loop splits the weight copies by wave: the first four copy each wave column's first half
         f32x16v acc0, acc1, acc2, acc3;
         if constexpr (HWS) {
-            asm volatile(
+            if constexpr (RAG) {
+                asm volatile(
+#include "gemm_flat_hw_rag_loop.inc"
+                    : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
+                    : LP_ASM_INPUTS, LP_ASM_INPUTS_RAG
+                    : LP_ASM_CLOBBERS, LP_ASM_CLOBBERS_RAG, "s87", "s89", "s90", "s91", "s92");
+            } else {
+                asm volatile(
 #include "gemm_flat_hw_loop.inc"
-                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
-                : LP_ASM_INPUTS
-                : LP_ASM_CLOBBERS, "s87", "s89", "s90", "s91", "s92");
+                    : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
+                    : LP_ASM_INPUTS
+                    : LP_ASM_CLOBBERS, "s87", "s89", "s90", "s91", "s92");
+            }
         } else {
-            asm volatile(
+            if constexpr (RAG) {
+                asm volatile(
+#include "gemm_flat_rag_loop.inc"
+                    : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
+                    : LP_ASM_INPUTS, LP_ASM_INPUTS_RAG
+                    : LP_ASM_CLOBBERS, LP_ASM_CLOBBERS_RAG, "s87", "s89", "s90", "s91", "s92");
+            } else {
+                asm volatile(
 #include "gemm_flat_loop.inc"
-                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
-                : LP_ASM_INPUTS
-                : LP_ASM_CLOBBERS, "s87", "s89", "s90", "s91", "s92");
+                    : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
+                    : LP_ASM_INPUTS
+                    : LP_ASM_CLOBBERS, "s87", "s89", "s90", "s91", "s92");
+            }
         }
         accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3;
     } else if constexpr (HWS && NBW == 8) {
@@ -575,12 +623,21 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
                 : LP_ASM_INPUTS
                 : LP_ASM_CLOBBERS);
         } else {
-            asm volatile(
+            if constexpr (RAG) {
+                asm volatile(
+#include "gemm_big_hw_rag_loop.inc"
+                    : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3),
+                      "=&{v[192:207]}"(acc4), "=&{v[208:223]}"(acc5), "=&{v[224:239]}"(acc6), "=&{v[240:255]}"(acc7)
+                    : LP_ASM_INPUTS, LP_ASM_INPUTS_RAG
+                    : LP_ASM_CLOBBERS, LP_ASM_CLOBBERS_RAG);
+            } else {
+                asm volatile(
 #include "gemm_big_hw_loop.inc"
-                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3),
-                  "=&{v[192:207]}"(acc4), "=&{v[208:223]}"(acc5), "=&{v[224:239]}"(acc6), "=&{v[240:255]}"(acc7)
-                : LP_ASM_INPUTS
-                : LP_ASM_CLOBBERS);
+                    : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3),
+                      "=&{v[192:207]}"(acc4), "=&{v[208:223]}"(acc5), "=&{v[224:239]}"(acc6), "=&{v[240:255]}"(acc7)
+                    : LP_ASM_INPUTS
+                    : LP_ASM_CLOBBERS);
+            }
         }
         accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3;
         accs[4] = acc4; accs[5] = acc5; accs[6] = acc6; accs[7] = acc7;
@@ -610,20 +667,37 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
         accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3;
     } else if constexpr (HWS) {
         f32x16v acc0, acc1, acc2, acc3;
-        asm volatile(
+        if constexpr (RAG) {
+            asm volatile(
+#include "gemm_mid_hw_rag_loop.inc"
+                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
+                : LP_ASM_INPUTS, LP_ASM_INPUTS_RAG
+                : LP_ASM_CLOBBERS, LP_ASM_CLOBBERS_RAG);
+        } else {
+            asm volatile(
 #include "gemm_mid_hw_loop.inc"
-            : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
-            : LP_ASM_INPUTS
-            : LP_ASM_CLOBBERS);
+                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
+                : LP_ASM_INPUTS
+                : LP_ASM_CLOBBERS);
+        }
         accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3;
     } else if constexpr (NBW == 8) {
         f32x16v acc0, acc1, acc2, acc3, acc4, acc5, acc6, acc7;
-        asm volatile(
+        if constexpr (RAG) {
+            asm volatile(
+#include "gemm_big_rag_loop.inc"
+                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3),
+                  "=&{v[192:207]}"(acc4), "=&{v[208:223]}"(acc5), "=&{v[224:239]}"(acc6), "=&{v[240:255]}"(acc7)
+                : LP_ASM_INPUTS, LP_ASM_INPUTS_RAG
+                : LP_ASM_CLOBBERS, LP_ASM_CLOBBERS_RAG);
+        } else {
+            asm volatile(
 #include "gemm_big_loop.inc"
-            : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3),
-              "=&{v[192:207]}"(acc4), "=&{v[208:223]}"(acc5), "=&{v[224:239]}"(acc6), "=&{v[240:255]}"(acc7)
-            : LP_ASM_INPUTS
-            : LP_ASM_CLOBBERS);
+                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3),
+                  "=&{v[192:207]}"(acc4), "=&{v[208:223]}"(acc5), "=&{v[224:239]}"(acc6), "=&{v[240:255]}"(acc7)
+                : LP_ASM_INPUTS
+                : LP_ASM_CLOBBERS);
+        }
         accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3;
         accs[4] = acc4; accs[5] = acc5; accs[6] = acc6; accs[7] = acc7;
     } else if constexpr (NBW == 6) {
@@ -638,11 +712,19 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
         accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3; accs[4] = acc4; accs[5] = acc5;
     } else if constexpr (KSUB == 1) {
         f32x16v acc0, acc1, acc2, acc3;
-        asm volatile(
+        if constexpr (RAG) {
+            asm volatile(
+#include "gemm_mid_rag_loop.inc"
+                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
+                : LP_ASM_INPUTS, LP_ASM_INPUTS_RAG
+                : LP_ASM_CLOBBERS, LP_ASM_CLOBBERS_RAG);
+        } else {
+            asm volatile(
 #include "gemm_mid_loop.inc"
-            : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
-            : LP_ASM_INPUTS
-            : LP_ASM_CLOBBERS);
+                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
+                : LP_ASM_INPUTS
+                : LP_ASM_CLOBBERS);
+        }
         accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3;
     } else {
         f32x16v acc0, acc1, acc2, acc3;
@@ -897,7 +979,7 @@ __device__ __forceinline__ void tile_quad(uint8_t *smem, const uint8_t *__restri
 
 #pragma clang diagnostic pop
 
-template <int TM, int TN, int KSUB, bool HWS = false, int NST = 2>
+template <int TM, int TN, int KSUB, bool HWS = false, int NST = 2, bool RAG = false>
 __global__ __launch_bounds__(TM * 2) void gemm_asm(const uint8_t *__restrict__ Aq, const float *__restrict__ As,
                                                    const uint8_t *__restrict__ Bq, const float *__restrict__ Bs, int64_t M,
                                                    int64_t N, int64_t K, int64_t tiles_m, int64_t tiles_n,
@@ -906,7 +988,7 @@ __global__ __launch_bounds__(TM * 2) void gemm_asm(const uint8_t *__restrict__ A
     __shared__ __attribute__((aligned(1024))) uint8_t smem[AsmTile<TM, TN, KSUB, NST>::LDS_BYTES];
     int64_t tm, tn;
     if (!gemm::tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
-    tile_asm<TM, TN, KSUB, HWS, false, NST, false, true>(smem, Aq, As, Bq, Bs, tm * TM, M, tn * TN, N, K, C, ldc, out_dtype);
+    tile_asm<TM, TN, KSUB, HWS, false, NST, false, true, 2, false, false, RAG>(smem, Aq, As, Bq, Bs, tm * TM, M, tn * TN, N, K, C, ldc, out_dtype);
 }
 
 // The unscaled bf16 NT GEMM on the 256 x 256 loop (tile_asm with BF16): row_bytes = 2 K, every scale byte 2^0.
@@ -1030,7 +1112,7 @@ __global__ __launch_bounds__(256) void gemm_asm_rowscale_grouped(const uint8_t *
 //   2  what PART 1 leaves, i.e. the last M_e % 256 rows, in tiles of TM
 // Launching 1 with 256 x 256 tiles and then 2 with 128 x 128 tiles keeps the large tiles full and bounds the
 // padding of an expert by 127 rows.
-template <int TM, int TN, int KSUB, int PART, bool HWS = false>
+template <int TM, int TN, int KSUB, int PART, bool HWS = false, bool RAG = false>
 __global__ __launch_bounds__(TM * 2) void gemm_asm_grouped(const uint8_t *__restrict__ Aq, const float *__restrict__ As,
                                                            const uint8_t *__restrict__ Bq, const float *__restrict__ Bs,
                                                            const int32_t *__restrict__ m_offsets, int E, int64_t M_total,
@@ -1084,7 +1166,7 @@ __global__ __launch_bounds__(TM * 2) void gemm_asm_grouped(const uint8_t *__rest
     const int64_t first = PART == 2 ? row_begin + (row_end - row_begin) / 256 * 256 : row_begin;
     const int64_t kblocks = K / KB;
     const float *bs_e = (const float *)((const char *)Bs + (int64_t)e * (N / 128) * kblocks * (HWS ? 1 : 4));
-    tile_asm<TM, TN, KSUB, HWS, false, 2, false, true>(smem, Aq, As, Bq + (int64_t)e * N * K, bs_e, first + (gmt - found_first) * TM, row_end,
+    tile_asm<TM, TN, KSUB, HWS, false, 2, false, true, 2, false, false, RAG>(smem, Aq, As, Bq + (int64_t)e * N * K, bs_e, first + (gmt - found_first) * TM, row_end,
                                 tn * TN, N, K, C, N, out_dtype);
 }
 
@@ -1102,7 +1184,7 @@ constexpr int kMixedMaxExperts = 512;
 
 // NN: expert e's weight is stored [K, N] (the layer's own [out, in] weight read for the data gradient dX = dY W: K = out
 // features = the contraction, N = in features = the columns of C), its scale bytes [K / 128, N / 128].
-template <bool HWS, bool NN = false>
+template <bool HWS, bool NN = false, bool RAG = false>
 __global__ __launch_bounds__(512) void gemm_asm_grouped_mixed(const uint8_t *__restrict__ Aq, const float *__restrict__ As,
                                                               const uint8_t *__restrict__ Bq, const float *__restrict__ Bs,
                                                               const int32_t *__restrict__ m_offsets, int E, int64_t M_total,
@@ -1145,7 +1227,7 @@ __global__ __launch_bounds__(512) void gemm_asm_grouped_mixed(const uint8_t *__r
     tot_small = __builtin_amdgcn_readfirstlane(tot_small);
     // ---- which class and which tile of it this workgroup takes (32-bit arithmetic: the grid is below 2^31, and 64-bit
     // divisions by run-time values would cost this prologue about a microsecond per workgroup)
-    const uint32_t tiles_n = (uint32_t)(N >> 8);
+    const uint32_t tiles_n = (uint32_t)((N + 255) >> 8);                   // the last column tile may be half empty
     auto padded_slots = [](uint32_t tiles) -> uint32_t {                   // workgroups per XCD for that many tiles
         const uint32_t chunks = (tiles + gemm::CHUNK - 1) / gemm::CHUNK;
         return ((chunks + 7) / 8) * gemm::CHUNK;
@@ -1240,9 +1322,9 @@ __global__ __launch_bounds__(512) void gemm_asm_grouped_mixed(const uint8_t *__r
             const uint8_t *bq_e = Bq + (int64_t)e * N * K;
             __syncthreads();                            // every wave is done with the previous tile's use of the stage memory
             if (ex >> 30)
-                tile_asm<256, 256, 1, HWS, false, 2, false, true, 2, NN>(smem, Aq, As, bq_e, bs_e, m0, row_end, n0, N, K, C, N, out_dtype);
+                tile_asm<256, 256, 1, HWS, false, 2, false, true, 2, NN, false, RAG>(smem, Aq, As, bq_e, bs_e, m0, row_end, n0, N, K, C, N, out_dtype);
             else
-                tile_asm<128, 256, 1, HWS, false, 3, false, true, 4, NN>(smem, Aq, As, bq_e, bs_e, m0, row_end, n0, N, K, C, N, out_dtype);
+                tile_asm<128, 256, 1, HWS, false, 3, false, true, 4, NN, false, RAG>(smem, Aq, As, bq_e, bs_e, m0, row_end, n0, N, K, C, N, out_dtype);
         }
     }
 }
@@ -1264,13 +1346,24 @@ int launch_nb(const void *Aq, const void *As, const void *Bq, const void *Bs, in
 namespace lowp {
 namespace gemm {
 
-// The hand-scheduled loop addresses operands with 32-bit offsets and moves scales in 16-byte groups
-// of four K steps.
+// The hand-scheduled loops address operands with 32-bit offsets.
+static bool asm_size_ok(const void *As, const void *Bs, int64_t M, int64_t N, int64_t K, int scale_dtype)
+{
+    const uintptr_t align = scale_dtype == LP_E8M0 ? 0 : 3;
+    return K % 128 == 0 && (((uintptr_t)As | (uintptr_t)Bs) & align) == 0 && M * K < 0xFFFFFFFFll && N * K < 0xFFFFFFFFll &&
+           M * (K / 128) * 4 < 0xFFFFFFFFll;
+}
+
+// All but the RAG loops move scales in aligned groups of four K steps; what does not fit that (K % 512, or a scale table that
+// starts off its alignment) takes a RAG loop.  Before, such shapes ran on the compiler-scheduled 128 x 128 kernels, which are
+// left with operands of 4 GiB and more (one MI355X, us, fp32 / e8m0 scales, before -> now: 1000 x 4992 x 2944 38.8 / 43.0 ->
+// 26.9 / 22.2, 4096 x 4096 x 4224 95 / 109 -> 70 / 60, 8192 x 7168 x 2176 176 / 207 -> 126 / 112; grouped, 32 experts, 4096 rows,
+// N = 4096, K = 1920 116 / 131 -> 75 / 72).  Where K is a multiple of 512 the aligned loops stay 1 - 4 % ahead per K block
+// (4096 x 4096 x 4096: 64.8 / 55.6 us = 2.12 / 2.47 PFLOP/s, x 4224: 2.02 / 2.35).
 static bool asm_shape_ok(const void *As, const void *Bs, int64_t M, int64_t N, int64_t K, int scale_dtype = LP_F32)
 {
     const uintptr_t align = scale_dtype == LP_E8M0 ? 3 : 15;          // one group of four scales per access
-    return K % 512 == 0 && (((uintptr_t)As | (uintptr_t)Bs) & align) == 0 && M * K < 0xFFFFFFFFll && N * K < 0xFFFFFFFFll &&
-           M * (K / 128) * 4 < 0xFFFFFFFFll;
+    return K % 512 == 0 && (((uintptr_t)As | (uintptr_t)Bs) & align) == 0 && asm_size_ok(As, Bs, M, N, K, scale_dtype);
 }
 
 // Picks the tile width whose last round of tiles wastes the fewest CU slots.
@@ -1306,6 +1399,17 @@ int launch_big(const void *Aq, const void *As, const void *Bq, const void *Bs, i
         return launch_nb<SDT, 4>(Aq, As, Bq, Bs, M, N, K, C, ldc, out_dtype, st);                            \
     } while (0)
     static const bool no_asm = getenv("LP_GEMM_NO_ASM") != nullptr;       // tuning / test aid
+    if (!no_asm && tn == 256 && !asm_shape_ok(As, Bs, M, N, K, scale_dtype) && asm_size_ok(As, Bs, M, N, K, scale_dtype)) {
+        const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + 255) / 256;
+        const int64_t grid = gemm::padded_grid(tiles_m, tiles_n);
+        if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_block: problem too large");
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(THREADS), 0, st, (const uint8_t *)Aq, (const float *)As, (const uint8_t *)Bq,
+                               (const float *)Bs, M, N, K, tiles_m, tiles_n, C, ldc, out_dtype);
+        };
+        scale_dtype == LP_E8M0 ? go(gemm_asm<256, 256, 1, true, 2, true>) : go(gemm_asm<256, 256, 1, false, 2, true>);
+        return check_launch("lp_gemm_fp8_block(asm, any K)");
+    }
     if (!no_asm && scale_dtype == LP_E8M0 && tn == 256 && asm_shape_ok(As, Bs, M, N, K, LP_E8M0)) {
         // e8m0 scales: the matrix cores apply them (no fold, accumulation in place)
         const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + 255) / 256;
@@ -1434,7 +1538,7 @@ bool launch_mixed(const void *Aq, const void *As, const void *Bq, const void *Bs
 bool mid_asm_ok(const void *As, const void *Bs, int scale_dtype, int64_t M, int64_t N, int64_t K)
 {
     static const bool no_asm = getenv("LP_GEMM_NO_ASM") != nullptr || getenv("LP_GEMM_NO_MID") != nullptr;
-    return !no_asm && (scale_dtype == LP_F32 || scale_dtype == LP_E8M0) && asm_shape_ok(As, Bs, M, N, K, scale_dtype);
+    return !no_asm && (scale_dtype == LP_F32 || scale_dtype == LP_E8M0) && asm_size_ok(As, Bs, M, N, K, scale_dtype);
 }
 
 int launch_mid_asm(const void *Aq, const void *As, const void *Bq, const void *Bs, int scale_dtype, int64_t M, int64_t N,
@@ -1443,6 +1547,14 @@ int launch_mid_asm(const void *Aq, const void *As, const void *Bq, const void *B
     const int64_t tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128;
     const int64_t grid = gemm::padded_grid(tiles_m, tiles_n);
     if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_block: problem too large");
+    if (!asm_shape_ok(As, Bs, M, N, K, scale_dtype)) {
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), 0, st, (const uint8_t *)Aq, (const float *)As, (const uint8_t *)Bq,
+                               (const float *)Bs, M, N, K, tiles_m, tiles_n, C, ldc, out_dtype);
+        };
+        scale_dtype == LP_E8M0 ? go(gemm_asm<128, 128, 1, true, 2, true>) : go(gemm_asm<128, 128, 1, false, 2, true>);
+        return check_launch("lp_gemm_fp8_block(asm128, any K)");
+    }
     // At most one tile per CU: split K inside the workgroup (needs whole scale groups of 512 in each half).  With
     // more tiles than CUs the 512-thread workgroups would need a second round where 256-thread ones share the CUs
     // (288 tiles at K = 7168: 90 us with the split against 60 without).
@@ -1525,12 +1637,11 @@ int launch_rowscale_grouped_asm(const void *Aq, const void *As, const void *Bq, 
     return check_launch("lp_gemm_fp8_rowscale_grouped(asm)");
 }
 
-// Grouped problems on the hand-scheduled kernel: fp32 scales, N a multiple of 256, offsets that fit 32 bits.
+// Grouped problems on the hand-scheduled kernels: offsets that fit 32 bits.
 bool big_grouped_ok(const void *As, const void *Bs, int scale_dtype, int64_t M_total, int64_t N, int64_t K)
 {
     static const bool no_asm = getenv("LP_GEMM_NO_ASM") != nullptr;
-    return !no_asm && (scale_dtype == LP_F32 || scale_dtype == LP_E8M0) && N % 256 == 0 &&
-           asm_shape_ok(As, Bs, M_total, N, K, scale_dtype);
+    return !no_asm && (scale_dtype == LP_F32 || scale_dtype == LP_E8M0) && asm_size_ok(As, Bs, M_total, N, K, scale_dtype);
 }
 
 // CUs of the current device (0 if it cannot be asked); asked once per device
@@ -1547,23 +1658,27 @@ static int compute_units()
     return cached[dev] > 0 ? cached[dev] : 0;
 }
 
-// The data gradient of the grouped linear on the stored weights (no transposed copy): e8m0 scales, N a multiple of 256,
-// K of 512, the scale table's rows a multiple of 4 bytes apart and 4-byte aligned, at most kMixedMaxExperts experts.
+// The data gradient of the grouped linear on the stored weights (no transposed copy): e8m0 scales, at most
+// kMixedMaxExperts experts.
 bool grouped_nn_ok(const void *As, const void *Bs, int scale_dtype, int E, int64_t M_total, int64_t N, int64_t K)
 {
-    return scale_dtype == LP_E8M0 && E <= kMixedMaxExperts && N % 256 == 0 && (N / 128) % 4 == 0 && ((uintptr_t)Bs & 3) == 0 &&
-           asm_shape_ok(As, Bs, M_total, N, K, LP_E8M0);
+    return scale_dtype == LP_E8M0 && E <= kMixedMaxExperts && asm_size_ok(As, Bs, M_total, N, K, LP_E8M0);
 }
 
 int launch_grouped_nn(const void *Aq, const void *As, const void *Bq, const void *Bs, const int32_t *m_offsets, int E,
                       int64_t M_total, int64_t N, int64_t K, void *C, int out_dtype, hipStream_t st)
 {
-    int64_t grid = padded_grid(M_total / 256 + E, N / 256) + 2 * 8 * CHUNK;
+    int64_t grid = padded_grid(M_total / 256 + E, (N + 255) / 256) + 2 * 8 * CHUNK;
     if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_grouped_nn: problem too large");
     const int cus = compute_units();
     if (cus >= 8 && grid > cus) grid = cus / 8 * 8;            // one workgroup per CU walks the tile slots, as in the forward launch
-    hipLaunchKernelGGL((gemm_asm_grouped_mixed<true, true>), dim3((unsigned)grid), dim3(512), 0, st, (const uint8_t *)Aq,
-                       (const float *)As, (const uint8_t *)Bq, (const float *)Bs, m_offsets, E, M_total, N, K, C, out_dtype, 4);
+    // the loop without RAG takes the dword around a scale byte: rows of the weight's scale table a multiple of 4 bytes apart
+    const bool rag = !asm_shape_ok(As, Bs, M_total, N, K, LP_E8M0) || N % 512;
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(512), 0, st, (const uint8_t *)Aq, (const float *)As, (const uint8_t *)Bq,
+                           (const float *)Bs, m_offsets, E, M_total, N, K, C, out_dtype, 4);
+    };
+    rag ? go(gemm_asm_grouped_mixed<true, true, true>) : go(gemm_asm_grouped_mixed<true, true, false>);
     return check_launch("lp_gemm_fp8_grouped_nn");
 }
 
@@ -1584,11 +1699,13 @@ int launch_big_grouped(const void *Aq, const void *As, const void *Bq, const voi
     // 17.8 us; 16 experts, N = 4096, K = 1536: 37.4 against 32.9 the other way).  Decode-sized batches pass the same test
     // with their flat tiles alone: 256 experts of 1 .. 127 rows, gate_up shape, 1.10 - 1.30 ms against 1.26 - 1.49 on the
     // 128 x 128 kernel (three LDS stages of streamed weights against two); 8 such experts stay there, 45 against 72 us.
-    const bool enough_tiles = (M_total / 256 + E / 2) * (N / 256) >= 256;
+    const int64_t tiles_n = (N + 255) / 256;
+    const bool enough_tiles = (M_total / 256 + E / 2) * tiles_n >= 256;
+    const bool rag = !asm_shape_ok(As, Bs, M_total, N, K, scale_dtype);
     if (mode == 2 || (mode < 0 && E <= kMixedMaxExperts && enough_tiles)) {
         // an expert with r rows has r / 256 tiles plus one when rows are left over, big or small: M_total / 256 + E row
         // tiles at most over both classes, each class rounded up to whole groups of 8 x 32 workgroups
-        int64_t grid = padded_grid(M_total / 256 + E, N / 256) + 2 * 8 * CHUNK;
+        int64_t grid = padded_grid(M_total / 256 + E, tiles_n) + 2 * 8 * CHUNK;
         if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_grouped: problem too large");
         if (E <= kMixedMaxExperts) {
             // one workgroup per CU that works through every grid-th slot (a workgroup owns its CU: the tiles' LDS)
@@ -1600,25 +1717,26 @@ int launch_big_grouped(const void *Aq, const void *As, const void *Bq, const voi
             if (cus >= 8 && grid > cus) grid = cus / 8 * 8;
             static const char *order_env = getenv("LP_GEMM_GROUPED_ORDER");     // tuning aid: XCDs that take their small tiles first (0: classes dealt alternately)
             const int small_first = order_env ? atoi(order_env) : 4;
-            if (scale_dtype == LP_E8M0)
-                hipLaunchKernelGGL((gemm_asm_grouped_mixed<true>), dim3((unsigned)grid), dim3(512), 0, st, (const uint8_t *)Aq,
-                                   (const float *)As, (const uint8_t *)Bq, (const float *)Bs, m_offsets, E, M_total, N, K, C, out_dtype, small_first);
-            else
-                hipLaunchKernelGGL((gemm_asm_grouped_mixed<false>), dim3((unsigned)grid), dim3(512), 0, st, (const uint8_t *)Aq,
-                                   (const float *)As, (const uint8_t *)Bq, (const float *)Bs, m_offsets, E, M_total, N, K, C, out_dtype, small_first);
+            auto go = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(512), 0, st, (const uint8_t *)Aq, (const float *)As, (const uint8_t *)Bq,
+                                   (const float *)Bs, m_offsets, E, M_total, N, K, C, out_dtype, small_first);
+            };
+            if (scale_dtype == LP_E8M0) rag ? go(gemm_asm_grouped_mixed<true, false, true>) : go(gemm_asm_grouped_mixed<true>);
+            else rag ? go(gemm_asm_grouped_mixed<false, false, true>) : go(gemm_asm_grouped_mixed<false>);
             return check_launch("lp_gemm_fp8_grouped(asm mixed heights)");
         }
     }
-    if (scale_dtype == LP_E8M0) {
-        // e8m0 scales: 128 x 128 tiles on the kernel whose matrix instructions apply the scales
+    auto go128 = [&](auto kernel) {
         const int64_t mtiles = M_total / 128 + E;
         const int64_t grid = padded_grid(mtiles, N / 128);
         if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_grouped: problem too large");
-        hipLaunchKernelGGL((gemm_asm_grouped<128, 128, 1, 0, true>), dim3((unsigned)grid), dim3(256), 0, st, (const uint8_t *)Aq,
-                           (const float *)As, (const uint8_t *)Bq, (const float *)Bs, m_offsets, E, M_total, N, K, mtiles, N / 128, C,
-                           out_dtype);
-        return check_launch("lp_gemm_fp8_grouped(asm 128 e8m0)");
-    }
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), 0, st, (const uint8_t *)Aq, (const float *)As, (const uint8_t *)Bq,
+                           (const float *)Bs, m_offsets, E, M_total, N, K, mtiles, N / 128, C, out_dtype);
+        return check_launch("lp_gemm_fp8_grouped(asm 128)");
+    };
+    // e8m0 scales: 128 x 128 tiles on the kernel whose matrix instructions apply the scales
+    if (scale_dtype == LP_E8M0) return rag ? go128(gemm_asm_grouped<128, 128, 1, 0, true, true>) : go128(gemm_asm_grouped<128, 128, 1, 0, true>);
+    if (rag) return go128(gemm_asm_grouped<128, 128, 1, 0, false, true>);
     // Few rows per expert on average: the weights of most experts are read for one or two row tiles, so the launch
     // is as much a weight stream as a GEMM.  128 x 128 tiles (two workgroups per CU, tiles taken from both ends
     // of the expert list) let streaming tiles and compute-bound tiles overlap and bound the padding per expert
@@ -1627,10 +1745,10 @@ int launch_big_grouped(const void *Aq, const void *As, const void *Bq, const voi
     const bool split = mode >= 0 ? mode == 1 : M_total >= (int64_t)E * 1024;
     if (split) {
         const int64_t big_mtiles = M_total / 256;
-        const int64_t grid = padded_grid(big_mtiles, N / 256);
+        const int64_t grid = padded_grid(big_mtiles, tiles_n);
         if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_grouped: problem too large");
         hipLaunchKernelGGL((gemm_asm_grouped<256, 256, 1, 1>), dim3((unsigned)grid), dim3(512), 0, st, (const uint8_t *)Aq,
-                           (const float *)As, (const uint8_t *)Bq, (const float *)Bs, m_offsets, E, M_total, N, K, big_mtiles, N / 256,
+                           (const float *)As, (const uint8_t *)Bq, (const float *)Bs, m_offsets, E, M_total, N, K, big_mtiles, tiles_n,
                            C, out_dtype);
         const int rc = check_launch("lp_gemm_fp8_grouped(asm 256)");
         if (rc) return rc;
@@ -1643,13 +1761,7 @@ int launch_big_grouped(const void *Aq, const void *As, const void *Bq, const voi
                            C, out_dtype);
         return check_launch("lp_gemm_fp8_grouped(asm 128)");
     }
-    const int64_t mtiles = M_total / 128 + E;
-    const int64_t grid = padded_grid(mtiles, N / 128);
-    if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_grouped: problem too large");
-    hipLaunchKernelGGL((gemm_asm_grouped<128, 128, 1, 0>), dim3((unsigned)grid), dim3(256), 0, st, (const uint8_t *)Aq,
-                       (const float *)As, (const uint8_t *)Bq, (const float *)Bs, m_offsets, E, M_total, N, K, mtiles, N / 128, C,
-                       out_dtype);
-    return check_launch("lp_gemm_fp8_grouped(asm 128)");
+    return go128(gemm_asm_grouped<128, 128, 1, 0>);
 }
 
 }  // namespace gemm

@@ -36,13 +36,23 @@ MB = 4                                     # 16-row blocks per wave (64 activati
 
 
 def configure(tm, tn, waves_m, waves_n, ksub, hw=False, nstage=2, brow=False, early=False, wide=False, idle=False, pingpong=False, nn=False,
-              bf16=False):
+              bf16=False, rag=False):
     """Tile tm x tn, waves_m x waves_n waves of 64 x (tn / waves_n); a stage holds ksub K blocks of 128; nstage
     stages in LDS (2: the copies of the next stage overlap this one; 4 with ksub 1: three K steps are in flight,
     for problems of about one tile per CU whose time is the chain of K steps)."""
     global A_BYTES, B_BYTES, SCL_LDS, SCL_HALF, NB, WAVES, KSUB, SPLIT, HW, NSTAGE, BROW, EARLY, WIDE, lines
     global ACC, P, AF, SC, SC2, SAN, WFB, RA0, RA1, RB0, RB1, SRD0, SRD, WS1, WS2, WSCUR, HALFSPLIT, ROT, WITH_IDLE, IDLE, PINGPONG, GRP, SPREAD, NN, BF, RBN
-    global WIDE_GROUP, WIDE_PART, BF16
+    global WIDE_GROUP, WIDE_PART, BF16, RAG
+    # rag: any number of K blocks (the other loops need a multiple of four: their scale groups).  Three things differ.  The
+    # operand bases stop at the last K block (s93 / s94 = their low halves there), so the requests of a last trip of fewer than
+    # four blocks re-read that block instead of running past the matrices, and every counted wait stays as it is.  The last trip
+    # is left behind its last block (s97 = how many it has, 0: all four).  And a row of scales starts anywhere, so a group cannot
+    # be copied into LDS by one aligned request: the copying waves load it into registers (unaligned loads; a short last group
+    # element by element, nothing is read past the table) when the trip begins and write it to the same place in LDS two steps
+    # later.  Weight scales: fp32 by scalar loads of the group's length; e8m0 by a vector load of one address for all lanes.
+    # nn: the scale bytes of the stored weight lie a table row apart, four byte loads per group, whatever that row's length.
+    RAG = rag
+    assert not rag or (early and not wide and not brow and not bf16)
     # bf16: the operands are bf16 values (a K step of 128 bytes is 64 of them) and every matrix instruction of the
     # hardware-scaled loop becomes two v_mfma_f32_16x16x32_bf16 on the halves of the same fragment registers, accumulating
     # in place: a lane's first four registers hold values 16 lq .. 16 lq + 7 of its row and the other four 16 lq + 8 .. + 15,
@@ -179,7 +189,7 @@ def emit(s):
     if IDLE:
         # such a wave keeps its share of the copies, the barriers and the counters, and drops the arithmetic: fragment
         # and scale reads, matrix instructions, folds, scale products, and the waits that only order those
-        if s.startswith(("ds_read", "v_mfma", "v_fmac", "v_mul_f32", "v_mov_b32", "v_add_u32", "s_load_dword", "s_waitcnt lgkmcnt", "s_setprio")):
+        if s.startswith(("ds_read", "ds_write", "v_lshl_or", "v_mfma", "v_fmac", "v_mul_f32", "v_mov_b32", "v_add_u32", "s_load_dword", "s_waitcnt lgkmcnt", "s_setprio")):
             return
         s = s.replace("%=", "i%=")
     elif GRP == 1:
@@ -247,12 +257,18 @@ def dma(stage, part="all"):
         if HALFSPLIT and part != "all":
             emit(f"Lnoh{_uid}%=:")
         if part in ("all", "mid"):
-            emit("s_add_u32 s40, s40, 128")
+            if RAG:
+                emit("s_cmp_eq_u32 s40, s93")
+                emit("s_cselect_b32 s96, 0, 128")
+            emit(f"s_add_u32 s40, s40, {'s96' if RAG else 128}")
             emit("s_addc_u32 s41, s41, 0")
         if part in ("all", "end"):
             for i in range(ncopies if WIDE else 1):
                 lo = int(WB_EXTRA[i][2:4])
-                emit(f"s_add_u32 s{lo}, s{lo}, {'s66' if NN else 128}")      # nn: 128 rows of the stored weight further on
+                if RAG:
+                    emit("s_cmp_eq_u32 s42, s94")
+                    emit(f"s_cselect_b32 s96, 0, {'s66' if NN else 128}")
+                emit(f"s_add_u32 s{lo}, s{lo}, {'s96' if RAG else 's66' if NN else 128}")      # nn: 128 rows of the stored weight further on
                 emit(f"s_addc_u32 s{lo + 1}, s{lo + 1}, 0")
 
 
@@ -351,9 +367,121 @@ def wait_copies(c, at_end, extra=""):
         emit(f"Lwj{tag}%=:")
 
 
+RSA, RSB, RZERO = 104, 108, 112     # rag, e8m0: activation / weight scales of the next group on their way, a zero offset
+RSA_F32 = 36                        # rag, fp32: the lane's four activation scales of the next group
+
+
+def rag_short(label):
+    """Branch to `label` unless the group being loaded (the one after this trip's; the first one in the prologue) is the
+    last one and short: one trip is left and the number of K blocks is no multiple of four (s95 = the remainder)."""
+    emit("s_cmp_lg_u32 s49, 1")
+    emit(f"s_cbranch_scc1 {label}")
+    emit("s_cmp_eq_u32 s95, 0")
+    emit(f"s_cbranch_scc1 {label}")
+
+
+def rag_elements(dst, load, offset, base, size, join):
+    """Loads of a short group's one to three elements, one by one; ends behind the label `join`."""
+    for i in range(3):
+        if i:
+            emit(f"s_cmp_lt_u32 s95, {i + 1}")
+            emit(f"s_cbranch_scc1 {join}")
+        emit(f"{load} v{dst + i}, {offset}, {base} offset:{i * size}")
+
+
+def rag_scale_load(tag):
+    """Request the scales of the next group (see configure: rag)."""
+    emit("s_cmp_eq_u32 s53, 0")
+    emit(f"s_cbranch_scc1 Lra{tag}%=")
+    if HW:
+        for i in (1, 2):
+            emit(f"v_mov_b32 v{RSA + i}, 0")
+    rag_short(f"Lrf{tag}%=")
+    if HW:
+        rag_elements(RSA, "global_load_ubyte", "%[soff]", "s[44:45]", 1, f"Lra{tag}%=")
+    else:
+        rag_elements(RSA_F32, "global_load_dword", "%[soff]", "s[44:45]", 4, f"Lra{tag}%=")
+    emit(f"s_branch Lra{tag}%=")
+    emit(f"Lrf{tag}%=:")
+    if HW:
+        emit(f"global_load_dword v{RSA}, %[soff], s[44:45]")
+    else:
+        emit(f"global_load_dwordx4 {vr(RSA_F32, 4)}, %[soff], s[44:45]")
+    emit(f"Lra{tag}%=:")
+    emit(f"s_add_u32 s44, s44, {4 if HW else 16}")
+    emit("s_addc_u32 s45, s45, 0")
+    if HW:
+        for i in range(1, 4):
+            emit(f"v_mov_b32 v{RSB + i}, 0")
+    if NN:
+        # four bytes a table row (s64 bytes) apart; a short last group has s95 of them
+        for i in range(4):
+            if i:
+                emit(f"s_cmp_lg_u32 s49, 1")
+                emit(f"s_cbranch_scc1 Lrn{i}{tag}%=")
+                emit(f"s_cmp_eq_u32 s95, {i}")
+                emit(f"s_cbranch_scc1 Lrb{tag}%=")
+                emit(f"Lrn{i}{tag}%=:")
+            emit(f"global_load_ubyte v{RSB + i}, v{RZERO}, s[46:47]")
+            emit("s_add_u32 s46, s46, s64")
+            emit("s_addc_u32 s47, s47, 0")
+        emit(f"Lrb{tag}%=:")
+        return
+    rag_short(f"Lrg{tag}%=")
+    if HW:
+        rag_elements(RSB, "global_load_ubyte", f"v{RZERO}", "s[46:47]", 1, f"Lrb{tag}%=")
+    else:
+        emit("s_cmp_eq_u32 s95, 1")
+        emit(f"s_cbranch_scc0 Lrh{tag}%=")
+        emit("s_load_dword s60, s[46:47], 0x0")
+        emit(f"s_branch Lrb{tag}%=")
+        emit(f"Lrh{tag}%=:")
+        emit("s_load_dwordx2 s[60:61], s[46:47], 0x0")
+        emit("s_cmp_eq_u32 s95, 2")
+        emit(f"s_cbranch_scc1 Lrb{tag}%=")
+        emit("s_load_dword s62, s[46:47], 0x8")
+    emit(f"s_branch Lrb{tag}%=")
+    emit(f"Lrg{tag}%=:")
+    if HW:
+        emit(f"global_load_dword v{RSB}, v{RZERO}, s[46:47]")
+    else:
+        emit("s_load_dwordx4 s[60:63], s[46:47], 0x0")
+    emit(f"Lrb{tag}%=:")
+    emit(f"s_add_u32 s46, s46, {4 if HW else 16}")
+    emit("s_addc_u32 s47, s47, 0")
+
+
+def rag_scale_write(tag):
+    """The group requested by rag_scale_load has landed: put a short group's bytes together and write the activation scales
+    to LDS (half s54), where read_scales finds them."""
+    if HW:
+        if not NN:
+            rag_short(f"Lrc{tag}%=")
+        for base in (RSA, RSB) if not NN else (RSB,):
+            for i in range(1, 4 if NN else 3):
+                emit(f"v_lshl_or_b32 v{base}, v{base + i}, {8 * i}, v{base}")
+        if NN:
+            rag_short(f"Lrc{tag}%=")
+            for i in (1, 2):
+                emit(f"v_lshl_or_b32 v{RSA}, v{RSA + i}, {8 * i}, v{RSA}")
+        emit(f"Lrc{tag}%=:")
+    emit("s_cmp_eq_u32 s53, 0")
+    emit(f"s_cbranch_scc1 Lrw{tag}%=")
+    addr = RZERO + 1 if HW else P
+    emit(f"v_add_u32 v{addr}, s54, %[swr]")
+    if HW:
+        emit(f"ds_write_b32 v{addr}, v{RSA}")
+    else:
+        emit(f"ds_write_b128 v{addr}, {vr(RSA_F32, 4)}")
+    emit(f"Lrw{tag}%=:")
+
+
 def scale_group_copy(tag):
     """Copy the activation scales of the next group of four K steps into LDS (waves 0..3, one row per
     lane, 16 bytes each)."""
+    if RAG:
+        rag_scale_load(tag)
+        return
     emit("s_cmp_eq_u32 s53, 0")
     emit(f"s_cbranch_scc1 Lnosc{tag}%=")
     emit("s_add_u32 m0, s48, s54")
@@ -370,7 +498,7 @@ def scale_group_copy(tag):
 
 def weight_scale_load():
     """The four weight scales of the next group into s[60:63] (and those of the second scale row into s[68:71])."""
-    if BROW:
+    if BROW or RAG:
         return                                            # they travel with the activation scales, see scale_group_copy
     if NN:
         # one byte per K step, a table row (s64 bytes) apart: the aligned dword around each, taken apart at the top of the loop
@@ -499,6 +627,13 @@ def step(c):
         scale_group_copy("b")
         weight_scale_load()
         emit("Lnogrp%=:")
+    if RAG and c == 2:
+        # the next group's scales were requested when the trip began: in front of the copies of steps 0 and 1
+        emit("s_cmp_eq_u32 s50, 1")
+        emit("s_cbranch_scc1 Lnorw%=")
+        emit(f"s_waitcnt vmcnt({2 * sum(copies_per_part())})")
+        rag_scale_write("b")
+        emit("Lnorw%=:")
     if c == 3:
         # the next step belongs to the next group
         emit(f"s_xor_b32 s55, s55, {SCL_HALF}")
@@ -642,6 +777,8 @@ def loop_body():
         if BROW:
             for nb in range(NB):
                 emit(f"v_mov_b32 v{WSN + nb}, v{WSC + nb}")
+        elif RAG:
+            emit(f"v_mov_b32 {WS1}, v{RSB}")
         elif NN:
             # byte (address & 3) of each of the four dwords -> the four scale bytes of this group in one register
             for i in range(4):
@@ -665,8 +802,13 @@ def loop_body():
     emit("s_sub_u32 s49, s49, 1")
     emit("s_cmp_eq_u32 s49, 0")
     emit("s_cselect_b32 s50, 1, 0")
+    if RAG:
+        emit("s_cselect_b32 s97, s95, 0")
     for c in range(4):
         step(c)
+        if RAG and c < 3:
+            emit(f"s_cmp_eq_u32 s97, {c + 1}")
+            lines.append("s_cbranch_scc1 Ldone%=")             # one label for all bodies
     emit("s_cmp_lg_u32 s50, 1")
     emit("s_cbranch_scc1 Lloop%=")
 
@@ -702,6 +844,17 @@ def generate():
                 emit(f"s_mul_i32 s87, %[bstride], {WIDE_GROUP[i]}")
             emit(f"s_add_u32 s{lo}, s42, s87")
             emit(f"s_addc_u32 s{lo + 1}, s43, 0")
+    if RAG:
+        emit("s_add_u32 s93, s40, %[klast]")               # low half of the last K block's activation address
+        if NN:
+            emit("s_lshr_b32 s96, %[klast], 7")
+            emit("s_mul_i32 s96, s96, %[bstep]")
+            emit("s_add_u32 s94, s42, s96")
+        else:
+            emit("s_add_u32 s94, s42, %[klast]")
+        emit("s_mov_b32 s95, %[krem]")
+        if HW:
+            emit(f"v_mov_b32 v{RZERO}, 0")
     if HALFSPLIT:
         emit("s_bfe_u32 s87, %[flags], 0x10003")           # bit 3 of the wave flags: first half of the waves
     emit("s_mov_b32 s48, %[m0base]")
@@ -718,7 +871,8 @@ def generate():
         for b in range(NB):
             emit(f"v_mov_b32 {RBN[b]}, %[brdn{b}]")
         emit("s_mov_b32 s64, %[bsstride]")                 # bytes between two rows of the weight-scale table
-        emit("s_mov_b32 s65, %[bsbfe]")                    # s_bfe_u32 operand: 8 bits from bit 8 * (table address & 3)
+        if not RAG:
+            emit("s_mov_b32 s65, %[bsbfe]")                # s_bfe_u32 operand: 8 bits from bit 8 * (table address & 3)
         emit("s_mov_b32 s66, %[bstep]")                    # bytes between two K steps of the stored weight
     if BROW:
         emit("s_mov_b32 s51, %[sdst]")
@@ -742,6 +896,9 @@ def generate():
             emit("s_mov_b32 s89, 0")
             emit("s_mov_b32 s90, 0")
         emit(f"s_waitcnt vmcnt({(NSTAGE - 1) * sum(copies_per_part())}) lgkmcnt(0)")
+        if RAG:
+            rag_scale_write("a")                           # the oldest requests of all
+            emit("s_waitcnt lgkmcnt(0)")
         emit("s_barrier")
     else:
         dma(0)
@@ -786,7 +943,7 @@ def generate():
         IDLE = True
         loop_body()
         IDLE = False
-    if WITH_IDLE or PINGPONG:
+    if WITH_IDLE or PINGPONG or RAG:
         emit("Ldone%=:")
     if PINGPONG:
         emit("s_setprio 0")
@@ -817,7 +974,15 @@ def main():
                       ("gemm_mid_hwrow_loop.inc", (128, 128, 2, 2, 1, True, 2, True, True)),
                       ("gemm_big_hw_nn_loop.inc", (256, 256, 4, 2, 1, True, 2, False, True, False, True, PP, True)),
                       ("gemm_flat_hw_nn_loop.inc", (128, 256, 2, 4, 1, True, 3, False, True, False, True, False, True)),
-                      ("gemm_big_bf16_loop.inc", (256, 256, 4, 2, 1, True, 2, False, True, False, True, PP, False, True))):
+                      ("gemm_big_bf16_loop.inc", (256, 256, 4, 2, 1, True, 2, False, True, False, True, PP, False, True)),
+                      ("gemm_big_rag_loop.inc", (256, 256, 4, 2, 1, False, 2, False, True, False, True, PP, False, False, True)),
+                      ("gemm_big_hw_rag_loop.inc", (256, 256, 4, 2, 1, True, 2, False, True, False, True, PP, False, False, True)),
+                      ("gemm_mid_rag_loop.inc", (128, 128, 2, 2, 1, False, 2, False, True, False, False, False, False, False, True)),
+                      ("gemm_mid_hw_rag_loop.inc", (128, 128, 2, 2, 1, True, 2, False, True, False, False, False, False, False, True)),
+                      ("gemm_flat_rag_loop.inc", (128, 256, 2, 4, 1, False, 3, False, True, False, True, False, False, False, True)),
+                      ("gemm_flat_hw_rag_loop.inc", (128, 256, 2, 4, 1, True, 3, False, True, False, True, False, False, False, True)),
+                      ("gemm_big_hw_nn_rag_loop.inc", (256, 256, 4, 2, 1, True, 2, False, True, False, True, PP, True, False, True)),
+                      ("gemm_flat_hw_nn_rag_loop.inc", (128, 256, 2, 4, 1, True, 3, False, True, False, True, False, True, False, True))):
         configure(*cfg)
         generate()
         write(here, name)

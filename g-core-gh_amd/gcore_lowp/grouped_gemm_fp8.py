@@ -87,8 +87,8 @@ def grouped_gemm_fp8_nn(xq, xs, wq, ws, m_offsets: torch.Tensor, out: torch.Tens
     """out_e = x_e W_e on weights stored [E, K, N] (K = the contraction): the data gradient of the grouped linear on the
     layer's own [out, in] weights, general_grouped_gemm(..., layout="NN") at gpatch_v4/models/deepseek_v4/fp8.py:301-313.
     xq [M, K] e4m3fn with xs [M, K/128], wq [E, K, N] e4m3fn with ws [E, K/128, N/128], all scales e8m0.
-    The kernel turns the weight operand while it reads it out of LDS; shapes it does not take (N or K not a multiple of
-    512, more than 512 experts) go through a transposed copy of the weights and grouped_gemm_fp8."""
+    The kernel turns the weight operand while it reads it out of LDS; what it does not take (more than 512 experts, an
+    expert's weight or the activations of 4 GiB) goes through a transposed copy of the weights and grouped_gemm_fp8."""
     M, K = xq.shape
     E, K2, N = wq.shape
     assert K == K2 and K % 128 == 0 and N % 128 == 0

@@ -277,8 +277,8 @@ int lp_gemm_fp8_grouped(const void *Aq, const void *As, const void *Bq, const vo
  * contraction) and its 128 x 128 scales Ws [E,K/128,N/128], scales e8m0 on both operands.  This is the data gradient
  * of the grouped linear, dX_e = dY_e W_e on the layer's own [out, in] weight (K = out features, N = in features),
  * without a transposed copy of the weights: the matrix cores' operand is turned while it is read out of LDS.
- * Aq [M_total,K], As [M_total,K/128] (dY quantised 1 x 128 along K), C [M_total,N].  Needs N % 512 == 0, K % 512 == 0,
- * Ws 4-byte aligned, E <= 512; LP_ERR_UNSUPPORTED otherwise (transpose and call lp_gemm_fp8_grouped).
+ * Aq [M_total,K], As [M_total,K/128] (dY quantised 1 x 128 along K), C [M_total,N].  Needs E <= 512 and operands below
+ * 4 GiB; LP_ERR_UNSUPPORTED otherwise (transpose and call lp_gemm_fp8_grouped).
  * Replaces the dgrad of _MyTeGroupedLinear.backward, general_grouped_gemm(..., layout="NN")
  * (gpatch_v4/models/deepseek_v4/fp8.py:301-313).
  */
