@@ -126,13 +126,12 @@ __global__ __launch_bounds__(256) void quant_tile128(const void *__restrict__ xi
 // A 256-thread workgroup owns 16 groups per pass and PASSES passes.
 // CHECKED = false: every group of the workgroup exists (no bounds tests).
 template <bool IS_BF16, int MODE, int PASSES, bool CHECKED>
-__global__ __launch_bounds__(256) void quant_group128(const void *__restrict__ xin, int64_t group0, int64_t n_groups,
-                                                      uint8_t *__restrict__ q, void *__restrict__ scale_out,
-                                                      int scale_dtype, float amax_floor, int zero_rule,
-                                                      int32_t *nan_count)
+__device__ __forceinline__ void quant_groups(const void *__restrict__ xin, int64_t n_groups, uint8_t *__restrict__ q,
+                                             void *__restrict__ scale_out, int scale_dtype, float amax_floor, int zero_rule,
+                                             int32_t *nan_count)
 {
     const int t = threadIdx.x;
-    const int64_t g0 = group0 + (int64_t)blockIdx.x * (16 * PASSES) + (t >> 4);
+    const int64_t g0 = (int64_t)blockIdx.x * (16 * PASSES) + (t >> 4);
     const int lane16 = t & 15;
 
     u32x4 w[PASSES][IS_BF16 ? 1 : 2];
@@ -159,13 +158,14 @@ __global__ __launch_bounds__(256) void quant_group128(const void *__restrict__ x
         float v[8];
         uint32_t mbits = 0;
         if (IS_BF16) {
+            u16x2 m = {0, 0};                       // the two halves of a word compared at once (as in quant_tile128)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                uint32_t lo = w[p][0][j] << 16, hi = w[p][0][j] & 0xFFFF0000u;
-                v[2 * j] = u2f(lo); v[2 * j + 1] = u2f(hi);
-                uint32_t a = lo & 0x7FFFFFFFu, b = hi & 0x7FFFFFFFu;
-                mbits = a > mbits ? a : mbits; mbits = b > mbits ? b : mbits;
+                v[2 * j] = u2f(w[p][0][j] << 16);
+                v[2 * j + 1] = u2f(w[p][0][j] & 0xFFFF0000u);
+                m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, w[p][0][j] & 0x7FFF7FFFu));
             }
+            mbits = (uint32_t)(m.x > m.y ? m.x : m.y) << 16;
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
@@ -198,6 +198,20 @@ __global__ __launch_bounds__(256) void quant_group128(const void *__restrict__ x
             }
         }
     }
+}
+
+// Bound by HBM from about 10^5 groups on (65536 x 7168 bf16: 5.9 - 6.4 TB/s), below that by one trip to memory plus the
+// passes a workgroup makes one after the other.  One launch: only the workgroup that holds the ragged end tests bounds (that
+// end used to be a launch of its own, 3 - 4 us).
+template <bool IS_BF16, int MODE, int PASSES>
+__global__ __launch_bounds__(256) void quant_group128(const void *__restrict__ xin, int64_t n_groups, uint8_t *__restrict__ q,
+                                                      void *__restrict__ scale_out, int scale_dtype, float amax_floor,
+                                                      int zero_rule, int32_t *nan_count)
+{
+    if (((int64_t)blockIdx.x + 1) * (16 * PASSES) <= n_groups)
+        quant_groups<IS_BF16, MODE, PASSES, false>(xin, n_groups, q, scale_out, scale_dtype, amax_floor, zero_rule, nan_count);
+    else
+        quant_groups<IS_BF16, MODE, PASSES, true>(xin, n_groups, q, scale_out, scale_dtype, amax_floor, zero_rule, nan_count);
 }
 
 // ------------------------------------------------------------------ generic
@@ -261,27 +275,22 @@ int launch_mode(const void *x, bool is_bf16, int64_t rows, int64_t cols, int bm,
             hipLaunchKernelGGL((quant_tile128<false, MODE>), dim3((unsigned)tiles), dim3(256), 0, st, x, cols, tiles_c,
                                q, scale_out, scale_dtype, amax_floor, zero_rule, nan_count);
     } else if (bm == 1 && bn == 128 && aligned16) {
-        constexpr int PASSES = 4;
-        const int64_t groups = rows * (cols / 128), per_wg = 16 * PASSES;
-        const int64_t full = groups / per_wg, tail0 = full * per_wg;
-        if (full > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_quant_fp8_block: too many groups");
-        // full workgroups run without bounds tests; the ragged end is a one-workgroup launch
-        if (full > 0) {
-            if (is_bf16)
-                hipLaunchKernelGGL((quant_group128<true, MODE, PASSES, false>), dim3((unsigned)full), dim3(256), 0, st, x,
-                                   (int64_t)0, groups, q, scale_out, scale_dtype, amax_floor, zero_rule, nan_count);
-            else
-                hipLaunchKernelGGL((quant_group128<false, MODE, PASSES, false>), dim3((unsigned)full), dim3(256), 0, st, x,
-                                   (int64_t)0, groups, q, scale_out, scale_dtype, amax_floor, zero_rule, nan_count);
-        }
-        if (tail0 < groups) {
-            if (is_bf16)
-                hipLaunchKernelGGL((quant_group128<true, MODE, PASSES, true>), dim3(1), dim3(256), 0, st, x, tail0, groups, q,
-                                   scale_out, scale_dtype, amax_floor, zero_rule, nan_count);
-            else
-                hipLaunchKernelGGL((quant_group128<false, MODE, PASSES, true>), dim3(1), dim3(256), 0, st, x, tail0, groups, q,
-                                   scale_out, scale_dtype, amax_floor, zero_rule, nan_count);
-        }
+        // Passes per workgroup: one up to 2^17 groups, where a launch has few workgroups per CU and what counts is that all
+        // of it is on its way at once (us with one / four passes: 1 x 7168 2.1 / 3.4, 64 x 7168 2.5 / 3.7, 1000 x 2944 4.0 / 4.9,
+        // 2048 x 7168 10.6 / 11.3, the largest where one is level or ahead).  Beyond, enough loads in flight per wave: two passes
+        // with the cheap power-of-two arithmetic, four with the division (16384 x 4096: 34.6 with two against 36.9 and 39.5 with
+        // four and one; 4096 x 18432 divided: 41.6 with four against 44.2 and 46.2).
+        constexpr int MANY = div_like(MODE) ? 4 : 2;
+        const int64_t groups = rows * (cols / 128);
+        const bool few = groups <= (1 << 17);
+        const int64_t wgs = (groups + (few ? 16 : 16 * MANY) - 1) / (few ? 16 : 16 * MANY);
+        if (wgs > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_quant_fp8_block: too many groups");
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), 0, st, x, groups, q, scale_out, scale_dtype, amax_floor, zero_rule,
+                               nan_count);
+        };
+        if (is_bf16) few ? go(quant_group128<true, MODE, 1>) : go(quant_group128<true, MODE, MANY>);
+        else few ? go(quant_group128<false, MODE, 1>) : go(quant_group128<false, MODE, MANY>);
     } else {
         int64_t blocks_c = cols / bn, blocks = (rows / bm) * blocks_c;
         if (blocks > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_quant_fp8_block: too many blocks");
