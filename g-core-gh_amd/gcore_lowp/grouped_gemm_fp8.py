@@ -8,6 +8,9 @@
 """
 from __future__ import annotations
 
+from array import array
+from itertools import accumulate
+
 import torch
 
 from . import _abi as A
@@ -221,23 +224,32 @@ def gemm_fp8_rowscale_grouped(aq, a_s, bq, b_s, k_blocks, M, N, out: torch.Tenso
     E = len(k_blocks)
     assert out.is_contiguous() and tuple(out.shape) == (E, M, N) and out.dtype in (torch.bfloat16, torch.float32)
     launches, empty = rowscale_launches(k_blocks)
-    if empty:
-        out[torch.tensor(empty, device=out.device)] = 0
+    for e in empty:
+        out[e].zero_()
     odt = A.BF16 if out.dtype == torch.bfloat16 else A.F32
     with torch.cuda.device(out.device):
+        table = host_table([w for groups, _ in launches for g in groups for w in g], out.device)
+        first = table.data_ptr()
         for groups, multiple in launches:
-            table = torch.tensor(groups, dtype=torch.int32).to(out.device)
             A.check(A.lib().lp_gemm_fp8_rowscale_grouped(aq.data_ptr(), a_s.data_ptr(), bq.data_ptr(), b_s.data_ptr(), A.E8M0,
-                                                         table.data_ptr(), len(groups), max(g[1] for g in groups), multiple,
+                                                         first, len(groups), max(g[1] for g in groups), multiple,
                                                          M, N, out.data_ptr(), odt, A.stream_ptr()))
-            table.record_stream(torch.cuda.current_stream())
+            first += 16 * len(groups)
+    return out
+
+
+def host_table(words, dev) -> torch.Tensor:
+    """A list of host integers as an int32 tensor on `dev` (the current device), without a copy the stream and the host would
+    wait for (lp_host_table)."""
+    src = array("i", words)
+    out = torch.empty(len(src), dtype=torch.int32, device=dev)
+    A.check(A.lib().lp_host_table(src.buffer_info()[0], len(src), out.data_ptr(), A.stream_ptr()))
     return out
 
 
 def _offsets(m_splits, dev):
-    offs = torch.zeros(len(m_splits) + 1, dtype=torch.int32)
-    offs[1:] = torch.cumsum(torch.tensor(m_splits, dtype=torch.int64), 0).to(torch.int32)
-    return offs.to(dev)
+    with torch.cuda.device(dev):
+        return host_table(accumulate(m_splits, initial=0), dev)
 
 
 class _GroupedGemmFp8(torch.autograd.Function):

@@ -334,6 +334,14 @@ int lp_quant_fp8_colwise_t(const void *x, int x_dtype, int64_t rows, int64_t col
                            int E, int64_t padded_blocks, int pad_rows, void *qT, void *sT, int scale_dtype,
                            lp_stream_t stream);
 
+/*
+ * n int32 words of HOST memory at src -> device memory at dst, ordered on the stream like a kernel: the words are taken
+ * before the call returns (src may be reused at once) and neither the host nor the stream waits, as a copy from pageable
+ * memory would.  For the small tables the grouped entries read: row offsets, problem lists.  The reference hands the row
+ * counts over as a host list (fp8.py:193).
+ */
+int lp_host_table(const int32_t *src, int64_t n, int32_t *dst, lp_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
