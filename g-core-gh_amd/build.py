@@ -1,5 +1,6 @@
 """Builds the gfx950 C-ABI library in-tree: csrc/*.hip + api.cpp -> gcore_lowp/_lib/liblowp.so, and the
 measurement / self-test aids of include/lowp_probe.h as a second library: csrc/probe/*.hip -> liblowp_probe.so.
+csrc/host/native.cpp, host code against torch's headers, becomes the Python extension gcore_lowp/_lib/_lowp_native.so.
 
 Usage: python g-core-gh_amd/build.py [--force]
 hipcc cross-compiles without a GPU.  The library links against the HIP runtime
@@ -20,6 +21,7 @@ OBJ = os.path.join(HERE, "build")
 LIBDIR = os.path.join(HERE, "gcore_lowp", "_lib")
 LIB = os.path.join(LIBDIR, "liblowp.so")
 PROBE_LIB = os.path.join(LIBDIR, "liblowp_probe.so")
+NATIVE = os.path.join(LIBDIR, "_lowp_native.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 COMMON = [
@@ -109,13 +111,32 @@ def _audit_asm_operands():
         raise RuntimeError("gemm_fp8_big.hip: an asm operand shares a register with the loop it feeds; not linking")
 
 
+def _build_native(force: bool) -> None:
+    src = os.path.join(CSRC, "host", "native.cpp")
+    deps = [src, os.path.join(HERE, "..", "include", "lowp.h")]
+    if not force and os.path.exists(NATIVE) and os.path.getmtime(NATIVE) >= max(os.path.getmtime(d) for d in deps):
+        return
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-I" + sysconfig.get_paths()["include"], "-isystem", os.path.join(root, "include"),
+           "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"), "-isystem", "/opt/rocm/include", src, "-o", NATIVE,
+           "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for host/native.cpp:\n{r.stderr}")
+
+
 def build(force: bool = False) -> str:
     _generate()
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
     srcs, psrcs = sources(), probe_sources()
-    with ThreadPoolExecutor(max_workers=min(8, len(srcs) + len(psrcs))) as ex:
+    with ThreadPoolExecutor(max_workers=min(8, len(srcs) + len(psrcs) + 1)) as ex:
+        native = ex.submit(_build_native, force)
         all_objs = list(ex.map(lambda s: _compile(s, force), srcs + psrcs))
+        native.result()
     objs, pobjs = all_objs[:len(srcs)], all_objs[len(srcs):]
     if force or not os.path.exists(LIB) or any(os.path.getmtime(o) > os.path.getmtime(LIB) for o in objs):
         _audit_asm_operands()

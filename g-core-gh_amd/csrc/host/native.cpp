@@ -1,0 +1,215 @@
+// The calls a decode or conversion loop makes thousands of times, from Python's arguments to the C ABI in one step.
+//
+// Every function takes what its wrapper in gcore_lowp/ has in hand and answers None unless the call is the plain one: exact
+// torch tensors, contiguous, on the current GPU, of the types and shapes the kernels take as they are, and accepted by the C
+// ABI.  The wrapper then goes through its own checks, conversions and errors as if this file did not exist.  What it saves is
+// the interpreter's work per call (attribute look-ups, four or five tensor methods that do nothing, a device guard, ctypes
+// conversions).
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../../include/lowp.h"
+
+namespace {
+
+// addresses in the library that ctypes has loaded (bind)
+decltype(&lp_quant_fp8_block) p_quant_fp8;
+decltype(&lp_dequant_fp8_block) p_dequant_fp8;
+decltype(&lp_dequant_fp4_block) p_dequant_fp4;
+decltype(&lp_fp4_to_fp8_amax) p_fp4_amax;
+decltype(&lp_fp4_to_fp8_rebase) p_fp4_rebase;
+decltype(&lp_gemm_fp8_block) p_gemm;
+decltype(&lp_gemm_workspace_bytes) p_gemm_ws;
+
+PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    void *a[7];
+    if (n != 7) { PyErr_SetString(PyExc_TypeError, "bind: seven addresses"); return nullptr; }
+    for (int i = 0; i < 7; ++i) {
+        a[i] = PyLong_AsVoidPtr(args[i]);
+        if (!a[i]) { if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "bind: null address"); return nullptr; }
+    }
+    p_quant_fp8 = (decltype(p_quant_fp8))a[0];
+    p_dequant_fp8 = (decltype(p_dequant_fp8))a[1];
+    p_dequant_fp4 = (decltype(p_dequant_fp4))a[2];
+    p_fp4_amax = (decltype(p_fp4_amax))a[3];
+    p_fp4_rebase = (decltype(p_fp4_rebase))a[4];
+    p_gemm = (decltype(p_gemm))a[5];
+    p_gemm_ws = (decltype(p_gemm_ws))a[6];
+    Py_RETURN_NONE;
+}
+
+// A tensor the kernels can take as it is; nullptr otherwise.
+const at::Tensor *plain(PyObject *o)
+{
+    if (!THPVariable_CheckExact(o)) return nullptr;
+    const at::Tensor &t = THPVariable_Unpack(o);
+    if (!t.is_cuda() || !t.is_contiguous() || t.numel() == 0 || t.is_conj() || t.is_neg()) return nullptr;
+    return &t;
+}
+
+// All of them on the device that is current (the kernels are launched there).
+template <class... T>
+bool here(c10::DeviceIndex dev, const T *...t) { return dev == c10::hip::current_device() && ((t->get_device() == dev) && ...); }
+
+at::Tensor make(at::IntArrayRef sizes, at::ScalarType type, c10::DeviceIndex dev)
+{
+    return at::detail::empty_cuda(sizes, type, c10::Device(c10::kCUDA, dev), std::nullopt);
+}
+
+void *stream(c10::DeviceIndex dev) { return (void *)c10::hip::getCurrentHIPStream(dev).stream(); }
+
+int scale_code(at::ScalarType t)
+{
+    switch (t) {
+    case at::kFloat: return LP_F32;
+    case at::kBFloat16: return LP_BF16;
+    case at::kFloat8_e8m0fnu: return LP_E8M0;
+    default: return -1;
+    }
+}
+
+at::ScalarType scale_type(int code) { return code == LP_F32 ? at::kFloat : code == LP_BF16 ? at::kBFloat16 : at::kFloat8_e8m0fnu; }
+
+PyObject *pair(const at::Tensor &a, const at::Tensor &b)
+{
+    PyObject *x = THPVariable_Wrap(a), *y = x ? THPVariable_Wrap(b) : nullptr;
+    PyObject *r = y ? PyTuple_Pack(2, x, y) : nullptr;
+    Py_XDECREF(x);
+    Py_XDECREF(y);
+    return r;
+}
+
+bool ints(PyObject *const *args, int n, long *out)
+{
+    for (int i = 0; i < n; ++i) {
+        out[i] = PyLong_AsLong(args[i]);
+        if (out[i] == -1 && PyErr_Occurred()) { PyErr_Clear(); return false; }
+    }
+    return true;
+}
+
+#define GUARDED(...)                                                                                                              \
+    try {                                                                                                                         \
+        __VA_ARGS__                                                                                                               \
+    } catch (const std::exception &e) {                                                                                           \
+        PyErr_SetString(PyExc_RuntimeError, e.what());                                                                            \
+        return nullptr;                                                                                                           \
+    }
+
+// (x, bm, bn, scale_mode, scale code, zero_rule, amax_floor) -> (codes, scales)
+PyObject *quant_fp8(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    long v[5];
+    if (n != 7 || !ints(args + 1, 5, v)) Py_RETURN_NONE;
+    const double floor = PyFloat_AsDouble(args[6]);
+    if (PyErr_Occurred()) { PyErr_Clear(); Py_RETURN_NONE; }
+    GUARDED(
+        const at::Tensor *x = plain(args[0]);
+        if (!x) Py_RETURN_NONE;
+        const c10::DeviceIndex dev = x->get_device();
+        if (!here(dev, x) || x->dim() < 2 || (x->scalar_type() != at::kBFloat16 && x->scalar_type() != at::kFloat)) Py_RETURN_NONE;
+        const int64_t rows = x->size(-2), cols = x->size(-1), bm = v[0], bn = v[1];
+        if (bm <= 0 || bn <= 0 || rows % bm || cols % bn || v[3] < 0 || v[3] > LP_E8M0) Py_RETURN_NONE;
+        at::DimVector grid(x->sizes().begin(), x->sizes().end());
+        grid[grid.size() - 2] = rows / bm;
+        grid[grid.size() - 1] = cols / bn;
+        at::Tensor q = make(x->sizes(), at::kFloat8_e4m3fn, dev), s = make(grid, scale_type((int)v[3]), dev);
+        if (p_quant_fp8(x->const_data_ptr(), x->scalar_type() == at::kFloat ? LP_F32 : LP_BF16, x->numel() / cols, cols, (int)bm, (int)bn,
+                        (int)v[2], (float)floor, (int)v[4], q.data_ptr(), s.data_ptr(), (int)v[3], nullptr, stream(dev)))
+            Py_RETURN_NONE;
+        return pair(q, s);
+    )
+}
+
+// (codes, scales, fp4, FP4 zero rule, out code) -> values; the block is the ratio of the two shapes
+PyObject *dequant(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    long v[3];
+    if (n != 5 || !ints(args + 2, 3, v)) Py_RETURN_NONE;
+    GUARDED(
+        const at::Tensor *c = plain(args[0]), *s = plain(args[1]);
+        if (!c || !s) Py_RETURN_NONE;
+        const c10::DeviceIndex dev = c->get_device();
+        if (!here(dev, c, s) || c->dim() < 2 || s->dim() != c->dim() || c->element_size() != 1) Py_RETURN_NONE;
+        const int sc = scale_code(s->scalar_type());
+        const int64_t rows = c->size(-2), cols = c->size(-1) * (v[0] ? 2 : 1), sr = s->size(-2), scol = s->size(-1);
+        if (sc < 0 || rows % sr || cols % scol || (v[2] != LP_F32 && v[2] != LP_BF16)) Py_RETURN_NONE;
+        for (int64_t d = 0; d + 2 < c->dim(); ++d)
+            if (c->size(d) != s->size(d)) Py_RETURN_NONE;
+        at::DimVector shape(c->sizes().begin(), c->sizes().end());
+        shape[shape.size() - 1] = cols;
+        at::Tensor out = make(shape, v[2] == LP_F32 ? at::kFloat : at::kBFloat16, dev);
+        const int64_t all_rows = c->numel() / c->size(-1);
+        const int bm = (int)(rows / sr), bn = (int)(cols / scol);
+        const int rc = v[0] ? p_dequant_fp4(c->const_data_ptr(), s->const_data_ptr(), sc, all_rows, cols, bm, bn, (int)v[1], out.data_ptr(), (int)v[2], stream(dev))
+                            : p_dequant_fp8(c->const_data_ptr(), s->const_data_ptr(), sc, all_rows, cols, bm, bn, out.data_ptr(), (int)v[2], stream(dev));
+        if (rc) Py_RETURN_NONE;
+        return THPVariable_Wrap(out);
+    )
+}
+
+// (packed, e8m0 scales, kind, scale_mode, zero_rule, scale code of the result, amax_floor) -> (codes, scales); kind 0: re-based,
+// kind 1: requantised by amax
+PyObject *fp4_to_fp8(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    long v[4];
+    if (n != 7 || !ints(args + 2, 4, v)) Py_RETURN_NONE;
+    const double floor = PyFloat_AsDouble(args[6]);
+    if (PyErr_Occurred()) { PyErr_Clear(); Py_RETURN_NONE; }
+    GUARDED(
+        const at::Tensor *x = plain(args[0]), *s = plain(args[1]);
+        if (!x || !s) Py_RETURN_NONE;
+        const c10::DeviceIndex dev = x->get_device();
+        if (!here(dev, x, s) || x->dim() != 2 || s->dim() != 2 || x->scalar_type() != at::kChar || s->scalar_type() != at::kFloat8_e8m0fnu)
+            Py_RETURN_NONE;
+        const int64_t rows = x->size(0), cols = x->size(1) * 2;
+        if (rows % 128 || cols % 128 || s->size(0) != rows || s->size(1) != cols / 32 || v[3] < 0 || v[3] > LP_E8M0) Py_RETURN_NONE;
+        at::Tensor q = make({rows, cols}, at::kFloat8_e4m3fn, dev), so = make({rows / 128, cols / 128}, scale_type((int)v[3]), dev);
+        const int rc = v[0] ? p_fp4_amax(x->const_data_ptr(), s->const_data_ptr(), rows, cols, (int)v[1], (float)floor, (int)v[2], q.data_ptr(),
+                                         so.data_ptr(), (int)v[3], nullptr, stream(dev))
+                            : p_fp4_rebase(x->const_data_ptr(), s->const_data_ptr(), rows, cols, q.data_ptr(), so.data_ptr(), (int)v[3], stream(dev));
+        if (rc) Py_RETURN_NONE;
+        return pair(q, so);
+    )
+}
+
+// (Aq, As, Bq, Bs, out code) -> C
+PyObject *gemm(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    long out_code;
+    if (n != 5 || !ints(args + 4, 1, &out_code)) Py_RETURN_NONE;
+    GUARDED(
+        const at::Tensor *a = plain(args[0]), *sa = plain(args[1]), *b = plain(args[2]), *sb = plain(args[3]);
+        if (!a || !sa || !b || !sb) Py_RETURN_NONE;
+        const c10::DeviceIndex dev = a->get_device();
+        if (!here(dev, a, sa, b, sb) || a->dim() != 2 || sa->dim() != 2 || b->dim() != 2 || sb->dim() != 2) Py_RETURN_NONE;
+        if (a->scalar_type() != at::kFloat8_e4m3fn || b->scalar_type() != at::kFloat8_e4m3fn || sa->scalar_type() != sb->scalar_type() ||
+            (sa->scalar_type() != at::kFloat && sa->scalar_type() != at::kFloat8_e8m0fnu) || (out_code != LP_BF16 && out_code != LP_F32))
+            Py_RETURN_NONE;
+        const int64_t M = a->size(0), K = a->size(1), N = b->size(0);
+        if (b->size(1) != K || K % 128 || N % 128 || sa->size(0) != M || sa->size(1) != K / 128 || sb->size(0) != N / 128 || sb->size(1) != K / 128)
+            Py_RETURN_NONE;
+        at::Tensor c = make({M, N}, out_code == LP_BF16 ? at::kBFloat16 : at::kFloat, dev), ws;
+        const int64_t need = p_gemm_ws(M, N, K);
+        if (need > 0) ws = make({need}, at::kByte, dev);
+        if (p_gemm(a->const_data_ptr(), sa->const_data_ptr(), b->const_data_ptr(), sb->const_data_ptr(), scale_code(sa->scalar_type()), M, N, K,
+                   c.data_ptr(), (int)out_code, need > 0 ? ws.data_ptr() : nullptr, need, stream(dev)))
+            Py_RETURN_NONE;
+        return THPVariable_Wrap(c);
+    )
+}
+
+#define ENTRY(f) {#f, (PyCFunction)(void (*)(void))f, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {ENTRY(bind), ENTRY(quant_fp8), ENTRY(dequant), ENTRY(fp4_to_fp8), ENTRY(gemm), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_lowp_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+extern "C" __attribute__((visibility("default"))) PyObject *PyInit__lowp_native() { return PyModule_Create(&module); }

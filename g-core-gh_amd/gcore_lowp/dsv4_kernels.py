@@ -4,9 +4,11 @@ from __future__ import annotations
 
 import torch
 
+from . import _abi as A
 from . import ops
 import re
 
+from ._native import fast
 from .eager_quant_kernels import (dequant_fp4_e2m1_fp8_scale_e8m0_packed, quant_fp4_e2m1_scale_e8m0_packed,
                                   quant_fp8_e4m3_scale_e8m0)
 
@@ -42,6 +44,9 @@ def dequant_fp8_block(weight: torch.Tensor, scale: torch.Tensor) -> torch.Tensor
 
 def cast_e2m1fn_to_e4m3fn(x: torch.Tensor, scale: torch.Tensor):
     """kernels.py:91-126: lossless FP4 -> e4m3fn, 128 x 128 e8m0 outer scale = max(e8m0)/64."""
+    r = fast.fp4_to_fp8(x, scale, 0, 0, 0, A.E8M0, 0.0)
+    if r is not None:
+        return r
     assert x.dtype == torch.int8
     assert x.ndim == 2
     out_dim, in_dim = x.size()
@@ -54,6 +59,9 @@ def cast_e2m1fn_to_e4m3fn(x: torch.Tensor, scale: torch.Tensor):
 
 def official_expert_to_sgl(weight: torch.Tensor, scale: torch.Tensor):
     """kernels.py:129-133: as above with the outer scale widened to fp32."""
+    r = fast.fp4_to_fp8(weight, scale, 0, 0, 0, A.F32, 0.0)
+    if r is not None:
+        return r
     assert weight.dtype == torch.int8
     assert weight.ndim == 2
     out_dim, in_dim = weight.size()
@@ -97,6 +105,10 @@ def sgl_expert_to_official(weight: torch.Tensor, scale: torch.Tensor):
 def fp4_to_fp8_blockwise(x: torch.Tensor, scale: torch.Tensor, *, return_bf16: bool = False):
     """FP4 (1 x 32 e8m0) -> bf16 -> e4m3fn with a 128 x 128 fp32 scale = max(amax, 1e-12)/448, fused:
     byte-identical to cast_e2m1fn_to_bf16 followed by the divide-form 128 x 128 quantiser."""
+    if not return_bf16:
+        r = fast.fp4_to_fp8(x, scale, 1, A.SCALE_DIV, A.ZERO_NONE, A.F32, 1e-12)
+        if r is not None:
+            return r
     assert x.dtype == torch.int8 and x.ndim == 2
     out_dim, in_dim = x.size()
     in_dim *= 2

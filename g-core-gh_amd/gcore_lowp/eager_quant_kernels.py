@@ -9,6 +9,7 @@ import torch
 
 from . import _abi as A
 from . import ops
+from ._native import fast
 
 __all__ = ["quant_fp4_e2m1_scale_e8m0_packed", "quant_fp8_e4m3_scale_e8m0", "dequant_fp4_e2m1_fp8_scale_e8m0_packed"]
 
@@ -48,6 +49,10 @@ def dequant_fp4_e2m1_fp8_scale_e8m0_packed(quantized: torch.Tensor, scales: torc
     float4_e2m1fn_x2 inputs are packed FP4 (code 8 = -0.0), anything else is
     read as e4m3fn; result dtype = scales.dtype if it is a float of >= 2 bytes,
     else bf16."""
+    if quantized.dtype == ops.E4M3 or quantized.dtype == torch.int8:
+        out = fast.dequant(quantized, scales, quantized.dtype == torch.int8, A.FP4_NEG_ZERO, A.F32 if scales.dtype == torch.float32 else A.BF16)
+        if out is not None:
+            return out
     fp4x2 = getattr(torch, "float4_e2m1fn_x2", None)
     is_fp4 = quantized.dtype == torch.int8 or (fp4x2 is not None and quantized.dtype == fp4x2)
     out_dtype = scales.dtype if scales.dtype.is_floating_point and scales.element_size() >= 2 else torch.bfloat16

@@ -13,6 +13,7 @@ import torch
 
 from . import _abi as A
 from . import ops
+from ._native import fast
 
 __all__ = ["quantize_fp8_blockwise", "quant_1d", "quant_2d", "quant_act", "quant_weight"]
 
@@ -56,7 +57,8 @@ def _div_quant(x, block, *, round_sf, amax_floor, zero_rule):
 def quant_1d(x: torch.Tensor, block_size: int = 128, *, round_sf: bool = False):
     """Row-wise 1 x block_size activation quant, s = max(amax, 1e-12)/448 (round_sf: rounded up to a power of two).
     Returns (e4m3fn [M, K], fp32 scale [M, K/block_size])."""
-    return _div_quant(x, (1, block_size), round_sf=round_sf, amax_floor=1e-12, zero_rule=A.ZERO_NONE)
+    r = fast.quant_fp8(x, 1, block_size, A.SCALE_POW2 if round_sf else A.SCALE_DIV, A.F32, A.ZERO_NONE, 1e-12)
+    return r if r is not None else _div_quant(x, (1, block_size), round_sf=round_sf, amax_floor=1e-12, zero_rule=A.ZERO_NONE)
 
 
 def quant_2d(w: torch.Tensor, block_size: tuple[int, int] = (128, 128), *, round_sf: bool = False):

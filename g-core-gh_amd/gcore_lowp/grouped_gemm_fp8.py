@@ -15,6 +15,7 @@ import torch
 
 from . import _abi as A
 from . import ops
+from ._native import fast
 
 __all__ = ["grouped_gemm_fp8", "grouped_gemm_fp8_nn", "m_grouped_gemm_fp8_fp8_bf16_nt_contiguous", "MyTeGroupedLinearFp8",
            "quant_fp8_colwise_t", "gemm_fp8_rowscale"]
@@ -26,6 +27,9 @@ def _quant_pow2(value: torch.Tensor, block_size):
     and so stalls the stream once per call: inside the grouped linear (three quantisations per step and layer) a NaN
     simply propagates into the product, as it does in the reference, whose layer quantises inside TransformerEngine
     (fp8.py:180-343) without such a check."""
+    r = fast.quant_fp8(value, *block_size, A.SCALE_POW2, A.E8M0, A.ZERO_NONE, 0.0)
+    if r is not None:
+        return r
     q, s, _ = ops.quant_fp8_block(value, block_size, scale_mode=A.SCALE_POW2, scale_dtype=ops.E8M0, count_nan=False)
     return q, s
 
