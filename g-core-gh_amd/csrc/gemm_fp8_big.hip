@@ -1176,10 +1176,7 @@ __global__ __launch_bounds__(TM * 2) void gemm_asm_grouped(const uint8_t *__rest
 // bytes it pulls through the L2 -> LDS copies, and an expert with few rows is a stream of its weights: the flat tile
 // moves 48 KB per K step and 256 weight rows where two 128 x 128 tiles move 64 KB.
 // The tile list is built on the device from m_offsets (at most 512 experts): one scan gives every thread the two class
-// totals and the running tile counts of its expert, from which the workgroup finds its class, its tile and the expert
-// that owns it.  Within every XCD's sequence of workgroup ids the two classes are dealt in the ratio of their sizes
-// (1 big : ps small), and each class keeps the 8(M) x 4(N) blocks of neighbouring tiles per XCD that let operand panels
-// be re-used out of one L2.
+// totals and the running tile counts of its expert, from which a workgroup finds its tiles and the experts that own them.
 constexpr int kMixedMaxExperts = 512;
 
 // NN: expert e's weight is stored [K, N] (the layer's own [out, in] weight read for the data gradient dX = dY W: K = out
@@ -1188,7 +1185,7 @@ template <bool HWS, bool NN = false, bool RAG = false>
 __global__ __launch_bounds__(512) void gemm_asm_grouped_mixed(const uint8_t *__restrict__ Aq, const float *__restrict__ As,
                                                               const uint8_t *__restrict__ Bq, const float *__restrict__ Bs,
                                                               const int32_t *__restrict__ m_offsets, int E, int64_t M_total,
-                                                              int64_t N, int64_t K, void *__restrict__ C, int out_dtype, int small_first)
+                                                              int64_t N, int64_t K, void *__restrict__ C, int out_dtype)
 {
     constexpr int LDS_BIG = AsmTile<256, 256, 1>::LDS_BYTES, LDS_FLAT = AsmTile<128, 256, 1, 3, 4>::LDS_BYTES;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[LDS_BIG > LDS_FLAT ? LDS_BIG : LDS_FLAT];
@@ -1225,59 +1222,52 @@ __global__ __launch_bounds__(512) void gemm_asm_grouped_mixed(const uint8_t *__r
     }
     tot_big = __builtin_amdgcn_readfirstlane(tot_big);
     tot_small = __builtin_amdgcn_readfirstlane(tot_small);
-    // ---- which class and which tile of it this workgroup takes (32-bit arithmetic: the grid is below 2^31, and 64-bit
-    // divisions by run-time values would cost this prologue about a microsecond per workgroup)
+    // ---- this workgroup's tiles (32-bit arithmetic: the host keeps the tile count below 2^31)
+    // Tiles of a class are numbered expert by expert (expert e owns tiles_n numbers per row tile).  Each XCD takes an eighth of
+    // both classes, one run of numbers each, so the tiles it runs together belong to one expert or to neighbours.  Inside the
+    // XCD its P workgroups, one per CU, share both runs in advance as a longest-first list scheduler would: first the big
+    // tiles in rounds -- r workgroups end up with one more than the others -- then every small tile goes to the workgroup with
+    // the least work so far, a big tile counting as one and a half small ones (measured, K = 7168 / 2048: 115 / 35 us against
+    // 72 / 22).  In rounds that gives the P - r workgroups without the extra big tile two small ones each before the r others
+    // get their first, and from there on everybody one per round: small tile j of the XCD has a closed form.
+    // Dealing both classes in rounds of 32 padded to whole blocks per XCD, as before, left XCDs and CUs with twice the work of
+    // others when a class has few tiles per CU (32 experts, 4096 rows, N = 4096, K = 2048: 77 us before).
     const uint32_t tiles_n = (uint32_t)((N + 255) >> 8);                   // the last column tile may be half empty
-    auto padded_slots = [](uint32_t tiles) -> uint32_t {                   // workgroups per XCD for that many tiles
-        const uint32_t chunks = (tiles + gemm::CHUNK - 1) / gemm::CHUNK;
-        return ((chunks + 7) / 8) * gemm::CHUNK;
-    };
-    const uint32_t slots_big = padded_slots((uint32_t)tot_big * tiles_n), slots_small = padded_slots((uint32_t)tot_small * tiles_n);
-    // A workgroup takes slots blockIdx.x, blockIdx.x + gridDim.x, ...: with one workgroup per CU (grid = number of CUs, a
-    // multiple of 8, so a workgroup stays on its XCD's share of the slots) the scan above is paid once per CU instead of
-    // once per tile; with a grid of all slots the loop below runs once.  The workgroup's tiles are looked up kTable slots at a
-    // time, one slot per thread, and listed in LDS: between two tiles only a table entry is read (a workgroup has its CU to
-    // itself, so whatever happens between two K loops is time the matrix cores stand still).
+    const uint32_t P = gridDim.x >> 3, xcd = blockIdx.x & 7, wg = blockIdx.x >> 3;
+    const uint32_t all_big = (uint32_t)tot_big * tiles_n, all_small = (uint32_t)tot_small * tiles_n;
+    // the first all_big % 8 XCDs have one big tile more, the last all_small % 8 one small tile more
+    const uint32_t eb = all_big & 7, es = all_small & 7;
+    const uint32_t first_big = xcd * (all_big >> 3) + (xcd < eb ? xcd : eb), n_big = (all_big >> 3) + (xcd < eb ? 1 : 0);
+    const uint32_t first_small = xcd * (all_small >> 3) + (xcd > 8 - es ? xcd - (8 - es) : 0), n_small = (all_small >> 3) + (xcd >= 8 - es ? 1 : 0);
+    const uint32_t rounds = n_big / P, r = n_big - rounds * P;
+    const bool extra = wg < r;
+    const uint32_t mine_big = rounds + (extra ? 1 : 0);
+    // number of this workgroup's k-th small tile: k P + shift, except for k = 0 without the extra big tile
+    const int32_t shift = extra ? (int32_t)(2 * (P - r) + wg) : (int32_t)wg - 2 * (int32_t)r;
+    const int32_t zeroth = extra ? shift : (int32_t)(wg - r);
+    uint32_t mine_small = 0;
+    if (zeroth < (int32_t)n_small) {
+        const int32_t rest = (int32_t)n_small - shift;                     // tiles k with k P < rest
+        mine_small = 1 + (rest > (int32_t)P ? (uint32_t)(rest - 1) / P : 0);
+    }
+    const uint32_t mine = mine_big + mine_small;
+    // Half of the XCDs take their small tiles first, the others last: at any time some stream weights while others compute,
+    // each class with an L2 to itself.
+    const uint32_t lead = xcd < 4 ? mine_small : mine_big;
+    // The tiles are looked up kTable at a time, one per thread, and listed in LDS: between two tiles only a table entry is read
+    // (a workgroup has its CU to itself, so whatever happens between two K loops is time the matrix cores stand still).
     __syncthreads();                                    // the running counts are written
-    const uint32_t slots = slots_big + slots_small;
-    const uint64_t all_slots = (uint64_t)slots * 8;     // below 2^31
     const int64_t kblocks = K / KB;
-    for (uint64_t first = blockIdx.x; first < all_slots; first += (uint64_t)kTable * gridDim.x) {
+    for (uint32_t first = 0; first < mine; first += kTable) {
         __syncthreads();                                // every thread has read the previous batch's last entry
         if (t < kTable) {
-            const uint64_t slot64 = first + (uint64_t)t * gridDim.x;
+            const uint32_t at = first + (uint32_t)t;
             int4 entry = {-1, 0, 0, 0};                 // expert (-1: no tile; bit 30: 256-row tile), first row, end of the expert's rows, first column
-            if (slot64 < all_slots) {
-                const uint32_t slot = (uint32_t)slot64;
-                const uint32_t xcd = slot & 7, sidx = slot >> 3;
-                bool big;
-                uint32_t idx;
-                if (small_first > 0) {
-                    // XCDs below small_first work through their small tiles first and then their big ones, the others the
-                    // other way round: every XCD has the same share of both classes, and at any time some XCDs stream weights
-                    // while the others compute, each class with an L2 to itself
-                    if (xcd < (uint32_t)small_first) { big = sidx >= slots_small; idx = big ? sidx - slots_small : sidx; }
-                    else { big = sidx < slots_big; idx = big ? sidx : sidx - slots_big; }
-                } else {
-                    // the classes dealt alternately in the ratio of their sizes (1 big : ps small)
-                    uint32_t ps = slots_big > 0 ? (slots_small + slots_big / 2) / slots_big : 1;
-                    if (ps < 1) ps = 1;
-                    const uint32_t period = 1 + ps;
-                    const uint32_t rounds = slots_big < slots_small / ps ? slots_big : slots_small / ps;      // periods in which both classes have tiles
-                    if (sidx < rounds * period) {
-                        const uint32_t q = sidx / period, rr = sidx - q * period;
-                        big = rr == 0;
-                        idx = big ? q : q * ps + (rr - 1);
-                    } else {
-                        const uint32_t w = sidx - rounds * period, left_big = slots_big - rounds;
-                        big = w < left_big;
-                        idx = big ? rounds + w : rounds * ps + (w - left_big);
-                    }
-                }
-                // Tiles of a class are numbered expert by expert (expert e owns tiles_n numbers per row tile) and an XCD takes
-                // 32 consecutive numbers at a time, so the tiles it runs together belong to one expert, or to neighbours.
-                const uint32_t lin = ((idx / gemm::CHUNK) * 8 + xcd) * gemm::CHUNK + idx % gemm::CHUNK;
-                if (lin < (uint32_t)(big ? tot_big : tot_small) * tiles_n) {
+            if (at < mine) {
+                const bool big = (xcd < 4) == (at >= lead);
+                const uint32_t k = at < lead ? at : at - lead;
+                const uint32_t lin = big ? first_big + k * P + wg : first_small + (k == 0 ? (uint32_t)zeroth : (uint32_t)((int32_t)(k * P) + shift));
+                if (lin < (big ? all_big : all_small)) {
                     const int gmt = (int)(lin / tiles_n);
                     // the expert that owns row tile gmt of the class: the first whose running count exceeds gmt
                     const int *upto = big ? upto_big : upto_small;
@@ -1311,7 +1301,7 @@ __global__ __launch_bounds__(512) void gemm_asm_grouped_mixed(const uint8_t *__r
         }
         __syncthreads();
         for (int i = 0; i < kTable; ++i) {
-            if (first + (uint64_t)i * gridDim.x >= all_slots) break;
+            if (first + (uint32_t)i >= mine) break;
             const int4 entry = table[i];
             const int ex = __builtin_amdgcn_readfirstlane(entry.x);
             if (ex < 0) continue;
@@ -1658,6 +1648,17 @@ static int compute_units()
     return cached[dev] > 0 ? cached[dev] : 0;
 }
 
+// Workgroups of a launch with two tile heights: one per CU (it owns its CU: the tiles' LDS) that walks its tiles, or one per
+// tile when there are fewer tiles than that or the CUs are not known.  An expert has M_e / 256 row tiles plus one when rows are
+// left over, big or small: M_total / 256 + E over both classes.  A multiple of 8 (the XCDs); 0: too many tiles for the
+// kernel's arithmetic.
+static int64_t mixed_grid(int64_t M_total, int E, int64_t tiles_n, int cus)
+{
+    const int64_t tiles = (M_total / 256 + E) * tiles_n, grid = (tiles + 7) / 8 * 8;
+    if (tiles > 0x3FFFFFFF) return 0;
+    return cus >= 8 && grid > cus ? cus / 8 * 8 : grid;
+}
+
 // The data gradient of the grouped linear on the stored weights (no transposed copy): e8m0 scales, at most
 // kMixedMaxExperts experts.
 bool grouped_nn_ok(const void *As, const void *Bs, int scale_dtype, int E, int64_t M_total, int64_t N, int64_t K)
@@ -1668,15 +1669,13 @@ bool grouped_nn_ok(const void *As, const void *Bs, int scale_dtype, int E, int64
 int launch_grouped_nn(const void *Aq, const void *As, const void *Bq, const void *Bs, const int32_t *m_offsets, int E,
                       int64_t M_total, int64_t N, int64_t K, void *C, int out_dtype, hipStream_t st)
 {
-    int64_t grid = padded_grid(M_total / 256 + E, (N + 255) / 256) + 2 * 8 * CHUNK;
-    if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_grouped_nn: problem too large");
-    const int cus = compute_units();
-    if (cus >= 8 && grid > cus) grid = cus / 8 * 8;            // one workgroup per CU walks the tile slots, as in the forward launch
+    const int64_t grid = mixed_grid(M_total, E, (N + 255) / 256, compute_units());
+    if (grid <= 0) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_grouped_nn: problem too large");
     // the loop without RAG takes the dword around a scale byte: rows of the weight's scale table a multiple of 4 bytes apart
     const bool rag = !asm_shape_ok(As, Bs, M_total, N, K, LP_E8M0) || N % 512;
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(512), 0, st, (const uint8_t *)Aq, (const float *)As, (const uint8_t *)Bq,
-                           (const float *)Bs, m_offsets, E, M_total, N, K, C, out_dtype, 4);
+                           (const float *)Bs, m_offsets, E, M_total, N, K, C, out_dtype);
     };
     rag ? go(gemm_asm_grouped_mixed<true, true, true>) : go(gemm_asm_grouped_mixed<true, true, false>);
     return check_launch("lp_gemm_fp8_grouped_nn");
@@ -1703,23 +1702,16 @@ int launch_big_grouped(const void *Aq, const void *As, const void *Bq, const voi
     const bool enough_tiles = (M_total / 256 + E / 2) * tiles_n >= 256;
     const bool rag = !asm_shape_ok(As, Bs, M_total, N, K, scale_dtype);
     if (mode == 2 || (mode < 0 && E <= kMixedMaxExperts && enough_tiles)) {
-        // an expert with r rows has r / 256 tiles plus one when rows are left over, big or small: M_total / 256 + E row
-        // tiles at most over both classes, each class rounded up to whole groups of 8 x 32 workgroups
-        int64_t grid = padded_grid(M_total / 256 + E, tiles_n) + 2 * 8 * CHUNK;
-        if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_grouped: problem too large");
         if (E <= kMixedMaxExperts) {
-            // one workgroup per CU that works through every grid-th slot (a workgroup owns its CU: the tiles' LDS)
-            // (LP_GEMM_GROUPED_PERSIST, read at every call so that a test can change it: 0 = one workgroup per slot, n >= 8 =
-            // that many workgroups, e.g. few enough that each walks more slots than one table holds)
+            // LP_GEMM_GROUPED_PERSIST, read at every call so that a test can change it: 0 = one workgroup per tile, n >= 8 = that
+            // many workgroups, e.g. few enough that each walks more tiles than one table holds
             const char *persist_env = getenv("LP_GEMM_GROUPED_PERSIST");
             const int forced = persist_env ? atoi(persist_env) : -1;
-            const int cus = forced == 0 ? 0 : (forced >= 8 ? forced : compute_units());
-            if (cus >= 8 && grid > cus) grid = cus / 8 * 8;
-            static const char *order_env = getenv("LP_GEMM_GROUPED_ORDER");     // tuning aid: XCDs that take their small tiles first (0: classes dealt alternately)
-            const int small_first = order_env ? atoi(order_env) : 4;
+            const int64_t grid = mixed_grid(M_total, E, tiles_n, forced == 0 ? 0 : (forced >= 8 ? forced : compute_units()));
+            if (grid <= 0) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_grouped: problem too large");
             auto go = [&](auto kernel) {
                 hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(512), 0, st, (const uint8_t *)Aq, (const float *)As, (const uint8_t *)Bq,
-                                   (const float *)Bs, m_offsets, E, M_total, N, K, C, out_dtype, small_first);
+                                   (const float *)Bs, m_offsets, E, M_total, N, K, C, out_dtype);
             };
             if (scale_dtype == LP_E8M0) rag ? go(gemm_asm_grouped_mixed<true, false, true>) : go(gemm_asm_grouped_mixed<true>);
             else rag ? go(gemm_asm_grouped_mixed<false, false, true>) : go(gemm_asm_grouped_mixed<false>);

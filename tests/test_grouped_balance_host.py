@@ -1,0 +1,42 @@
+"""How the grouped launch with two tile heights shares its tiles (gemm_asm_grouped_mixed in csrc/gemm_fp8_big.hip), restated on the
+host: every tile of both classes is taken by exactly one workgroup of the XCD whose run it lies in, and no workgroup has
+more work than a longest-first list schedule would give it: at most one small tile above the least loaded one of its XCD (a big
+tile counts 3, a small one 2)."""
+import pytest
+
+
+def share(all_big, all_small, grid):
+    """-> per workgroup (XCD, big tile numbers, small tile numbers)"""
+    out = []
+    for b in range(grid):
+        P, x, wg = grid >> 3, b & 7, b >> 3
+        eb, es = all_big & 7, all_small & 7
+        first_big, n_big = x * (all_big >> 3) + min(x, eb), (all_big >> 3) + (x < eb)
+        first_small, n_small = x * (all_small >> 3) + max(0, x - (8 - es)), (all_small >> 3) + (x >= 8 - es)
+        rounds, r = divmod(n_big, P)
+        extra = wg < r
+        shift = 2 * (P - r) + wg if extra else wg - 2 * r
+        zeroth = shift if extra else wg - r
+        mine_small = 0
+        if zeroth < n_small:
+            rest = n_small - shift
+            mine_small = 1 + ((rest - 1) // P if rest > P else 0)
+        big = [first_big + k * P + wg for k in range(rounds + extra)]
+        small = [first_small + (zeroth if k == 0 else k * P + shift) for k in range(mine_small)]
+        out.append((x, big, small))
+    return out
+
+
+@pytest.mark.parametrize("grid", [8, 16, 256, 304])
+@pytest.mark.parametrize("all_small", [0, 1, 7, 9, 31, 32, 255, 416, 513, 2048, 5000])
+def test_every_tile_once_and_balanced(grid, all_small):
+    for all_big in (0, 1, 8, 63, 64, 160, 255, 256, 257, 300, 1000, 3333):
+        got = share(all_big, all_small, grid)
+        assert sorted(t for _, b, _ in got for t in b) == list(range(all_big)), (all_big, all_small, grid)
+        assert sorted(t for _, _, s in got for t in s) == list(range(all_small)), (all_big, all_small, grid)
+        for x in range(8):
+            load = [(3 * len(b) + 2 * len(s), len(s)) for xx, b, s in got if xx == x]
+            least = min(w for w, _ in load)
+            assert all(w - 2 <= least for w, small in load if small), (all_big, all_small, grid, load)
+            runs = [t for xx, b, _ in got if xx == x for t in b]
+            assert not runs or max(runs) - min(runs) + 1 == len(runs)          # one run of numbers per XCD
