@@ -70,8 +70,8 @@ int launch_big(const void *Aq, const void *As, const void *Bq, const void *Bs, i
                int64_t K, void *C, int64_t ldc, int out_dtype, int tn, hipStream_t st);
 
 bool rowscale_asm_ok(const void *As, const void *Bs, int scale_dtype, int64_t M, int64_t N, int64_t K);
-int launch_rowscale_asm(const void *Aq, const void *As, const void *Bq, const void *Bs, int64_t M, int64_t N, int64_t K, void *C,
-                        int out_dtype, hipStream_t st);
+int launch_rowscale_asm(const void *Aq, const void *As, const void *Bq, const void *Bs, const int32_t *groups, int G, int max_k_blocks,
+                        int multiple, int64_t M, int64_t N, void *C, int out_dtype, hipStream_t st);
 
 // gemm_skinny.hip: at most 64 activation rows
 constexpr int kSkinnyBlocks = 7;          // K blocks one workgroup handles
@@ -90,8 +90,6 @@ int64_t skinny_workspace_bytes(int64_t N, int splits);
 int launch_skinny(const void *Aq, const void *As, const void *Bq, const void *Bs, int scale_dtype, int64_t M, int64_t N,
                   int64_t K, void *C, int out_dtype, float *ws, int splits, int per, hipStream_t st);
 
-int launch_rowscale_grouped_asm(const void *Aq, const void *As, const void *Bq, const void *Bs, const int32_t *groups, int G, int max_k_blocks, int64_t M,
-                                int64_t N, void *C, int out_dtype, hipStream_t st);
 int launch_nt_unit_scales(const void *A, const void *B, const void *ones, int64_t M, int64_t N, int64_t K, void *C, int out_dtype,
                           hipStream_t st, bool bf16 = false);
 bool nt_unit_scales_ok(const void *ones, int64_t M, int64_t N, int64_t K);

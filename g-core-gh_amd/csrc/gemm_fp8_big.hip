@@ -328,8 +328,8 @@ struct AsmTile {
 // since requesting scales that start at any address takes registers, a second write to LDS and a dozen scalar instructions
 // per trip (see gen_gemm_loop.py).
 // BROW: the weights carry an e8m0 scale per row and K block ([N, K/128] bytes) instead of per 128 rows; the matrix
-// instruction takes a scale per operand row anyway, so the loop only fetches them differently (hardware-scaled
-// 128 x 128 loop: waves 2 and 3 copy the weight-scale dwords of a group while waves 0 and 1 copy the activations').
+// instruction takes a scale per operand row anyway, so the loop only fetches them differently (the second half of the waves
+// loads the weight scales of a group while the first half loads the activations').
 // STAGED: bf16 results leave through LDS, so that a store instruction writes 16 bytes per lane and whole runs of a row
 // (4 rows x 256 contiguous bytes for a 128-column wave tile) instead of 16 rows x 32 bytes.  Each wave turns its own
 // 64-row sub-tile in a region of its own (the stage memory, free after the loop), so only the barrier that ends the
@@ -351,7 +351,7 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
 {
     using T = AsmTile<TM, TN, KSUB, NST, WN>;
     constexpr int WAVES = T::WAVES, NBW = T::NBW;
-    static_assert(!RAG || (KSUB == 1 && !DUAL && !BROW && !BF16 && ((NST == 2 && TM == TN) || WN == 4)), "any K: the 128 x 128, 256 x 256 and flat tiles");
+    static_assert(!RAG || (KSUB == 1 && !DUAL && !BF16 && ((NST == 2 && TM == TN) || WN == 4)), "any K: the 128 x 128, 256 x 256 and flat tiles");
     static_assert(WN == 2 || (WN == 4 && TM == 128 && TN == 256 && KSUB == 1 && !DUAL && NST == 3 && !BROW), "four waves along N: the 128 x 256 tile, three stages");
     // NN: Bq is the weight as stored for C = A W, [K, N] row-major (row pitch N), Bs its [K / 128, N / 128] scale bytes:
     // the 256-row and the flat tile with e8m0 scales (the data gradient of the grouped linear)
@@ -359,7 +359,7 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
                   "weights stored [K, N]: hardware-scaled 256 x 256 and 128 x 256 tiles");
     static_assert(!DUAL || (TM == 128 && TN == 128), "the K split inside a workgroup is built for the 128 x 128 tile");
     static_assert(NST == 2 || (NST == 3 && WN == 4) || (NST == 4 && TM == 128 && TN == 128 && KSUB == 1 && !DUAL), "three stages: flat tile, four: 128 x 128 tile");
-    static_assert(!BROW || (HWS && TM == 128 && TN == 128 && KSUB == 1 && !DUAL && NST == 2), "row-scaled weights: hardware-scaled 128 x 128 loop");
+    static_assert(!BROW || (HWS && RAG && TM == TN && KSUB == 1 && !DUAL && NST == 2), "row-scaled weights: hardware-scaled 128 x 128 and 256 x 256 loops for any K");
     static_assert((TM / 8 / WAVES == 4 || (WN == 4 && TM / 8 / WAVES == 2)) && (TN / 8 / WAVES == 4 || TN / 8 / WAVES == 3),
                   "copies per operand and wave");
     constexpr int NBC = TN / 8 / WAVES;                 // weight copies per wave and K block
@@ -491,15 +491,14 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
     // RAG: bytes from the first to the last K block of an operand row, K blocks of the last trip (0: four), and where this
     // lane writes the scales of the row it loads (see srd)
     const uint32_t klast = __builtin_amdgcn_readfirstlane((kblocks - 1) * KB), krem = __builtin_amdgcn_readfirstlane(kblocks & 3);
-    const uint32_t swr = lds0 + T::S_LDS + wave * 1024 + lane * (HWS ? 4 : 16);
+    const uint32_t swr = lds0 + T::S_LDS + (copies_weights ? TM * 16 : 0) + wave * 1024 + lane * (HWS ? 4 : 16);
     (void)klast; (void)krem; (void)swr;
     (void)bsn_u; (void)bsbfe; (void)bsstride; (void)bstep;
     // scale staging: 16 bytes per activation row (fp32, four K steps), or 4 bytes per row in 1 KB per copying wave (e8m0)
     const uint32_t srd = HWS ? lds0 + T::S_LDS + wm * 1024 + l16 * 4 : lds0 + T::S_LDS + arow_l * 16;
-    // row-scaled weights: their dwords live behind the two activation halves, 1 KB per copying wave like those
-    const uint32_t sdst = __builtin_amdgcn_readfirstlane((uint32_t)(T::S_LDS + (copies_weights ? 2048 : 0)));
-    const uint32_t srdb = lds0 + T::S_LDS + 4096 + wn * 1024 + l16 * 4;
-    (void)sdst; (void)srdb;
+    // row-scaled weights: their dwords live behind the two activation halves, 1 KB per copying wave (64 rows) like those
+    const uint32_t srdb = lds0 + T::S_LDS + TM * 32 + wn * (TN / WN * 16) + l16 * 4;
+    (void)srdb;
 
     f32x16v accs[NBW];
     if constexpr (TN == 288) {
@@ -611,6 +610,16 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
             }
         }
         accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3;
+    } else if constexpr (BROW && TM == 256) {
+        f32x16v acc0, acc1, acc2, acc3, acc4, acc5, acc6, acc7;
+        asm volatile(
+#include "gemm_big_hwrow_rag_loop.inc"
+            : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3),
+              "=&{v[192:207]}"(acc4), "=&{v[208:223]}"(acc5), "=&{v[224:239]}"(acc6), "=&{v[240:255]}"(acc7)
+            : LP_ASM_INPUTS, LP_ASM_INPUTS_RAG, [srdb] "v"(srdb)
+            : LP_ASM_CLOBBERS, LP_ASM_CLOBBERS_RAG);
+        accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3;
+        accs[4] = acc4; accs[5] = acc5; accs[6] = acc6; accs[7] = acc7;
     } else if constexpr (HWS && NBW == 8) {
         f32x16v acc0, acc1, acc2, acc3, acc4, acc5, acc6, acc7;
         if constexpr (BF16) {
@@ -644,10 +653,10 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
     } else if constexpr (BROW) {
         f32x16v acc0, acc1, acc2, acc3;
         asm volatile(
-#include "gemm_mid_hwrow_loop.inc"
+#include "gemm_mid_hwrow_rag_loop.inc"
             : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
-            : LP_ASM_INPUTS, [sdst] "s"(sdst), [srdb] "v"(srdb)
-            : LP_ASM_CLOBBERS);
+            : LP_ASM_INPUTS, LP_ASM_INPUTS_RAG, [srdb] "v"(srdb)
+            : LP_ASM_CLOBBERS, LP_ASM_CLOBBERS_RAG);
         accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3;
     } else if constexpr (HWS && NST == 4) {
         f32x16v acc0, acc1, acc2, acc3;
@@ -1067,41 +1076,31 @@ __global__ __launch_bounds__(512) void gemm_asm_mixed(const uint8_t *__restrict_
     }
 }
 
-// 128 x 128 tiles, e8m0 scales per row and K block on both operands (the weight-gradient GEMM of the grouped linear).
-__global__ __launch_bounds__(256) void gemm_asm_rowscale(const uint8_t *__restrict__ Aq, const float *__restrict__ As,
-                                                         const uint8_t *__restrict__ Bq, const float *__restrict__ Bs, int64_t M,
-                                                         int64_t N, int64_t K, int64_t tiles_m, int64_t tiles_n,
-                                                         void *__restrict__ C, int64_t ldc, int out_dtype)
+// e8m0 scales per row and K block on both operands (the weight-gradient GEMM of the grouped linear): one problem, or a list of
+// problems that share M and N and differ in K (the weight gradients of the experts).  Entry g of `groups` = {output slot, K
+// blocks of 128, K blocks of all problems before it in the operand buffers, unused}: problem g reads Aq + M * 128 * before (its
+// [M, K_g] codes), As + M * before, the same for B with N, and writes C + slot * M * N.  per_group workgroups (a multiple of
+// 256) belong to each entry.
+template <int TM>
+__global__ __launch_bounds__(TM * 2) void gemm_asm_rowscale(const uint8_t *__restrict__ Aq, const float *__restrict__ As,
+                                                            const uint8_t *__restrict__ Bq, const float *__restrict__ Bs,
+                                                            const int32_t *__restrict__ groups, int64_t M, int64_t N,
+                                                            int64_t tiles_m, int64_t tiles_n, int64_t per_group,
+                                                            void *__restrict__ C, int out_dtype, int max_k_blocks, int multiple)
 {
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[AsmTile<128, 128, 1>::LDS_BYTES + 4096];
-    int64_t tm, tn;
-    if (!gemm::tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
-    tile_asm<128, 128, 1, true, false, 2, true, true>(smem, Aq, As, Bq, Bs, tm * 128, M, tn * 128, N, K, C, ldc, out_dtype);
-}
-
-// The same for a list of problems that share M and N and differ in K (the weight gradients of the experts of a grouped
-// linear): entry g of `groups` = {output slot, K blocks of 128, K blocks of all problems before it in the operand
-// buffers, unused}.  Problem g reads Aq + M * 128 * before (its [M, K_g] codes), As + M * before, the same for B with
-// N, and writes C + slot * M * N.  per_group workgroups (a multiple of 256) belong to each entry.
-__global__ __launch_bounds__(256) void gemm_asm_rowscale_grouped(const uint8_t *__restrict__ Aq, const float *__restrict__ As,
-                                                                 const uint8_t *__restrict__ Bq, const float *__restrict__ Bs,
-                                                                 const int32_t *__restrict__ groups, int64_t M, int64_t N,
-                                                                 int64_t tiles_m, int64_t tiles_n, int64_t per_group,
-                                                                 void *__restrict__ C, int out_dtype, int max_k_blocks)
-{
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[AsmTile<128, 128, 1>::LDS_BYTES + 4096];
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[AsmTile<TM, TM, 1>::LDS_BYTES + TM * 32];
     const int64_t g = blockIdx.x / per_group, local = blockIdx.x - g * per_group;
     int64_t tm, tn;
     if (!gemm::tile_coords(local, tiles_m, tiles_n, tm, tn)) return;
-    const int64_t slot = groups[4 * g], kb = groups[4 * g + 1], before = groups[4 * g + 2];
+    const int64_t slot = groups ? groups[4 * g] : 0, before = groups ? groups[4 * g + 2] : 0;
+    const int kb = groups ? groups[4 * g + 1] : max_k_blocks;
     // an entry that breaks the caller's promise writes nothing: more K blocks than max_k_blocks (on which the host checked
-    // that the operands fit 32-bit offsets), a count that is not a multiple of four (the loop works in groups of four
-    // K blocks and would silently drop the rest), a negative slot or offset
-    if (kb <= 0 || kb > max_k_blocks || (kb & 3) || slot < 0 || before < 0) return;
+    // that the operands fit 32-bit offsets), a count that is no multiple of the promised one, a negative slot or offset
+    if (kb <= 0 || kb > max_k_blocks || kb % multiple || slot < 0 || before < 0) return;
     char *c = (char *)C + slot * M * N * (out_dtype == LP_BF16 ? 2 : 4);
-    tile_asm<128, 128, 1, true, false, 2, true, true>(smem, Aq + M * 128 * before, (const float *)((const char *)As + M * before),
-                                                      Bq + N * 128 * before, (const float *)((const char *)Bs + N * before), tm * 128, M,
-                                                      tn * 128, N, kb * 128, c, N, out_dtype);
+    tile_asm<TM, TM, 1, true, false, 2, true, true, 2, false, false, true>(
+        smem, Aq + M * 128 * before, (const float *)((const char *)As + M * before), Bq + N * 128 * before,
+        (const float *)((const char *)Bs + N * before), tm * TM, M, tn * TM, N, (int64_t)kb * 128, c, N, out_dtype);
 }
 
 // Grouped variant: expert e owns rows m_offsets[e] .. m_offsets[e+1]-1 and the weight matrix e of Bq / Bs.
@@ -1597,34 +1596,31 @@ int launch_mid_asm(const void *Aq, const void *As, const void *Bq, const void *B
     return check_launch("lp_gemm_fp8_block(asm128)");
 }
 
-// Row-scaled weights on the hardware-scaled loop: e8m0 scales, K in whole groups of four blocks, 32-bit operand offsets.
+// Row-scaled operands on the hardware-scaled loops: e8m0 scales, 32-bit operand offsets.
 bool rowscale_asm_ok(const void *As, const void *Bs, int scale_dtype, int64_t M, int64_t N, int64_t K)
 {
     static const bool no_asm = getenv("LP_GEMM_NO_ASM") != nullptr;
-    return !no_asm && scale_dtype == LP_E8M0 && K % 512 == 0 && (uintptr_t)As % 4 == 0 && (uintptr_t)Bs % 4 == 0 &&
-           M * K < 0xFFFFFFFFLL && N * K < 0xFFFFFFFFLL;
+    return !no_asm && scale_dtype == LP_E8M0 && asm_size_ok(As, Bs, M, N, K, scale_dtype);
 }
 
-int launch_rowscale_asm(const void *Aq, const void *As, const void *Bq, const void *Bs, int64_t M, int64_t N, int64_t K, void *C,
-                        int out_dtype, hipStream_t st)
+// groups == nullptr: one problem of max_k_blocks K blocks.
+int launch_rowscale_asm(const void *Aq, const void *As, const void *Bq, const void *Bs, const int32_t *groups, int G, int max_k_blocks,
+                        int multiple, int64_t M, int64_t N, void *C, int out_dtype, hipStream_t st)
 {
-    const int64_t tiles_m = (M + 127) / 128, tiles_n = N / 128;
-    const int64_t grid = gemm::padded_grid(tiles_m, tiles_n);
-    if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_rowscale: problem too large");
-    hipLaunchKernelGGL(gemm_asm_rowscale, dim3((unsigned)grid), dim3(256), 0, st, (const uint8_t *)Aq, (const float *)As,
-                       (const uint8_t *)Bq, (const float *)Bs, M, N, K, tiles_m, tiles_n, C, N, out_dtype);
-    return check_launch("lp_gemm_fp8_rowscale(asm)");
-}
-
-int launch_rowscale_grouped_asm(const void *Aq, const void *As, const void *Bq, const void *Bs, const int32_t *groups, int G, int max_k_blocks, int64_t M,
-                                int64_t N, void *C, int out_dtype, hipStream_t st)
-{
-    const int64_t tiles_m = (M + 127) / 128, tiles_n = N / 128;
+    // 256 x 256 tiles (us per problem of 4096 x 4096 with 3 / 4 / 8 / 16 / 32 K blocks: 11.0 / 12.1 / 17.2 / 29.1 / 51.0 against
+    // 12.4 / 13.3 / 18.6 / 31.3 / 58.6 on 128 x 128 ones), unless they would cover more than a tenth beyond the matrix or leave
+    // CUs without one.
+    const int64_t big = ((M + 255) / 256) * ((N + 255) / 256);
+    const int tm = big * 65536 * 10 <= M * N * 11 && big * G >= 256 ? 256 : 128;
+    const int64_t tiles_m = (M + tm - 1) / tm, tiles_n = (N + tm - 1) / tm;
     const int64_t per_group = gemm::padded_grid(tiles_m, tiles_n), grid = per_group * G;
-    if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_rowscale_grouped: problem too large");
-    hipLaunchKernelGGL(gemm_asm_rowscale_grouped, dim3((unsigned)grid), dim3(256), 0, st, (const uint8_t *)Aq, (const float *)As,
-                       (const uint8_t *)Bq, (const float *)Bs, groups, M, N, tiles_m, tiles_n, per_group, C, out_dtype, max_k_blocks);
-    return check_launch("lp_gemm_fp8_rowscale_grouped(asm)");
+    if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_rowscale: problem too large");
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(tm * 2), 0, st, (const uint8_t *)Aq, (const float *)As, (const uint8_t *)Bq,
+                           (const float *)Bs, groups, M, N, tiles_m, tiles_n, per_group, C, out_dtype, max_k_blocks, multiple);
+    };
+    tm == 256 ? go(gemm_asm_rowscale<256>) : go(gemm_asm_rowscale<128>);
+    return check_launch("lp_gemm_fp8_rowscale(asm)");
 }
 
 // Grouped problems on the hand-scheduled kernels: offsets that fit 32 bits.

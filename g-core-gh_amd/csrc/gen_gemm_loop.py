@@ -42,7 +42,7 @@ def configure(tm, tn, waves_m, waves_n, ksub, hw=False, nstage=2, brow=False, ea
     for problems of about one tile per CU whose time is the chain of K steps)."""
     global A_BYTES, B_BYTES, SCL_LDS, SCL_HALF, NB, WAVES, KSUB, SPLIT, HW, NSTAGE, BROW, EARLY, WIDE, lines
     global ACC, P, AF, SC, SC2, SAN, WFB, RA0, RA1, RB0, RB1, SRD0, SRD, WS1, WS2, WSCUR, HALFSPLIT, ROT, WITH_IDLE, IDLE, PINGPONG, GRP, SPREAD, NN, BF, RBN
-    global WIDE_GROUP, WIDE_PART, BF16, RAG
+    global WIDE_GROUP, WIDE_PART, BF16, RAG, WSC
     # rag: any number of K blocks (the other loops need a multiple of four: their scale groups).  Three things differ.  The
     # operand bases stop at the last K block (s93 / s94 = their low halves there), so the requests of a last trip of fewer than
     # four blocks re-read that block instead of running past the matrices, and every counted wait stays as it is.  The last trip
@@ -52,7 +52,8 @@ def configure(tm, tn, waves_m, waves_n, ksub, hw=False, nstage=2, brow=False, ea
     # later.  Weight scales: fp32 by scalar loads of the group's length; e8m0 by a vector load of one address for all lanes.
     # nn: the scale bytes of the stored weight lie a table row apart, four byte loads per group, whatever that row's length.
     RAG = rag
-    assert not rag or (early and not wide and not brow and not bf16)
+    # brow: the weight scales take the activation scales' way, loaded by the other half of the waves.
+    assert not rag or (early and not wide and not bf16)
     # bf16: the operands are bf16 values (a K step of 128 bytes is 64 of them) and every matrix instruction of the
     # hardware-scaled loop becomes two v_mfma_f32_16x16x32_bf16 on the halves of the same fragment registers, accumulating
     # in place: a lane's first four registers hold values 16 lq .. 16 lq + 7 of its row and the other four 16 lq + 8 .. + 15,
@@ -132,7 +133,7 @@ def configure(tm, tn, waves_m, waves_n, ksub, hw=False, nstage=2, brow=False, ea
     assert not ROT or not wide
     NSTAGE = nstage
     BROW = brow                 # weight scales per row and K step (e8m0, hardware-scaled loop only) instead of per 128 rows
-    assert not brow or (hw and tm == 128 and tn == 128)
+    assert not brow or (hw and rag and tm == tn)
     assert nstage == 2 or (nstage in (3, 4) and ksub == 1)
     assert tm == 64 * waves_m
     WAVES = waves_m * waves_n
@@ -141,6 +142,7 @@ def configure(tm, tn, waves_m, waves_n, ksub, hw=False, nstage=2, brow=False, ea
     SCL_LDS = nstage * ksub * (A_BYTES + B_BYTES)          # activation-scale buffer: 2 halves x tm rows x 16 bytes
     SCL_HALF = tm * 16        # (the e8m0 variant uses 4 of every 16 bytes: one wave writes 64 rows x 4 bytes per KB)
     NB = tn // waves_n // 16
+    WSC = WSN + NB
     RBN = [f"v{96 + b}" for b in range(NB)]               # nn: fragment read address of block b (the fp32 loops' result registers are free)
     # a wave whose columns are not a multiple of 128 wide can straddle two weight-scale blocks: two scale rows
     # are loaded and each pair of 16-column blocks takes the one the set-up code selected for it
@@ -163,7 +165,7 @@ def b_lds(stage, sub):
 
 SCP = (44, 224, 228)        # scale products per pair of 16-column blocks when a wave straddles two weight-scale blocks
 SRDB0, SRDB = 37, 38        # row-scaled weights: LDS address of the lane's weight-scale dwords (half 0, half in use)
-WSN, WSC = 96, 100          # ... the dwords of this group / of the next one, one per 16-row block
+WSN, WSC = 96, 100          # ... the dwords of this group / of the next one, one per 16-row block (WSC = WSN + blocks of a wave)
 WB_EXTRA = ("s[42:43]", "s[78:79]", "s[80:81]", "s[82:83]", "s[84:85]")     # wide: weight base per copy
 # wide, 288 columns: the 36 groups of 8 weight rows are dealt to the waves so that the early hand-back can request the
 # first 64 rows of both wave columns (groups 0..7 and 18..25: the rows blocks 0..3 read) half way through a step and the
@@ -367,7 +369,7 @@ def wait_copies(c, at_end, extra=""):
         emit(f"Lwj{tag}%=:")
 
 
-RSA, RSB, RZERO = 104, 108, 112     # rag, e8m0: activation / weight scales of the next group on their way, a zero offset
+RSA, RSB, RZERO = 112, 116, 120     # rag, e8m0: activation / weight scales of the next group on their way, a zero offset
 RSA_F32 = 36                        # rag, fp32: the lane's four activation scales of the next group
 
 
@@ -410,6 +412,8 @@ def rag_scale_load(tag):
     emit(f"Lra{tag}%=:")
     emit(f"s_add_u32 s44, s44, {4 if HW else 16}")
     emit("s_addc_u32 s45, s45, 0")
+    if BROW:
+        return
     if HW:
         for i in range(1, 4):
             emit(f"v_mov_b32 v{RSB + i}, 0")
@@ -457,7 +461,7 @@ def rag_scale_write(tag):
     if HW:
         if not NN:
             rag_short(f"Lrc{tag}%=")
-        for base in (RSA, RSB) if not NN else (RSB,):
+        for base in (RSB,) if NN else (RSA,) if BROW else (RSA, RSB):
             for i in range(1, 4 if NN else 3):
                 emit(f"v_lshl_or_b32 v{base}, v{base + i}, {8 * i}, v{base}")
         if NN:
@@ -485,10 +489,7 @@ def scale_group_copy(tag):
     emit("s_cmp_eq_u32 s53, 0")
     emit(f"s_cbranch_scc1 Lnosc{tag}%=")
     emit("s_add_u32 m0, s48, s54")
-    if BROW:
-        emit("s_add_u32 m0, m0, s51")                     # activation rows or weight rows: the set-up code says where
-    else:
-        emit(f"s_add_u32 m0, m0, {SCL_LDS}")
+    emit(f"s_add_u32 m0, m0, {SCL_LDS}")
     emit("s_nop 0")
     emit("global_load_lds_dword %[soff], s[44:45]" if HW else "global_load_lds_dwordx4 %[soff], s[44:45]")
     emit(f"Lnosc{tag}%=:")
@@ -498,8 +499,8 @@ def scale_group_copy(tag):
 
 def weight_scale_load():
     """The four weight scales of the next group into s[60:63] (and those of the second scale row into s[68:71])."""
-    if BROW or RAG:
-        return                                            # they travel with the activation scales, see scale_group_copy
+    if RAG:
+        return                                            # they travel with the activation scales, see rag_scale_load
     if NN:
         # one byte per K step, a table row (s64 bytes) apart: the aligned dword around each, taken apart at the top of the loop
         for i in range(4):
@@ -548,7 +549,7 @@ def read_scales(col):
                 emit(f"ds_read_b32 v{SC + mb}, {SRD} offset:{mb * 64}")
             if BROW:
                 for nb in range(NB):
-                    emit(f"ds_read_b32 v{WSC + nb}, v{SRDB} offset:{nb * 64}")
+                    emit(f"ds_read_b32 v{WSC + nb}, v{SRDB} offset:{(nb >> 2) * 1024 + (nb & 3) * 64}")
         return
     for mb in range(MB):
         emit(f"ds_read_b32 v{SAN + mb}, {SRD} offset:{mb * 256 + col * 4}")
@@ -875,7 +876,6 @@ def generate():
             emit("s_mov_b32 s65, %[bsbfe]")                # s_bfe_u32 operand: 8 bits from bit 8 * (table address & 3)
         emit("s_mov_b32 s66, %[bstep]")                    # bytes between two K steps of the stored weight
     if BROW:
-        emit("s_mov_b32 s51, %[sdst]")
         emit(f"v_mov_b32 v{SRDB0}, %[srdb]")
         emit(f"v_mov_b32 v{SRDB}, %[srdb]")
     for r in range(16 * NB):
@@ -918,7 +918,7 @@ def generate():
         emit(f"ds_read_b32 v{(SC if HW else SAN) + mb}, {SRD} offset:{mb * (64 if HW else 256)}")
     if BROW:
         for nb in range(NB):
-            emit(f"ds_read_b32 v{WSC + nb}, v{SRDB} offset:{nb * 64}")
+            emit(f"ds_read_b32 v{WSC + nb}, v{SRDB} offset:{(nb >> 2) * 1024 + (nb & 3) * 64}")
     emit("s_waitcnt lgkmcnt(0)")
     read_bfrag(WFB[0], 0, 0)
     for mb in range(MB):
@@ -971,7 +971,6 @@ def main():
                       ("gemm_flat_loop.inc", (128, 256, 2, 4, 1, False, 3, False, True, False, True)),
                       ("gemm_flat_hw_loop.inc", (128, 256, 2, 4, 1, True, 3, False, True, False, True)),
                       ("gemm_mid4_loop.inc", (128, 128, 2, 2, 1, False, 4)), ("gemm_mid4_hw_loop.inc", (128, 128, 2, 2, 1, True, 4)),
-                      ("gemm_mid_hwrow_loop.inc", (128, 128, 2, 2, 1, True, 2, True, True)),
                       ("gemm_big_hw_nn_loop.inc", (256, 256, 4, 2, 1, True, 2, False, True, False, True, PP, True)),
                       ("gemm_flat_hw_nn_loop.inc", (128, 256, 2, 4, 1, True, 3, False, True, False, True, False, True)),
                       ("gemm_big_bf16_loop.inc", (256, 256, 4, 2, 1, True, 2, False, True, False, True, PP, False, True)),
@@ -981,6 +980,8 @@ def main():
                       ("gemm_mid_hw_rag_loop.inc", (128, 128, 2, 2, 1, True, 2, False, True, False, False, False, False, False, True)),
                       ("gemm_flat_rag_loop.inc", (128, 256, 2, 4, 1, False, 3, False, True, False, True, False, False, False, True)),
                       ("gemm_flat_hw_rag_loop.inc", (128, 256, 2, 4, 1, True, 3, False, True, False, True, False, False, False, True)),
+                      ("gemm_mid_hwrow_rag_loop.inc", (128, 128, 2, 2, 1, True, 2, True, True, False, False, False, False, False, True)),
+                      ("gemm_big_hwrow_rag_loop.inc", (256, 256, 4, 2, 1, True, 2, True, True, False, True, PP, False, False, True)),
                       ("gemm_big_hw_nn_rag_loop.inc", (256, 256, 4, 2, 1, True, 2, False, True, False, True, PP, True, False, True)),
                       ("gemm_flat_hw_nn_rag_loop.inc", (128, 256, 2, 4, 1, True, 3, False, True, False, True, False, True, False, True))):
         configure(*cfg)

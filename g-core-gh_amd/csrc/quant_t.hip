@@ -4,7 +4,7 @@
 // so both operands are needed with that dimension contiguous and scaled per 128 of it.  This kernel takes a
 // row-major [rows, cols] tensor whose rows are grouped by expert (m_offsets) and writes, per expert, the
 // transposed codes [cols, P_e] with one power-of-two scale per (column, 128 rows), P_e = M_e rounded up to a
-// multiple of pad_rows (128, or 512 so that the row-scaled GEMM can run its K loop in whole groups of four blocks).  Blocks restart at every expert; the rows that pad the last block are zero codes and take no
+// multiple of pad_rows.  Blocks restart at every expert; the rows that pad the last block are zero codes and take no
 // part in the block's amax.  Expert e's matrices start at cols * (P_0 + .. + P_{e-1}) in the code buffer and at
 // that over 128 in the scale buffer, so each expert's pair is a contiguous operand for lp_gemm_fp8_rowscale.
 // One workgroup (256 threads) = 128 rows x 128 columns.  A thread owns 8 consecutive rows x 8 consecutive columns
@@ -31,7 +31,7 @@ __device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b)
 }
 
 // 128-row blocks an expert of `rows` rows takes: rows rounded up to pad_rows, or with pad_rows = LP_PAD_MIXED to 128 up to
-// 256 rows and to 512 beyond (short experts then run the row-scaled GEMM's one- and two-block kernel, the others its loop)
+// 256 rows and to 512 beyond
 __device__ __forceinline__ int padded_blocks_of(int rows, int pad_rows)
 {
     if (pad_rows == LP_PAD_MIXED) return rows <= 256 ? (rows + 127) >> 7 : ((rows + 511) >> 9) << 2;

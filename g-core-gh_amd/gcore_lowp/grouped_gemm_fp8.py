@@ -159,11 +159,9 @@ def padded_blocks(rows: int, pad_rows: int) -> int:
 
 
 def choose_colwise_pad(m_splits) -> int:
-    """How the experts' rows are padded in the column-wise operands: A.PAD_MIXED -- experts of at most 256 rows to 128 or
-    256 (the row-scaled GEMM has a kernel without a K loop for problems of one and two K blocks: a weight gradient of a
-    short expert is a write of N x K values more than a GEMM), the others to multiples of 512 (its hand-scheduled loop
-    needs K in multiples of 512).  256 experts of [4096, 7168] with 0 .. 7163 rows: 6.7 ms with every expert padded to
-    512, 9.7 ms with every expert padded to 128 (the experts above 256 rows then run on the compiler-scheduled kernel)."""
+    """The default padding of quant_fp8_colwise_t: A.PAD_MIXED, 128 or 256 rows for experts of at most 256 rows and multiples of
+    512 beyond.  The grouped linear pads to whole blocks of 128 instead: the row-scaled loops take any number of K blocks, and
+    every padded block is multiplied."""
     return A.PAD_MIXED
 
 
@@ -221,13 +219,17 @@ def rowscale_launches(k_blocks):
 
 def gemm_fp8_rowscale_grouped(aq, a_s, bq, b_s, k_blocks, M, N, out: torch.Tensor) -> torch.Tensor:
     """out[e] [M, N] = the row-scaled product of problem e, whose operands ([M, K_e] / [N, K_e] codes and their e8m0
-    scales, K_e = 128 * k_blocks[e]) lie one after the other in aq / a_s / bq / b_s.  The problems whose K is a multiple
-    of 512 go to the hand-scheduled loop in one launch, those of one and of two K blocks to the kernel without a K loop
-    (a launch each), the others to the compiler-scheduled kernel; problems with no K blocks are zero-filled.  (The
-    reference issues one grouped GEMM call: fp8.py:325-341.)"""
+    scales, K_e = 128 * k_blocks[e]) lie one after the other in aq / a_s / bq / b_s.  The problems of one and of two K blocks
+    go to the kernel without a K loop (a launch each), the others to the hand-scheduled loop in one launch, longest first (a
+    long problem started last would run alone at the end); problems with no K blocks are zero-filled.  (The reference issues
+    one grouped GEMM call: fp8.py:325-341.)"""
     E = len(k_blocks)
     assert out.is_contiguous() and tuple(out.shape) == (E, M, N) and out.dtype in (torch.bfloat16, torch.float32)
-    launches, empty = rowscale_launches(k_blocks)
+    kinds, empty = rowscale_launches(k_blocks)
+    looped = [g for groups, _ in kinds for g in groups if g[1] > 2]
+    launches = [(g, m) for g, m in kinds if g[0][1] == m and m < 3 and all(x[1] == m for x in g)]
+    if looped:
+        launches.insert(0, (sorted(looped, key=lambda g: -g[1]), 1))
     for e in empty:
         out[e].zero_()
     odt = A.BF16 if out.dtype == torch.bfloat16 else A.F32
@@ -264,10 +266,10 @@ class _GroupedGemmFp8(torch.autograd.Function):
                                   scaling is its own transpose, its table is read by column); no transposed copy;
       wgrad  dW_e = dY_e^T X_e    (layout NT over column-wise operands): dY and X quantised per (column, 128 rows of
                                   the expert), transposed, the experts' row-scaled GEMMs in one launch per kind of
-                                  expert (rowscale_launches: at most four) straight into dW.
+                                  expert (at most three) straight into dW.
     The reference pads every expert to a multiple of 16 rows for TE (fp8.py:29-58); here a ragged expert needs no
     padding in the forward and dgrad (tiles are masked), and the column-wise operands are zero-padded to whole blocks
-    of 128 rows (choose_colwise_pad), which does not change any block's amax or sum."""
+    of 128 rows, which does not change any block's amax or sum."""
 
     @staticmethod
     def forward(ctx, inp, weight, wq, ws, m_splits, out_dtype):
@@ -280,7 +282,7 @@ class _GroupedGemmFp8(torch.autograd.Function):
         ctx.need_dgrad = inp.requires_grad
         saved = [wq.view(torch.uint8), ws.view(torch.uint8), offs]
         if ctx.need_wgrad:
-            ctx.pad_rows = choose_colwise_pad(m_splits)
+            ctx.pad_rows = 128
             xtq, xts, _ = quant_fp8_colwise_t(x.detach(), offs, m_splits, ctx.pad_rows)
             saved += [xtq, xts.view(torch.uint8)]
         ctx.save_for_backward(*saved)

@@ -303,14 +303,14 @@ int lp_gemm_fp8_rowscale(const void *Aq, const void *As, const void *Bq, const v
  * {output slot, K blocks of 128 of this problem, K blocks of all problems stored before it, unused}.  Problem g
  * reads Aq + M * 128 * before (its [M, K_g] codes), As + M * before scales, Bq / Bs likewise with N, and writes
  * C + slot * M * N elements.  max_k_blocks bounds every entry's K blocks (argument checks); k_blocks_multiple is
- * the caller's promise that every entry's K block count is a multiple of it (4 selects the hand-scheduled loop
- * with e8m0 scales; max_k_blocks = k_blocks_multiple = 1 or 2, i.e. every entry has exactly that many blocks,
- * selects the kernel without a K loop for short experts, whose entries of any other size write nothing).  A caller
- * with problems of several kinds makes one call per kind (gcore_lowp/grouped_gemm_fp8.py: rowscale_launches).
+ * the caller's promise that every entry's K block count is a multiple of it (max_k_blocks = k_blocks_multiple = 1 or
+ * 2, i.e. every entry has exactly that many blocks, selects the kernel without a K loop for short experts, whose entries
+ * of any other size write nothing; otherwise e8m0 scales run on the hand-scheduled loop).  A caller with problems of
+ * several kinds makes one call per kind (gcore_lowp/grouped_gemm_fp8.py: gemm_fp8_rowscale_grouped).
  * M must be a multiple of 128.  Entries with 0 blocks write nothing.  The table lives in device memory, so the
  * host cannot check it: an entry that breaks these promises (more K blocks than max_k_blocks, a count that is not
- * a multiple of 4 on the hand-scheduled kernel, a negative slot or offset) computes and writes nothing -- its C_g
- * keeps what it held.
+ * a multiple of k_blocks_multiple on the hand-scheduled kernel, a negative slot or offset) computes and writes nothing --
+ * its C_g keeps what it held.
  */
 int lp_gemm_fp8_rowscale_grouped(const void *Aq, const void *As, const void *Bq, const void *Bs, int scale_dtype,
                                  const int32_t *groups, int G, int max_k_blocks, int k_blocks_multiple, int64_t M,
@@ -319,10 +319,8 @@ int lp_gemm_fp8_rowscale_grouped(const void *Aq, const void *As, const void *Bq,
 /*
  * Column-wise quantiser with transposed output for expert-grouped rows.  x: device [rows, cols]
  * (LP_BF16 or LP_F32), rows of expert e = m_offsets[e] .. m_offsets[e+1]-1 (device int32 [E+1]),
- * cols % 128 == 0.  Per expert, P_e = ceil(M_e / pad_rows) * pad_rows (pad_rows 128, 256 or 512; with 512
- * lp_gemm_fp8_rowscale runs on its hand-scheduled kernel), or with pad_rows = LP_PAD_MIXED: M_e rounded up to 128 for
- * experts of at most 256 rows and to 512 for the others (lp_gemm_fp8_rowscale_grouped has a kernel for problems of one
- * and two K blocks, which most experts of a routed batch are), and
+ * cols % 128 == 0.  Per expert, P_e = ceil(M_e / pad_rows) * pad_rows (pad_rows 128, 256 or 512), or with
+ * pad_rows = LP_PAD_MIXED: M_e rounded up to 128 for experts of at most 256 rows and to 512 for the others, and
  *   qT block e: [cols, P_e] e4m3fn at byte offset cols * (P_0 + .. + P_{e-1}), zero codes in the pad,
  *   sT block e: [cols, P_e / 128] scales at element offset cols * (P_0 + .. + P_{e-1}) / 128,
  * scale = 2^ceil(log2(amax / 448)) per (column, 128 rows of the expert), 1 for an all-zero block
