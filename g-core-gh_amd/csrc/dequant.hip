@@ -5,6 +5,8 @@
 //
 // Arithmetic: out = cast(fl32(fl32(code) * fl32(scale))) -- the fp32 product is
 // formed and rounded first, then narrowed to bf16 with RNE (two roundings).
+#include <type_traits>
+
 #include "lowp_device.h"
 
 using namespace lowp;
@@ -55,11 +57,12 @@ __device__ __forceinline__ void decode_fp8x4(uint32_t w, float v[4])
     }
 }
 
-// Chunks (8 elements) per lane: a workgroup converts 256 * PASSES consecutive chunks.  Few passes = many small
-// workgroups, which the memory system likes better on large tensors (measured on [18432, 7168] FP8 -> bf16:
-// 5.9 / 6.1 / 6.4 TB/s with 8 / 4 / 2 passes; packed FP4 is best at 4); small tensors are launch-bound and
-// keep 8 (a quarter of the workgroups).
-constexpr int kMaxPasses = 8;
+// Chunks (8 elements) per lane: a workgroup converts 256 * PASSES consecutive chunks.  Few passes = many small workgroups,
+// which the memory system likes better on large tensors (measured on [18432, 7168] FP8 -> bf16: 5.9 / 6.1 / 6.4 TB/s with 8 / 4 /
+// 2 passes; packed FP4 is best at 4) and which put a small one on more CUs at once (us with 8 / 4 / 2 / 1 passes: 256 x 256 7.1 /
+// 4.3 / 2.7 / 2.5, 2048 x 2048 8.0 / 6.0 / 4.4 / 5.5, 4096 x 4096 12.3 / 9.8 / 10.9 / 14.0): two passes, four for large packed
+// tensors.
+constexpr int kMaxPasses = 4;
 
 // Scale index of chunk c (8 consecutive elements of one row).  With one-row blocks (bm == 1) and
 // cols % bn == 0 the scale grid is just the element index divided by bn: no row / column split.
@@ -76,12 +79,11 @@ __device__ __forceinline__ int64_t scale_index(uint32_t c, uint32_t chunks_per_r
 // chunks_per_row = cols / 8; bm, bn powers of two given as shifts; bn >= 8.
 // CHECKED = false: every chunk of the workgroup exists (no bounds tests at all).
 template <bool OUT_BF16, bool CHECKED, bool ROWSCALE, int kPasses>
-__global__ __launch_bounds__(256) void dequant_fp8_fast(const uint8_t *__restrict__ q, const void *__restrict__ scale,
-                                                        int scale_dtype, uint32_t chunk0, uint32_t n_chunks,
-                                                        uint32_t chunks_per_row, int bm_shift, int bn_shift,
-                                                        uint32_t scale_cols, void *__restrict__ out)
+__device__ __forceinline__ void dequant_fp8_chunks(const uint8_t *__restrict__ q, const void *__restrict__ scale, int scale_dtype,
+                                                   uint32_t n_chunks, uint32_t chunks_per_row, int bm_shift, int bn_shift,
+                                                   uint32_t scale_cols, void *__restrict__ out)
 {
-    const uint32_t base = chunk0 + blockIdx.x * (256u * kPasses) + threadIdx.x;
+    const uint32_t base = blockIdx.x * (256u * kPasses) + threadIdx.x;
     u32x2 w[kPasses];
     float s[kPasses];
 #pragma unroll
@@ -110,12 +112,11 @@ __global__ __launch_bounds__(256) void dequant_fp8_fast(const uint8_t *__restric
 // FP4: each lane owns 4 packed bytes = 8 consecutive elements of one row.
 // chunks_per_row = cols / 8 (logical columns); bn >= 8.
 template <bool OUT_BF16, bool CHECKED, bool ROWSCALE, int kPasses>
-__global__ __launch_bounds__(256) void dequant_fp4_fast(const uint8_t *__restrict__ packed, const void *__restrict__ scale,
-                                                        int scale_dtype, uint32_t chunk0, uint32_t n_chunks,
-                                                        uint32_t chunks_per_row, int bm_shift, int bn_shift,
-                                                        uint32_t scale_cols, int neg_zero, void *__restrict__ out)
+__device__ __forceinline__ void dequant_fp4_chunks(const uint8_t *__restrict__ packed, const void *__restrict__ scale, int scale_dtype,
+                                                   uint32_t n_chunks, uint32_t chunks_per_row, int bm_shift, int bn_shift,
+                                                   uint32_t scale_cols, int neg_zero, void *__restrict__ out)
 {
-    const uint32_t base = chunk0 + blockIdx.x * (256u * kPasses) + threadIdx.x;
+    const uint32_t base = blockIdx.x * (256u * kPasses) + threadIdx.x;
     uint32_t w[kPasses];
     float s[kPasses];
 #pragma unroll
@@ -139,6 +140,24 @@ __global__ __launch_bounds__(256) void dequant_fp4_fast(const uint8_t *__restric
         for (int j = 0; j < 8; ++j) v[j] = v[j] * s[p];
         if (!CHECKED || c < n_chunks) store8<OUT_BF16>(out, (int64_t)c * 8, v);
     }
+}
+
+// One launch: only the workgroup with the ragged end tests bounds.
+template <bool IS_FP4, bool OUT_BF16, bool ROWSCALE, int kPasses>
+__global__ __launch_bounds__(256) void dequant_fast(const uint8_t *__restrict__ codes, const void *__restrict__ scale, int scale_dtype,
+                                                    uint32_t n_chunks, uint32_t chunks_per_row, int bm_shift, int bn_shift,
+                                                    uint32_t scale_cols, int neg_zero, void *__restrict__ out)
+{
+    auto go = [&](auto checked) {
+        if constexpr (IS_FP4)
+            dequant_fp4_chunks<OUT_BF16, decltype(checked)::value, ROWSCALE, kPasses>(codes, scale, scale_dtype, n_chunks, chunks_per_row, bm_shift,
+                                                                                      bn_shift, scale_cols, neg_zero, out);
+        else
+            dequant_fp8_chunks<OUT_BF16, decltype(checked)::value, ROWSCALE, kPasses>(codes, scale, scale_dtype, n_chunks, chunks_per_row, bm_shift,
+                                                                                      bn_shift, scale_cols, out);
+    };
+    if ((blockIdx.x + 1u) * (256u * kPasses) <= n_chunks) go(std::false_type{});
+    else go(std::true_type{});
 }
 
 // any block shape, one element per thread per step
@@ -189,43 +208,23 @@ int dequant_common(const char *name, bool is_fp4, const void *codes, const void 
                       (uintptr_t)codes % 8 == 0 && (uintptr_t)out % 16 == 0;
     const bool bf = out_dtype == LP_BF16;
     if (fast) {
-        // full workgroups run without bounds tests; the ragged end (< one workgroup of chunks) is a second launch
-        const bool large = n_chunks >= (1ll << 23);
-        const int passes = !large ? 8 : (is_fp4 ? 4 : 2);
-        const uint32_t per_wg = 256 * passes;
-        const uint32_t full_wgs = (uint32_t)(n_chunks / per_wg), tail0 = full_wgs * per_wg;
+        const int passes = is_fp4 && n_chunks >= (1ll << 23) ? 4 : 2;
+        const uint32_t wgs = (uint32_t)((n_chunks + 256 * passes - 1) / (256 * passes));
         const uint32_t cpr = (uint32_t)(cols / 8), sc = (uint32_t)(cols / bn);
-        const bool rowscale = bm == 1;
-#define LP_DQ(KERNEL, BF, CHK, RS, P, GRID, C0, ...)                                                                     \
-    hipLaunchKernelGGL((KERNEL<BF, CHK, RS, P>), dim3(GRID), dim3(256), 0, st, (const uint8_t *)codes, scale, scale_dtype, \
-                       (uint32_t)(C0), (uint32_t)n_chunks, cpr, bm_shift, bn_shift, sc, ##__VA_ARGS__, out)
-#define LP_DQ_P(KERNEL, BF, CHK, RS, GRID, C0, ...)                                                                   \
-    do {                                                                                                              \
-        if (passes == 8) LP_DQ(KERNEL, BF, CHK, RS, 8, GRID, C0, ##__VA_ARGS__);                                      \
-        else if (passes == 4) LP_DQ(KERNEL, BF, CHK, RS, 4, GRID, C0, ##__VA_ARGS__);                                 \
-        else LP_DQ(KERNEL, BF, CHK, RS, 2, GRID, C0, ##__VA_ARGS__);                                                  \
-    } while (0)
-#define LP_DQ_ALL(KERNEL, ...)                                                                                        \
-    do {                                                                                                              \
-        for (int part = 0; part < 2; ++part) {                                                                        \
-            const bool chk = part == 1;                                                                               \
-            const uint32_t grid = chk ? (tail0 < n_chunks ? 1u : 0u) : full_wgs, c0 = chk ? tail0 : 0u;               \
-            if (!grid) continue;                                                                                      \
-            if (bf && !chk && rowscale) LP_DQ_P(KERNEL, true, false, true, grid, c0, ##__VA_ARGS__);                  \
-            else if (bf && !chk) LP_DQ_P(KERNEL, true, false, false, grid, c0, ##__VA_ARGS__);                        \
-            else if (bf && rowscale) LP_DQ_P(KERNEL, true, true, true, grid, c0, ##__VA_ARGS__);                      \
-            else if (bf) LP_DQ_P(KERNEL, true, true, false, grid, c0, ##__VA_ARGS__);                                 \
-            else if (!chk && rowscale) LP_DQ_P(KERNEL, false, false, true, grid, c0, ##__VA_ARGS__);                  \
-            else if (!chk) LP_DQ_P(KERNEL, false, false, false, grid, c0, ##__VA_ARGS__);                             \
-            else if (rowscale) LP_DQ_P(KERNEL, false, true, true, grid, c0, ##__VA_ARGS__);                           \
-            else LP_DQ_P(KERNEL, false, true, false, grid, c0, ##__VA_ARGS__);                                        \
-        }                                                                                                             \
-    } while (0)
-        if (is_fp4) LP_DQ_ALL(dequant_fp4_fast, neg_zero);
-        else LP_DQ_ALL(dequant_fp8_fast);
-#undef LP_DQ_ALL
-#undef LP_DQ_P
-#undef LP_DQ
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, st, (const uint8_t *)codes, scale, scale_dtype, (uint32_t)n_chunks, cpr, bm_shift,
+                               bn_shift, sc, neg_zero, out);
+        };
+        auto type = [&](auto bf16, auto rowscale) {
+            constexpr bool BF = decltype(bf16)::value, RS = decltype(rowscale)::value;
+            if (!is_fp4) go(dequant_fast<false, BF, RS, 2>);
+            else if (passes == 2) go(dequant_fast<true, BF, RS, 2>);
+            else go(dequant_fast<true, BF, RS, 4>);
+        };
+        if (bf && bm == 1) type(std::true_type{}, std::true_type{});
+        else if (bf) type(std::true_type{}, std::false_type{});
+        else if (bm == 1) type(std::false_type{}, std::true_type{});
+        else type(std::false_type{}, std::false_type{});
     } else {
         int64_t n = rows * cols;
         unsigned wgs = (unsigned)((n + 255) / 256 < 65536 ? (n + 255) / 256 : 65536);
