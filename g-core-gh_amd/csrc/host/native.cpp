@@ -8,7 +8,10 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <chrono>
+
 #include <ATen/ATen.h>
+#include <ATen/EmptyTensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
@@ -26,12 +29,14 @@ decltype(&lp_fp4_to_fp8_amax) p_fp4_amax;
 decltype(&lp_fp4_to_fp8_rebase) p_fp4_rebase;
 decltype(&lp_gemm_fp8_block) p_gemm;
 decltype(&lp_gemm_workspace_bytes) p_gemm_ws;
+decltype(&lp_host_flag) p_flag;
 
 PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
-    void *a[7];
-    if (n != 7) { PyErr_SetString(PyExc_TypeError, "bind: seven addresses"); return nullptr; }
-    for (int i = 0; i < 7; ++i) {
+    constexpr int count = 8;
+    void *a[count];
+    if (n != count) { PyErr_SetString(PyExc_TypeError, "bind: eight addresses"); return nullptr; }
+    for (int i = 0; i < count; ++i) {
         a[i] = PyLong_AsVoidPtr(args[i]);
         if (!a[i]) { if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "bind: null address"); return nullptr; }
     }
@@ -42,6 +47,7 @@ PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n)
     p_fp4_rebase = (decltype(p_fp4_rebase))a[4];
     p_gemm = (decltype(p_gemm))a[5];
     p_gemm_ws = (decltype(p_gemm_ws))a[6];
+    p_flag = (decltype(p_flag))a[7];
     Py_RETURN_NONE;
 }
 
@@ -103,13 +109,27 @@ bool ints(PyObject *const *args, int n, long *out)
         return nullptr;                                                                                                           \
     }
 
-// (x, bm, bn, scale_mode, scale code, zero_rule, amax_floor) -> (codes, scales)
+// Waits until the flag lp_host_flag raises is up.  Watching it for the length of a kernel beats the runtime's own wait (12 us
+// against 14 - 20 for a quantisation of 256 x 256 with the check); behind a long queue the runtime waits.
+bool wait_flag(const int32_t *flag, hipStream_t st)
+{
+    const auto begin = std::chrono::steady_clock::now();
+    for (int i = 0; !__atomic_load_n(flag, __ATOMIC_ACQUIRE); ++i) {
+        if ((i & 63) == 63 && std::chrono::steady_clock::now() - begin > std::chrono::microseconds(200)) return hipStreamSynchronize(st) == hipSuccess;
+        __builtin_ia32_pause();
+    }
+    return true;
+}
+
+// (x, bm, bn, scale_mode, scale code, zero_rule, amax_floor, check) -> (codes, scales), with `check` (codes, scales, whether a
+// block holds a NaN), which waits for the result
 PyObject *quant_fp8(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
     long v[5];
-    if (n != 7 || !ints(args + 1, 5, v)) Py_RETURN_NONE;
+    if (n != 8 || !ints(args + 1, 5, v)) Py_RETURN_NONE;
     const double floor = PyFloat_AsDouble(args[6]);
     if (PyErr_Occurred()) { PyErr_Clear(); Py_RETURN_NONE; }
+    const bool check = args[7] == Py_True;
     GUARDED(
         const at::Tensor *x = plain(args[0]);
         if (!x) Py_RETURN_NONE;
@@ -117,14 +137,38 @@ PyObject *quant_fp8(PyObject *, PyObject *const *args, Py_ssize_t n)
         if (!here(dev, x) || x->dim() < 2 || (x->scalar_type() != at::kBFloat16 && x->scalar_type() != at::kFloat)) Py_RETURN_NONE;
         const int64_t rows = x->size(-2), cols = x->size(-1), bm = v[0], bn = v[1];
         if (bm <= 0 || bn <= 0 || rows % bm || cols % bn || v[3] < 0 || v[3] > LP_E8M0) Py_RETURN_NONE;
+        const hipStream_t st = c10::hip::getCurrentHIPStream(dev).stream();
+        at::Tensor words;                                // NaN count, flag
+        int32_t *host = nullptr;
+        if (check) {
+            hipStreamCaptureStatus capturing;
+            if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) Py_RETURN_NONE;
+            words = at::detail::empty_cpu({2}, at::kInt, true);
+            host = words.data_ptr<int32_t>();
+            host[0] = host[1] = 0;
+        }
         at::DimVector grid(x->sizes().begin(), x->sizes().end());
         grid[grid.size() - 2] = rows / bm;
         grid[grid.size() - 1] = cols / bn;
         at::Tensor q = make(x->sizes(), at::kFloat8_e4m3fn, dev), s = make(grid, scale_type((int)v[3]), dev);
         if (p_quant_fp8(x->const_data_ptr(), x->scalar_type() == at::kFloat ? LP_F32 : LP_BF16, x->numel() / cols, cols, (int)bm, (int)bn,
-                        (int)v[2], (float)floor, (int)v[4], q.data_ptr(), s.data_ptr(), (int)v[3], nullptr, stream(dev)))
+                        (int)v[2], (float)floor, (int)v[4], q.data_ptr(), s.data_ptr(), (int)v[3], host, st))
             Py_RETURN_NONE;
-        return pair(q, s);
+        if (!check) return pair(q, s);
+        bool done;
+        // the counter and the flag stay allocated until the GPU is through with them
+        if (p_flag(host + 1, st)) {
+            done = hipStreamSynchronize(st) == hipSuccess;
+        } else {
+            Py_BEGIN_ALLOW_THREADS
+            done = wait_flag(host + 1, st);
+            Py_END_ALLOW_THREADS
+        }
+        if (!done) { PyErr_SetString(PyExc_RuntimeError, "lp_quant_fp8_block: the GPU reported an error"); return nullptr; }
+        PyObject *two = pair(q, s);
+        PyObject *r = two ? PyTuple_Pack(3, PyTuple_GET_ITEM(two, 0), PyTuple_GET_ITEM(two, 1), host[0] ? Py_True : Py_False) : nullptr;
+        Py_XDECREF(two);
+        return r;
     )
 }
 

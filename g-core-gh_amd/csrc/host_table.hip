@@ -32,3 +32,16 @@ extern "C" int lp_host_table(const int32_t *src, int64_t n, int32_t *dst, lp_str
     }
     return lowp::check_launch("lp_host_table");
 }
+
+namespace {
+
+__global__ void raise_flag(int32_t *flag) { __hip_atomic_store(flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM); }
+
+}  // namespace
+
+extern "C" int lp_host_flag(int32_t *flag, lp_stream_t stream)
+{
+    LP_REQUIRE(flag, "lp_host_flag: null pointer");
+    hipLaunchKernelGGL(raise_flag, dim3(1), dim3(1), 0, (hipStream_t)stream, flag);
+    return lowp::check_launch("lp_host_flag");
+}

@@ -49,6 +49,7 @@ PROTOTYPES = {
     "lp_gemm_fp8_grouped": (_i32, [_p, _p, _p, _p, _i32, _p, _i32, _i64, _i64, _i64, _p, _i32, _p]),
     "lp_gemm_fp8_grouped_nn": (_i32, [_p, _p, _p, _p, _i32, _p, _i32, _i64, _i64, _i64, _p, _i32, _p]),
     "lp_host_table": (_i32, [_p, _i64, _p, _p]),
+    "lp_host_flag": (_i32, [_p, _p]),
     "lp_gemm_workspace_bytes": (_i64, [_i64, _i64, _i64]),
 }
 

@@ -13,7 +13,7 @@ from . import _abi as A
 
 PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "_lowp_native.so")
 _BOUND = ("lp_quant_fp8_block", "lp_dequant_fp8_block", "lp_dequant_fp4_block", "lp_fp4_to_fp8_amax", "lp_fp4_to_fp8_rebase",
-          "lp_gemm_fp8_block", "lp_gemm_workspace_bytes")
+          "lp_gemm_fp8_block", "lp_gemm_workspace_bytes", "lp_host_flag")
 
 
 def _load():

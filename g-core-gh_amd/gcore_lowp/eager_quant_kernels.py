@@ -38,8 +38,10 @@ def quant_fp8_e4m3_scale_e8m0(value: torch.Tensor, block_size: tuple[int, int] =
     m, n = value.shape[-2:]
     bm, bn = block_size
     assert m % bm == 0 and n % bn == 0, f"value shape ({m}, {n}) not divisible by block ({bm}, {bn})"
-    q, s, n_nan = ops.quant_fp8_block(value, (bm, bn), scale_mode=A.SCALE_POW2, scale_dtype=ops.E8M0,
-                                      count_nan=True)
+    r = fast.quant_fp8(value, bm, bn, A.SCALE_POW2, A.E8M0, A.ZERO_NONE, 0.0, True)
+    if r is None:
+        r = ops.quant_fp8_block(value, (bm, bn), scale_mode=A.SCALE_POW2, scale_dtype=ops.E8M0, count_nan=True)
+    q, s, n_nan = r
     assert n_nan == 0, "quant_fp8_e4m3_scale_e8m0: input contains NaN"
     return q, s
 

@@ -57,7 +57,7 @@ def _div_quant(x, block, *, round_sf, amax_floor, zero_rule):
 def quant_1d(x: torch.Tensor, block_size: int = 128, *, round_sf: bool = False):
     """Row-wise 1 x block_size activation quant, s = max(amax, 1e-12)/448 (round_sf: rounded up to a power of two).
     Returns (e4m3fn [M, K], fp32 scale [M, K/block_size])."""
-    r = fast.quant_fp8(x, 1, block_size, A.SCALE_POW2 if round_sf else A.SCALE_DIV, A.F32, A.ZERO_NONE, 1e-12)
+    r = fast.quant_fp8(x, 1, block_size, A.SCALE_POW2 if round_sf else A.SCALE_DIV, A.F32, A.ZERO_NONE, 1e-12, False)
     return r if r is not None else _div_quant(x, (1, block_size), round_sf=round_sf, amax_floor=1e-12, zero_rule=A.ZERO_NONE)
 
 

@@ -27,7 +27,7 @@ def _quant_pow2(value: torch.Tensor, block_size):
     and so stalls the stream once per call: inside the grouped linear (three quantisations per step and layer) a NaN
     simply propagates into the product, as it does in the reference, whose layer quantises inside TransformerEngine
     (fp8.py:180-343) without such a check."""
-    r = fast.quant_fp8(value, *block_size, A.SCALE_POW2, A.E8M0, A.ZERO_NONE, 0.0)
+    r = fast.quant_fp8(value, *block_size, A.SCALE_POW2, A.E8M0, A.ZERO_NONE, 0.0, False)
     if r is not None:
         return r
     q, s, _ = ops.quant_fp8_block(value, block_size, scale_mode=A.SCALE_POW2, scale_dtype=ops.E8M0, count_nan=False)

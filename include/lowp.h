@@ -91,7 +91,7 @@ const char *lp_last_error(void);
  * One scale per bm x bn block; rows % bm == 0, cols % bn == 0.
  * q_out: device u8 [rows, cols].  scale_out: device [rows/bm, cols/bn] of
  * scale_dtype (LP_F32, LP_BF16 or LP_E8M0).  nan_count: optional device
- * int32 that is incremented once per block that holds a NaN (caller zeroes it).
+ * int32 (or one in pinned host memory) that is incremented once per block that holds a NaN (caller zeroes it).
  * Replaces quant_fp8_e4m3_scale_e8m0 (eager_quant_kernels.py:132-181),
  * quantize_fp8_blockwise (qwen3_mtp_fp8_postprocess.py:102-151) and the
  * 1 x 128 / 128 x 128 fp32-scale quantisers used around the GEMM
@@ -339,6 +339,15 @@ int lp_quant_fp8_colwise_t(const void *x, int x_dtype, int64_t rows, int64_t col
  * counts over as a host list (fp8.py:193).
  */
 int lp_host_table(const int32_t *src, int64_t n, int32_t *dst, lp_stream_t stream);
+
+/*
+ * Sets *flag (int32 in pinned host memory, device accessible) to 1 when everything queued on the stream before this call is
+ * done, so that a host that waits for one result can watch a word instead of synchronising the stream: with a NaN counter in
+ * pinned memory as well (nan_count above may point there), the quantiser's NaN check costs the host half of a read-back.
+ * For callers that have to look at a result before they go on; no counterpart in the reference, whose check is an eager
+ * assertion (eager_quant_kernels.py:156-161).
+ */
+int lp_host_flag(int32_t *flag, lp_stream_t stream);
 
 #ifdef __cplusplus
 }
