@@ -85,6 +85,46 @@ __device__ __forceinline__ Geometry geometry(int64_t super, int64_t supers_c, in
 // that neighbours sharing scale cache lines sit behind the same L2.
 __device__ __forceinline__ int64_t xcd_remap(int64_t b, int64_t per_xcd) { return (b & 7) * per_xcd + (b >> 3); }
 
+__device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+
+// value of the e2m1 code in the top nibble
+__device__ __forceinline__ float fp4_top(uint32_t x) { const f32x2 t = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(x, 1.0f, 3); return t.y; }
+
+// The e4m3 codes of a lane's 8 elements from its packed word and the 8-entry code table of its scale byte (magnitude code ->
+// e4m3 code, low four in `lo`): byte permutes look the nibbles up.  Zero magnitudes carry no sign (fp4_pos_zero).
+__device__ __forceinline__ u32x2 lookup8(uint32_t w, uint32_t lo, uint32_t hi)
+{
+    // even elements sit in the low nibbles of the four bytes, odd elements in the high nibbles
+    uint32_t ce = __builtin_amdgcn_perm(hi, lo, w & 0x07070707u);
+    uint32_t co = __builtin_amdgcn_perm(hi, lo, (w >> 4) & 0x07070707u);
+    ce |= (w & 0x08080808u) << 4;
+    co |= w & 0x80808080u;
+    return u32x2{__builtin_amdgcn_perm(co, ce, 0x05010400u), __builtin_amdgcn_perm(co, ce, 0x07030602u)};
+}
+
+// Code table at the scale byte where half a unit, t1 / 2, is the smallest normal e4m3 number's binade: t1 and t3 (the images
+// of 1 and 1.5) are given there, the other entries are theirs times powers of two, 8 per power in the code.  Every scale byte
+// `up` steps higher has each entry 8 up higher: rounding to e4m3 is the same in every binade of normal numbers, and no
+// element's quotient passes 448.  Entries that no element of a block uses may overflow into the entries above them, which are
+// larger and so are not used either; entry 0 is zero and stays zero.
+struct CodeTable {
+    uint32_t lo, hi;
+    __device__ __forceinline__ CodeTable(float t1, float t3)
+    {
+        const uint32_t c = cvt4(t1, t3, 0.0f, 0.0f), b1 = c & 0xFFu, b3 = (c >> 8) & 0xFFu;
+        lo = ((b1 - 8u) << 8) | (b1 << 16) | (b3 << 24);
+        hi = (b1 + 8u) | ((b3 + 8u) << 8) | ((b1 + 16u) << 16) | ((b3 + 16u) << 24);
+    }
+    __device__ __forceinline__ u32x2 codes(uint32_t w, int up) const
+    {
+        const uint32_t u = (uint32_t)up << 3;
+        return lookup8(w, lo + __builtin_amdgcn_perm(0u, u, 0x0000000Cu), hi + __builtin_amdgcn_perm(0u, u, 0x00000000u));
+    }
+};
+
 template <int NT>
 __global__ __launch_bounds__(NT) void fp4_rebase(const uint8_t *__restrict__ packed, const uint8_t *__restrict__ scale,
                                                   int64_t cols, int64_t supers_c, int64_t n_supers, int64_t per_xcd,
@@ -148,6 +188,11 @@ __global__ __launch_bounds__(NT) void fp4_rebase(const uint8_t *__restrict__ pac
 
 // ---------------------------------------------------------------- fused amax
 
+// A whole layer in one launch is bound by HBM; one expert's tensor (a few MB, a launch of its own in a loader's loop) by the
+// arithmetic of the two or three waves a SIMD gets, since nothing else covers it: what was 63 vector operations per 8 elements
+// is 38 with one conversion for the maximum and the moved code table.  us a launch, back to back: 2048 x 7168 6.96 -> 5.85, 512 x
+// 1024 4.3 -> 3.8, 65536 x 7168 137.6 -> 135.3 (256 threads; 512 level with it, 1024 behind: 6.6 and 149).
+
 template <int MODE, bool WRITE_BF16, int NT>
 __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packed, const uint8_t *__restrict__ scale,
                                                 int64_t cols, int64_t supers_c, int64_t n_supers, int64_t per_xcd,
@@ -156,6 +201,7 @@ __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packe
 {
     constexpr int kRowsPerPass = NT / 32, kPasses = 128 / kRowsPerPass;
     __shared__ uint32_t lds[2][16];
+    asm volatile("" ::"s"(packed), "s"(scale));              // fetched with the other arguments, not behind the test below
     const int64_t super = xcd_remap(blockIdx.x, per_xcd);
     if (super >= n_supers) return;
     const int t = threadIdx.x;
@@ -177,18 +223,22 @@ __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packe
     // amax of |table(code)| * 2^(sb-127).  The product is exact in fp32 (and
     // in bf16) for scale bytes 2..252; any other byte sends the whole super
     // tile down the literal slow path.
-    uint32_t mbits = 0;
-    uint32_t edge = 0;
+    // The largest of a word's eight magnitude codes is the largest magnitude: folded in the top nibble of each half and then of
+    // the word (what lies below that nibble does not matter to the maximum), so one element of eight is converted.
+    float amax_lane = 0.0f;
+    uint32_t sb_min = 255u, sb_max = 0u;
 #pragma unroll
     for (int p = 0; p < kPasses; ++p) {
-        float v[8];
-        fp4_decode8(w[p], v);
-        float m = fmaxf(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))),
-                        fmaxf(fmaxf(fabsf(v[4]), fabsf(v[5])), fmaxf(fabsf(v[6]), fabsf(v[7]))));
-        uint32_t prod = f2u(m * u2f(sb[p] << 23));
-        mbits = prod > mbits ? prod : mbits;
-        edge |= (sb[p] < 2u || sb[p] > 252u) ? 1u : 0u;
+        const uint32_t x = w[p] & 0x77777777u;
+        uint32_t h = max_u16x2(max_u16x2(x, x << 4), max_u16x2(x << 8, x << 12));
+        const uint32_t h16 = h << 16;
+        h = h > h16 ? h : h16;
+        amax_lane = fmaxf(amax_lane, fp4_top(h) * u2f(sb[p] << 23));
+        sb_min = sb[p] < sb_min ? sb[p] : sb_min;
+        sb_max = sb[p] > sb_max ? sb[p] : sb_max;
     }
+    const uint32_t mbits = f2u(amax_lane);
+    const bool edge = sb_min < 2u || sb_max > 252u;
     // Every thread of the workgroup must take the same number of barriers, so both slow decisions
     // (edge scale bytes, tile scale outside the fast range) are made for the super tile as a whole -- by
     // every lane for both tiles, from one reduction: an edge byte travels as the key 0xFFFFFFFF (products
@@ -229,16 +279,31 @@ __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packe
         if (!g.active) return;
         // All 8 elements of a pass share one scale byte sb, so their codes are eight numbers per pass:
         //   magnitude 0 .5 1 1.5 2 3 4 6  ->  e4m3(0, t1/2, t1, t3, 2 t1, 2 t3, 4 t1, 4 t3),  t = c * 2^(sb-127).
-        // Four conversions build that table in two registers and byte permutes look the nibbles up: no
-        // decode, no multiply per element (a conversion costs about 3 plain VALU instructions, measured).
+        // Where t1 / 2 is a normal e4m3 number (scale bytes within 11 or so of the largest that counts), the table of the tile
+        // moved up by 8 per power of two is that table: two permutes and two additions.
+        const uint32_t c1b = f2u(c1), c3b = f2u(c3);
+        const int cf = (int)(c1b >> 23);
+        const int sb0 = 249 - cf;                                  // c1 * 2^(sb0 - 127) / 2 = 1.x * 2^-6
+        if (!WRITE_BF16 && !__any((int)sb_min < sb0)) {
+            const uint32_t to5 = (uint32_t)(122 - cf) << 23;       // c1, c3 at sb0
+            const CodeTable tab(u2f(c1b + to5), u2f(c3b + to5));
+#pragma unroll
+            for (int p = 0; p < kPasses; ++p) {
+                const int64_t r = g.row0 + p * kRowsPerPass;
+                uint32_t wp = w[p];
+                asm volatile("" : "+v"(wp));                   // keep the packed word, not values derived before the barrier
+                __builtin_nontemporal_store(tab.codes(wp, (int)sb[p] - sb0), (u32x2 *)(q + r * cols + (g.colb << 1)));
+            }
+            return;
+        }
+        // Otherwise four conversions build the table of each pass in two registers (a conversion costs about 3 plain VALU
+        // instructions, measured).
         // The factors are formed by adding to the exponent field.  c1 and c3 are normal here (exponent
         // field cf, c3's at most cf + 1), so t1/2 .. 4 t3 are normal floats for sb in [129 - cf, 378 - cf],
         // and clamping sb to that range changes no result: a non-zero block has 2^(sb-127) <= 2 amax,
         // i.e. sb <= 264 - cf, so above the range every element is zero (and zero maps to table entry 0);
         // below it every quotient is under 2^-120 in magnitude and becomes a signed zero with the clamped
         // factor as with the true one.
-        const uint32_t c1b = f2u(c1), c3b = f2u(c3);
-        const int cf = (int)(c1b >> 23);
         const int sb_lo = 129 - cf, sb_hi = 378 - cf;
         const uint32_t c1adj = c1b - (127u << 23), c3adj = c3b - (127u << 23);
 #pragma unroll
@@ -251,12 +316,7 @@ __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packe
             const uint32_t tab_hi = cvt4(u2f(t1 + (1u << 23)), u2f(t3 + (1u << 23)), u2f(t1 + (2u << 23)), u2f(t3 + (2u << 23)));
             uint32_t wp = w[p];
             asm volatile("" : "+v"(wp));                       // keep the packed word, not values derived before the barrier
-            // even elements sit in the low nibbles of the four bytes, odd elements in the high nibbles
-            uint32_t ce = __builtin_amdgcn_perm(tab_hi, tab_lo, wp & 0x07070707u);
-            uint32_t co = __builtin_amdgcn_perm(tab_hi, tab_lo, (wp >> 4) & 0x07070707u);
-            ce |= (wp & 0x08080808u) << 4;                     // signs (zero magnitudes carry none, see fp4_pos_zero)
-            co |= wp & 0x80808080u;
-            u32x2 out = {__builtin_amdgcn_perm(co, ce, 0x05010400u), __builtin_amdgcn_perm(co, ce, 0x07030602u)};
+            const u32x2 out = lookup8(wp, tab_lo, tab_hi);
             __builtin_nontemporal_store(out, (u32x2 *)(q + r * cols + (g.colb << 1)));
             if (WRITE_BF16) {
                 const float s = u2f(sb[p] << 23);            // sb in 2..252: a normal power of two
