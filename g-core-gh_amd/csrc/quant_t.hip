@@ -14,6 +14,11 @@
 // contiguous bytes of the transposed output) go to a 16 KB LDS tile [column][row], swizzled so that neither side has
 // bank conflicts, and leave from there as whole 128-byte lines, 16 bytes per lane (measured 5-13 % faster than letting
 // the 16 threads of 4 waves that share a line store 8 bytes each).  A block that is padding only loads nothing.
+//
+// With ROWS the same pass also writes the 1 x 128 quantisation of the rows (codes and scales as lp_quant_fp8_block with
+// LP_SCALE_POW2 writes them): the 16 lanes that cover a row of the tile hold one of its groups.  A training step needs both
+// of x and of dY: 16384 x 4096 bf16 60 us where the two kernels take 36 + 43 (134 MB read once instead of twice; what bounds
+// it is the arithmetic of two quantisations beside 4.5 TB/s of traffic).
 #include <stdlib.h>
 
 #include "lowp_device.h"
@@ -38,10 +43,45 @@ __device__ __forceinline__ int padded_blocks_of(int rows, int pad_rows)
     return (rows + pad_rows - 1) / pad_rows * (pad_rows >> 7);
 }
 
+// The power-of-two scale of a block whose largest |value| has the bits m; bf16 values without the division:
+// s = 2^ceil(log2(amax / 448)), amax = f * 2^k with 1 <= f < 2 and 448 = 1.75 * 2^8, so the exponent is k - 8, and one more
+// when f > 1.75.  (fl32(amax / 448) is a power of two only for f = 1.75: a bf16 f is no closer than 1 / 224 to it otherwise,
+// far beyond the rounding of the division.)  amax below the smallest normal counts as that, a zero block gets the scale 1.
 template <bool IS_BF16>
+__device__ __forceinline__ BlockScale block_scale(uint32_t m, bool special)
+{
+    if (IS_BF16 && !special) {
+        BlockScale bs;
+        const uint32_t ab = m < 0x00800000u ? 0x00800000u : m;
+        const int e = m == 0u ? 0 : (int)(ab >> 23) - 135 + ((ab & 0x7FFFFFu) > 0x600000u ? 1 : 0);
+        bs.stored = e < -126 ? u2f(1u << (e + 149)) : u2f((uint32_t)(e + 127) << 23);
+        bs.div = 1.0f; bs.recip = 1.0f; bs.exp2 = e; bs.fast = true;
+        return bs;
+    }
+    return derive_scale<LP_SCALE_POW2>(u2f(m > 0x7F800000u ? 0x7FC00000u : m), 0.0f, LP_ZERO_NONE);
+}
+
+// 8 finite values over the scale, as codes: |x| <= amax <= 448 * 2^e and x * 2^-e is exact, no quotient leaves the e4m3
+// range, nothing to clamp.  2^-e is no normal float at the ends of the range: rare, and exact either way.
+template <class F>
+__device__ __forceinline__ u32x2 codes8(F value, int exp2)
+{
+    float y[8];
+    if (exp2 < -126 || exp2 > 126) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[i] = ldexpf(value(i), -exp2);
+    } else {
+        const float f = u2f((uint32_t)(127 - exp2) << 23);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[i] = value(i) * f;
+    }
+    return u32x2{cvt4(y[0], y[1], y[2], y[3]), cvt4(y[4], y[5], y[6], y[7])};
+}
+
+template <bool IS_BF16, bool ROWS>
 __global__ __launch_bounds__(256) void quant_colwise_t(const void *__restrict__ x, int64_t cols, const int32_t *__restrict__ m_offsets,
                                                        int E, int pad_rows, uint8_t *__restrict__ qT, void *__restrict__ sT, int scale_dtype,
-                                                       int cols_fastest)
+                                                       int cols_fastest, uint8_t *__restrict__ q, void *__restrict__ s)
 {
     __shared__ u32x4 wave_max[4][16][2];                 // [wave][column chunk][8 columns as fp32-bit maxima, 4 + 4]
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -86,8 +126,8 @@ __global__ __launch_bounds__(256) void quant_colwise_t(const void *__restrict__ 
     // ---- loads: row rg * 8 + i, columns c0 + 8 cc .. + 7; rows past the expert's end repeat its last row and
     // are zeroed afterwards (no branch between the loads)
     // The loaded words stay as they are; bf16 pairs are unpacked where they are used (32 registers instead of 64 live
-    // across the barrier); with the other waves' maxima read one wave at a time below, a thread needs 69 registers and
-    // seven workgroups share a CU (96 and five with those reads unrolled, 123 and four with floats kept).
+    // across the barrier): a thread needs 74 registers (78 with ROWS) and
+    // six workgroups share a CU (123 registers and four with floats kept; 104 and four where the rows are unpacked at once).
     constexpr int W = IS_BF16 ? 4 : 8;
     uint32_t rw[8][W];
     {
@@ -116,6 +156,57 @@ __global__ __launch_bounds__(256) void quant_colwise_t(const void *__restrict__ 
         if (IS_BF16) return u2f((j & 1) ? rw[i][(j >> 1) & 3] & 0xFFFF0000u : rw[i][(j >> 1) & 3] << 16);
         return u2f(rw[i][j & (W - 1)]);
     };
+    // ---- the rows' own groups (row rg * 8 + i: the 16 lanes of a DPP row hold its 128 values)
+    uint32_t literal_rows = 0;                           // rows with inf or NaN: done at the end
+    if constexpr (ROWS) {
+        uint32_t rmax[8];
+        if constexpr (IS_BF16) {
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) {
+                // two rows' maxima share a word through the four exchanges
+                uint32_t a = 0, b = 0;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    a = pk_max_u16(a, rw[i][k] & 0x7FFF7FFFu);
+                    b = pk_max_u16(b, rw[i + 1][k] & 0x7FFF7FFFu);
+                }
+                uint32_t w = pk_max_u16(__builtin_amdgcn_perm(b, a, 0x05040100u), __builtin_amdgcn_perm(b, a, 0x07060302u));
+                w = pk_max_u16(w, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x128, 0xF, 0xF, false));
+                w = pk_max_u16(w, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x124, 0xF, 0xF, false));
+                w = pk_max_u16(w, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x122, 0xF, 0xF, false));
+                w = pk_max_u16(w, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x121, 0xF, 0xF, false));
+                rmax[i] = w << 16;
+                rmax[i + 1] = w & 0xFFFF0000u;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                uint32_t a = 0;
+#pragma unroll
+                for (int k = 0; k < W; ++k) {
+                    const uint32_t b = rw[i][k] & 0x7FFFFFFFu;
+                    a = b > a ? b : a;
+                }
+                rmax[i] = row16_max_u32(a);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if (rg * 8 + i >= valid) continue;
+            const int64_t r = r0 + rg * 8 + i;
+            const bool special = rmax[i] >= 0x7F800000u;
+            const BlockScale bs = block_scale<IS_BF16>(rmax[i], special);
+            if (cc == 0) store_scale(s, scale_dtype, r * (cols >> 7) + (c0 >> 7), bs.stored);
+            if (special) literal_rows |= 1u << i;
+            else __builtin_nontemporal_store(codes8([&](int j) { return elem(i, j); }, bs.exp2), (u32x2 *)(q + r * cols + c0 + cc * 8));
+            // one row after the other, and nothing unpacked is kept for the columns: registers for the workgroups of a CU
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int k = 0; k < W; ++k) asm volatile("" : "+v"(rw[i][k]));
+    }
     // ---- column maxima of |x| as integers on the sign-cleared bits (inf / NaN sort above every finite value).
     // The kernel is bound by its arithmetic, not by memory (with loads and stores taken out it ran in three quarters
     // of its time), so bf16 maxima are taken on the packed words, two columns per instruction (16-bit integer max).
@@ -187,43 +278,19 @@ __global__ __launch_bounds__(256) void quant_colwise_t(const void *__restrict__ 
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const bool special = m[j] >= 0x7F800000u;        // inf or NaN in the block: literal arithmetic
-        const float amax = u2f(m[j] > 0x7F800000u ? 0x7FC00000u : m[j]);
-        BlockScale bs;
-        if (IS_BF16 && !special) {
-            // s = 2^ceil(log2(amax / 448)) without the division: amax = f * 2^k with 1 <= f < 2 and 448 = 1.75 * 2^8, so the
-            // exponent is k - 8, and one more when f > 1.75.  (fl32(amax / 448) is a power of two only for f = 1.75: a bf16 f
-            // is no closer than 1 / 224 to it otherwise, far beyond the rounding of the division.)  amax below the
-            // smallest normal counts as that, a zero block gets the scale 1.
-            const uint32_t ab = m[j] < 0x00800000u ? 0x00800000u : m[j];
-            const int e = m[j] == 0u ? 0 : (int)(ab >> 23) - 135 + ((ab & 0x7FFFFFu) > 0x600000u ? 1 : 0);
-            bs.stored = e < -126 ? u2f(1u << (e + 149)) : u2f((uint32_t)(e + 127) << 23);
-            bs.div = 1.0f; bs.recip = 1.0f; bs.exp2 = e; bs.fast = true;
-        } else {
-            bs = derive_scale<LP_SCALE_POW2>(amax, 0.0f, LP_ZERO_NONE);
-        }
+        const BlockScale bs = block_scale<IS_BF16>(m[j], special);
         const int64_t c = c0 + cc * 8 + j;
         if (rg == 0) store_scale(sT, scale_dtype, cols * pb + c * nblk + lb, bs.stored);
-        uint32_t lo, hi;
+        uint32_t lo = 0, hi = 0;
         if (special) {
-            lo = hi = 0;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 lo |= (uint32_t)quant_slow<LP_SCALE_POW2>(elem(i, j), bs) << (8 * i);
                 hi |= (uint32_t)quant_slow<LP_SCALE_POW2>(elem(4 + i, j), bs) << (8 * i);
             }
         } else {
-            // |x| <= amax <= 448 * 2^e and x * 2^-e is exact: no quotient leaves the e4m3 range, nothing to clamp
-            float y[8];
-            if (bs.exp2 < -126 || bs.exp2 > 126) {                       // 2^-e is not a normal float: rare, and exact either way
-#pragma unroll
-                for (int i = 0; i < 8; ++i) y[i] = ldexpf(elem(i, j), -bs.exp2);
-            } else {
-                const float f = u2f((uint32_t)(127 - bs.exp2) << 23);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) y[i] = elem(i, j) * f;
-            }
-            lo = cvt4(y[0], y[1], y[2], y[3]);
-            hi = cvt4(y[4], y[5], y[6], y[7]);
+            const u32x2 c8 = codes8([&](int i) { return elem(i, j); }, bs.exp2);
+            lo = c8.x; hi = c8.y;
         }
         turned[(cc * 8 + j) * 16 + (rg ^ cc)] = u32x2{lo, hi};
     }
@@ -236,6 +303,51 @@ __global__ __launch_bounds__(256) void quant_colwise_t(const void *__restrict__ 
         const u32x4 out = (sw & 1) ? u32x4{raw[2], raw[3], raw[0], raw[1]} : raw;
         *(u32x4 *)(qT + base + (c0 + col) * P + (int64_t)lb * 128 + pair * 16) = out;
     }
+    if constexpr (ROWS) {
+#pragma unroll 1
+        for (; literal_rows; literal_rows &= literal_rows - 1) {
+            const int64_t off = (r0 + rg * 8 + __builtin_ctz(literal_rows)) * cols + c0 + cc * 8;
+            uint32_t any = 0;                            // the group's maximum again: inf divides by its own scale, NaN by NaN
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t a = IS_BF16 ? (uint32_t)(((const uint16_t *)x)[off + j] & 0x7FFFu) << 16 : ((const uint32_t *)x)[off + j] & 0x7FFFFFFFu;
+                any = a > any ? a : any;
+            }
+            quant_slow_span<LP_SCALE_POW2>(x, IS_BF16, off, 8, block_scale<IS_BF16>(row16_max_u32(any), true).stored, q);
+        }
+    }
+}
+
+}  // namespace
+
+namespace {
+
+// q, s: the rows' own quantisation too, or null
+int colwise(const char *name, const void *x, int x_dtype, int64_t rows, int64_t cols, const int32_t *m_offsets, int E, int64_t padded_blocks,
+            int pad_rows, void *qT, void *sT, void *q, void *s, int scale_dtype, hipStream_t st)
+{
+    LP_REQUIRE(pad_rows == 128 || pad_rows == 256 || pad_rows == 512 || pad_rows == LP_PAD_MIXED,
+               "%s: pad_rows must be 128, 256, 512 or LP_PAD_MIXED", name);
+    LP_REQUIRE(x_dtype == LP_BF16 || x_dtype == LP_F32, "%s: x_dtype must be LP_BF16 or LP_F32", name);
+    LP_REQUIRE(scale_dtype == LP_F32 || scale_dtype == LP_E8M0, "%s: scale_dtype must be LP_F32 or LP_E8M0", name);
+    LP_REQUIRE(rows >= 0 && cols >= 0 && E >= 0 && padded_blocks >= 0, "%s: bad shape", name);
+    LP_REQUIRE(cols % 128 == 0, "%s: cols (%lld) must be a multiple of 128", name, (long long)cols);
+    if (cols == 0 || padded_blocks == 0 || E == 0) return LP_OK;
+    LP_REQUIRE(x && m_offsets && qT && sT, "%s: null pointer", name);
+    LP_REQUIRE((uintptr_t)qT % 16 == 0, "%s: qT must be 16-byte aligned", name);
+    LP_REQUIRE(padded_blocks <= 0x7FFFFFFF && cols / 128 <= 65535, "%s: problem too large", name);
+    // Workgroups that run together should read whole rows between them: the column blocks of one row block are
+    // numbered consecutively (217 -> 187 us on a [65536, 4096] gradient against row blocks first, whose concurrent
+    // reads were 256-byte pieces 8 KB apart).  The grid's second dimension holds 65535 at most.
+    static const int order_env = getenv("LP_COLWISE_ROWS_FIRST") ? atoi(getenv("LP_COLWISE_ROWS_FIRST")) : 0;
+    const int cols_fastest = !order_env && padded_blocks <= 65535 ? 1 : 0;
+    const dim3 grid = cols_fastest ? dim3((unsigned)(cols / 128), (unsigned)padded_blocks) : dim3((unsigned)padded_blocks, (unsigned)(cols / 128));
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, x, cols, m_offsets, E, pad_rows, (uint8_t *)qT, sT, scale_dtype, cols_fastest,
+                           (uint8_t *)q, s);
+    };
+    if (x_dtype == LP_BF16) q ? go(quant_colwise_t<true, true>) : go(quant_colwise_t<true, false>);
+    else q ? go(quant_colwise_t<false, true>) : go(quant_colwise_t<false, false>);
+    return check_launch(name);
 }
 
 }  // namespace
@@ -243,27 +355,19 @@ __global__ __launch_bounds__(256) void quant_colwise_t(const void *__restrict__ 
 extern "C" int lp_quant_fp8_colwise_t(const void *x, int x_dtype, int64_t rows, int64_t cols, const int32_t *m_offsets, int E,
                                       int64_t padded_blocks, int pad_rows, void *qT, void *sT, int scale_dtype, lp_stream_t stream)
 {
-    LP_REQUIRE(pad_rows == 128 || pad_rows == 256 || pad_rows == 512 || pad_rows == LP_PAD_MIXED,
-               "lp_quant_fp8_colwise_t: pad_rows must be 128, 256, 512 or LP_PAD_MIXED");
-    LP_REQUIRE(x_dtype == LP_BF16 || x_dtype == LP_F32, "lp_quant_fp8_colwise_t: x_dtype must be LP_BF16 or LP_F32");
-    LP_REQUIRE(scale_dtype == LP_F32 || scale_dtype == LP_E8M0, "lp_quant_fp8_colwise_t: scale_dtype must be LP_F32 or LP_E8M0");
-    LP_REQUIRE(rows >= 0 && cols >= 0 && E >= 0 && padded_blocks >= 0, "lp_quant_fp8_colwise_t: bad shape");
-    LP_REQUIRE(cols % 128 == 0, "lp_quant_fp8_colwise_t: cols (%lld) must be a multiple of 128", (long long)cols);
-    if (cols == 0 || padded_blocks == 0 || E == 0) return LP_OK;
-    LP_REQUIRE(x && m_offsets && qT && sT, "lp_quant_fp8_colwise_t: null pointer");
-    LP_REQUIRE((uintptr_t)qT % 16 == 0, "lp_quant_fp8_colwise_t: qT must be 16-byte aligned");
-    LP_REQUIRE(padded_blocks <= 0x7FFFFFFF && cols / 128 <= 65535, "lp_quant_fp8_colwise_t: problem too large");
-    // Workgroups that run together should read whole rows between them: the column blocks of one row block are
-    // numbered consecutively (217 -> 187 us on a [65536, 4096] gradient against row blocks first, whose concurrent
-    // reads were 256-byte pieces 8 KB apart).  The grid's second dimension holds 65535 at most.
-    static const int order_env = getenv("LP_COLWISE_ROWS_FIRST") ? atoi(getenv("LP_COLWISE_ROWS_FIRST")) : 0;
-    const int cols_fastest = !order_env && padded_blocks <= 65535 ? 1 : 0;
-    const dim3 grid = cols_fastest ? dim3((unsigned)(cols / 128), (unsigned)padded_blocks) : dim3((unsigned)padded_blocks, (unsigned)(cols / 128));
-    if (x_dtype == LP_BF16)
-        hipLaunchKernelGGL(quant_colwise_t<true>, grid, dim3(256), 0, (hipStream_t)stream, x, cols, m_offsets, E, pad_rows, (uint8_t *)qT, sT,
-                           scale_dtype, cols_fastest);
-    else
-        hipLaunchKernelGGL(quant_colwise_t<false>, grid, dim3(256), 0, (hipStream_t)stream, x, cols, m_offsets, E, pad_rows, (uint8_t *)qT, sT,
-                           scale_dtype, cols_fastest);
-    return check_launch("lp_quant_fp8_colwise_t");
+    return colwise("lp_quant_fp8_colwise_t", x, x_dtype, rows, cols, m_offsets, E, padded_blocks, pad_rows, qT, sT, nullptr, nullptr, scale_dtype,
+                   (hipStream_t)stream);
+}
+
+extern "C" int lp_quant_fp8_row_colwise_t(const void *x, int x_dtype, int64_t rows, int64_t cols, const int32_t *m_offsets, int E,
+                                          int64_t padded_blocks, int pad_rows, void *q, void *s, void *qT, void *sT, int scale_dtype,
+                                          lp_stream_t stream)
+{
+    if (rows > 0 && cols > 0 && padded_blocks > 0 && E > 0) {
+        LP_REQUIRE(q && s, "lp_quant_fp8_row_colwise_t: null pointer");
+        LP_REQUIRE((uintptr_t)q % 8 == 0, "lp_quant_fp8_row_colwise_t: q must be 8-byte aligned");
+        LP_REQUIRE((uintptr_t)x % 16 == 0, "lp_quant_fp8_row_colwise_t: x must be 16-byte aligned");
+    }
+    return colwise("lp_quant_fp8_row_colwise_t", x, x_dtype, rows, cols, m_offsets, E, padded_blocks, pad_rows, qT, sT, q, s, scale_dtype,
+                   (hipStream_t)stream);
 }

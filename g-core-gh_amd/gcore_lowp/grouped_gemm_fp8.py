@@ -188,6 +188,25 @@ def quant_fp8_colwise_t(x: torch.Tensor, m_offsets: torch.Tensor, m_splits, pad_
     return q, s, nblk
 
 
+def _quant_rows_and_columns(x: torch.Tensor, offs: torch.Tensor, m_splits, pad_rows: int):
+    """Both quantisations a training step needs of x (or of dY), whose rows all belong to an expert, from one read of it: ->
+    (codes [rows, cols], e8m0 scales [rows, cols / 128], then quant_fp8_colwise_t's three)."""
+    rows, cols = x.shape
+    if not (x.is_contiguous() and x.dtype in (torch.bfloat16, torch.float32) and x.data_ptr() % 16 == 0 and cols % 128 == 0):
+        return *_quant_pow2(x, (1, 128)), *quant_fp8_colwise_t(x, offs, m_splits, pad_rows)
+    nblk = [padded_blocks(m, pad_rows) for m in m_splits]
+    total = sum(nblk)
+    q = torch.empty((rows, cols), dtype=ops.E4M3, device=x.device)
+    s = torch.empty((rows, cols // 128), dtype=ops.E8M0, device=x.device)
+    qt = torch.empty(cols * total * 128, dtype=torch.uint8, device=x.device)
+    st = torch.empty(cols * total, dtype=ops.E8M0, device=x.device)
+    with torch.cuda.device(x.device):
+        A.check(A.lib().lp_quant_fp8_row_colwise_t(x.data_ptr(), A.BF16 if x.dtype == torch.bfloat16 else A.F32, rows, cols,
+                                                   offs.data_ptr(), len(nblk), total, pad_rows, q.data_ptr(), s.data_ptr(),
+                                                   qt.data_ptr(), st.data_ptr(), A.E8M0, A.stream_ptr()))
+    return q, s, qt, st, nblk
+
+
 def gemm_fp8_rowscale(aq, a_s, bq, b_s, M, N, K, out: torch.Tensor) -> torch.Tensor:
     """out[M, N] = sum over K blocks of (aq . bq^T) * a_s[m, kb] * b_s[n, kb]: e8m0 scales per row and 128 of K on
     both operands; aq / bq are flat uint8 views of [M, K] / [N, K]."""
@@ -275,16 +294,17 @@ class _GroupedGemmFp8(torch.autograd.Function):
     def forward(ctx, inp, weight, wq, ws, m_splits, out_dtype):
         E, n_out, k_in = wq.shape
         x = inp.reshape(-1, k_in)
-        xq, xs = _quant_pow2(x, (1, 128))
-        offs = _offsets(m_splits, x.device)
-        out = grouped_gemm_fp8(xq, xs, wq, ws, offs, out_dtype=out_dtype, total_rows=sum(m_splits))
         ctx.need_wgrad = weight is not None and weight.requires_grad
         ctx.need_dgrad = inp.requires_grad
+        offs = _offsets(m_splits, x.device)
         saved = [wq.view(torch.uint8), ws.view(torch.uint8), offs]
         if ctx.need_wgrad:
             ctx.pad_rows = 128
-            xtq, xts, _ = quant_fp8_colwise_t(x.detach(), offs, m_splits, ctx.pad_rows)
+            xq, xs, xtq, xts, _ = _quant_rows_and_columns(x.detach(), offs, m_splits, ctx.pad_rows)
             saved += [xtq, xts.view(torch.uint8)]
+        else:
+            xq, xs = _quant_pow2(x, (1, 128))
+        out = grouped_gemm_fp8(xq, xs, wq, ws, offs, out_dtype=out_dtype, total_rows=sum(m_splits))
         ctx.save_for_backward(*saved)
         ctx.m_splits, ctx.inp_shape, ctx.dims, ctx.out_dtype = m_splits, inp.shape, (E, n_out, k_in), out_dtype
         return out.view(*inp.shape[:-1], n_out)
@@ -295,13 +315,17 @@ class _GroupedGemmFp8(torch.autograd.Function):
         wq, ws, offs = ctx.saved_tensors[:3]
         dy = grad_output.contiguous().view(-1, n_out)
         dgrad = wgrad = None
-        if ctx.need_dgrad:
+        if ctx.need_wgrad and ctx.need_dgrad:
+            dyq, dys, dtq, dts, nblk = _quant_rows_and_columns(dy, offs, ctx.m_splits, ctx.pad_rows)       # padded like X^T in the forward
+        elif ctx.need_wgrad:
+            dtq, dts, nblk = quant_fp8_colwise_t(dy, offs, ctx.m_splits, ctx.pad_rows)
+        elif ctx.need_dgrad:
             dyq, dys = _quant_pow2(dy, (1, 128))
+        if ctx.need_dgrad:
             dgrad = grouped_gemm_fp8_nn(dyq, dys, wq.view(ops.E4M3), ws.view(ops.E8M0), offs, out_dtype=ctx.out_dtype,
                                         total_rows=sum(ctx.m_splits)).view(ctx.inp_shape)
         if ctx.need_wgrad:
             xtq, xts = ctx.saved_tensors[3:5]
-            dtq, dts, nblk = quant_fp8_colwise_t(dy, offs, ctx.m_splits, ctx.pad_rows)       # padded like X^T in the forward
             wgrad = torch.empty((E, n_out, k_in), dtype=ctx.out_dtype, device=dy.device)
             gemm_fp8_rowscale_grouped(dtq, dts.view(torch.uint8), xtq, xts, nblk, n_out, k_in, wgrad)
         return dgrad, wgrad, None, None, None, None

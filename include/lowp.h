@@ -333,6 +333,16 @@ int lp_quant_fp8_colwise_t(const void *x, int x_dtype, int64_t rows, int64_t col
                            lp_stream_t stream);
 
 /*
+ * Both quantisations of an expert-grouped tensor from one read of it: qT, sT as lp_quant_fp8_colwise_t writes them, and q
+ * [rows, cols], s [rows, cols / 128] as lp_quant_fp8_block writes them for 1 x 128 groups with LP_SCALE_POW2 (rows that
+ * belong to no expert are left as they are).  x 16-byte aligned, q 8-byte aligned; one scale_dtype for both.  Replaces
+ * tex.split_quantize with both usages set (gpatch_v4/models/deepseek_v4/fp8.py:231,292-294).
+ */
+int lp_quant_fp8_row_colwise_t(const void *x, int x_dtype, int64_t rows, int64_t cols, const int32_t *m_offsets,
+                               int E, int64_t padded_blocks, int pad_rows, void *q, void *s, void *qT, void *sT,
+                               int scale_dtype, lp_stream_t stream);
+
+/*
  * n int32 words of HOST memory at src -> device memory at dst, ordered on the stream like a kernel: the words are taken
  * before the call returns (src may be reused at once) and neither the host nor the stream waits, as a copy from pageable
  * memory would.  For the small tables the grouped entries read: row offsets, problem lists.  The reference hands the row
