@@ -1,14 +1,18 @@
-// Row-scaled FP8 GEMM for problems of one or two K blocks: the weight gradients dW_e = dY_e^T X_e of experts with at most
-// 256 rows (gpatch_v4/models/deepseek_v4/fp8.py:325-341), which are most experts of a routed batch.  Such a problem is a
-// write of M x N results more than a GEMM: a 128 x 128 tile reads 32 KB (or 64 KB) and writes 32 KB of bf16.  No K loop
-// and no pipeline inside a workgroup: it requests its whole operand tiles (LDS-direct loads, 8 rows x 128 bytes per
-// request), waits once, multiplies with the scale bytes of both operands applied by the matrix cores, stages the results
-// through the same LDS and stores whole 128-byte lines.  What overlaps one workgroup's wait and stores is the other
-// workgroups of its CU: 36 KB of LDS and 64 accumulators per lane let four of them (one K block) or two (two blocks)
-// share it.  LDS rows and chunks are laid out as in gemm_fp8_big.hip (the 16 lanes of a fragment read cover whole
-// 256-byte lines).
+// Row-scaled FP8 GEMM for problems of one K block (gemm_rowscale_small) and of two (gemm_rowscale_strip): the weight
+// gradients dW_e = dY_e^T X_e of experts with at most 256 rows (gpatch_v4/models/deepseek_v4/fp8.py:325-341), which are most
+// experts of a routed batch.  Such a problem is a write of M x N results more than a GEMM: a 128 x 128 tile reads 32 KB (or
+// 64 KB) and writes 32 KB of bf16.  With one K block there is no pipeline inside a workgroup: it requests its whole operand
+// tiles (LDS-direct loads, 8 rows x 128 bytes per request), waits once, multiplies with the scale bytes of both operands
+// applied by the matrix cores, stages the results through the same LDS and stores whole 128-byte lines.  What overlaps one
+// workgroup's wait and stores is the other workgroups of its CU: 36 KB of LDS and 64 accumulators per lane let four of them
+// share it.  LDS rows and chunks are laid out as in gemm_fp8_big.hip (the 16 lanes of a fragment read cover whole 256-byte
+// lines).
+//
+// Two K blocks leave room for two workgroups only, too few to cover each other's wait for 64 KB: that way 15 problems of
+// 4096 x 4096 took 159 us, 3.2 TB/s of results, where the strips take 114 (bound by their stores: 40 problems of 7168 x 4096
+// reach 5.4 TB/s).  gemm_rowscale_strip keeps a workgroup's activation rows in registers and walks a strip of weight columns, the
+// next tile's operand on its way while this one is multiplied and stored.
 #include "gemm_common.h"
-#include <utility>
 
 using namespace lowp;
 
@@ -30,31 +34,26 @@ __device__ __forceinline__ int swz(int r, int chunk) { return chunk ^ (r & 7); }
 // lanes to a row, so that a store instruction writes 8 whole rows of 128 bytes.
 constexpr int kPitch = 64 * 2 + 16, kWaveStage = 64 * kPitch;
 
-// Tried: two to four K blocks passing one after the other through one block's worth of LDS (four workgroups per CU whatever
-// the K): the weight gradient of config 4's layer 4.31 ms against 4.21 with both blocks requested at once, and four-block
-// problems 4.74 against 4.21 on the hand-scheduled loop.
-template <int KBS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KBS == 1 ? 4 : 2, KBS == 1 ? 4 : 2))) void gemm_rowscale_small(const uint8_t *__restrict__ Aq, const uint8_t *__restrict__ As,
-                                                           const uint8_t *__restrict__ Bq, const uint8_t *__restrict__ Bs,
-                                                           const int32_t *__restrict__ groups, int64_t M, int64_t N, int64_t tiles_m,
-                                                           int64_t tiles_n, int64_t per_group, void *__restrict__ C, int out_dtype)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void gemm_rowscale_small(
+    const uint8_t *__restrict__ Aq, const uint8_t *__restrict__ As, const uint8_t *__restrict__ Bq, const uint8_t *__restrict__ Bs,
+    const int32_t *__restrict__ groups, int64_t M, int64_t N, int64_t tiles_m, int64_t tiles_n, int64_t per_group, void *__restrict__ C,
+    int out_dtype)
 {
-    constexpr int TILE = 128 * 128, OPER = KBS * TILE, PITCH = KBS * 128;
-    constexpr int LDS_BYTES = 2 * OPER > 4 * kWaveStage ? 2 * OPER : 4 * kWaveStage;
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[LDS_BYTES];
+    constexpr int TILE = 128 * 128, PITCH = 128;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * TILE > 4 * kWaveStage ? 2 * TILE : 4 * kWaveStage];
     const int64_t g = blockIdx.x / per_group, local = blockIdx.x - g * per_group;
     int64_t tm, tn;
     if (!gemm::tile_coords(local, tiles_m, tiles_n, tm, tn)) return;
-    // no table: one problem of KBS blocks
-    const int64_t slot = groups ? groups[4 * g] : 0, kb = groups ? groups[4 * g + 1] : KBS, before = groups ? groups[4 * g + 2] : 0;
+    // no table: one problem
+    const int64_t slot = groups ? groups[4 * g] : 0, kb = groups ? groups[4 * g + 1] : 1, before = groups ? groups[4 * g + 2] : 0;
     // an entry of another size (or one that breaks the caller's promises) is not this launch's: nothing is written
-    if (kb != KBS || slot < 0 || before < 0) return;
+    if (kb != 1 || slot < 0 || before < 0) return;
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave >> 1, wn = wave & 1, l16 = lane & 15, lq = lane >> 4;
     const int64_t m0 = tm * 128, n0 = tn * 128;
     const uint8_t *a_g = Aq + M * 128 * before + m0 * PITCH, *b_g = Bq + N * 128 * before + n0 * PITCH;
-    const uint8_t *as_g = As + M * before + m0 * KBS, *bs_g = Bs + N * before + n0 * KBS;
+    const uint8_t *as_g = As + M * before + m0, *bs_g = Bs + N * before + n0;
 
     // requests: group q of 8 LDS rows of an operand block is wave q % 4's; lane -> row lane / 8 of the group, slot lane % 8
     const int ld_row = lane >> 3, ld_slot = lane & 7;
@@ -64,23 +63,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KBS == 1 ? 
         const int row = tile_row(8 * (wave + 4 * i) + ld_row);
         off[i] = (uint32_t)(row * PITCH + swz(row, ld_slot) * 16);
     }
-    auto request = [&](int j, int buf) {                 // K block j of both operands into block buffer buf
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int q = wave + 4 * i;
-            __builtin_amdgcn_global_load_lds(GLB_PTR(a_g + off[i] + j * 128), LDS_PTR(smem + buf * TILE + q * 1024), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(GLB_PTR(b_g + off[i] + j * 128), LDS_PTR(smem + OPER + buf * TILE + q * 1024), 16, 0, 0);
-        }
-    };
-#pragma unroll
-    for (int j = 0; j < KBS; ++j) request(j, j);
-    // scale bytes of the lane's rows: byte j of the register = K block j (picked by the instruction's op_sel)
-    int sa[4], sb[4];
+    for (int i = 0; i < 4; ++i) {
+        const int q = wave + 4 * i;
+        __builtin_amdgcn_global_load_lds(GLB_PTR(a_g + off[i]), LDS_PTR(smem + q * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds(GLB_PTR(b_g + off[i]), LDS_PTR(smem + TILE + q * 1024), 16, 0, 0);
+    }
+    int sa[4], sb[4];                                    // scale bytes of the lane's rows
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-        const int ra = wm * 64 + b * 16 + l16, rb = wn * 64 + b * 16 + l16;
-        if (KBS == 1) { sa[b] = as_g[ra]; sb[b] = bs_g[rb]; }
-        else { sa[b] = *(const uint16_t *)(as_g + 2 * ra); sb[b] = *(const uint16_t *)(bs_g + 2 * rb); }
+        sa[b] = as_g[wm * 64 + b * 16 + l16];
+        sb[b] = bs_g[wn * 64 + b * 16 + l16];
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -95,21 +88,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KBS == 1 ? 
         const u32x4 x1 = *(const u32x4 *)(base + lds_row(row) * 128 + swz(row, 2 * lq + 1) * 16);
         return i32x8{(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w, (int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
     };
-    auto block = [&](auto jc) {
-        constexpr int j = decltype(jc)::value, buf = j;
-        // fragments are read where they are used (the activation side four times over): registers for four workgroups per CU
+    // fragments are read where they are used (the activation side four times over): registers for four workgroups per CU
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-            const i32x8 bf = frag(smem + OPER + buf * TILE, wn * 64 + nb * 16 + l16);
+    for (int nb = 0; nb < 4; ++nb) {
+        const i32x8 bf = frag(smem + TILE, wn * 64 + nb * 16 + l16);
 #pragma unroll
-            for (int mb = 0; mb < 4; ++mb) {
-                const i32x8 af = frag(smem + buf * TILE, wm * 64 + mb * 16 + l16);
-                acc[mb][nb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf, af, acc[mb][nb], 0, 0, j, sb[nb], j, sa[mb]);
-            }
+        for (int mb = 0; mb < 4; ++mb) {
+            const i32x8 af = frag(smem, wm * 64 + mb * 16 + l16);
+            acc[mb][nb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf, af, acc[mb][nb], 0, 0, 0, sb[nb], 0, sa[mb]);
         }
-    };
-    block(std::integral_constant<int, 0>{});
-    if constexpr (KBS == 2) block(std::integral_constant<int, 1>{});
+    }
 
     const int64_t row0 = m0 + wm * 64, col0 = n0 + wn * 64;
     char *c_g = (char *)C + slot * M * N * (out_dtype == LP_BF16 ? 2 : 4);
@@ -141,6 +129,139 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KBS == 1 ? 
         }
 }
 
+// Problems of two K blocks: a 128-row panel of A against `strip` 128-column tiles of B, one after the other.  The panel's
+// fragments stay in registers (64 of them); B tiles go through two 32 KB halves of LDS, tile i + 1 requested before tile i is
+// multiplied.  When a tile's fragments have been read its half takes the bf16 results (64 x 64 per wave, 128-byte rows,
+// 16-byte chunks swizzled so that neither side has bank conflicts) on their way to whole-line stores.  The wait for the next
+// tile stands in front of those stores (loads and stores share the request counter, and stores acknowledge late).
+constexpr int kStripTile = 128 * 128, kStripHalf = 2 * kStripTile;
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_rowscale_strip(
+    const uint8_t *__restrict__ Aq, const uint8_t *__restrict__ As, const uint8_t *__restrict__ Bq, const uint8_t *__restrict__ Bs,
+    const int32_t *__restrict__ groups, int G, int64_t M, int64_t N, int tiles_m, int tiles_n, int strip, void *__restrict__ C, int out_dtype)
+{
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * kStripHalf];
+    // an XCD (workgroup id modulo 8) is handed whole units of 8 row panels x one strip, which share operands in its L2
+    const int strips = (tiles_n + strip - 1) / strip, parts = (tiles_m + 7) / 8;
+    const int in_xcd = blockIdx.x >> 3, unit = (in_xcd >> 3) * 8 + (blockIdx.x & 7);
+    const int g = unit / (strips * parts), rest = unit - g * (strips * parts);
+    const int first_n = (rest / parts) * strip, tm = (rest % parts) * 8 + (in_xcd & 7);
+    if (g >= G || tm >= tiles_m) return;
+    const int count = tiles_n - first_n < strip ? tiles_n - first_n : strip;
+    // no table: one problem.  An entry of another size (or one that breaks the caller's promises) is not this launch's:
+    // nothing is written
+    const int64_t slot = groups ? groups[4 * g] : 0, kb = groups ? groups[4 * g + 1] : 2, before = groups ? groups[4 * g + 2] : 0;
+    if (kb != 2 || slot < 0 || before < 0) return;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wave >> 1, wn = wave & 1, l16 = lane & 15, lq = lane >> 4;
+    const int64_t m0 = (int64_t)tm * 128, n0 = (int64_t)first_n * 128;
+    const uint8_t *a_g = Aq + M * 128 * before + m0 * 256, *b_g = Bq + N * 128 * before + n0 * 256;
+    const uint8_t *as_g = As + M * before + m0 * 2, *bs_g = Bs + N * before + n0 * 2;
+
+    // requests as in gemm_rowscale_small: group q of 8 LDS rows of a K block is wave q % 4's
+    uint32_t off[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = tile_row(8 * (wave + 4 * i) + (lane >> 3));
+        off[i] = (uint32_t)(row * 256 + swz(row, lane & 7) * 16);
+    }
+    const uint32_t lds0 = (uint32_t)(uintptr_t)LDS_PTR(smem) + (uint32_t)wave * 1024;
+    // (not the builtin: behind it the compiler waits for the request in front of every LDS read)
+    auto request = [&](const uint8_t *tile, int half) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                             :: "s"(lds0 + (uint32_t)(half * kStripHalf + j * kStripTile + i * 4096)), "v"(off[i]), "s"(tile + j * 128)
+                             : "memory", "m0");
+    };
+    auto frag = [&](const uint8_t *base, int row) -> i32x8 {
+        const u32x4 x0 = *(const u32x4 *)(base + lds_row(row) * 128 + swz(row, 2 * lq) * 16);
+        const u32x4 x1 = *(const u32x4 *)(base + lds_row(row) * 128 + swz(row, 2 * lq + 1) * 16);
+        return i32x8{(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w, (int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
+    };
+    request(a_g, 1);
+    request(b_g, 0);
+    // scale bytes of the lane's rows: byte j of the register = K block j (picked by the instruction's op_sel)
+    int sa[4], sb[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        sa[b] = *(const uint16_t *)(as_g + 2 * (wm * 64 + b * 16 + l16));
+        sb[b] = *(const uint16_t *)(bs_g + 2 * (wn * 64 + b * 16 + l16));
+    }
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" : "+v"(sa[0]), "+v"(sa[1]), "+v"(sa[2]), "+v"(sa[3]), "+v"(sb[0]), "+v"(sb[1]), "+v"(sb[2]), "+v"(sb[3]) :: "memory");
+    i32x8 af[2][4];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb) af[j][mb] = frag(smem + kStripHalf + j * kStripTile, wm * 64 + mb * 16 + l16);
+    const int64_t esz = out_dtype == LP_BF16 ? 2 : 4;
+    char *c_g = (char *)C + (slot * M * N + (m0 + wm * 64) * N + n0 + wn * 64) * esz;
+    for (int i = 0; i < count; ++i) {
+        // every wave is through with the other half (the A panel, or the results of the tile before), and this tile has landed
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        uint8_t *half = smem + (i & 1) * kStripHalf;
+        const bool more = i + 1 < count;
+        int sn[4] = {0, 0, 0, 0};
+        if (more) {
+            request(b_g + (int64_t)(i + 1) * (128 * 256), (i + 1) & 1);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) sn[b] = *(const uint16_t *)(bs_g + (int64_t)(i + 1) * 256 + 2 * (wn * 64 + b * 16 + l16));
+        }
+        f32x4v acc[4][4];
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) acc[mb][nb] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) {
+            const i32x8 b0 = frag(half, wn * 64 + nb * 16 + l16), b1 = frag(half + kStripTile, wn * 64 + nb * 16 + l16);
+#pragma unroll
+            for (int mb = 0; mb < 4; ++mb)
+                acc[mb][nb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b0, af[0][mb], acc[mb][nb], 0, 0, 0, sb[nb], 0, sa[mb]);
+#pragma unroll
+            for (int mb = 0; mb < 4; ++mb)
+                acc[mb][nb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b1, af[1][mb], acc[mb][nb], 0, 0, 1, sb[nb], 1, sa[mb]);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // every wave has read this tile's fragments
+        if (out_dtype == LP_BF16) {
+            uint8_t *stage = half + wave * (64 * 128);
+#pragma unroll
+            for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+                for (int nb = 0; nb < 4; ++nb) {
+                    const u32x2 o = {pack_bf16(acc[mb][nb].x, acc[mb][nb].y), pack_bf16(acc[mb][nb].z, acc[mb][nb].w)};
+                    const int row = mb * 16 + l16, chunk = nb * 2 + (lq >> 1);
+                    *(u32x2 *)(stage + row * 128 + (chunk ^ ((row >> 1) & 7)) * 16 + (lq & 1) * 8) = o;
+                }
+        }
+        // the next tile has landed (and the stores of the tile before are done); a wave reads back only what it wrote
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : "+v"(sn[0]), "+v"(sn[1]), "+v"(sn[2]), "+v"(sn[3]) :: "memory");
+#pragma unroll
+        for (int b = 0; b < 4; ++b) sb[b] = sn[b];
+        char *c_t = c_g + (int64_t)i * 128 * esz;
+        if (out_dtype == LP_BF16) {
+            const uint8_t *stage = half + wave * (64 * 128);
+#pragma unroll
+            for (int p = 0; p < 8; ++p) {
+                const int row = p * 8 + (lane >> 3), chunk = lane & 7;
+                const u32x4 v = *(const u32x4 *)(stage + row * 128 + (chunk ^ ((row >> 1) & 7)) * 16);
+                __builtin_nontemporal_store(v, (u32x4 *)((uint16_t *)c_t + (int64_t)row * N + chunk * 8));
+            }
+        } else {
+#pragma unroll
+            for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+                for (int nb = 0; nb < 4; ++nb) {
+                    const u32x4 o = {f2u(acc[mb][nb].x), f2u(acc[mb][nb].y), f2u(acc[mb][nb].z), f2u(acc[mb][nb].w)};
+                    *(u32x4 *)((float *)c_t + (int64_t)(mb * 16 + l16) * N + nb * 16 + 4 * lq) = o;
+                }
+        }
+    }
+}
+
 }  // namespace
 
 namespace lowp {
@@ -152,15 +273,22 @@ int launch_rowscale_small(const void *Aq, const void *As, const void *Bq, const 
                           int64_t M, int64_t N, void *C, int out_dtype, hipStream_t st)
 {
     const int64_t tiles_m = M / 128, tiles_n = N / 128;
+    if (k_blocks == 2) {
+        // At most 8 tiles a strip, all strips alike: the panel's load and the first tile's wait spread over 8 tiles while a weight
+        // of 4096 columns still cuts into 4 (40 x 7168 x 4096, strips of 2 / 4 / 8 / 16 tiles: 535 / 476 / 433 / 471 us; 15 x 4096 x
+        // 4096: 117 / 122 / 114 / 128).
+        const int64_t per_row = (tiles_n + 7) / 8, strip = per_row ? (tiles_n + per_row - 1) / per_row : 1;
+        const int64_t units = G * ((tiles_n + strip - 1) / strip) * ((tiles_m + 7) / 8), wgs = (units + 7) / 8 * 64;
+        if (wgs > 0x7FFFFFFF || tiles_n > 0x7FFFFF || tiles_m > 0x7FFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_rowscale_grouped: problem too large");
+        hipLaunchKernelGGL(gemm_rowscale_strip, dim3((unsigned)wgs), dim3(256), 0, st, (const uint8_t *)Aq, (const uint8_t *)As, (const uint8_t *)Bq,
+                           (const uint8_t *)Bs, groups, G, M, N, (int)tiles_m, (int)tiles_n, (int)strip, C, out_dtype);
+        return check_launch("lp_gemm_fp8_rowscale_grouped(two K blocks)");
+    }
     const int64_t per_group = padded_grid(tiles_m, tiles_n), grid = per_group * G;
     if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_rowscale_grouped: problem too large");
-    auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), 0, st, (const uint8_t *)Aq, (const uint8_t *)As, (const uint8_t *)Bq,
-                           (const uint8_t *)Bs, groups, M, N, tiles_m, tiles_n, per_group, C, out_dtype);
-    };
-    if (k_blocks == 1) go(gemm_rowscale_small<1>);
-    else go(gemm_rowscale_small<2>);
-    return check_launch("lp_gemm_fp8_rowscale_grouped(small K)");
+    hipLaunchKernelGGL(gemm_rowscale_small, dim3((unsigned)grid), dim3(256), 0, st, (const uint8_t *)Aq, (const uint8_t *)As, (const uint8_t *)Bq,
+                       (const uint8_t *)Bs, groups, M, N, tiles_m, tiles_n, per_group, C, out_dtype);
+    return check_launch("lp_gemm_fp8_rowscale_grouped(one K block)");
 }
 
 }  // namespace gemm
