@@ -19,6 +19,21 @@ __device__ __forceinline__ float scale_at(const void *s, int64_t idx)
 // modulo 8) is handed whole blocks, so panels are re-used out of one L2.
 constexpr int GROUP_M = 8, GROUP_N = 4, CHUNK = GROUP_M * GROUP_N;
 
+// Tile `lin` of the numbering.
+__device__ __forceinline__ void tile_of(int64_t lin, int64_t tiles_m, int64_t tiles_n, int64_t &tm, int64_t &tn)
+{
+    // groups of GROUP_M m-tiles (the last may be short); inside a group, blocks of
+    // GROUP_N n-tiles (the last may be narrow); inside a block m runs fastest
+    const int64_t per_group = GROUP_M * tiles_n;
+    const int64_t grp = lin / per_group, in_grp = lin - grp * per_group;
+    const int64_t left = tiles_m - grp * GROUP_M;
+    const int64_t gm = left < GROUP_M ? left : GROUP_M;
+    const int64_t per_nblock = gm * GROUP_N;
+    const int64_t nblk = in_grp / per_nblock, in_blk = in_grp - nblk * per_nblock;
+    tm = grp * GROUP_M + in_blk % gm;
+    tn = nblk * GROUP_N + in_blk / gm;
+}
+
 // ends_first: the chunks an XCD works through come alternately from the front and the back of the tile
 // list (grid = number of workgroups launched, a multiple of 8 * CHUNK).  Grouped problems list experts in
 // caller order; when the heavy experts sit at one end, this keeps compute-bound tiles and tiles that only
@@ -34,17 +49,35 @@ __device__ __forceinline__ bool tile_coords(int64_t b, int64_t tiles_m, int64_t 
     }
     const int64_t lin = (q * 8 + xcd) * CHUNK + s % CHUNK;
     if (lin >= tiles_m * tiles_n) return false;
-    // groups of GROUP_M m-tiles (the last may be short); inside a group, blocks of
-    // GROUP_N n-tiles (the last may be narrow); inside a block m runs fastest
-    const int64_t per_group = GROUP_M * tiles_n;
-    const int64_t grp = lin / per_group, in_grp = lin - grp * per_group;
-    const int64_t left = tiles_m - grp * GROUP_M;
-    const int64_t gm = left < GROUP_M ? left : GROUP_M;
-    const int64_t per_nblock = gm * GROUP_N;
-    const int64_t nblk = in_grp / per_nblock, in_blk = in_grp - nblk * per_nblock;
-    tm = grp * GROUP_M + in_blk % gm;
-    tn = nblk * GROUP_N + in_blk / gm;
+    tile_of(lin, tiles_m, tiles_n, tm, tn);
     return true;
+}
+
+// The tiles of G problems of one shape: every problem is cut into pieces of `piece` consecutive tiles, and the pieces of all
+// problems are dealt to the XCDs in turn.  (Numbered problem by problem as above, a problem of few tiles ran on few XCDs: 20
+// weight gradients of 1024 x 1408 with three K blocks, 24 tiles each, on one of eight: 131 us, dealt in turn 30.)  Workgroup b -> problem g and its tile; false: none.
+__device__ __forceinline__ bool list_coords(int64_t b, int64_t G, int64_t tiles_m, int64_t tiles_n, int piece, int64_t &g, int64_t &tm, int64_t &tn)
+{
+    const int64_t tiles = tiles_m * tiles_n, per = (tiles + piece - 1) / piece, s = b >> 3;
+    const int64_t p = s / piece * 8 + (b & 7);
+    g = p / per;
+    const int64_t lin = (p - g * per) * piece + s % piece;
+    if (g >= G || lin >= tiles) return false;
+    tile_of(lin, tiles_m, tiles_n, tm, tn);
+    return true;
+}
+
+// Whole chunks, whose operand panels are shared in an L2, where that leaves the XCDs alike; a quarter of one otherwise.
+inline int list_piece(int64_t G, int64_t tiles_m, int64_t tiles_n)
+{
+    const int64_t chunks = G * ((tiles_m * tiles_n + CHUNK - 1) / CHUNK);
+    return (chunks + 7) / 8 * 8 * 4 <= chunks * 5 ? CHUNK : GROUP_M;
+}
+
+inline int64_t list_grid(int64_t G, int64_t tiles_m, int64_t tiles_n, int piece)
+{
+    const int64_t pieces = G * ((tiles_m * tiles_n + piece - 1) / piece);
+    return (pieces + 7) / 8 * 8 * piece;
 }
 
 // Rows of expert e from the caller's offset table, made safe to use: both ends are clamped to [0, M_total] and a

@@ -1079,19 +1079,17 @@ __global__ __launch_bounds__(512) void gemm_asm_mixed(const uint8_t *__restrict_
 // e8m0 scales per row and K block on both operands (the weight-gradient GEMM of the grouped linear): one problem, or a list of
 // problems that share M and N and differ in K (the weight gradients of the experts).  Entry g of `groups` = {output slot, K
 // blocks of 128, K blocks of all problems before it in the operand buffers, unused}: problem g reads Aq + M * 128 * before (its
-// [M, K_g] codes), As + M * before, the same for B with N, and writes C + slot * M * N.  per_group workgroups (a multiple of
-// 256) belong to each entry.
+// [M, K_g] codes), As + M * before, the same for B with N, and writes C + slot * M * N.
 template <int TM>
 __global__ __launch_bounds__(TM * 2) void gemm_asm_rowscale(const uint8_t *__restrict__ Aq, const float *__restrict__ As,
                                                             const uint8_t *__restrict__ Bq, const float *__restrict__ Bs,
-                                                            const int32_t *__restrict__ groups, int64_t M, int64_t N,
-                                                            int64_t tiles_m, int64_t tiles_n, int64_t per_group,
+                                                            const int32_t *__restrict__ groups, int G, int64_t M, int64_t N,
+                                                            int64_t tiles_m, int64_t tiles_n, int piece,
                                                             void *__restrict__ C, int out_dtype, int max_k_blocks, int multiple)
 {
     __shared__ __attribute__((aligned(1024))) uint8_t smem[AsmTile<TM, TM, 1>::LDS_BYTES + TM * 32];
-    const int64_t g = blockIdx.x / per_group, local = blockIdx.x - g * per_group;
-    int64_t tm, tn;
-    if (!gemm::tile_coords(local, tiles_m, tiles_n, tm, tn)) return;
+    int64_t g, tm, tn;
+    if (!gemm::list_coords(blockIdx.x, G, tiles_m, tiles_n, piece, g, tm, tn)) return;
     const int64_t slot = groups ? groups[4 * g] : 0, before = groups ? groups[4 * g + 2] : 0;
     const int kb = groups ? groups[4 * g + 1] : max_k_blocks;
     // an entry that breaks the caller's promise writes nothing: more K blocks than max_k_blocks (on which the host checked
@@ -1613,11 +1611,12 @@ int launch_rowscale_asm(const void *Aq, const void *As, const void *Bq, const vo
     const int64_t big = ((M + 255) / 256) * ((N + 255) / 256);
     const int tm = big * 65536 * 10 <= M * N * 11 && big * G >= 256 ? 256 : 128;
     const int64_t tiles_m = (M + tm - 1) / tm, tiles_n = (N + tm - 1) / tm;
-    const int64_t per_group = gemm::padded_grid(tiles_m, tiles_n), grid = per_group * G;
+    const int piece = gemm::list_piece(G, tiles_m, tiles_n);
+    const int64_t grid = gemm::list_grid(G, tiles_m, tiles_n, piece);
     if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_rowscale: problem too large");
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(tm * 2), 0, st, (const uint8_t *)Aq, (const float *)As, (const uint8_t *)Bq,
-                           (const float *)Bs, groups, M, N, tiles_m, tiles_n, per_group, C, out_dtype, max_k_blocks, multiple);
+                           (const float *)Bs, groups, G, M, N, tiles_m, tiles_n, piece, C, out_dtype, max_k_blocks, multiple);
     };
     tm == 256 ? go(gemm_asm_rowscale<256>) : go(gemm_asm_rowscale<128>);
     return check_launch("lp_gemm_fp8_rowscale(asm)");

@@ -36,14 +36,13 @@ constexpr int kPitch = 64 * 2 + 16, kWaveStage = 64 * kPitch;
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void gemm_rowscale_small(
     const uint8_t *__restrict__ Aq, const uint8_t *__restrict__ As, const uint8_t *__restrict__ Bq, const uint8_t *__restrict__ Bs,
-    const int32_t *__restrict__ groups, int64_t M, int64_t N, int64_t tiles_m, int64_t tiles_n, int64_t per_group, void *__restrict__ C,
+    const int32_t *__restrict__ groups, int G, int64_t M, int64_t N, int64_t tiles_m, int64_t tiles_n, int piece, void *__restrict__ C,
     int out_dtype)
 {
     constexpr int TILE = 128 * 128, PITCH = 128;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * TILE > 4 * kWaveStage ? 2 * TILE : 4 * kWaveStage];
-    const int64_t g = blockIdx.x / per_group, local = blockIdx.x - g * per_group;
-    int64_t tm, tn;
-    if (!gemm::tile_coords(local, tiles_m, tiles_n, tm, tn)) return;
+    int64_t g, tm, tn;
+    if (!gemm::list_coords(blockIdx.x, G, tiles_m, tiles_n, piece, g, tm, tn)) return;
     // no table: one problem
     const int64_t slot = groups ? groups[4 * g] : 0, kb = groups ? groups[4 * g + 1] : 1, before = groups ? groups[4 * g + 2] : 0;
     // an entry of another size (or one that breaks the caller's promises) is not this launch's: nothing is written
@@ -284,10 +283,11 @@ int launch_rowscale_small(const void *Aq, const void *As, const void *Bq, const 
                            (const uint8_t *)Bs, groups, G, M, N, (int)tiles_m, (int)tiles_n, (int)strip, C, out_dtype);
         return check_launch("lp_gemm_fp8_rowscale_grouped(two K blocks)");
     }
-    const int64_t per_group = padded_grid(tiles_m, tiles_n), grid = per_group * G;
+    const int piece = list_piece(G, tiles_m, tiles_n);
+    const int64_t grid = list_grid(G, tiles_m, tiles_n, piece);
     if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_rowscale_grouped: problem too large");
     hipLaunchKernelGGL(gemm_rowscale_small, dim3((unsigned)grid), dim3(256), 0, st, (const uint8_t *)Aq, (const uint8_t *)As, (const uint8_t *)Bq,
-                       (const uint8_t *)Bs, groups, M, N, tiles_m, tiles_n, per_group, C, out_dtype);
+                       (const uint8_t *)Bs, groups, G, M, N, tiles_m, tiles_n, piece, C, out_dtype);
     return check_launch("lp_gemm_fp8_rowscale_grouped(one K block)");
 }
 

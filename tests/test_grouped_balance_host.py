@@ -1,7 +1,8 @@
-"""How the grouped launch with two tile heights shares its tiles (gemm_asm_grouped_mixed in csrc/gemm_fp8_big.hip), restated on the
-host: every tile of both classes is taken by exactly one workgroup of the XCD whose run it lies in, and no workgroup has
-more work than a longest-first list schedule would give it: at most one small tile above the least loaded one of its XCD (a big
-tile counts 3, a small one 2)."""
+"""How grouped launches share their tiles, restated on the host.  Two tile heights (gemm_asm_grouped_mixed in
+csrc/gemm_fp8_big.hip): every tile of both classes is taken by exactly one workgroup of the XCD whose run it lies in, and no
+workgroup has more work than a longest-first list schedule would give it: at most one small tile above the least loaded one of
+its XCD (a big tile counts 3, a small one 2).  Lists of problems of one shape (list_coords in csrc/gemm_common.h): every tile
+once, dealt to the XCDs in turn."""
 import pytest
 
 
@@ -40,3 +41,28 @@ def test_every_tile_once_and_balanced(grid, all_small):
             assert all(w - 2 <= least for w, small in load if small), (all_big, all_small, grid, load)
             runs = [t for xx, b, _ in got if xx == x for t in b]
             assert not runs or max(runs) - min(runs) + 1 == len(runs)          # one run of numbers per XCD
+
+
+def list_tiles(G, tiles_m, tiles_n):
+    """list_piece, list_grid and list_coords of csrc/gemm_common.h -> per XCD the (problem, tile number) of its workgroups"""
+    tiles, chunks = tiles_m * tiles_n, G * -(-(tiles_m * tiles_n) // 32)
+    piece = 32 if -(-chunks // 8) * 8 * 4 <= chunks * 5 else 8
+    per = -(-tiles // piece)
+    out = [[] for _ in range(8)]
+    for b in range(-(-(G * per) // 8) * 8 * piece):
+        s, xcd = b >> 3, b & 7
+        p = s // piece * 8 + xcd
+        g = p // per
+        lin = (p - g * per) * piece + s % piece
+        if g < G and lin < tiles:
+            out[xcd].append((g, lin))
+    return piece, out
+
+
+@pytest.mark.parametrize("G", [1, 2, 3, 15, 20, 64])
+@pytest.mark.parametrize("tiles_m,tiles_n", [(1, 1), (2, 2), (4, 4), (4, 6), (8, 8), (8, 11), (9, 23), (16, 16), (32, 32)])
+def test_problem_lists_cover_every_tile_once_on_all_xcds(G, tiles_m, tiles_n):
+    piece, per_xcd = list_tiles(G, tiles_m, tiles_n)
+    assert sorted(t for x in per_xcd for t in x) == [(g, lin) for g in range(G) for lin in range(tiles_m * tiles_n)]
+    # a deal in turn: no XCD has more than its share of whole pieces and one piece more
+    assert max(map(len, per_xcd)) <= -(-(G * -(-(tiles_m * tiles_n) // piece)) // 8) * piece
