@@ -221,9 +221,9 @@ def rowscale_launches(k_blocks):
     """How the row-scaled problems of a grouped weight gradient are dealt to kernels: -> (launches, empty) with launches a
     list of (table, multiple) -- table rows {problem, K blocks, K blocks of the problems before it, 0} as
     lp_gemm_fp8_rowscale_grouped reads them, multiple = what every K block count of the table is a multiple of -- and
-    empty the problems without K blocks (their outputs are zeros).  Problems whose K is a multiple of 512 share the
-    hand-scheduled loop, those of one K block and those of two the kernel without a K loop, whatever is left the
-    compiler-scheduled kernel."""
+    empty the problems without K blocks (their outputs are zeros).  Problems of one K block and those of two have a
+    kernel each; the others run on the hand-scheduled loop, which gemm_fp8_rowscale_grouped launches once for both of
+    their lists."""
     before, fast, one, two, rest, empty = 0, [], [], [], [], []
     for e, kb in enumerate(k_blocks):
         kb = int(kb)
