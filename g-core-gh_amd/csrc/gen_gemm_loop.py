@@ -184,14 +184,17 @@ _uid = 0
 
 
 IDLE = False        # emitting the loop body of a wave whose rows of the tile are all missing (see generate)
+STAGING = False     # emitting what brings the next group's scales into LDS (rag)
 GRP = 0             # which half of the waves the body being emitted is for (see configure: pingpong)
 
 
 def emit(s):
     if IDLE:
         # such a wave keeps its share of the copies, the barriers and the counters, and drops the arithmetic: fragment
-        # and scale reads, matrix instructions, folds, scale products, and the waits that only order those
-        if s.startswith(("ds_read", "ds_write", "v_lshl_or", "v_mfma", "v_fmac", "v_mul_f32", "v_mov_b32", "v_add_u32", "s_load_dword", "s_waitcnt lgkmcnt", "s_setprio")):
+        # and scale reads, matrix instructions, folds, scale products, and the waits that only order those.  The activation
+        # scales it would stage belong to rows at or behind its own, which do not exist; row-scaled weights' scales (brow)
+        # belong to the whole tile's columns, and it stages them like any other wave.
+        if not (BROW and STAGING) and s.startswith(("ds_read", "ds_write", "v_lshl_or", "v_mfma", "v_fmac", "v_mul_f32", "v_mov_b32", "v_add_u32", "s_load_dword", "s_waitcnt lgkmcnt", "s_setprio")):
             return
         s = s.replace("%=", "i%=")
     elif GRP == 1:
@@ -391,6 +394,16 @@ def rag_elements(dst, load, offset, base, size, join):
         emit(f"{load} v{dst + i}, {offset}, {base} offset:{i * size}")
 
 
+def staging(f):
+    def emitting(tag):
+        global STAGING
+        STAGING = True
+        f(tag)
+        STAGING = False
+    return emitting
+
+
+@staging
 def rag_scale_load(tag):
     """Request the scales of the next group (see configure: rag)."""
     emit("s_cmp_eq_u32 s53, 0")
@@ -455,6 +468,7 @@ def rag_scale_load(tag):
     emit("s_addc_u32 s47, s47, 0")
 
 
+@staging
 def rag_scale_write(tag):
     """The group requested by rag_scale_load has landed: put a short group's bytes together and write the activation scales
     to LDS (half s54), where read_scales finds them."""

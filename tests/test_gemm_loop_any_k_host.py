@@ -1,7 +1,10 @@
 """The loops of the GEMM kernels that take any number of K blocks (csrc/gen_gemm_loop.py: rag), walked on the host: the scalar
 program of the generated text is executed for one wave -- bases, counters, branches, copy requests and counted waits -- and
 checked for what the device cannot report: every request stays inside its operand and every scale inside its table, the
-fragments of step k are read from a stage whose copies of block k have landed, and there are exactly as many steps as blocks."""
+fragments of step k are read from a stage whose copies of block k have landed, there are exactly as many steps as blocks, and
+every wave that stages scales other waves read writes every group of them to the right half of LDS, before the barrier behind
+which it is read.  A wave none of whose activation rows exist stages nothing anybody reads, except with row-scaled weights,
+whose scales the second half of the waves stages for the whole tile."""
 import importlib.util
 import os
 import re
@@ -48,7 +51,8 @@ class Wave:
         self.pairs = dict(abase=ABASE, bbase=BBASE, sbase=SBASE, bsptr=BSBASE)
         self.s, self.v, self.scc, self.m0 = {}, {}, 0, 0
         self.queue, self.landed, self.scales_on_way = [], {}, None
-        self.step, self.mfma, self.groups, self.lds_group = 0, 0, [], {}
+        self.step, self.mfma, self.groups = 0, 0, []
+        self.staged, self.unsettled, self.staging = [], False, []        # LDS halves written; a write not waited for; the instructions on staged scales
 
     def val(self, t):
         t = t.strip()
@@ -163,10 +167,15 @@ class Wave:
                 self.request(("copy", self.m0, block))
             elif op.startswith("global_load") or op.startswith("s_load"):
                 self.scale_request(ln)
+                self.staging.append(ln)
+            elif op in ("v_mov_b32", "v_lshl_or_b32") and gen.HW and re.match(r"v1(1[2-9]|2[01])\b", a[0]):
+                self.staging.append(ln)                      # registers of the scales on their way (e8m0 loops)
             elif op == "s_waitcnt":
                 m = re.search(r"vmcnt\((\d+)\)", ln)
                 if m:
                     self.settle(int(m.group(1)))
+                if "lgkmcnt(0)" in ln:
+                    self.unsettled = False
             elif op == "v_mov_b32" and a[1].startswith("%["):
                 self.v[int(a[0][1:])] = self.ops.get(a[1][2:-1], 0)
             elif op == "v_add_u32" and a[2].startswith("%[") and a[2][2:-1] in self.ops:
@@ -174,6 +183,11 @@ class Wave:
             elif op.startswith("ds_write"):
                 # the group just written belongs to the trip after this one (to the first in the prologue)
                 assert not self.in_flight("scale"), "scales are written to LDS while they are on their way"
+                self.staged.append(self.s[54])
+                self.unsettled = True
+                self.staging.append(ln)
+            elif op == "s_barrier":
+                assert not self.unsettled, "a barrier with scales still on their way to LDS"
             elif op.startswith("ds_read_b128") or op.startswith("ds_read_b64_tr"):
                 addr = self.val(a[-1].split()[0]) + int(re.search(r"offset:(\d+)", ln).group(1))
                 is_a = addr < g.NSTAGE * g.A_BYTES
@@ -197,6 +211,7 @@ def test_requests_stay_inside_and_every_block_is_multiplied_once(name):
     gen.configure(*LOOPS[name])
     gen.generate()
     lines = [ln.replace("%=", "") for ln in gen.lines]
+    staging = {}
     ss_total = lambda kb: {("b", k) for k in range(kb)}
     for kblocks in (1, 2, 3, 4, 5, 6, 7, 8, 9, 11, 14, 23):
         for copies in (0, 1):
@@ -204,8 +219,15 @@ def test_requests_stay_inside_and_every_block_is_multiplied_once(name):
                 for idle in ((0, 1) if gen.WITH_IDLE else (0,)):
                     w = Wave(lines, kblocks, copies, idle, second)
                     w.run()
+                    if copies and (not idle or gen.BROW):
+                        assert w.staged == [gen.SCL_HALF * (i & 1) for i in range((kblocks + 3) // 4)], (kblocks, idle, w.staged)
+                        assert {x for x in w.groups if x[0] == "a"} == {("a", k) for k in range(kblocks)}
+                    if gen.BROW:
+                        staging.setdefault((kblocks, copies), []).append(w.staging)
                     if not idle:
                         assert w.step == kblocks and w.mfma == kblocks * gen.NB * gen.MB, (kblocks, w.step)
                         got = set(w.groups)
                         assert {x for x in got if x[0] == "b"} == (set() if gen.BROW else ss_total(kblocks)), (kblocks, sorted(got))
                         assert {x for x in got if x[0] == "a"} == ({("a", k) for k in range(kblocks)} if copies else set())
+    for key, ways in staging.items():
+        assert all(x == ways[0] for x in ways), ("an idle wave handles the scales it stages otherwise than a live one", key)

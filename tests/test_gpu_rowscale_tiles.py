@@ -1,5 +1,6 @@
 """The row-scaled grouped GEMM on both tile sizes of its loop (256 x 256 tiles need at least 256 of them and at most a tenth beyond
-the matrix): matrices that end inside a tile, three K blocks up to two trips of four and each remainder, an unaligned scale
+the matrix): matrices that end inside a tile, in rows (where half of the waves have no row of their own and still stage the scales
+of the tile's columns), in columns and in both, three K blocks up to two trips of four and each remainder, an unaligned scale
 table (an odd number of blocks in front).  Bound as in tests/test_gpu_any_k.py."""
 import pytest
 import torch
@@ -9,7 +10,8 @@ from tests.test_gpu_any_k import close, deq
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M,N", [(384, 640), (2048, 2176), (2304, 4096)], ids=["tiles128", "tiles256_ragged", "tiles256"])
+@pytest.mark.parametrize("M,N", [(384, 640), (2048, 2176), (2304, 4096), (1408, 2048), (2176, 2048), (2688, 2688)],
+                         ids=["tiles128", "tiles256_ragged_columns", "tiles256", "tiles256_ragged_rows", "tiles256_ragged_rows_9", "tiles256_ragged_both"])
 def test_problems_of_any_length(M, N):
     import gcore_lowp as G
     k_blocks = [3, 9, 1, 4, 5, 2, 8, 6, 7, 0, 11]
@@ -30,3 +32,31 @@ def test_problems_of_any_length(M, N):
             assert not out[e].any()
         else:
             close(out[e], deq(o[0], o[1], 1) @ deq(o[2], o[3], 1).t(), ("rowscale", M, N, k_blocks[e]))
+
+
+def test_weight_gradient_of_a_layer_whose_width_ends_inside_a_tile():
+    """The grouped linear's dW, 1408 = 5.5 x 256 output features, experts of 513 .. 1100 rows (5 to 9 K blocks): expert by expert
+    against the product of the same quantised operands in fp32, dequantised from the column-wise quantiser's own output."""
+    import importlib
+    import gcore_lowp as G
+    L = importlib.import_module("gcore_lowp.grouped_gemm_fp8")
+    m_splits, n_out, k_in = [513, 1100, 640, 0, 769, 1024, 600, 900, 700, 1025, 300, 513], 1408, 2048
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rows, E = sum(m_splits), len(m_splits)
+    x = torch.randn(rows, k_in, generator=g, device="cuda", dtype=torch.bfloat16)
+    w = (torch.randn(E, n_out, k_in, generator=g, device="cuda", dtype=torch.bfloat16) * 0.02).requires_grad_(True)
+    dy = torch.randn(rows, n_out, generator=g, device="cuda", dtype=torch.bfloat16) * 1e-3
+    out = G.MyTeGroupedLinearFp8(E)(x, w, m_splits)
+    dw, = torch.autograd.grad(out, w, dy)
+    offs = L._offsets(m_splits, x.device)
+    (xq, xs, nblk), (dq, ds, _) = L.quant_fp8_colwise_t(x, offs, m_splits, 128), L.quant_fp8_colwise_t(dy, offs, m_splits, 128)
+    before = 0
+    for e, nb in enumerate(nblk):
+        if not nb:
+            assert not dw[e].any()
+            continue
+        def operand(q, s, n):
+            q = q.view(torch.float8_e4m3fn)[n * 128 * before:n * 128 * (before + nb)].view(n, 128 * nb)
+            return deq(q, s.view(torch.float8_e8m0fnu)[n * before:n * (before + nb)].view(n, nb), 1)
+        close(dw[e], operand(dq, ds, n_out) @ operand(xq, xs, k_in).t(), ("dW", e, m_splits[e]))
+        before += nb
