@@ -137,15 +137,15 @@ constexpr int kStripTile = 128 * 128, kStripHalf = 2 * kStripTile;
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_rowscale_strip(
     const uint8_t *__restrict__ Aq, const uint8_t *__restrict__ As, const uint8_t *__restrict__ Bq, const uint8_t *__restrict__ Bs,
-    const int32_t *__restrict__ groups, int G, int64_t M, int64_t N, int tiles_m, int tiles_n, int strip, void *__restrict__ C, int out_dtype)
+    const int32_t *__restrict__ groups, int G, int64_t M, int64_t N, int tiles_m, int tiles_n, int strip, int piece, void *__restrict__ C, int out_dtype)
 {
     __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * kStripHalf];
-    // an XCD (workgroup id modulo 8) is handed whole units of 8 row panels x one strip, which share operands in its L2
-    const int strips = (tiles_n + strip - 1) / strip, parts = (tiles_m + 7) / 8;
-    const int in_xcd = blockIdx.x >> 3, unit = (in_xcd >> 3) * 8 + (blockIdx.x & 7);
-    const int g = unit / (strips * parts), rest = unit - g * (strips * parts);
-    const int first_n = (rest / parts) * strip, tm = (rest % parts) * 8 + (in_xcd & 7);
-    if (g >= G || tm >= tiles_m) return;
+    // The strips of all problems are numbered problem by problem and strip by strip, row panels running fastest, and pieces of
+    // `piece` consecutive ones, which share a strip of B in an L2, are dealt to the XCDs (workgroup id modulo 8) in turn.
+    const int runs = tiles_m * ((tiles_n + strip - 1) / strip), in_xcd = blockIdx.x >> 3;
+    const int id = (in_xcd / piece * 8 + (blockIdx.x & 7)) * piece + in_xcd % piece, g = id / runs, run = id - g * runs;
+    if (g >= G) return;
+    const int first_n = run / tiles_m * strip, tm = run % tiles_m;
     const int count = tiles_n - first_n < strip ? tiles_n - first_n : strip;
     // no table: one problem.  An entry of another size (or one that breaks the caller's promises) is not this launch's:
     // nothing is written
@@ -275,12 +275,19 @@ int launch_rowscale_small(const void *Aq, const void *As, const void *Bq, const 
     if (k_blocks == 2) {
         // At most 8 tiles a strip, all strips alike: the panel's load and the first tile's wait spread over 8 tiles while a weight
         // of 4096 columns still cuts into 4 (40 x 7168 x 4096, strips of 2 / 4 / 8 / 16 tiles: 535 / 476 / 433 / 471 us; 15 x 4096 x
-        // 4096: 117 / 122 / 114 / 128).
-        const int64_t per_row = (tiles_n + 7) / 8, strip = per_row ? (tiles_n + per_row - 1) / per_row : 1;
-        const int64_t units = G * ((tiles_n + strip - 1) / strip) * ((tiles_m + 7) / 8), wgs = (units + 7) / 8 * 64;
+        // 4096: 117 / 122 / 114 / 128).  Few small problems are cut shorter, until two workgroups per CU have one, and dealt
+        // out in smaller pieces, until every XCD has one (one problem of 1024 x 1024 / 2048 x 2048 / 7168 x 2048, strips of 8 tiles: 14.2 /
+        // 14.2 / 14.2 us, as cut here 4.7 / 5.4 / 9.6; 8 problems of 1024 x 1024 13.9 / 6.9; one of 384 x 384 in a piece of 8 7.1, in pieces of
+        // one 4.5.  Below ten tiles a workgroup without a strip's two barriers more would be 0.2 us ahead, 4.0 against 4.2).
+        const int64_t wanted = tiles_m && G ? (512 + G * tiles_m - 1) / (G * tiles_m) : 1, least = (tiles_n + 7) / 8;
+        const int64_t per_row = wanted <= least ? least : wanted < tiles_n ? wanted : tiles_n;
+        const int64_t strip = per_row ? (tiles_n + per_row - 1) / per_row : 1, runs = G * tiles_m * ((tiles_n + strip - 1) / strip);
+        int piece = GROUP_M;
+        while (piece > 1 && (runs + piece - 1) / piece < 8) piece /= 2;
+        const int64_t wgs = (runs + 8 * piece - 1) / (8 * piece) * (8 * piece);
         if (wgs > 0x7FFFFFFF || tiles_n > 0x7FFFFF || tiles_m > 0x7FFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_rowscale_grouped: problem too large");
         hipLaunchKernelGGL(gemm_rowscale_strip, dim3((unsigned)wgs), dim3(256), 0, st, (const uint8_t *)Aq, (const uint8_t *)As, (const uint8_t *)Bq,
-                           (const uint8_t *)Bs, groups, G, M, N, (int)tiles_m, (int)tiles_n, (int)strip, C, out_dtype);
+                           (const uint8_t *)Bs, groups, G, M, N, (int)tiles_m, (int)tiles_n, (int)strip, piece, C, out_dtype);
         return check_launch("lp_gemm_fp8_rowscale_grouped(two K blocks)");
     }
     const int piece = list_piece(G, tiles_m, tiles_n);

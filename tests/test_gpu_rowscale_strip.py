@@ -1,6 +1,7 @@
 """Row-scaled problems of two K blocks, walked in strips of column tiles: one tile, strips that end in the matrix (9, 17 tiles),
 row panels that do not fill a group of eight, bf16 and fp32 results, problems out of order, a single problem without a table,
-and an entry of another size, whose slot stays as it was.  Bound as in tests/test_gpu_any_k.py."""
+and an entry of another size, whose slot stays as it was.  Few problems: strips cut shorter than eight tiles (one tile, two, uneven
+last ones) and dealt in pieces smaller than eight.  Bound as in tests/test_gpu_any_k.py."""
 import pytest
 import torch
 
@@ -10,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
-@pytest.mark.parametrize("M,N,E", [(128, 128, 1), (1152, 1152, 3), (384, 2176, 2), (2048, 1024, 5)])
+@pytest.mark.parametrize("M,N,E", [(128, 128, 1), (1152, 1152, 3), (384, 2176, 2), (2048, 1024, 5), (128, 1024, 1), (1408, 1024, 1), (256, 1664, 2), (1024, 2048, 4)])
 def test_two_k_blocks(M, N, E, dtype):
     import gcore_lowp as G
     g = torch.Generator(device="cuda").manual_seed(M + N)

@@ -2,7 +2,8 @@
 csrc/gemm_fp8_big.hip): every tile of both classes is taken by exactly one workgroup of the XCD whose run it lies in, and no
 workgroup has more work than a longest-first list schedule would give it: at most one small tile above the least loaded one of
 its XCD (a big tile counts 3, a small one 2).  Lists of problems of one shape (list_coords in csrc/gemm_common.h): every tile
-once, dealt to the XCDs in turn."""
+once, dealt to the XCDs in turn.  Problems of two K blocks (gemm_rowscale_strip in csrc/gemm_rowscale_small.hip): every tile once,
+and no fewer workgroups than the tiles or two per CU allow."""
 import pytest
 
 
@@ -66,3 +67,34 @@ def test_problem_lists_cover_every_tile_once_on_all_xcds(G, tiles_m, tiles_n):
     assert sorted(t for x in per_xcd for t in x) == [(g, lin) for g in range(G) for lin in range(tiles_m * tiles_n)]
     # a deal in turn: no XCD has more than its share of whole pieces and one piece more
     assert max(map(len, per_xcd)) <= -(-(G * -(-(tiles_m * tiles_n) // piece)) // 8) * piece
+
+
+def strips(G, tiles_m, tiles_n):
+    """launch_rowscale_small and gemm_rowscale_strip -> strip length, per XCD the (problem, row tile, column tiles) of its workgroups"""
+    wanted, least = -(-512 // (G * tiles_m)), -(-tiles_n // 8)
+    per_row = max(least, min(wanted, tiles_n))
+    strip = -(-tiles_n // per_row)
+    runs = tiles_m * -(-tiles_n // strip)
+    piece = 8
+    while piece > 1 and -(-G * runs // piece) < 8:
+        piece //= 2
+    out = [[] for _ in range(8)]
+    for b in range(-(-G * runs // (8 * piece)) * 8 * piece):
+        in_xcd, xcd = b >> 3, b & 7
+        g, run = divmod((in_xcd // piece * 8 + xcd) * piece + in_xcd % piece, runs)
+        if g < G:
+            first = run // tiles_m * strip
+            out[xcd].append((g, run % tiles_m, range(first, min(first + strip, tiles_n))))
+    return strip, out
+
+
+@pytest.mark.parametrize("G", [1, 2, 4, 8, 15, 40])
+@pytest.mark.parametrize("tiles_m,tiles_n", [(1, 1), (1, 8), (3, 3), (4, 8), (8, 8), (11, 8), (11, 16), (16, 16), (9, 23), (32, 32), (56, 32)])
+def test_strips_cover_every_tile_once_and_fill_the_chip(G, tiles_m, tiles_n):
+    strip, per_xcd = strips(G, tiles_m, tiles_n)
+    tiles = [(g, m, n) for x in per_xcd for g, m, ns in x for n in ns]
+    assert sorted(tiles) == [(g, m, n) for g in range(G) for m in range(tiles_m) for n in range(tiles_n)]
+    busy = [len(x) for x in per_xcd]
+    assert strip <= 8 and sum(busy) * 2 > min(512, G * tiles_m * tiles_n)        # a cut of twice as many workgroups was not to be had
+    assert sum(1 for n in busy if n) == min(8, sum(busy))                        # one strip per XCD before any has more
+    assert max(busy) <= sum(busy) / 8 + 8
