@@ -240,7 +240,7 @@ def gemm_fp8_rowscale_grouped(aq, a_s, bq, b_s, k_blocks, M, N, out: torch.Tenso
     """out[e] [M, N] = the row-scaled product of problem e, whose operands ([M, K_e] / [N, K_e] codes and their e8m0
     scales, K_e = 128 * k_blocks[e]) lie one after the other in aq / a_s / bq / b_s.  The problems of one and of two K blocks
     go to the kernel without a K loop (a launch each), the others to the hand-scheduled loop in one launch, longest first (a
-    long problem started last would run alone at the end); problems with no K blocks are zero-filled.  (The reference issues
+    long problem started last would run alone at the end); problems with no K blocks are zero-filled, all in one launch.  (The reference issues
     one grouped GEMM call: fp8.py:325-341.)"""
     E = len(k_blocks)
     assert out.is_contiguous() and tuple(out.shape) == (E, M, N) and out.dtype in (torch.bfloat16, torch.float32)
@@ -249,17 +249,18 @@ def gemm_fp8_rowscale_grouped(aq, a_s, bq, b_s, k_blocks, M, N, out: torch.Tenso
     launches = [(g, m) for g, m in kinds if g[0][1] == m and m < 3 and all(x[1] == m for x in g)]
     if looped:
         launches.insert(0, (sorted(looped, key=lambda g: -g[1]), 1))
-    for e in empty:
-        out[e].zero_()
+    if not launches:
+        return out.zero_()
     odt = A.BF16 if out.dtype == torch.bfloat16 else A.F32
     with torch.cuda.device(out.device):
-        table = host_table([w for groups, _ in launches for g in groups for w in g], out.device)
+        table = host_table([w for groups, _ in launches for g in groups for w in g] + empty, out.device)
         first = table.data_ptr()
         for groups, multiple in launches:
             A.check(A.lib().lp_gemm_fp8_rowscale_grouped(aq.data_ptr(), a_s.data_ptr(), bq.data_ptr(), b_s.data_ptr(), A.E8M0,
                                                          first, len(groups), max(g[1] for g in groups), multiple,
                                                          M, N, out.data_ptr(), odt, A.stream_ptr()))
             first += 16 * len(groups)
+        A.check(A.lib().lp_zero_slots(out.data_ptr(), M * N * out.element_size(), E, first, len(empty), A.stream_ptr()))
     return out
 
 

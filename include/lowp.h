@@ -317,6 +317,14 @@ int lp_gemm_fp8_rowscale_grouped(const void *Aq, const void *As, const void *Bq,
                                  int64_t N, void *C, int out_dtype, lp_stream_t stream);
 
 /*
+ * Zeros for the problems without K blocks, which the call above leaves alone: clears C + slot * slot_bytes .. + slot_bytes for
+ * each of the n int32 slots listed in device memory at `slots`, in one launch.  total: slots in C; a listed slot outside
+ * 0 .. total - 1 clears nothing.  slot_bytes must be a multiple of 16.  The reference's grouped GEMM call fills the weight
+ * gradients of experts without rows (gpatch_v4/models/deepseek_v4/fp8.py:325-341).
+ */
+int lp_zero_slots(void *C, int64_t slot_bytes, int64_t total, const int32_t *slots, int n, lp_stream_t stream);
+
+/*
  * Column-wise quantiser with transposed output for expert-grouped rows.  x: device [rows, cols]
  * (LP_BF16 or LP_F32), rows of expert e = m_offsets[e] .. m_offsets[e+1]-1 (device int32 [E+1]),
  * cols % 128 == 0.  Per expert, P_e = ceil(M_e / pad_rows) * pad_rows (pad_rows 128, 256 or 512), or with
