@@ -1,0 +1,81 @@
+"""The native front end of the calls made most often (csrc/host/native.cpp): its answers are those of the wrappers' own way
+through the C ABI, and what goes wrong in it reaches Python as it does there."""
+import contextlib
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+E4M3, E8M0 = torch.float8_e4m3fn, torch.float8_e8m0fnu
+
+
+@pytest.fixture(scope="module")
+def G():
+    import gcore_lowp
+    return gcore_lowp
+
+
+def calls(G, rows=256, cols=1024):
+    """name -> a call of a public function on operands the front end takes"""
+    g = torch.Generator(device="cuda").manual_seed(rows + cols)
+    x = torch.randn(rows, cols, generator=g, device="cuda", dtype=torch.bfloat16)
+    q, s = G.quant_fp8_e4m3_scale_e8m0(x)
+    packed = torch.randint(-128, 128, (rows, cols // 2), generator=g, device="cuda", dtype=torch.int8)
+    fs = torch.randint(117, 128, (rows, cols // 32), generator=g, device="cuda", dtype=torch.uint8).view(E8M0)
+    aq, sa = G.quant_1d(x)
+    bq, sb = G.quant_2d(x)
+    return {
+        "quant_1d": lambda: G.quant_1d(x),
+        "quant_1d_pow2": lambda: G.quant_1d(x, round_sf=True),
+        "quant_e8m0": lambda: G.quant_fp8_e4m3_scale_e8m0(x),
+        "dequant_fp8": lambda: G.dequant_fp4_e2m1_fp8_scale_e8m0_packed(q, s),
+        "dequant_fp4": lambda: G.dequant_fp4_e2m1_fp8_scale_e8m0_packed(packed, fs),
+        "fp4_rebase": lambda: G.cast_e2m1fn_to_e4m3fn(packed, fs),
+        "fp4_rebase_f32": lambda: G.official_expert_to_sgl(packed, fs),
+        "fp4_amax": lambda: G.fp4_to_fp8_blockwise(packed, fs),
+        "gemm": lambda: G.gemm_fp8_block_scaling_impl(aq, sa, bq, sb),
+        "gemm_f32": lambda: G.gemm_fp8_block_scaling_impl(aq, sa, bq, sb, out_dtype=torch.float32),
+    }
+
+
+NAMES = ["quant_1d", "quant_1d_pow2", "quant_e8m0", "dequant_fp8", "dequant_fp4", "fp4_rebase", "fp4_rebase_f32", "fp4_amax", "gemm", "gemm_f32"]
+
+
+def parts(r):
+    return list(r) if isinstance(r, tuple) else [r]
+
+
+def bits(t):
+    return t.contiguous().view(torch.uint8)
+
+
+@contextlib.contextmanager
+def no_more_memory():
+    """The allocator has nothing of 16 MB left (a limit of its own: the card is not filled; what it has cached is taken)."""
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
+    taken = []
+    try:
+        with contextlib.suppress(torch.OutOfMemoryError):
+            while len(taken) < 1024:
+                taken.append(torch.empty(16 << 20, dtype=torch.uint8, device="cuda"))
+        yield
+    finally:
+        taken.clear()
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_out_of_memory_is_torchs_own_error(G, name):
+    """A caller that catches torch.OutOfMemoryError, frees and tries again."""
+    call = calls(G, 8192, 8192)[name]
+    print("[case]", name, flush=True)
+    want = [bits(t).clone() for t in parts(call())]
+    with no_more_memory():
+        with pytest.raises(torch.OutOfMemoryError):
+            call()
+    got = parts(call())
+    assert all(torch.equal(bits(a), b) for a, b in zip(got, want))
