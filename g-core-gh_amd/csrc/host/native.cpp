@@ -4,7 +4,8 @@
 // torch tensors, contiguous, on the current GPU, of the types and shapes the kernels take as they are, and accepted by the C
 // ABI.  The wrapper then goes through its own checks, conversions and errors as if this file did not exist.  What it saves is
 // the interpreter's work per call (attribute look-ups, four or five tensor methods that do nothing, a device guard, ctypes
-// conversions).
+// conversions).  Where it allocates, launches or waits the interpreter's lock is free, as it is in torch's allocations and in a
+// ctypes call: an allocation may wait for the device and a launch for room in a full queue.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -107,6 +108,12 @@ bool ints(PyObject *const *args, int n, long *out)
 // allocation among them).
 #define GUARDED(...) HANDLE_TH_ERRORS __VA_ARGS__ END_HANDLE_TH_ERRORS
 
+// Other Python threads run while one of these lives.
+struct Unlocked {
+    PyThreadState *state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
 // Waits until the flag lp_host_flag raises is up.  Watching it for the length of a kernel beats the runtime's own wait (12 us
 // against 14 - 20 for a quantisation of 256 x 256 with the check); behind a long queue the runtime waits.
 hipError_t wait_flag(const int32_t *flag, hipStream_t st)
@@ -136,33 +143,31 @@ PyObject *quant_fp8(PyObject *, PyObject *const *args, Py_ssize_t n)
         const int64_t rows = x->size(-2), cols = x->size(-1), bm = v[0], bn = v[1];
         if (bm <= 0 || bn <= 0 || rows % bm || cols % bn || v[3] < 0 || v[3] > LP_E8M0) Py_RETURN_NONE;
         const hipStream_t st = c10::hip::getCurrentHIPStream(dev).stream();
-        at::Tensor words;                                // NaN count, flag
+        at::Tensor q, s, words;                          // words: NaN count, flag
         int32_t *host = nullptr;
-        if (check) {
-            hipStreamCaptureStatus capturing;
-            if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) Py_RETURN_NONE;
-            words = at::detail::empty_cpu({2}, at::kInt, true);
-            host = words.data_ptr<int32_t>();
-            host[0] = host[1] = 0;
+        bool declined = false;
+        {
+            Unlocked u;
+            hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+            if (check) declined = hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone;
+            if (check && !declined) {
+                words = at::detail::empty_cpu({2}, at::kInt, true);
+                host = words.data_ptr<int32_t>();
+                host[0] = host[1] = 0;
+            }
+            if (!declined) {
+                at::DimVector grid(x->sizes().begin(), x->sizes().end());
+                grid[grid.size() - 2] = rows / bm;
+                grid[grid.size() - 1] = cols / bn;
+                q = make(x->sizes(), at::kFloat8_e4m3fn, dev), s = make(grid, scale_type((int)v[3]), dev);
+                declined = p_quant_fp8(x->const_data_ptr(), x->scalar_type() == at::kFloat ? LP_F32 : LP_BF16, x->numel() / cols, cols, (int)bm,
+                                       (int)bn, (int)v[2], (float)floor, (int)v[4], q.data_ptr(), s.data_ptr(), (int)v[3], host, st) != LP_OK;
+            }
+            // the counter and the flag stay allocated until the GPU is through with them
+            if (check && !declined) C10_HIP_CHECK(p_flag(host + 1, st) ? hipStreamSynchronize(st) : wait_flag(host + 1, st));
         }
-        at::DimVector grid(x->sizes().begin(), x->sizes().end());
-        grid[grid.size() - 2] = rows / bm;
-        grid[grid.size() - 1] = cols / bn;
-        at::Tensor q = make(x->sizes(), at::kFloat8_e4m3fn, dev), s = make(grid, scale_type((int)v[3]), dev);
-        if (p_quant_fp8(x->const_data_ptr(), x->scalar_type() == at::kFloat ? LP_F32 : LP_BF16, x->numel() / cols, cols, (int)bm, (int)bn,
-                        (int)v[2], (float)floor, (int)v[4], q.data_ptr(), s.data_ptr(), (int)v[3], host, st))
-            Py_RETURN_NONE;
+        if (declined) Py_RETURN_NONE;
         if (!check) return pair(q, s);
-        hipError_t done;
-        // the counter and the flag stay allocated until the GPU is through with them
-        if (p_flag(host + 1, st)) {
-            done = hipStreamSynchronize(st);
-        } else {
-            Py_BEGIN_ALLOW_THREADS
-            done = wait_flag(host + 1, st);
-            Py_END_ALLOW_THREADS
-        }
-        C10_HIP_CHECK(done);
         PyObject *two = pair(q, s);
         PyObject *r = two ? PyTuple_Pack(3, PyTuple_GET_ITEM(two, 0), PyTuple_GET_ITEM(two, 1), host[0] ? Py_True : Py_False) : nullptr;
         Py_XDECREF(two);
@@ -187,11 +192,16 @@ PyObject *dequant(PyObject *, PyObject *const *args, Py_ssize_t n)
             if (c->size(d) != s->size(d)) Py_RETURN_NONE;
         at::DimVector shape(c->sizes().begin(), c->sizes().end());
         shape[shape.size() - 1] = cols;
-        at::Tensor out = make(shape, v[2] == LP_F32 ? at::kFloat : at::kBFloat16, dev);
         const int64_t all_rows = c->numel() / c->size(-1);
         const int bm = (int)(rows / sr), bn = (int)(cols / scol);
-        const int rc = v[0] ? p_dequant_fp4(c->const_data_ptr(), s->const_data_ptr(), sc, all_rows, cols, bm, bn, (int)v[1], out.data_ptr(), (int)v[2], stream(dev))
-                            : p_dequant_fp8(c->const_data_ptr(), s->const_data_ptr(), sc, all_rows, cols, bm, bn, out.data_ptr(), (int)v[2], stream(dev));
+        at::Tensor out;
+        int rc;
+        {
+            Unlocked u;
+            out = make(shape, v[2] == LP_F32 ? at::kFloat : at::kBFloat16, dev);
+            rc = v[0] ? p_dequant_fp4(c->const_data_ptr(), s->const_data_ptr(), sc, all_rows, cols, bm, bn, (int)v[1], out.data_ptr(), (int)v[2], stream(dev))
+                      : p_dequant_fp8(c->const_data_ptr(), s->const_data_ptr(), sc, all_rows, cols, bm, bn, out.data_ptr(), (int)v[2], stream(dev));
+        }
         if (rc) Py_RETURN_NONE;
         return THPVariable_Wrap(out);
     )
@@ -213,10 +223,15 @@ PyObject *fp4_to_fp8(PyObject *, PyObject *const *args, Py_ssize_t n)
             Py_RETURN_NONE;
         const int64_t rows = x->size(0), cols = x->size(1) * 2;
         if (rows % 128 || cols % 128 || s->size(0) != rows || s->size(1) != cols / 32 || v[3] < 0 || v[3] > LP_E8M0) Py_RETURN_NONE;
-        at::Tensor q = make({rows, cols}, at::kFloat8_e4m3fn, dev), so = make({rows / 128, cols / 128}, scale_type((int)v[3]), dev);
-        const int rc = v[0] ? p_fp4_amax(x->const_data_ptr(), s->const_data_ptr(), rows, cols, (int)v[1], (float)floor, (int)v[2], q.data_ptr(),
-                                         so.data_ptr(), (int)v[3], nullptr, stream(dev))
-                            : p_fp4_rebase(x->const_data_ptr(), s->const_data_ptr(), rows, cols, q.data_ptr(), so.data_ptr(), (int)v[3], stream(dev));
+        at::Tensor q, so;
+        int rc;
+        {
+            Unlocked u;
+            q = make({rows, cols}, at::kFloat8_e4m3fn, dev), so = make({rows / 128, cols / 128}, scale_type((int)v[3]), dev);
+            rc = v[0] ? p_fp4_amax(x->const_data_ptr(), s->const_data_ptr(), rows, cols, (int)v[1], (float)floor, (int)v[2], q.data_ptr(),
+                                   so.data_ptr(), (int)v[3], nullptr, stream(dev))
+                      : p_fp4_rebase(x->const_data_ptr(), s->const_data_ptr(), rows, cols, q.data_ptr(), so.data_ptr(), (int)v[3], stream(dev));
+        }
         if (rc) Py_RETURN_NONE;
         return pair(q, so);
     )
@@ -238,12 +253,18 @@ PyObject *gemm(PyObject *, PyObject *const *args, Py_ssize_t n)
         const int64_t M = a->size(0), K = a->size(1), N = b->size(0);
         if (b->size(1) != K || K % 128 || N % 128 || sa->size(0) != M || sa->size(1) != K / 128 || sb->size(0) != N / 128 || sb->size(1) != K / 128)
             Py_RETURN_NONE;
-        at::Tensor c = make({M, N}, out_code == LP_BF16 ? at::kBFloat16 : at::kFloat, dev), ws;
-        const int64_t need = p_gemm_ws(M, N, K);
-        if (need > 0) ws = make({need}, at::kByte, dev);
-        if (p_gemm(a->const_data_ptr(), sa->const_data_ptr(), b->const_data_ptr(), sb->const_data_ptr(), scale_code(sa->scalar_type()), M, N, K,
-                   c.data_ptr(), (int)out_code, need > 0 ? ws.data_ptr() : nullptr, need, stream(dev)))
-            Py_RETURN_NONE;
+        at::Tensor c;
+        int rc;
+        {
+            Unlocked u;
+            at::Tensor ws;
+            c = make({M, N}, out_code == LP_BF16 ? at::kBFloat16 : at::kFloat, dev);
+            const int64_t need = p_gemm_ws(M, N, K);
+            if (need > 0) ws = make({need}, at::kByte, dev);
+            rc = p_gemm(a->const_data_ptr(), sa->const_data_ptr(), b->const_data_ptr(), sb->const_data_ptr(), scale_code(sa->scalar_type()), M, N, K,
+                        c.data_ptr(), (int)out_code, need > 0 ? ws.data_ptr() : nullptr, need, stream(dev));
+        }
+        if (rc) Py_RETURN_NONE;
         return THPVariable_Wrap(c);
     )
 }

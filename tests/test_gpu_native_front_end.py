@@ -1,6 +1,10 @@
 """The native front end of the calls made most often (csrc/host/native.cpp): its answers are those of the wrappers' own way
-through the C ABI, and what goes wrong in it reaches Python as it does there."""
+through the C ABI, what goes wrong in it reaches Python as it does there, and other threads run meanwhile."""
 import contextlib
+import ctypes
+import subprocess
+import threading
+import time
 
 import pytest
 import torch
@@ -79,3 +83,63 @@ def test_out_of_memory_is_torchs_own_error(G, name):
             call()
     got = parts(call())
     assert all(torch.equal(bits(a), b) for a, b in zip(got, want))
+
+
+# What the front end calls instead of the library: waits (two seconds at most) until another thread says go, and refuses.
+STAND_IN = """
+#include <unistd.h>
+volatile int inside, go, late;
+int stand_in(void) { inside = 1; for (int i = 0; i < 2000; ++i) { if (go) return -1; usleep(1000); } late = 1; return -1; }
+"""
+
+
+@pytest.fixture(scope="module")
+def stand_in(tmp_path_factory):
+    d = tmp_path_factory.mktemp("stand_in")
+    (d / "s.c").write_text(STAND_IN)
+    subprocess.check_call(["gcc", "-O1", "-shared", "-fPIC", "-o", str(d / "s.so"), str(d / "s.c")])
+    return ctypes.CDLL(str(d / "s.so"))
+
+
+@contextlib.contextmanager
+def bound(function):
+    """The front end's module with `function` in the place of the library's entries that launch."""
+    from gcore_lowp import _abi as A, _native
+    mod = _native._load()
+    real = [ctypes.cast(getattr(A.lib(), n), ctypes.c_void_p).value for n in _native._BOUND]
+    fake = ctypes.cast(function, ctypes.c_void_p).value
+    mod.bind(*[a if n in ("lp_gemm_workspace_bytes", "lp_host_flag") else fake for n, a in zip(_native._BOUND, real)])
+    try:
+        yield mod
+    finally:
+        mod.bind(*real)
+
+
+@pytest.mark.parametrize("name", ["quant_fp8", "quant_fp8_checked", "dequant", "fp4_to_fp8", "gemm"])
+def test_other_threads_run_while_a_launch_waits(G, stand_in, name):
+    """A launch can wait for room in a full queue, an allocation for the device."""
+    from gcore_lowp import _abi as A
+    x = torch.zeros(128, 256, device="cuda", dtype=torch.bfloat16)
+    (q, s), packed = G.quant_2d(x), torch.zeros(128, 128, device="cuda", dtype=torch.int8)
+    fs, (aq, sa) = torch.ones(128, 8, device="cuda").to(E8M0), G.quant_1d(x)
+    word = {n: ctypes.c_int.in_dll(stand_in, n) for n in ("inside", "go", "late")}
+    for w in word.values():
+        w.value = 0
+
+    def other():
+        while not word["inside"].value and not word["late"].value:
+            time.sleep(0.001)
+        word["go"].value = 1
+
+    with bound(stand_in.stand_in) as mod:
+        call = {"quant_fp8": lambda: mod.quant_fp8(x, 1, 128, A.SCALE_DIV, A.F32, A.ZERO_NONE, 1e-12, False),
+                "quant_fp8_checked": lambda: mod.quant_fp8(x, 128, 128, A.SCALE_POW2, A.E8M0, A.ZERO_NONE, 0.0, True),
+                "dequant": lambda: mod.dequant(q, s, False, A.FP4_NEG_ZERO, A.BF16),
+                "fp4_to_fp8": lambda: mod.fp4_to_fp8(packed, fs, 1, A.SCALE_DIV, A.ZERO_NONE, A.F32, 1e-12),
+                "gemm": lambda: mod.gemm(aq, sa, q, s, A.BF16)}[name]
+        t = threading.Thread(target=other)
+        t.start()
+        r = call()
+        t.join()
+    assert word["inside"].value == 1 and r is None
+    assert not word["late"].value, "no other thread ran during the call"
