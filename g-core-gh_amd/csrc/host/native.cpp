@@ -160,10 +160,13 @@ PyObject *quant_fp8(PyObject *, PyObject *const *args, Py_ssize_t n)
                 grid[grid.size() - 2] = rows / bm;
                 grid[grid.size() - 1] = cols / bn;
                 q = make(x->sizes(), at::kFloat8_e4m3fn, dev), s = make(grid, scale_type((int)v[3]), dev);
-                declined = p_quant_fp8(x->const_data_ptr(), x->scalar_type() == at::kFloat ? LP_F32 : LP_BF16, x->numel() / cols, cols, (int)bm,
-                                       (int)bn, (int)v[2], (float)floor, (int)v[4], q.data_ptr(), s.data_ptr(), (int)v[3], host, st) != LP_OK;
+                const int rc = p_quant_fp8(x->const_data_ptr(), x->scalar_type() == at::kFloat ? LP_F32 : LP_BF16, x->numel() / cols, cols, (int)bm,
+                                       (int)bn, (int)v[2], (float)floor, (int)v[4], q.data_ptr(), s.data_ptr(), (int)v[3], host, st);
+                declined = rc != LP_OK;
+                // an error of the runtime may be an earlier call's: the kernel may be running
+                if (check && rc == LP_ERR_HIP) (void)hipStreamSynchronize(st);
             }
-            // the counter and the flag stay allocated until the GPU is through with them
+            // the counter and the flag stay allocated until the GPU is through with them (above too)
             if (check && !declined) C10_HIP_CHECK(p_flag(host + 1, st) ? hipStreamSynchronize(st) : wait_flag(host + 1, st));
         }
         if (declined) Py_RETURN_NONE;

@@ -89,6 +89,7 @@ def test_out_of_memory_is_torchs_own_error(G, name):
 STAND_IN = """
 #include <unistd.h>
 volatile int inside, go, late;
+int failed_launch(void) { return %d; }
 int stand_in(void) { inside = 1; for (int i = 0; i < 2000; ++i) { if (go) return -1; usleep(1000); } late = 1; return -1; }
 """
 
@@ -96,7 +97,7 @@ int stand_in(void) { inside = 1; for (int i = 0; i < 2000; ++i) { if (go) return
 @pytest.fixture(scope="module")
 def stand_in(tmp_path_factory):
     d = tmp_path_factory.mktemp("stand_in")
-    (d / "s.c").write_text(STAND_IN)
+    (d / "s.c").write_text(STAND_IN % -3)
     subprocess.check_call(["gcc", "-O1", "-shared", "-fPIC", "-o", str(d / "s.so"), str(d / "s.c")])
     return ctypes.CDLL(str(d / "s.so"))
 
@@ -143,3 +144,14 @@ def test_other_threads_run_while_a_launch_waits(G, stand_in, name):
         t.join()
     assert word["inside"].value == 1 and r is None
     assert not word["late"].value, "no other thread ran during the call"
+
+
+def test_counter_outlives_a_launch_that_reports_an_error(G, stand_in):
+    """The runtime's last error may be an earlier call's, the quantiser queued all the same and the NaN counter in pinned memory
+    still to be written: the call ends behind everything queued, and the counter's memory is given back only then."""
+    from gcore_lowp import _abi as A
+    x = torch.zeros(128, 128, device="cuda", dtype=torch.bfloat16)
+    with bound(stand_in.failed_launch) as mod:
+        torch.cuda._sleep(20_000_000)
+        assert mod.quant_fp8(x, 128, 128, A.SCALE_POW2, A.E8M0, A.ZERO_NONE, 0.0, True) is None
+        assert torch.cuda.current_stream().query()
