@@ -111,21 +111,33 @@ def _audit_asm_operands():
         raise RuntimeError("gemm_fp8_big.hip: an asm operand shares a register with the loop it feeds; not linking")
 
 
+def _native_built_for() -> str:
+    """What the extension's layouts and symbols depend on besides its sources (gcore_lowp/_native.py asks for the same)."""
+    import sysconfig
+    import torch
+    return f"torch {torch.__version__} {torch.version.git_version} {sysconfig.get_config_var('SOABI')}"
+
+
 def _build_native(force: bool) -> None:
     src = os.path.join(CSRC, "host", "native.cpp")
     deps = [src, os.path.join(HERE, "..", "include", "lowp.h")]
-    if not force and os.path.exists(NATIVE) and os.path.getmtime(NATIVE) >= max(os.path.getmtime(d) for d in deps):
+    key, key_file = _native_built_for(), os.path.join(OBJ, "_lowp_native.built_for")
+    made_for = open(key_file).read() if os.path.exists(key_file) else None
+    if not force and made_for == key and os.path.exists(NATIVE) and os.path.getmtime(NATIVE) >= max(os.path.getmtime(d) for d in deps):
         return
     import sysconfig
     import torch
     root = os.path.dirname(torch.__file__)
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f'-DLOWP_BUILT_FOR="{key}"',
            "-I" + sysconfig.get_paths()["include"], "-isystem", os.path.join(root, "include"),
            "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"), "-isystem", "/opt/rocm/include", src, "-o", NATIVE,
            "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"g++ failed for host/native.cpp:\n{r.stderr}")
+    with open(key_file, "w") as f:
+        f.write(key)
 
 
 def build(force: bool = False) -> str:

@@ -278,4 +278,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_lowp_native", nullptr, -1, method
 
 }  // namespace
 
-extern "C" __attribute__((visibility("default"))) PyObject *PyInit__lowp_native() { return PyModule_Create(&module); }
+extern "C" __attribute__((visibility("default"))) PyObject *PyInit__lowp_native()
+{
+    PyObject *m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "built_for", LOWP_BUILT_FOR)) Py_CLEAR(m);
+    return m;
+}
