@@ -155,3 +155,208 @@ def test_counter_outlives_a_launch_that_reports_an_error(G, stand_in):
         torch.cuda._sleep(20_000_000)
         assert mod.quant_fp8(x, 128, 128, A.SCALE_POW2, A.E8M0, A.ZERO_NONE, 0.0, True) is None
         assert torch.cuda.current_stream().query()
+
+
+class Counted:
+    """Counts what the front end answered and what it left to the wrapper."""
+
+    def __init__(self, monkeypatch):
+        from gcore_lowp import _native
+        mod = _native._load()
+        self.answered, self.left = 0, 0
+        for n in _native._ENTRIES:
+            monkeypatch.setattr(_native.fast, n, self.counting(getattr(mod, n)), raising=False)
+
+    def counting(self, f):
+        def entry(*args):
+            r = f(*args)
+            if r is None:
+                self.left += 1
+            else:
+                self.answered += 1
+            return r
+        return entry
+
+
+@pytest.fixture
+def counted(monkeypatch):
+    return Counted(monkeypatch)
+
+
+@contextlib.contextmanager
+def without_front_end(monkeypatch):
+    from gcore_lowp import _native
+    with monkeypatch.context() as m:
+        for n in _native._ENTRIES:
+            m.setattr(_native.fast, n, lambda *args: None, raising=False)
+        yield
+
+
+def same(a, b):
+    return all(x.dtype == y.dtype and x.shape == y.shape and x.stride() == y.stride() and x.device == y.device
+               and torch.equal(bits(x), bits(y)) for x, y in zip(parts(a), parts(b))) and len(parts(a)) == len(parts(b))
+
+
+@pytest.mark.parametrize("name", NAMES)
+@pytest.mark.parametrize("rows,cols", [(128, 128), (256, 1024), (1152, 640)])
+def test_answers_are_the_wrappers(G, counted, monkeypatch, name, rows, cols):
+    call = calls(G, rows, cols)[name]
+    before = counted.answered
+    got = call()
+    assert counted.answered == before + 1 and not counted.left, "the front end takes this call"
+    with without_front_end(monkeypatch):
+        want = call()
+    assert same(got, want)
+
+
+def views(t):
+    """the values of t in other clothes: a stride in rows, in columns, an offset that is not aligned"""
+    wide = torch.zeros(t.shape[0], t.shape[1] * 2, dtype=t.dtype, device=t.device)
+    wide[:, :t.shape[1]].copy_(t)
+    apart = torch.zeros(t.shape[1], t.shape[0], dtype=t.dtype, device=t.device)
+    apart.copy_(t.t())
+    shifted = torch.zeros(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+    shifted.copy_(t)
+    return {"rows apart": wide[:, :t.shape[1]], "transposed": apart.t(), "shifted": shifted}
+
+
+@pytest.mark.parametrize("clothes", ["rows apart", "transposed", "shifted", "on the host", "half", "leading dims"])
+def test_what_is_not_plain_is_answered_as_before(G, monkeypatch, counted, clothes):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(256, 384, generator=g, device="cuda", dtype=torch.bfloat16)
+    if clothes == "on the host":
+        y = x.cpu()
+    elif clothes == "half":
+        y = x.half()
+    elif clothes == "leading dims":
+        y = x.view(2, 128, 384)
+    else:
+        y = views(x)[clothes]
+    for f in (G.quant_1d, G.quant_fp8_e4m3_scale_e8m0, lambda t: G.quant_fp8_e4m3_scale_e8m0(t, (1, 128)), lambda t: G.quant_1d(t, 32)):
+        got = f(y)
+        with without_front_end(monkeypatch):
+            want = f(y)
+        assert same(got, want), clothes
+    if clothes in ("rows apart", "transposed", "on the host", "half"):
+        assert not counted.answered
+    if clothes in ("rows apart", "transposed"):
+        q, s = G.quant_fp8_e4m3_scale_e8m0(x)
+        v = views(q.view(torch.uint8))[clothes].view(E4M3) if clothes == "rows apart" else q.t().contiguous().t()
+        before = counted.answered
+        assert same(G.dequant_fp4_e2m1_fp8_scale_e8m0_packed(v, s), G.dequant_fp4_e2m1_fp8_scale_e8m0_packed(q, s))
+        assert counted.answered == before + 1                      # the plain one alone
+
+
+def test_refusals_are_the_wrappers(G, counted):
+    x = torch.zeros(128, 256, device="cuda", dtype=torch.bfloat16)
+    q, s = G.quant_fp8_e4m3_scale_e8m0(x)
+    aq, sa = G.quant_1d(x)
+    bq, sb = G.quant_2d(x)
+    counted.answered = 0
+    with pytest.raises(ValueError, match="not divisible"):
+        G.dequant_fp4_e2m1_fp8_scale_e8m0_packed(q, s.view(torch.uint8).repeat(3, 1).view(E8M0))
+    with pytest.raises(ValueError, match="leading dims"):
+        G.dequant_fp4_e2m1_fp8_scale_e8m0_packed(q.view(torch.uint8).expand(2, 128, 256).contiguous().view(E4M3),
+                                                 s.view(torch.uint8).expand(3, 1, 2).contiguous().view(E8M0))
+    with pytest.raises(AssertionError):
+        G.quant_fp8_e4m3_scale_e8m0(x[:100])
+    with pytest.raises(AssertionError):
+        G.gemm_fp8_block_scaling_impl(aq, sa[:64], bq, sb)
+    with pytest.raises(AssertionError):
+        G.gemm_fp8_block_scaling_impl(aq, sa, bq, sb, out_dtype=torch.float16)
+    with pytest.raises(AssertionError):
+        G.cast_e2m1fn_to_e4m3fn(torch.zeros(100, 64, device="cuda", dtype=torch.int8), torch.ones(100, 4, device="cuda").to(E8M0))
+    for empty in (x[:0], x[:, :0]):
+        with contextlib.suppress(Exception):
+            G.quant_1d(empty)
+    assert not counted.answered
+
+
+@pytest.mark.parametrize("bad", [None, 0, 1000, 16383])
+@pytest.mark.parametrize("queue", ["empty", "long"])
+def test_nan_check_on_a_stream_of_its_own(G, counted, bad, queue):
+    """The flag is waited for on the stream the call was made on, for longer than it is watched (200 us) where much is queued in
+    front of it; every call has a counter of its own."""
+    side = torch.cuda.Stream()
+    x = torch.randn(128, 16384, device="cuda", dtype=torch.bfloat16)
+    if bad is not None:
+        x[7, bad] = float("nan")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            if queue == "long":
+                torch.cuda._sleep(20_000_000)
+            queued = torch.cuda.Event()
+            queued.record()
+            if bad is None:
+                q, s = G.quant_fp8_e4m3_scale_e8m0(x)
+                assert queued.query(), "the answer is that of everything queued before"
+            else:
+                with pytest.raises(AssertionError, match="contains NaN"):
+                    G.quant_fp8_e4m3_scale_e8m0(x)
+    assert counted.answered == 3
+    if bad is None:
+        torch.cuda.synchronize()
+        want = G.quant_fp8_e4m3_scale_e8m0(x)
+        assert same((q, s), want)
+
+
+def test_every_block_with_a_nan_is_seen(G):
+    x = torch.zeros(1024, 2048, device="cuda", dtype=torch.bfloat16)
+    for r in range(0, 1024, 128):
+        for c in range(0, 2048, 128):
+            x.zero_()
+            x[r + 77, c + 11] = float("nan")
+            with pytest.raises(AssertionError, match="contains NaN"):
+                G.quant_fp8_e4m3_scale_e8m0(x)
+
+
+@pytest.mark.parametrize("name", [n for n in NAMES if n != "quant_e8m0"])
+def test_captured_calls(G, counted, name):
+    """Under capture the front end answers too; replays, with other work between them, give the eager result each time."""
+    call = calls(G)[name]
+    want = [bits(t).clone() for t in parts(call())]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    before = counted.answered
+    with torch.cuda.graph(graph):
+        got = parts(call())
+    assert counted.answered == before + 1
+    for _ in range(3):
+        for t in got:
+            bits(t).zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(bits(a), b) for a, b in zip(got, want)), name
+        call()
+
+
+def test_threads_with_streams_of_their_own(G):
+    """Calls from several threads at once, each on its own stream and its own operands."""
+    wrong = []
+
+    def work(seed):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                g = torch.Generator(device="cuda").manual_seed(seed)
+                x = torch.randn(256, 512 + 128 * seed, generator=g, device="cuda", dtype=torch.bfloat16)
+                first = None
+                for _ in range(20):
+                    q, s = G.quant_fp8_e4m3_scale_e8m0(x)
+                    aq, sa = G.quant_1d(x)
+                    c = G.gemm_fp8_block_scaling_impl(aq, sa, *G.quant_2d(x))
+                    back = G.dequant_fp4_e2m1_fp8_scale_e8m0_packed(q, s)
+                    r = [bits(t).clone() for t in (q, s, aq, sa, c, back)]
+                    first = first or r
+                    if not all(torch.equal(a, b) for a, b in zip(r, first)):
+                        wrong.append((seed, "differs from its first result"))
+                assert (back.float() - x.float()).abs().max() <= x.float().abs().max() / 16
+        except BaseException as e:
+            wrong.append((seed, repr(e)))
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not wrong, wrong
