@@ -20,16 +20,17 @@ __device__ __forceinline__ float scale_at(const void *s, int64_t idx)
 constexpr int GROUP_M = 8, GROUP_N = 4, CHUNK = GROUP_M * GROUP_N;
 
 // Tile `lin` of the numbering.
-__device__ __forceinline__ void tile_of(int64_t lin, int64_t tiles_m, int64_t tiles_n, int64_t &tm, int64_t &tn)
+template <class I>
+__device__ __forceinline__ void tile_of(I lin, I tiles_m, I tiles_n, int64_t &tm, int64_t &tn)
 {
     // groups of GROUP_M m-tiles (the last may be short); inside a group, blocks of
     // GROUP_N n-tiles (the last may be narrow); inside a block m runs fastest
-    const int64_t per_group = GROUP_M * tiles_n;
-    const int64_t grp = lin / per_group, in_grp = lin - grp * per_group;
-    const int64_t left = tiles_m - grp * GROUP_M;
-    const int64_t gm = left < GROUP_M ? left : GROUP_M;
-    const int64_t per_nblock = gm * GROUP_N;
-    const int64_t nblk = in_grp / per_nblock, in_blk = in_grp - nblk * per_nblock;
+    const I per_group = GROUP_M * tiles_n;
+    const I grp = lin / per_group, in_grp = lin - grp * per_group;
+    const I left = tiles_m - grp * GROUP_M;
+    const I gm = left < GROUP_M ? left : GROUP_M;
+    const I per_nblock = gm * GROUP_N;
+    const I nblk = in_grp / per_nblock, in_blk = in_grp - nblk * per_nblock;
     tm = grp * GROUP_M + in_blk % gm;
     tn = nblk * GROUP_N + in_blk / gm;
 }
@@ -49,35 +50,39 @@ __device__ __forceinline__ bool tile_coords(int64_t b, int64_t tiles_m, int64_t 
     }
     const int64_t lin = (q * 8 + xcd) * CHUNK + s % CHUNK;
     if (lin >= tiles_m * tiles_n) return false;
-    tile_of(lin, tiles_m, tiles_n, tm, tn);
+    tile_of<int64_t>(lin, tiles_m, tiles_n, tm, tn);
     return true;
 }
 
-// The tiles of G problems of one shape: every problem is cut into pieces of `piece` consecutive tiles, and the pieces of all
-// problems are dealt to the XCDs in turn.  (Numbered problem by problem as above, a problem of few tiles ran on few XCDs: 20
-// weight gradients of 1024 x 1408 with three K blocks, 24 tiles each, on one of eight: 131 us, dealt in turn 30.)  Workgroup b -> problem g and its tile; false: none.
-__device__ __forceinline__ bool list_coords(int64_t b, int64_t G, int64_t tiles_m, int64_t tiles_n, int piece, int64_t &g, int64_t &tm, int64_t &tn)
+// The tiles of G problems of one shape, numbered problem by problem: pieces of 2^shift consecutive ones are dealt to the XCDs in
+// turn.  (With every problem dealt from XCD 0 on as above, a problem of few tiles ran on few XCDs: 20 weight gradients of 1024 x
+// 1408 with three K blocks, 24 tiles each, on one of eight: 131 us, dealt in turn 30.  With pieces that end with their problem, the
+// last and smaller ones could all fall to the same XCDs: 32 problems of 1408 x 2048 with
+// sixteen K blocks, 48 tiles each, 200 us, across problems 166.)  Workgroup b ->
+// problem g and its tile; false: none.  In 32 bits, which hold the grid and so every number here: the divisions stand in front of
+// a workgroup's first request, and in 64 bits they took 0.4 us (one problem of 128 x 256 with eight K blocks 6.6 us, so 6.1).
+__device__ __forceinline__ bool list_coords(uint32_t b, uint32_t G, uint32_t tiles_m, uint32_t tiles_n, int shift, int64_t &g, int64_t &tm, int64_t &tn)
 {
-    const int64_t tiles = tiles_m * tiles_n, per = (tiles + piece - 1) / piece, s = b >> 3;
-    const int64_t p = s / piece * 8 + (b & 7);
-    g = p / per;
-    const int64_t lin = (p - g * per) * piece + s % piece;
-    if (g >= G || lin >= tiles) return false;
-    tile_of(lin, tiles_m, tiles_n, tm, tn);
+    const uint32_t tiles = tiles_m * tiles_n, s = b >> 3;
+    const uint32_t id = (((s >> shift) * 8 + (b & 7)) << shift) + (s & ((1u << shift) - 1)), problem = id / tiles;
+    if (problem >= G) return false;
+    g = problem;
+    tile_of<uint32_t>(id - problem * tiles, tiles_m, tiles_n, tm, tn);
     return true;
 }
 
 // Whole chunks, whose operand panels are shared in an L2, where that leaves the XCDs alike; a quarter of one otherwise.
-inline int list_piece(int64_t G, int64_t tiles_m, int64_t tiles_n)
+inline int list_shift(int64_t G, int64_t tiles_m, int64_t tiles_n)
 {
-    const int64_t chunks = G * ((tiles_m * tiles_n + CHUNK - 1) / CHUNK);
-    return (chunks + 7) / 8 * 8 * 4 <= chunks * 5 ? CHUNK : GROUP_M;
+    static_assert(CHUNK == 1 << 5 && GROUP_M == 1 << 3);
+    const int64_t chunks = (G * tiles_m * tiles_n + CHUNK - 1) / CHUNK;
+    return (chunks + 7) / 8 * 8 * 4 <= chunks * 5 ? 5 : 3;
 }
 
-inline int64_t list_grid(int64_t G, int64_t tiles_m, int64_t tiles_n, int piece)
+inline int64_t list_grid(int64_t G, int64_t tiles_m, int64_t tiles_n, int shift)
 {
-    const int64_t pieces = G * ((tiles_m * tiles_n + piece - 1) / piece);
-    return (pieces + 7) / 8 * 8 * piece;
+    const int64_t round = 8ll << shift;
+    return (G * tiles_m * tiles_n + round - 1) / round * round;
 }
 
 // Rows of expert e from the caller's offset table, made safe to use: both ends are clamped to [0, M_total] and a

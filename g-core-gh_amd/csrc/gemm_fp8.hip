@@ -478,7 +478,7 @@ extern "C" int lp_gemm_fp8_rowscale(const void *Aq, const void *As, const void *
         ((uintptr_t)Aq | (uintptr_t)Bq) % 16 == 0)
         return gemm::launch_rowscale_small(Aq, As, Bq, Bs, nullptr, 1, (int)(K / 128), M, N, C, out_dtype, st);
     if (gemm::rowscale_asm_ok(As, Bs, scale_dtype, M, N, K))
-        return gemm::launch_rowscale_asm(Aq, As, Bq, Bs, nullptr, 1, (int)(K / 128), 1, M, N, C, out_dtype, st);
+        return gemm::launch_rowscale_asm(Aq, As, Bq, Bs, nullptr, 1, (int)(K / 128), K % 512 ? 1 : 4, M, N, C, out_dtype, st);
     if (scale_dtype == LP_F32)
         hipLaunchKernelGGL((gemm_dense<LP_F32, true>), dim3((unsigned)grid), dim3(256), 0, st, (const uint8_t *)Aq, As,
                            (const uint8_t *)Bq, Bs, scale_dtype, M, N, K, tiles_m, tiles_n, C, N, out_dtype);

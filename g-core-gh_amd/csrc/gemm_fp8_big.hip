@@ -359,7 +359,7 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
                   "weights stored [K, N]: hardware-scaled 256 x 256 and 128 x 256 tiles");
     static_assert(!DUAL || (TM == 128 && TN == 128), "the K split inside a workgroup is built for the 128 x 128 tile");
     static_assert(NST == 2 || (NST == 3 && WN == 4) || (NST == 4 && TM == 128 && TN == 128 && KSUB == 1 && !DUAL), "three stages: flat tile, four: 128 x 128 tile");
-    static_assert(!BROW || (HWS && RAG && TM == TN && KSUB == 1 && !DUAL && NST == 2), "row-scaled weights: hardware-scaled 128 x 128 and 256 x 256 loops for any K");
+    static_assert(!BROW || (HWS && (RAG || TM == 128) && TM == TN && KSUB == 1 && !DUAL && NST == 2), "row-scaled weights: hardware-scaled 128 x 128 loops, 256 x 256 for any K");
     static_assert((TM / 8 / WAVES == 4 || (WN == 4 && TM / 8 / WAVES == 2)) && (TN / 8 / WAVES == 4 || TN / 8 / WAVES == 3),
                   "copies per operand and wave");
     constexpr int NBC = TN / 8 / WAVES;                 // weight copies per wave and K block
@@ -498,7 +498,8 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
     const uint32_t srd = HWS ? lds0 + T::S_LDS + wm * 1024 + l16 * 4 : lds0 + T::S_LDS + arow_l * 16;
     // row-scaled weights: their dwords live behind the two activation halves, 1 KB per copying wave (64 rows) like those
     const uint32_t srdb = lds0 + T::S_LDS + TM * 32 + wn * (TN / WN * 16) + l16 * 4;
-    (void)srdb;
+    const uint32_t sdst = __builtin_amdgcn_readfirstlane((uint32_t)(T::S_LDS + (copies_weights ? TM * 16 : 0)));
+    (void)srdb; (void)sdst;
 
     f32x16v accs[NBW];
     if constexpr (TN == 288) {
@@ -652,11 +653,19 @@ __device__ __forceinline__ void tile_asm(uint8_t *smem, const uint8_t *__restric
         accs[4] = acc4; accs[5] = acc5; accs[6] = acc6; accs[7] = acc7;
     } else if constexpr (BROW) {
         f32x16v acc0, acc1, acc2, acc3;
-        asm volatile(
+        if constexpr (RAG) {
+            asm volatile(
 #include "gemm_mid_hwrow_rag_loop.inc"
-            : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
-            : LP_ASM_INPUTS, LP_ASM_INPUTS_RAG, [srdb] "v"(srdb)
-            : LP_ASM_CLOBBERS, LP_ASM_CLOBBERS_RAG);
+                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
+                : LP_ASM_INPUTS, LP_ASM_INPUTS_RAG, [srdb] "v"(srdb)
+                : LP_ASM_CLOBBERS, LP_ASM_CLOBBERS_RAG);
+        } else {
+            asm volatile(
+#include "gemm_mid_hwrow_loop.inc"
+                : "=&{v[128:143]}"(acc0), "=&{v[144:159]}"(acc1), "=&{v[160:175]}"(acc2), "=&{v[176:191]}"(acc3)
+                : LP_ASM_INPUTS, [sdst] "s"(sdst), [srdb] "v"(srdb)
+                : LP_ASM_CLOBBERS);
+        }
         accs[0] = acc0; accs[1] = acc1; accs[2] = acc2; accs[3] = acc3;
     } else if constexpr (HWS && NST == 4) {
         f32x16v acc0, acc1, acc2, acc3;
@@ -1080,23 +1089,23 @@ __global__ __launch_bounds__(512) void gemm_asm_mixed(const uint8_t *__restrict_
 // problems that share M and N and differ in K (the weight gradients of the experts).  Entry g of `groups` = {output slot, K
 // blocks of 128, K blocks of all problems before it in the operand buffers, unused}: problem g reads Aq + M * 128 * before (its
 // [M, K_g] codes), As + M * before, the same for B with N, and writes C + slot * M * N.
-template <int TM>
+template <int TM, bool RAG>
 __global__ __launch_bounds__(TM * 2) void gemm_asm_rowscale(const uint8_t *__restrict__ Aq, const float *__restrict__ As,
                                                             const uint8_t *__restrict__ Bq, const float *__restrict__ Bs,
                                                             const int32_t *__restrict__ groups, int G, int64_t M, int64_t N,
-                                                            int64_t tiles_m, int64_t tiles_n, int piece,
+                                                            uint32_t tiles_m, uint32_t tiles_n, int shift,
                                                             void *__restrict__ C, int out_dtype, int max_k_blocks, int multiple)
 {
     __shared__ __attribute__((aligned(1024))) uint8_t smem[AsmTile<TM, TM, 1>::LDS_BYTES + TM * 32];
     int64_t g, tm, tn;
-    if (!gemm::list_coords(blockIdx.x, G, tiles_m, tiles_n, piece, g, tm, tn)) return;
+    if (!gemm::list_coords(blockIdx.x, (uint32_t)G, tiles_m, tiles_n, shift, g, tm, tn)) return;
     const int64_t slot = groups ? groups[4 * g] : 0, before = groups ? groups[4 * g + 2] : 0;
     const int kb = groups ? groups[4 * g + 1] : max_k_blocks;
     // an entry that breaks the caller's promise writes nothing: more K blocks than max_k_blocks (on which the host checked
     // that the operands fit 32-bit offsets), a count that is no multiple of the promised one, a negative slot or offset
     if (kb <= 0 || kb > max_k_blocks || kb % multiple || slot < 0 || before < 0) return;
     char *c = (char *)C + slot * M * N * (out_dtype == LP_BF16 ? 2 : 4);
-    tile_asm<TM, TM, 1, true, false, 2, true, true, 2, false, false, true>(
+    tile_asm<TM, TM, 1, true, false, 2, true, true, 2, false, false, RAG>(
         smem, Aq + M * 128 * before, (const float *)((const char *)As + M * before), Bq + N * 128 * before,
         (const float *)((const char *)Bs + N * before), tm * TM, M, tn * TM, N, (int64_t)kb * 128, c, N, out_dtype);
 }
@@ -1605,20 +1614,28 @@ bool rowscale_asm_ok(const void *As, const void *Bs, int scale_dtype, int64_t M,
 int launch_rowscale_asm(const void *Aq, const void *As, const void *Bq, const void *Bs, const int32_t *groups, int G, int max_k_blocks,
                         int multiple, int64_t M, int64_t N, void *C, int out_dtype, hipStream_t st)
 {
-    // 256 x 256 tiles (us per problem of 4096 x 4096 with 3 / 4 / 8 / 16 / 32 K blocks: 11.0 / 12.1 / 17.2 / 29.1 / 51.0 against
-    // 12.4 / 13.3 / 18.6 / 31.3 / 58.6 on 128 x 128 ones), unless they would cover more than a tenth beyond the matrix or leave
-    // CUs without one.
-    const int64_t big = ((M + 255) / 256) * ((N + 255) / 256);
-    const int tm = big * 65536 * 10 <= M * N * 11 && big * G >= 256 ? 256 : 128;
+    // 256 x 256 tiles where their rounds of one per CU cost less than 128 x 128 ones do, which four times as many share the CUs with
+    // little loss at the end (in hundredths of a full round of either).  The large ones are the better the longer the K loop is, and
+    // with a short one only where their stores run beside another round (us, 128 / 256: 4096 x 4096 with 4 / 8 / 11 / 16 / 32 K blocks
+    // 13.6 / 14.6, 22.1 / 20.5, 27.3 / 25.1, 34.5 / 31.5, 61.9 / 53.7; 8 of them with 4 100 / 96; 7168 x 7168, 3.06 rounds that take four, with
+    // 8 60.8 / 68.2; 32 x 1408 x 2048 with 16 180 / 166, 8 of them, 1.5 rounds, 48.7 / 53.3).
+    // The 128 x 128 loop for K in whole groups of four blocks starts without the scales' way through registers: up to 8 % where
+    // there is about one tile per CU (128 x 256 with 8 K blocks 6.6 -> 6.1 us, 1152 x 128 with 12 8.2 -> 7.6), level from ten rounds on.
+    const int64_t big = ((M + 255) / 256) * ((N + 255) / 256) * G, small = ((M + 127) / 128) * ((N + 127) / 128) * G;
+    const int64_t rounds = (big + 255) / 256, kb = max_k_blocks;
+    const int64_t cost = kb >= 32 ? 83 : kb >= 16 ? 88 : kb >= 11 ? 90 : kb >= 8 ? 92 : kb >= 5 ? 92 + 6 / rounds : 98 + 10 / rounds;
+    const int tm = big >= 256 && rounds * cost < small * 100 / 1024 + 8 ? 256 : 128;
+    const bool aligned = multiple % 4 == 0 && asm_shape_ok(As, Bs, M, N, (int64_t)max_k_blocks * 128, LP_E8M0);
     const int64_t tiles_m = (M + tm - 1) / tm, tiles_n = (N + tm - 1) / tm;
-    const int piece = gemm::list_piece(G, tiles_m, tiles_n);
-    const int64_t grid = gemm::list_grid(G, tiles_m, tiles_n, piece);
+    const int shift = gemm::list_shift(G, tiles_m, tiles_n);
+    const int64_t grid = gemm::list_grid(G, tiles_m, tiles_n, shift);
     if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_rowscale: problem too large");
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(tm * 2), 0, st, (const uint8_t *)Aq, (const float *)As, (const uint8_t *)Bq,
-                           (const float *)Bs, groups, G, M, N, tiles_m, tiles_n, piece, C, out_dtype, max_k_blocks, multiple);
+                           (const float *)Bs, groups, G, M, N, (uint32_t)tiles_m, (uint32_t)tiles_n, shift, C, out_dtype, max_k_blocks, multiple);
     };
-    tm == 256 ? go(gemm_asm_rowscale<256>) : go(gemm_asm_rowscale<128>);
+    if (tm == 256) go(gemm_asm_rowscale<256, true>);
+    else aligned ? go(gemm_asm_rowscale<128, false>) : go(gemm_asm_rowscale<128, true>);
     return check_launch("lp_gemm_fp8_rowscale(asm)");
 }
 

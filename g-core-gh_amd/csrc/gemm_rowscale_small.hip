@@ -36,13 +36,13 @@ constexpr int kPitch = 64 * 2 + 16, kWaveStage = 64 * kPitch;
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void gemm_rowscale_small(
     const uint8_t *__restrict__ Aq, const uint8_t *__restrict__ As, const uint8_t *__restrict__ Bq, const uint8_t *__restrict__ Bs,
-    const int32_t *__restrict__ groups, int G, int64_t M, int64_t N, int64_t tiles_m, int64_t tiles_n, int piece, void *__restrict__ C,
+    const int32_t *__restrict__ groups, int G, int64_t M, int64_t N, uint32_t tiles_m, uint32_t tiles_n, int shift, void *__restrict__ C,
     int out_dtype)
 {
     constexpr int TILE = 128 * 128, PITCH = 128;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * TILE > 4 * kWaveStage ? 2 * TILE : 4 * kWaveStage];
     int64_t g, tm, tn;
-    if (!gemm::list_coords(blockIdx.x, G, tiles_m, tiles_n, piece, g, tm, tn)) return;
+    if (!gemm::list_coords(blockIdx.x, (uint32_t)G, tiles_m, tiles_n, shift, g, tm, tn)) return;
     // no table: one problem
     const int64_t slot = groups ? groups[4 * g] : 0, kb = groups ? groups[4 * g + 1] : 1, before = groups ? groups[4 * g + 2] : 0;
     // an entry of another size (or one that breaks the caller's promises) is not this launch's: nothing is written
@@ -290,11 +290,11 @@ int launch_rowscale_small(const void *Aq, const void *As, const void *Bq, const 
                            (const uint8_t *)Bs, groups, G, M, N, (int)tiles_m, (int)tiles_n, (int)strip, piece, C, out_dtype);
         return check_launch("lp_gemm_fp8_rowscale_grouped(two K blocks)");
     }
-    const int piece = list_piece(G, tiles_m, tiles_n);
-    const int64_t grid = list_grid(G, tiles_m, tiles_n, piece);
+    const int shift = list_shift(G, tiles_m, tiles_n);
+    const int64_t grid = list_grid(G, tiles_m, tiles_n, shift);
     if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_rowscale_grouped: problem too large");
     hipLaunchKernelGGL(gemm_rowscale_small, dim3((unsigned)grid), dim3(256), 0, st, (const uint8_t *)Aq, (const uint8_t *)As, (const uint8_t *)Bq,
-                       (const uint8_t *)Bs, groups, G, M, N, tiles_m, tiles_n, piece, C, out_dtype);
+                       (const uint8_t *)Bs, groups, G, M, N, (uint32_t)tiles_m, (uint32_t)tiles_n, shift, C, out_dtype);
     return check_launch("lp_gemm_fp8_rowscale_grouped(one K block)");
 }
 

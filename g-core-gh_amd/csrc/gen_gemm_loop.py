@@ -52,7 +52,7 @@ def configure(tm, tn, waves_m, waves_n, ksub, hw=False, nstage=2, brow=False, ea
     # later.  Weight scales: fp32 by scalar loads of the group's length; e8m0 by a vector load of one address for all lanes.
     # nn: the scale bytes of the stored weight lie a table row apart, four byte loads per group, whatever that row's length.
     RAG = rag
-    # brow: the weight scales take the activation scales' way, loaded by the other half of the waves.
+    # brow: the weight scales take the activation scales' way, loaded (rag) or copied by the other half of the waves.
     assert not rag or (early and not wide and not bf16)
     # bf16: the operands are bf16 values (a K step of 128 bytes is 64 of them) and every matrix instruction of the
     # hardware-scaled loop becomes two v_mfma_f32_16x16x32_bf16 on the halves of the same fragment registers, accumulating
@@ -133,7 +133,7 @@ def configure(tm, tn, waves_m, waves_n, ksub, hw=False, nstage=2, brow=False, ea
     assert not ROT or not wide
     NSTAGE = nstage
     BROW = brow                 # weight scales per row and K step (e8m0, hardware-scaled loop only) instead of per 128 rows
-    assert not brow or (hw and rag and tm == tn)
+    assert not brow or (hw and tm == tn and (rag or tm == 128))
     assert nstage == 2 or (nstage in (3, 4) and ksub == 1)
     assert tm == 64 * waves_m
     WAVES = waves_m * waves_n
@@ -503,7 +503,10 @@ def scale_group_copy(tag):
     emit("s_cmp_eq_u32 s53, 0")
     emit(f"s_cbranch_scc1 Lnosc{tag}%=")
     emit("s_add_u32 m0, s48, s54")
-    emit(f"s_add_u32 m0, m0, {SCL_LDS}")
+    if BROW:
+        emit("s_add_u32 m0, m0, s51")                     # activation rows or weight rows: the set-up code says where
+    else:
+        emit(f"s_add_u32 m0, m0, {SCL_LDS}")
     emit("s_nop 0")
     emit("global_load_lds_dword %[soff], s[44:45]" if HW else "global_load_lds_dwordx4 %[soff], s[44:45]")
     emit(f"Lnosc{tag}%=:")
@@ -513,8 +516,8 @@ def scale_group_copy(tag):
 
 def weight_scale_load():
     """The four weight scales of the next group into s[60:63] (and those of the second scale row into s[68:71])."""
-    if RAG:
-        return                                            # they travel with the activation scales, see rag_scale_load
+    if RAG or BROW:
+        return                                            # they travel with the activation scales, see rag_scale_load, scale_group_copy
     if NN:
         # one byte per K step, a table row (s64 bytes) apart: the aligned dword around each, taken apart at the top of the loop
         for i in range(4):
@@ -890,6 +893,8 @@ def generate():
             emit("s_mov_b32 s65, %[bsbfe]")                # s_bfe_u32 operand: 8 bits from bit 8 * (table address & 3)
         emit("s_mov_b32 s66, %[bstep]")                    # bytes between two K steps of the stored weight
     if BROW:
+        if not RAG:
+            emit("s_mov_b32 s51, %[sdst]")
         emit(f"v_mov_b32 v{SRDB0}, %[srdb]")
         emit(f"v_mov_b32 v{SRDB}, %[srdb]")
     for r in range(16 * NB):
@@ -985,6 +990,7 @@ def main():
                       ("gemm_flat_loop.inc", (128, 256, 2, 4, 1, False, 3, False, True, False, True)),
                       ("gemm_flat_hw_loop.inc", (128, 256, 2, 4, 1, True, 3, False, True, False, True)),
                       ("gemm_mid4_loop.inc", (128, 128, 2, 2, 1, False, 4)), ("gemm_mid4_hw_loop.inc", (128, 128, 2, 2, 1, True, 4)),
+                      ("gemm_mid_hwrow_loop.inc", (128, 128, 2, 2, 1, True, 2, True, True)),
                       ("gemm_big_hw_nn_loop.inc", (256, 256, 4, 2, 1, True, 2, False, True, False, True, PP, True)),
                       ("gemm_flat_hw_nn_loop.inc", (128, 256, 2, 4, 1, True, 3, False, True, False, True, False, True)),
                       ("gemm_big_bf16_loop.inc", (256, 256, 4, 2, 1, True, 2, False, True, False, True, PP, False, True)),

@@ -248,7 +248,7 @@ def gemm_fp8_rowscale_grouped(aq, a_s, bq, b_s, k_blocks, M, N, out: torch.Tenso
     looped = [g for groups, _ in kinds for g in groups if g[1] > 2]
     launches = [(g, m) for g, m in kinds if g[0][1] == m and m < 3 and all(x[1] == m for x in g)]
     if looped:
-        launches.insert(0, (sorted(looped, key=lambda g: -g[1]), 1))
+        launches.insert(0, (sorted(looped, key=lambda g: -g[1]), 1 if any(g[1] % 4 for g in looped) else 4))
     if not launches:
         return out.zero_()
     odt = A.BF16 if out.dtype == torch.bfloat16 else A.F32

@@ -45,28 +45,25 @@ def test_every_tile_once_and_balanced(grid, all_small):
 
 
 def list_tiles(G, tiles_m, tiles_n):
-    """list_piece, list_grid and list_coords of csrc/gemm_common.h -> per XCD the (problem, tile number) of its workgroups"""
-    tiles, chunks = tiles_m * tiles_n, G * -(-(tiles_m * tiles_n) // 32)
+    """list_shift, list_grid and list_coords of csrc/gemm_common.h -> tiles in a piece, per XCD the (problem, tile number) of its workgroups"""
+    tiles, chunks = tiles_m * tiles_n, -(-G * tiles_m * tiles_n // 32)
     piece = 32 if -(-chunks // 8) * 8 * 4 <= chunks * 5 else 8
-    per = -(-tiles // piece)
     out = [[] for _ in range(8)]
-    for b in range(-(-(G * per) // 8) * 8 * piece):
+    for b in range(-(-(G * tiles) // (8 * piece)) * 8 * piece):
         s, xcd = b >> 3, b & 7
-        p = s // piece * 8 + xcd
-        g = p // per
-        lin = (p - g * per) * piece + s % piece
-        if g < G and lin < tiles:
+        g, lin = divmod((s // piece * 8 + xcd) * piece + s % piece, tiles)
+        if g < G:
             out[xcd].append((g, lin))
     return piece, out
 
 
-@pytest.mark.parametrize("G", [1, 2, 3, 15, 20, 64])
-@pytest.mark.parametrize("tiles_m,tiles_n", [(1, 1), (2, 2), (4, 4), (4, 6), (8, 8), (8, 11), (9, 23), (16, 16), (32, 32)])
+@pytest.mark.parametrize("G", [1, 2, 3, 15, 20, 32, 64])
+@pytest.mark.parametrize("tiles_m,tiles_n", [(1, 1), (2, 2), (4, 4), (4, 6), (6, 8), (8, 8), (8, 11), (11, 16), (9, 23), (16, 16), (32, 32)])
 def test_problem_lists_cover_every_tile_once_on_all_xcds(G, tiles_m, tiles_n):
     piece, per_xcd = list_tiles(G, tiles_m, tiles_n)
     assert sorted(t for x in per_xcd for t in x) == [(g, lin) for g in range(G) for lin in range(tiles_m * tiles_n)]
-    # a deal in turn: no XCD has more than its share of whole pieces and one piece more
-    assert max(map(len, per_xcd)) <= -(-(G * -(-(tiles_m * tiles_n) // piece)) // 8) * piece
+    # a deal in turn: no XCD has more than its share of all tiles and one piece more
+    assert max(map(len, per_xcd)) <= G * tiles_m * tiles_n / 8 + piece
 
 
 def strips(G, tiles_m, tiles_n):
