@@ -1741,6 +1741,10 @@ int launch_big_grouped(const void *Aq, const void *As, const void *Bq, const voi
     // e8m0 scales: 128 x 128 tiles on the kernel whose matrix instructions apply the scales
     if (scale_dtype == LP_E8M0) return rag ? go128(gemm_asm_grouped<128, 128, 1, 0, true, true>) : go128(gemm_asm_grouped<128, 128, 1, 0, true>);
     if (rag) return go128(gemm_asm_grouped<128, 128, 1, 0, false, true>);
+    // Half of the last column's 256-row tiles empty: two launches only where 128 x 128 tiles would not fit the chip at once and
+    // 256-row ones nearly fill it, as in the dense dispatch (fp32 scales, us on 128 x 128 tiles / in two launches: E = 3, 6000 rows, N = 640,
+    // K = 4096 22 / 69; 1 x 4096, N = 1408, K = 2048 19 / 33, N = 3712, K = 4096 66 / 58).
+    if (N % 256 && !(M_total / 128 * (N / 128) > 512 && M_total / 256 * tiles_n > 192)) return go128(gemm_asm_grouped<128, 128, 1, 0>);
     // Few rows per expert on average: the weights of most experts are read for one or two row tiles, so the launch
     // is as much a weight stream as a GEMM.  128 x 128 tiles (two workgroups per CU, tiles taken from both ends
     // of the expert list) let streaming tiles and compute-bound tiles overlap and bound the padding per expert

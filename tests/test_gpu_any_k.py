@@ -55,7 +55,7 @@ def test_dense(G, M, N, blocks, pow2):
 
 @pytest.mark.parametrize("pow2", [False, True], ids=["f32scale", "e8m0scale"])
 @pytest.mark.parametrize("splits,N,K", [([700, 0, 3, 257, 128, 129, 1, 64] * 4, 2176, 384), ([1000, 1, 0, 260, 385, 60] * 6, 1152, 1408),
-                                        ([33, 0, 300, 1], 640, 640), ([5, 2, 0, 129, 64], 384, 1152), ([600, 0, 60, 1] * 20, 896, 1024)],
+                                        ([33, 0, 300, 1], 640, 640), ([5, 2, 0, 129, 64], 384, 1152), ([600, 0, 60, 1] * 20, 896, 1024), ([1100, 1283], 640, 512), ([2945], 384, 1024)],
                          ids=lambda v: str(v) if isinstance(v, int) else "E%d" % len(v))
 def test_grouped(G, splits, N, K, pow2):
     E, M = len(splits), sum(splits)
