@@ -719,17 +719,15 @@ def main():
         fnw = lambda: chk(L.lp_gemm_fp8_rowscale(a_w.data_ptr(), sa_w.data_ptr(), b_w.data_ptr(), sb_w.data_ptr(), A.E8M0,  # noqa: E731
                                                  4096, 7168, Pw, dw.data_ptr(), A.BF16, stream()))
         msw, _ = time_launches([fnw], 10, 3)
-        # the whole layer's weight gradient, one launch per kind of problem (K a multiple of 512; one K block; two K blocks):
-        # 256 problems [4096, 7168] x P_e, config 4's rows per expert padded as the wrapper pads them (experts of at most 256
-        # rows to 128 or 256, the others to multiples of 512); operands are random codes (the time does not depend on the
-        # values), 15 GB of bf16 out
-        from gcore_lowp.grouped_gemm_fp8 import choose_colwise_pad, padded_blocks, rowscale_launches
-        padw = choose_colwise_pad(m_splits.tolist())
+        # the whole layer's weight gradient, one launch per kind of problem (one K block; two; more, longest first):
+        # 256 problems [4096, 7168] x P_e, config 4's rows per expert padded as the layer pads them (to whole blocks of
+        # 128 rows); operands are random codes (the time does not depend on the values), 15 GB of bf16 out
+        from gcore_lowp.grouped_gemm_fp8 import padded_blocks, rowscale_launches
+        padw = 128
         nblkw = [padded_blocks(int(m), padw) for m in m_splits.tolist()]
         pbw = sum(nblkw)
         launches_w, _ = rowscale_launches(nblkw)
-        kinds_w = {"k_multiple_of_512": sum(1 for nb in nblkw if nb and nb % 4 == 0), "one_k_block": nblkw.count(1),
-                   "two_k_blocks": nblkw.count(2), "other": sum(1 for nb in nblkw if nb > 2 and nb % 4)}
+        kinds_w = {"looped": sum(1 for nb in nblkw if nb > 2), "one_k_block": nblkw.count(1), "two_k_blocks": nblkw.count(2)}
         aT = torch.randint(0, 120, (4096 * pbw * 128,), dtype=torch.uint8, device=dev)
         bT = torch.randint(0, 120, (7168 * pbw * 128,), dtype=torch.uint8, device=dev)
         saT = torch.full((4096 * pbw,), 120, dtype=torch.uint8, device=dev)
@@ -748,7 +746,7 @@ def main():
         del aT, bT, saT, sbT, dW, tabs
         extras["grouped_linear_backward"] = {
             "dgrad_grouped_256_experts_65536x4096_to_7168": dgrad_res,
-            "wgrad_grouped_256_experts_4096x7168": {"ms": msg, "rows_padded_to": "128 up to 256 rows, 512 beyond" if padw == 0 else padw,
+            "wgrad_grouped_256_experts_4096x7168": {"ms": msg, "rows_padded_to": padw,
                                                     "problems_by_kernel": kinds_w,
                                                     "tflops_on_padded_rows": flg / msg / 1e9,
                                                     "mfma_frac": flg / msg / 1e9 / FP8_PEAK_TFLOPS,

@@ -218,37 +218,33 @@ def gemm_fp8_rowscale(aq, a_s, bq, b_s, M, N, K, out: torch.Tensor) -> torch.Ten
 
 
 def rowscale_launches(k_blocks):
-    """How the row-scaled problems of a grouped weight gradient are dealt to kernels: -> (launches, empty) with launches a
-    list of (table, multiple) -- table rows {problem, K blocks, K blocks of the problems before it, 0} as
+    """The launches of the row-scaled problems of a grouped weight gradient: -> (launches, empty) with launches a list of
+    (table, multiple) -- table rows {problem, K blocks, K blocks of the problems before it, 0} as
     lp_gemm_fp8_rowscale_grouped reads them, multiple = what every K block count of the table is a multiple of -- and
     empty the problems without K blocks (their outputs are zeros).  Problems of one K block and those of two have a
-    kernel each; the others run on the hand-scheduled loop, which gemm_fp8_rowscale_grouped launches once for both of
-    their lists."""
-    before, fast, one, two, rest, empty = 0, [], [], [], [], []
+    kernel each; the others run on the hand-scheduled loop, longest first (a long problem started last would run alone at
+    the end)."""
+    before, looped, one, two, empty = 0, [], [], [], []
     for e, kb in enumerate(k_blocks):
         kb = int(kb)
         assert kb >= 0
         if kb == 0:
             empty.append(e)
         else:
-            (fast if kb % 4 == 0 else one if kb == 1 else two if kb == 2 else rest).append((e, kb, before, 0))
+            (one if kb == 1 else two if kb == 2 else looped).append((e, kb, before, 0))
         before += kb
-    return [(g, m) for g, m in ((fast, 4), (one, 1), (two, 2), (rest, 1)) if g], empty
+    looped.sort(key=lambda g: -g[1])
+    whole = 4 if all(g[1] % 4 == 0 for g in looped) else 1
+    return [(g, m) for g, m in ((looped, whole), (one, 1), (two, 2)) if g], empty
 
 
 def gemm_fp8_rowscale_grouped(aq, a_s, bq, b_s, k_blocks, M, N, out: torch.Tensor) -> torch.Tensor:
     """out[e] [M, N] = the row-scaled product of problem e, whose operands ([M, K_e] / [N, K_e] codes and their e8m0
-    scales, K_e = 128 * k_blocks[e]) lie one after the other in aq / a_s / bq / b_s.  The problems of one and of two K blocks
-    go to the kernel without a K loop (a launch each), the others to the hand-scheduled loop in one launch, longest first (a
-    long problem started last would run alone at the end); problems with no K blocks are zero-filled, all in one launch.  (The reference issues
-    one grouped GEMM call: fp8.py:325-341.)"""
+    scales, K_e = 128 * k_blocks[e]) lie one after the other in aq / a_s / bq / b_s.  At most three launches (rowscale_launches);
+    problems with no K blocks are zero-filled, all in one more.  (The reference issues one grouped GEMM call: fp8.py:325-341.)"""
     E = len(k_blocks)
     assert out.is_contiguous() and tuple(out.shape) == (E, M, N) and out.dtype in (torch.bfloat16, torch.float32)
-    kinds, empty = rowscale_launches(k_blocks)
-    looped = [g for groups, _ in kinds for g in groups if g[1] > 2]
-    launches = [(g, m) for g, m in kinds if g[0][1] == m and m < 3 and all(x[1] == m for x in g)]
-    if looped:
-        launches.insert(0, (sorted(looped, key=lambda g: -g[1]), 1 if any(g[1] % 4 for g in looped) else 4))
+    launches, empty = rowscale_launches(k_blocks)
     if not launches:
         return out.zero_()
     odt = A.BF16 if out.dtype == torch.bfloat16 else A.F32

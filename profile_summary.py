@@ -193,7 +193,7 @@ def floor_summary(b):
                      % (w, c1[f"read32MiB_write16MiB_{w}_workgroups_us"], c1[f"read16MiB_write32MiB_{w}_workgroups_us"]))
         L.append("   quant_tile128    %6.2f us = %.2f x the best bare stream (%.3f of 8 TB/s; the bare stream %.3f)"
                  % (ex["c1_quant_128x128"]["ms"] * 1e3, c1["quant_over_bare_stream"], ex["c1_quant_128x128"]["hbm_frac"], c1["bare_stream_hbm_frac"]["read32_write16"]))
-        L.append("   dequant_fp8_fast %6.2f us = %.2f x the best bare stream (%.3f of 8 TB/s; the bare stream %.3f)"
+        L.append("   dequant_fast     %6.2f us = %.2f x the best bare stream (%.3f of 8 TB/s; the bare stream %.3f)"
                  % (ex["c1_dequant_128x128"]["ms"] * 1e3, c1["dequant_over_bare_stream"], ex["c1_dequant_128x128"]["hbm_frac"], c1["bare_stream_hbm_frac"]["read16_write32"]))
         L.append("")
     if "c5_floor_probe" in ex:

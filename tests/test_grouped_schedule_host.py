@@ -177,24 +177,25 @@ def test_weight_gradient_padding_and_launch_split():
     assert [padded_blocks(r, 512) for r in rows] == [0, 4, 4, 4, 4, 4, 4, 8, 8, 12, 56]
     assert [padded_blocks(r, A.PAD_MIXED) for r in rows] == [0, 1, 1, 2, 2, 4, 4, 8, 8, 12, 56]
     assert choose_colwise_pad(rows) == A.PAD_MIXED
-    k_blocks = [4, 1, 0, 8, 3, 12, 0, 5, 2, 1, 2]
-    launches, empty = rowscale_launches(k_blocks)
-    assert empty == [2, 6]
-    seen = {}
-    for table, multiple in launches:
-        assert table and multiple in (1, 2, 4)
-        for e, kb, before, zero in table:
-            assert e not in seen and kb == k_blocks[e] and kb % multiple == 0 and zero == 0
-            assert before == sum(k_blocks[:e])
-            seen[e] = multiple
-        if multiple == 2:
-            assert all(kb == 2 for _, kb, _, _ in table)
-    assert sorted(seen) == [e for e, kb in enumerate(k_blocks) if kb]
-    assert {e for e, m in seen.items() if m == 4} == {0, 3, 5}
-    # the problems of one K block and the odd ones never share a table: the kernel without a K loop takes a table whose
-    # largest problem has one block
-    ones = [t for t, m in launches if m == 1 and all(kb == 1 for _, kb, _, _ in t)]
-    assert len(ones) == 1 and {e for e, _, _, _ in ones[0]} == {1, 9}
-    # a mixed padding never leaves a problem to the compiler-scheduled kernel
+    for k_blocks, whole in (([4, 1, 0, 8, 3, 12, 0, 5, 2, 1, 2], 1), ([4, 1, 0, 8, 16, 12, 0, 4, 2, 1, 2], 4), ([0, 0], None), ([2], None)):
+        launches, empty = rowscale_launches(k_blocks)
+        assert empty == [e for e, kb in enumerate(k_blocks) if kb == 0]
+        seen = {}
+        for table, multiple in launches:
+            assert table and multiple in (1, 2, 4)
+            for e, kb, before, zero in table:
+                assert e not in seen and kb == k_blocks[e] and kb % multiple == 0 and zero == 0
+                assert before == sum(k_blocks[:e])
+                seen[e] = table
+        assert sorted(seen) == [e for e, kb in enumerate(k_blocks) if kb]
+        # one launch a kind at most: the problems of one K block, those of two, and the looped ones, longest first, with the promise
+        # of whole groups of four exactly when all of them keep it
+        kinds = [sorted({min(kb, 3) for _, kb, _, _ in table}) for table, _ in launches]
+        assert all(len(k) == 1 for k in kinds) and len({k[0] for k in kinds}) == len(kinds)
+        for table, multiple in launches:
+            lengths = [kb for _, kb, _, _ in table]
+            assert multiple == (min(lengths[0], 3) if lengths[0] < 3 else whole)
+            assert lengths == sorted(lengths, reverse=True)
+    # padding to 512 beyond 256 rows leaves whole groups of four only
     launches, _ = rowscale_launches([padded_blocks(r, A.PAD_MIXED) for r in range(0, 3000, 37)])
     assert all(m in (2, 4) or all(kb == 1 for _, kb, _, _ in t) for t, m in launches)
