@@ -1,17 +1,14 @@
 """The device-side tile schedule of the grouped GEMM with two tile heights (gemm_asm_grouped_mixed in
-csrc/gemm_fp8_big.hip), restated on the host: from the rows per expert every workgroup derives its class, its
-expert, its row tile and its column tile.  Over the grid the host launches, every tile of every expert must come up
-exactly once, nothing else may come up, the grid bound must cover the schedule, and the tiles an XCD runs together
-must belong to one expert or to neighbours.  A mistake here shows on the GPU as missing or doubly written output
+csrc/gemm_fp8_big.hip), restated on the host: from the rows per expert every workgroup derives its tiles (how both classes are
+shared out: tests/test_grouped_balance_host.py) and for each its expert, its row tile and its column tile.  Over the grid the host
+launches, every tile of every expert must come up exactly once, nothing else may come up, the grid bound must cover the
+schedule, and the tiles an XCD runs together must belong to one expert or to neighbours.  A mistake here shows on the GPU as missing or doubly written output
 rows, so it is checked where a mistake costs nothing.  Also the wide tile's weight-copy plan (256 x 288 loop)."""
 import pytest
 
+from tests.test_grouped_balance_host import share
+
 CHUNK, GROUP_M = 32, 8
-
-
-def padded_grid(tiles_m, tiles_n):
-    chunks = (tiles_m * tiles_n + CHUNK - 1) // CHUNK
-    return (chunks + 7) // 8 * 8 * CHUNK
 
 
 def classes(rows):
@@ -19,60 +16,26 @@ def classes(rows):
     return (rows >> 8) + (1 if rem > 128 else 0), (1 if 0 < rem <= 128 else 0)
 
 
-def schedule(m_splits, N, small_first):
-    """-> list of (class, expert, local row tile, column tile) per workgroup that gets a tile; grid size."""
-    E, M_total, tiles_n = len(m_splits), sum(m_splits), N >> 8
-    nb = [classes(r)[0] for r in m_splits]
-    ns = [classes(r)[1] for r in m_splits]
-    tot_big, tot_small = sum(nb), sum(ns)
-    slots = lambda tiles: ((tiles + CHUNK - 1) // CHUNK + 7) // 8 * CHUNK
-    slots_big, slots_small = slots(tot_big * tiles_n), slots(tot_small * tiles_n)
-    grid = padded_grid(M_total // 256 + E, tiles_n) + 2 * 8 * CHUNK                     # what the host launches
-    assert grid >= 8 * (slots_big + slots_small), "host grid bound below the device schedule"
+def schedule(m_splits, N, grid):
+    """-> list of (class, expert, local row tile, column tile, XCD, position in the XCD's run of the class) of every tile a workgroup takes."""
+    tiles_n = -(-N // 256)
+    cnts = {"big": [classes(r)[0] for r in m_splits], "small": [classes(r)[1] for r in m_splits]}
     out = []
-    for b in range(grid):
-        xcd, sidx = b & 7, b >> 3
-        if sidx >= slots_big + slots_small:
-            continue
-        if small_first > 0:
-            if xcd < small_first:
-                big = sidx >= slots_small
-                idx = sidx - slots_small if big else sidx
-            else:
-                big = sidx < slots_big
-                idx = sidx if big else sidx - slots_big
-        else:
-            ps = max(1, (slots_small + slots_big // 2) // slots_big if slots_big > 0 else 1)
-            period = 1 + ps
-            rounds = min(slots_big, slots_small // ps)
-            if sidx < rounds * period:
-                r, q = sidx % period, sidx // period
-                big = r == 0
-                idx = q if big else q * ps + (r - 1)
-            else:
-                w, left_big = sidx - rounds * period, slots_big - rounds
-                big = w < left_big
-                idx = rounds + w if big else rounds * ps + (w - left_big)
-        lin = ((idx // CHUNK) * 8 + xcd) * CHUNK + idx % CHUNK
-        cnts = nb if big else ns
-        if lin >= (tot_big if big else tot_small) * tiles_n:
-            continue
-        gmt = lin // tiles_n
-        incl, e = 0, None
-        for i, c in enumerate(cnts):                       # the expert whose running count covers gmt
-            if incl <= gmt < incl + c:
-                e, first = i, incl
-            incl += c
-        assert e is not None
-        in_e = lin - first * tiles_n
-        per_group = GROUP_M * tiles_n
-        grp, in_grp = divmod(in_e, per_group)
-        gm = min(cnts[e] - grp * GROUP_M, GROUP_M)
-        gn = CHUNK // gm
-        nblk, in_blk = divmod(in_grp, gm * gn)
-        local, tn = grp * GROUP_M + in_blk % gm, nblk * gn + in_blk // gm
-        out.append(("big" if big else "small", e, local, tn, xcd, idx))
-    return out, grid
+    for xcd, big, small in share(sum(cnts["big"]) * tiles_n, sum(cnts["small"]) * tiles_n, grid):
+        for cls, numbers in (("big", big), ("small", small)):
+            for lin in numbers:
+                gmt, incl = lin // tiles_n, 0
+                for e, c in enumerate(cnts[cls]):                       # the expert whose running count covers gmt
+                    if incl <= gmt < incl + c:
+                        break
+                    incl += c
+                in_e = lin - incl * tiles_n
+                grp, in_grp = divmod(in_e, GROUP_M * tiles_n)
+                gm = min(c - grp * GROUP_M, GROUP_M)
+                gn = CHUNK // gm
+                nblk, in_blk = divmod(in_grp, gm * gn)
+                out.append((cls, e, grp * GROUP_M + in_blk % gm, nblk * gn + in_blk // gm, xcd, lin))
+    return out
 
 
 CASES = {
@@ -86,19 +49,23 @@ CASES = {
 
 
 @pytest.mark.parametrize("name", list(CASES))
-@pytest.mark.parametrize("small_first", [0, 4, 8])
-@pytest.mark.parametrize("N", [4096, 7168, 256])
-def test_every_tile_exactly_once(name, small_first, N):
+@pytest.mark.parametrize("grid", [0, 8, 256, 304])
+@pytest.mark.parametrize("N", [4096, 7168, 256, 4224, 128])
+def test_every_tile_exactly_once(name, grid, N):
+    """grid 0: a workgroup per tile, as the host launches where there are fewer tiles than CUs or the CUs are not known"""
     if CASES[name] is None:
         from tests._inputs import zipf_m_splits
         m_splits = zipf_m_splits().tolist()
     else:
         m_splits = CASES[name]
-    got, grid = schedule(m_splits, N, small_first)
+    tiles_n = -(-N // 256)
+    bound = (sum(m_splits) // 256 + len(m_splits)) * tiles_n                         # mixed_grid: tiles of both classes at most
+    assert sum(sum(classes(r)) for r in m_splits) * tiles_n <= bound
+    got = schedule(m_splits, N, min(grid or 1 << 30, -(-bound // 8) * 8))
     want = set()
     for e, r in enumerate(m_splits):
         b, s = classes(r)
-        for tn in range(N >> 8):
+        for tn in range(tiles_n):
             want |= {("big", e, m, tn) for m in range(b)} | {("small", e, 0, tn) for _ in range(s)}
     tiles = [g[:4] for g in got]
     assert len(tiles) == len(set(tiles)), "a tile is handed out twice"
@@ -110,35 +77,31 @@ def test_every_tile_exactly_once(name, small_first, N):
         assert covered == r, (e, r, b, s)
 
 
-@pytest.mark.parametrize("workgroups", [8, 256, 304, 1 << 20])
-@pytest.mark.parametrize("all_slots", [0, 8 * 32, 8 * 32 * 47, 8 * 32 * 300])
-def test_slot_walk_of_the_persistent_launch(workgroups, all_slots):
-    """With fewer workgroups than slots, workgroup b takes slots b, b + G, b + 2 G ... (G = workgroups rounded down to a
-    multiple of 8, what the host launches), looked up 256 at a time, one slot per thread: every slot comes up exactly once,
-    and always on the XCD (slot mod 8) of the workgroup that takes it, which keeps the per-XCD order of the schedule."""
-    K_TABLE = 256
-    G = workgroups // 8 * 8 if all_slots > workgroups else max(all_slots, 8)
-    seen = []
-    for b in range(min(G, all_slots)):
-        first = b
-        while first < all_slots:                            # one look-up batch
-            for t in range(K_TABLE):
-                slot = first + t * G
-                if slot < all_slots:
-                    assert slot % 8 == b % 8
-                    seen.append(slot)
-            first += K_TABLE * G
-    assert sorted(seen) == list(range(all_slots))
+@pytest.mark.parametrize("mine", [0, 1, 255, 256, 257, 1000])
+@pytest.mark.parametrize("lead", [0, 1, 300])
+def test_table_walk_of_a_workgroup(mine, lead):
+    """A workgroup's tiles are looked up 256 at a time, one per thread: first the `lead` tiles of one class, then the other's, every
+    position exactly once."""
+    K_TABLE, seen = 256, []
+    lead = min(lead, mine)
+    for first in range(0, mine, K_TABLE):
+        for t in range(K_TABLE):
+            at = first + t
+            if at < mine:
+                seen.append((at >= lead, at if at < lead else at - lead))
+    assert seen == [(False, k) for k in range(lead)] + [(True, k) for k in range(mine - lead)]
 
 
 def test_an_xcd_runs_neighbouring_tiles_together():
-    """32 consecutive positions of an XCD's sequence within a class are 32 consecutive tile numbers: at most two
-    experts unless experts have fewer than 16 tiles, and for an expert with at least 8 row tiles a block of 8 x 4."""
+    """32 consecutive tiles of an XCD's run of a class, which its workgroups take at the same time: at most three experts, and for an
+    expert with at least 8 row tiles a block of 8 x 4."""
     from tests._inputs import zipf_m_splits
-    got, _ = schedule(zipf_m_splits().tolist(), 4096, 4)
-    by = {}
-    for cls, e, m, tn, xcd, idx in got:
-        by.setdefault((cls, xcd, idx // CHUNK), []).append((e, m, tn))
+    got = schedule(zipf_m_splits().tolist(), 4096, 256)
+    by, start = {}, {}
+    for cls, e, m, tn, xcd, lin in got:
+        start[cls, xcd] = min(lin, start.get((cls, xcd), lin))
+    for cls, e, m, tn, xcd, lin in got:
+        by.setdefault((cls, xcd, (lin - start[cls, xcd]) // CHUNK), []).append((e, m, tn))
     for (cls, xcd, chunk), tiles in by.items():
         experts = {t[0] for t in tiles}
         assert len(experts) <= 3, (cls, xcd, chunk, experts)           # 16 column tiles per row tile: 32 numbers span <= 3 experts
