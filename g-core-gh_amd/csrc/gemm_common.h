@@ -55,7 +55,7 @@ __device__ __forceinline__ bool tile_coords(int64_t b, int64_t tiles_m, int64_t 
 }
 
 // The tiles of G problems of one shape, numbered problem by problem: pieces of 2^shift consecutive ones are dealt to the XCDs in
-// turn.  (With every problem dealt from XCD 0 on as above, a problem of few tiles ran on few XCDs: 20 weight gradients of 1024 x
+// turn, forwards and backwards: in a list sorted by length the XCD with the longest of one turn has the shortest of the next.  (With every problem dealt from XCD 0 on as above, a problem of few tiles ran on few XCDs: 20 weight gradients of 1024 x
 // 1408 with three K blocks, 24 tiles each, on one of eight: 131 us, dealt in turn 30.  With pieces that end with their problem, the
 // last and smaller ones could all fall to the same XCDs: 32 problems of 1408 x 2048 with
 // sixteen K blocks, 48 tiles each, 200 us, across problems 166.)  Workgroup b ->
@@ -64,7 +64,8 @@ __device__ __forceinline__ bool tile_coords(int64_t b, int64_t tiles_m, int64_t 
 __device__ __forceinline__ bool list_coords(uint32_t b, uint32_t G, uint32_t tiles_m, uint32_t tiles_n, int shift, int64_t &g, int64_t &tm, int64_t &tn)
 {
     const uint32_t tiles = tiles_m * tiles_n, s = b >> 3;
-    const uint32_t id = (((s >> shift) * 8 + (b & 7)) << shift) + (s & ((1u << shift) - 1)), problem = id / tiles;
+    const uint32_t turn = s >> shift, xcd = (b & 7) ^ (turn & 1 ? 7 : 0);
+    const uint32_t id = ((turn * 8 + xcd) << shift) + (s & ((1u << shift) - 1)), problem = id / tiles;
     if (problem >= G) return false;
     g = problem;
     tile_of<uint32_t>(id - problem * tiles, tiles_m, tiles_n, tm, tn);

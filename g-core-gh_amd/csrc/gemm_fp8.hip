@@ -217,7 +217,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     store_tile(acc, ta.m0, M, ta.n0, ldc, C, out_dtype);
 }
 
-// Row-scaled problems that share M and N and differ in K, one launch (see gemm_asm_rowscale_grouped for `groups`).
+// Row-scaled problems that share M and N and differ in K, one launch (see gemm_asm_rowscale in gemm_fp8_big.hip for `groups`): fp32 scales,
+// and operands of 4 GiB and more.
 template <int SDT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_rowscale_grouped(
     const uint8_t *__restrict__ Aq, const void *__restrict__ As, const uint8_t *__restrict__ Bq, const void *__restrict__ Bs,

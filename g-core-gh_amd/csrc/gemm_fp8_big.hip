@@ -1614,17 +1614,18 @@ bool rowscale_asm_ok(const void *As, const void *Bs, int scale_dtype, int64_t M,
 int launch_rowscale_asm(const void *Aq, const void *As, const void *Bq, const void *Bs, const int32_t *groups, int G, int max_k_blocks,
                         int multiple, int64_t M, int64_t N, void *C, int out_dtype, hipStream_t st)
 {
-    // 256 x 256 tiles where their rounds of one per CU cost less than 128 x 128 ones do, which four times as many share the CUs with
-    // little loss at the end (in hundredths of a full round of either).  The large ones are the better the longer the K loop is, and
-    // with a short one only where their stores run beside another round (us, 128 / 256: 4096 x 4096 with 4 / 8 / 11 / 16 / 32 K blocks
-    // 13.6 / 14.6, 22.1 / 20.5, 27.3 / 25.1, 34.5 / 31.5, 61.9 / 53.7; 8 of them with 4 100 / 96; 7168 x 7168, 3.06 rounds that take four, with
-    // 8 60.8 / 68.2; 32 x 1408 x 2048 with 16 180 / 166, 8 of them, 1.5 rounds, 48.7 / 53.3).
+    // 256 x 256 tiles where they cost less than 128 x 128 ones, in hundredths of a round of 256 of the former or 1024 of the latter.  The large
+    // ones are the better the longer the K loop is, and with a short one only where their stores run beside another round (us, 128 /
+    // 256: 4096 x 4096 with 4 / 5 / 8 / 11 / 16 / 32 K blocks 13.1 / 14.1, 17.0 / 15.7, 22.1 / 19.4, 27.3 / 23.8, 34.5 / 30.5, 61.9 / 53.2; 16 x 2048 x 2048
+    // with 4 51.3 / 49.4).  One problem pays its last round in full (7168 x 7168, 3.06 rounds that take four, with 8 60.0 / 65.2); in a
+    // list, longest first, shorter tiles fill it.
     // The 128 x 128 loop for K in whole groups of four blocks starts without the scales' way through registers: up to 8 % where
     // there is about one tile per CU (128 x 256 with 8 K blocks 6.6 -> 6.1 us, 1152 x 128 with 12 8.2 -> 7.6), level from ten rounds on.
     const int64_t big = ((M + 255) / 256) * ((N + 255) / 256) * G, small = ((M + 127) / 128) * ((N + 127) / 128) * G;
     const int64_t rounds = (big + 255) / 256, kb = max_k_blocks;
-    const int64_t cost = kb >= 32 ? 83 : kb >= 16 ? 88 : kb >= 11 ? 90 : kb >= 8 ? 92 : kb >= 5 ? 92 + 6 / rounds : 98 + 10 / rounds;
-    const int tm = big >= 256 && rounds * cost < small * 100 / 1024 + 8 ? 256 : 128;
+    const int64_t cost = kb >= 32 ? 83 : kb >= 16 ? 88 : kb >= 11 ? 90 : kb >= 8 ? 92 : kb >= 5 ? 92 + 4 / rounds : G == 1 ? 98 + 10 / rounds : 94 + 8 / rounds;
+    const int64_t paid = G == 1 ? rounds * cost : big * cost / 256 + 10;
+    const int tm = big >= 256 && paid < small * 100 / 1024 + 8 ? 256 : 128;
     const bool aligned = multiple % 4 == 0 && asm_shape_ok(As, Bs, M, N, (int64_t)max_k_blocks * 128, LP_E8M0);
     const int64_t tiles_m = (M + tm - 1) / tm, tiles_n = (N + tm - 1) / tm;
     const int shift = gemm::list_shift(G, tiles_m, tiles_n);

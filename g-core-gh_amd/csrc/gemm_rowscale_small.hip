@@ -273,15 +273,20 @@ int launch_rowscale_small(const void *Aq, const void *As, const void *Bq, const 
 {
     const int64_t tiles_m = M / 128, tiles_n = N / 128;
     if (k_blocks == 2) {
-        // At most 8 tiles a strip, all strips alike: the panel's load and the first tile's wait spread over 8 tiles while a weight
-        // of 4096 columns still cuts into 4 (40 x 7168 x 4096, strips of 2 / 4 / 8 / 16 tiles: 535 / 476 / 433 / 471 us; 15 x 4096 x
-        // 4096: 117 / 122 / 114 / 128).  Few small problems are cut shorter, until two workgroups per CU have one, and dealt
-        // out in smaller pieces, until every XCD has one (one problem of 1024 x 1024 / 2048 x 2048 / 7168 x 2048, strips of 8 tiles: 14.2 /
-        // 14.2 / 14.2 us, as cut here 4.7 / 5.4 / 9.6; 8 problems of 1024 x 1024 13.9 / 6.9; one of 384 x 384 in a piece of 8 7.1, in pieces of
-        // one 4.5.  Below ten tiles a workgroup without a strip's two barriers more would be 0.2 us ahead, 4.0 against 4.2).
-        const int64_t wanted = tiles_m && G ? (512 + G * tiles_m - 1) / (G * tiles_m) : 1, least = (tiles_n + 7) / 8;
-        const int64_t per_row = wanted <= least ? least : wanted < tiles_n ? wanted : tiles_n;
-        const int64_t strip = per_row ? (tiles_n + per_row - 1) / per_row : 1, runs = G * tiles_m * ((tiles_n + strip - 1) / strip);
+        // Strips of at most 8 tiles, all alike, cut so that rounds of two workgroups per CU x (their tiles + 2 for the panel's load and the
+        // first tile's wait) are fewest: 8 tiles for many problems (40 x 7168 x 4096, strips of 2 / 4 / 8 / 16 tiles: 535 / 476 / 433 / 471 us; 15 x
+        // 4096 x 4096: 117 / 122 / 114 / 128), down to one for few (one problem of 1024 x 1024 / 2048 x 2048 / 7168 x 2048, strips of 8: 14.2 us
+        // each, as cut here 4.6 / 5.6 / 9.7; 8 problems of 1024 x 1024 13.9 / 6.9), and dealt out in smaller pieces until every XCD has
+        // one (384 x 384 in a piece of 8 7.1, in pieces of one 4.4; below ten tiles a workgroup without a strip's two barriers more would be
+        // 0.2 us ahead).
+        int64_t strip = 1, best = INT64_MAX;
+        for (int64_t s = 1; s <= 8 && s <= tiles_n; ++s) {
+            const int64_t per_row = (tiles_n + s - 1) / s;
+            if ((tiles_n + per_row - 1) / per_row != s) continue;              // not alike: a shorter strip makes as many
+            const int64_t cost = (G * tiles_m * per_row + 511) / 512 * (s + 2);
+            if (cost <= best) best = cost, strip = s;
+        }
+        const int64_t runs = G * tiles_m * ((tiles_n + strip - 1) / strip);
         int piece = GROUP_M;
         while (piece > 1 && (runs + piece - 1) / piece < 8) piece /= 2;
         const int64_t wgs = (runs + 8 * piece - 1) / (8 * piece) * (8 * piece);
