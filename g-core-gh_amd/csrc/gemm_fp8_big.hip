@@ -1628,7 +1628,7 @@ int launch_rowscale_asm(const void *Aq, const void *As, const void *Bq, const vo
     const int tm = big >= 256 && paid < small * 100 / 1024 + 8 ? 256 : 128;
     const bool aligned = multiple % 4 == 0 && asm_shape_ok(As, Bs, M, N, (int64_t)max_k_blocks * 128, LP_E8M0);
     const int64_t tiles_m = (M + tm - 1) / tm, tiles_n = (N + tm - 1) / tm;
-    const int shift = gemm::list_shift(G, tiles_m, tiles_n);
+    const int shift = gemm::list_shift(G, tiles_m, tiles_n, tm == 128 ? 64 : 0);      // two 128 x 128 workgroups on each of an XCD's 32 CUs
     const int64_t grid = gemm::list_grid(G, tiles_m, tiles_n, shift);
     if (grid > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_gemm_fp8_rowscale: problem too large");
     auto go = [&](auto kernel) {

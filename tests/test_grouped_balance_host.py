@@ -44,10 +44,12 @@ def test_every_tile_once_and_balanced(grid, all_small):
             assert not runs or max(runs) - min(runs) + 1 == len(runs)          # one run of numbers per XCD
 
 
-def list_tiles(G, tiles_m, tiles_n):
+def list_tiles(G, tiles_m, tiles_n, slots):
     """list_shift, list_grid and list_coords of csrc/gemm_common.h -> tiles in a piece, per XCD the (problem, tile number) of its workgroups"""
     tiles, chunks = tiles_m * tiles_n, -(-G * tiles_m * tiles_n // 32)
-    piece = 32 if -(-chunks // 8) * 8 * 4 <= chunks * 5 else 8
+    most = -(-chunks // 8)
+    alike = most * 8 * 4 <= chunks * 5
+    piece = 32 if alike or slots and chunks >= 8 and -(-most * 32 // slots) <= -(-G * tiles // (8 * slots)) else 8
     out = [[] for _ in range(8)]
     for b in range(-(-(G * tiles) // (8 * piece)) * 8 * piece):
         s, xcd = b >> 3, b & 7
@@ -60,8 +62,9 @@ def list_tiles(G, tiles_m, tiles_n):
 
 @pytest.mark.parametrize("G", [1, 2, 3, 15, 20, 32, 64])
 @pytest.mark.parametrize("tiles_m,tiles_n", [(1, 1), (2, 2), (4, 4), (4, 6), (6, 8), (8, 8), (8, 11), (11, 16), (9, 23), (16, 16), (32, 32)])
-def test_problem_lists_cover_every_tile_once_on_all_xcds(G, tiles_m, tiles_n):
-    piece, per_xcd = list_tiles(G, tiles_m, tiles_n)
+@pytest.mark.parametrize("slots", [0, 64])
+def test_problem_lists_cover_every_tile_once_on_all_xcds(G, tiles_m, tiles_n, slots):
+    piece, per_xcd = list_tiles(G, tiles_m, tiles_n, slots)
     assert sorted(t for x in per_xcd for t in x) == [(g, lin) for g in range(G) for lin in range(tiles_m * tiles_n)]
     # a deal in turn: no XCD has more than its share of all tiles and one piece more
     assert max(map(len, per_xcd)) <= G * tiles_m * tiles_n / 8 + piece
