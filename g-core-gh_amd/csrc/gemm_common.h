@@ -137,10 +137,12 @@ bool launch_wide(const void *Aq, const void *As, const void *Bq, const void *Bs,
                  void *C, int64_t ldc, int out_dtype, hipStream_t st, int *rc);
 bool launch_mixed(const void *Aq, const void *As, const void *Bq, const void *Bs, int scale_dtype, int64_t M, int64_t N, int64_t K,
                   int64_t n_big, void *C, int64_t ldc, int out_dtype, hipStream_t st, int *rc);
-// A dense problem on 128 x 128 tiles of which those at or behind column n_whole are cut into `splits` ranges of `per` K blocks.
+// A dense problem on 128 x 128 tiles of which those at or behind column n_whole are cut into `splits` ranges of `per` K blocks; fold: e8m0
+// products are added up in fp32 (gemm_asm_split).
 struct SplitPlan {
     int64_t n_whole;
     int splits, per;
+    bool fold;
 };
 int launch_split(const void *Aq, const void *As, const void *Bq, const void *Bs, int scale_dtype, int64_t M, int64_t N, int64_t K,
                  const SplitPlan &plan, void *C, int out_dtype, float *ws, hipStream_t st);
