@@ -2,6 +2,8 @@
 lp_gemm_workspace_bytes, and asked for only where there is a K to cut."""
 import random
 
+import pytest
+
 
 def test_split_scratch_is_bounded():
     from gcore_lowp import _abi
@@ -24,3 +26,18 @@ def test_split_scratch_is_bounded():
     assert seen > 300
     assert L.lp_gemm_split_workspace_bytes(1, 4096, 7168) == 0 and L.lp_gemm_split_workspace_bytes(512, 4096, 1024) == 0
     assert [L.lp_gemm_split_workspace_bytes(*s) for s in ((0, 128, 128), (8, 100, 128), (8, 128, 100))] == [0, 0, 0]
+
+
+@pytest.mark.parametrize("M,N,K", [(47, 6528, 6528), (33, 8192, 6144), (64, 6144, 7168), (64, 8192, 7168), (33, 8192, 8064), (43, 8192, 14464), (17, 6144, 7296), (22, 6016, 7424),
+                                   (18, 5888, 13696), (24, 6144, 12032), (32, 5632, 9216), (23, 5376, 14336), (23, 5632, 18432), (65, 8192, 6144),
+                                   (512, 2048, 5632), (64, 4096, 7168), (128, 4096, 5504)], ids=str)
+def test_shapes_the_decode_kernels_are_faster_at_are_not_cut(M, N, K):
+    from gcore_lowp import _abi
+    assert _abi.lib().lp_gemm_split_workspace_bytes(M, N, K) == 0
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 5120, 6144), (56, 4224, 7168), (33, 5120, 7296), (44, 8192, 9216), (35, 7168, 16768), (24, 5120, 8192), (17, 5376, 14464), (24, 6144, 18432),
+                                   (96, 8192, 6144), (65, 4096, 5632), (512, 2048, 6144)], ids=str)
+def test_shapes_the_ranges_are_faster_at_are_cut(M, N, K):
+    from gcore_lowp import _abi
+    assert _abi.lib().lp_gemm_split_workspace_bytes(M, N, K) > 0
