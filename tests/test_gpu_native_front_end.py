@@ -102,27 +102,33 @@ def stand_in(tmp_path_factory):
     return ctypes.CDLL(str(d / "s.so"))
 
 
+HOST_ONLY = {"lp_gemm_split_workspace_bytes", "lp_host_flag"}          # answer on the host, without a launch
+
+
 @contextlib.contextmanager
 def bound(function):
     """The front end's module with `function` in the place of the library's entries that launch."""
     from gcore_lowp import _abi as A, _native
     mod = _native._load()
+    assert HOST_ONLY <= set(_native._BOUND)
     real = [ctypes.cast(getattr(A.lib(), n), ctypes.c_void_p).value for n in _native._BOUND]
     fake = ctypes.cast(function, ctypes.c_void_p).value
-    mod.bind(*[a if n in ("lp_gemm_workspace_bytes", "lp_host_flag") else fake for n, a in zip(_native._BOUND, real)])
+    mod.bind(*[a if n in HOST_ONLY else fake for n, a in zip(_native._BOUND, real)])
     try:
         yield mod
     finally:
         mod.bind(*real)
 
 
-@pytest.mark.parametrize("name", ["quant_fp8", "quant_fp8_checked", "dequant", "fp4_to_fp8", "gemm"])
+@pytest.mark.parametrize("name", ["quant_fp8", "quant_fp8_checked", "dequant", "fp4_to_fp8", "gemm", "grouped_forward", "grouped_backward"])
 def test_other_threads_run_while_a_launch_waits(G, stand_in, name):
     """A launch can wait for room in a full queue, an allocation for the device."""
     from gcore_lowp import _abi as A
     x = torch.zeros(128, 256, device="cuda", dtype=torch.bfloat16)
     (q, s), packed = G.quant_2d(x), torch.zeros(128, 128, device="cuda", dtype=torch.int8)
     fs, (aq, sa) = torch.ones(128, 8, device="cuda").to(E8M0), G.quant_1d(x)
+    experts = q.view(1, 128, 256), torch.ones(1, 1, 2, device="cuda").to(E8M0)
+    offsets = torch.tensor([0, 128], device="cuda", dtype=torch.int32)
     word = {n: ctypes.c_int.in_dll(stand_in, n) for n in ("inside", "go", "late")}
     for w in word.values():
         w.value = 0
@@ -137,7 +143,10 @@ def test_other_threads_run_while_a_launch_waits(G, stand_in, name):
                 "quant_fp8_checked": lambda: mod.quant_fp8(x, 128, 128, A.SCALE_POW2, A.E8M0, A.ZERO_NONE, 0.0, True),
                 "dequant": lambda: mod.dequant(q, s, False, A.FP4_NEG_ZERO, A.BF16),
                 "fp4_to_fp8": lambda: mod.fp4_to_fp8(packed, fs, 1, A.SCALE_DIV, A.ZERO_NONE, A.F32, 1e-12),
-                "gemm": lambda: mod.gemm(aq, sa, q, s, A.BF16)}[name]
+                "gemm": lambda: mod.gemm(aq, sa, q, s, A.BF16),
+                "grouped_forward": lambda: mod.grouped_forward(x, *experts, [128], A.BF16, False, False),
+                "grouped_backward": lambda: mod.grouped_backward(x[:, :128].contiguous(), *(t.view(torch.uint8) for t in experts), offsets, None, None, None,
+                                                                 [128], True, False, A.BF16)}[name]
         t = threading.Thread(target=other)
         t.start()
         r = call()
