@@ -34,7 +34,7 @@ decltype(&lp_dequant_fp4_block) p_dequant_fp4;
 decltype(&lp_fp4_to_fp8_amax) p_fp4_amax;
 decltype(&lp_fp4_to_fp8_rebase) p_fp4_rebase;
 decltype(&lp_gemm_fp8_block) p_gemm;
-decltype(&lp_gemm_split_workspace_bytes) p_gemm_ws;
+decltype(&lp_gemm_block_workspace_bytes) p_gemm_ws;
 decltype(&lp_host_flag) p_flag;
 decltype(&lp_host_table) p_table;
 decltype(&lp_quant_fp8_row_colwise_t) p_quant_both;
@@ -279,9 +279,10 @@ PyObject *gemm(PyObject *, PyObject *const *args, Py_ssize_t n)
             Unlocked u;
             at::Tensor ws;
             c = make({M, N}, out_code == LP_BF16 ? at::kBFloat16 : at::kFloat, dev);
-            const int64_t need = p_gemm_ws(M, N, K);
+            const int scales = scale_code(sa->scalar_type());
+            const int64_t need = p_gemm_ws(scales, M, N, K);
             if (need > 0) ws = make({need}, at::kByte, dev);
-            rc = p_gemm(a->const_data_ptr(), sa->const_data_ptr(), b->const_data_ptr(), sb->const_data_ptr(), scale_code(sa->scalar_type()), M, N, K,
+            rc = p_gemm(a->const_data_ptr(), sa->const_data_ptr(), b->const_data_ptr(), sb->const_data_ptr(), scales, M, N, K,
                         c.data_ptr(), (int)out_code, need > 0 ? ws.data_ptr() : nullptr, need, stream(dev));
         }
         if (rc) Py_RETURN_NONE;

@@ -54,6 +54,7 @@ PROTOTYPES = {
     "lp_host_table": (_i32, [_p, _i64, _p, _p]),
     "lp_host_flag": (_i32, [_p, _p]),
     "lp_gemm_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "lp_gemm_block_workspace_bytes": (_i64, [_i32, _i64, _i64, _i64]),
     "lp_gemm_split_workspace_bytes": (_i64, [_i64, _i64, _i64]),
 }
 

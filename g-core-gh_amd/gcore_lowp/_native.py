@@ -20,7 +20,7 @@ from . import _abi as A
 
 PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "_lowp_native.so")
 _BOUND = ("lp_quant_fp8_block", "lp_dequant_fp8_block", "lp_dequant_fp4_block", "lp_fp4_to_fp8_amax", "lp_fp4_to_fp8_rebase",
-          "lp_gemm_fp8_block", "lp_gemm_split_workspace_bytes", "lp_host_flag", "lp_host_table", "lp_quant_fp8_row_colwise_t",
+          "lp_gemm_fp8_block", "lp_gemm_block_workspace_bytes", "lp_host_flag", "lp_host_table", "lp_quant_fp8_row_colwise_t",
           "lp_gemm_fp8_grouped", "lp_gemm_fp8_grouped_nn", "lp_gemm_fp8_rowscale_grouped", "lp_zero_slots", "lp_gemm_fp8_grouped_rows")
 _ENTRIES = ("quant_fp8", "dequant", "fp4_to_fp8", "gemm", "grouped_forward", "grouped_backward")
 

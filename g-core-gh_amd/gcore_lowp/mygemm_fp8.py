@@ -61,7 +61,7 @@ def gemm_fp8_block_scaling_impl(Aq, As, Bq, Bs, BLK_M=64, BLK_N=128, BLK_K=128, 
         sa, sb, ca = sa.to(torch.float32), sb.to(torch.float32), A.F32
     C = torch.empty((M, N), dtype=out_dtype, device=dev)
     with torch.cuda.device(dev):
-        nws = A.lib().lp_gemm_split_workspace_bytes(M, N, K)
+        nws = A.lib().lp_gemm_block_workspace_bytes(ca, M, N, K)
         ws = _get_workspace(dev, nws)
         A.check(A.lib().lp_gemm_fp8_block(
             a.data_ptr(), sa.data_ptr(), b.data_ptr(), sb.data_ptr(), ca, M, N, K, C.data_ptr(),

@@ -102,7 +102,7 @@ def stand_in(tmp_path_factory):
     return ctypes.CDLL(str(d / "s.so"))
 
 
-HOST_ONLY = {"lp_gemm_split_workspace_bytes", "lp_host_flag"}          # answer on the host, without a launch
+HOST_ONLY = {"lp_gemm_block_workspace_bytes", "lp_host_flag"}          # answer on the host, without a launch
 
 
 @contextlib.contextmanager

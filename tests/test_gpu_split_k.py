@@ -119,3 +119,23 @@ def test_ranges_in_a_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, G.gemm_fp8_block_scaling_impl(xq, xs, wq, ws)), i
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_decode_kernels_get_no_scratch(monkeypatch, native):
+    """e8m0 scales at shapes whose fp32 form is cut: the call allocates its result and nothing else."""
+    import gcore_lowp as G
+    from gcore_lowp import mygemm_fp8
+    if not native:
+        class Nothing:
+            gemm = staticmethod(lambda *a: None)
+        monkeypatch.setattr(mygemm_fp8, "fast", Nothing)
+    M, N, K = 48, 8192, 9216
+    xq, xs = G.quant_fp8_e4m3_scale_e8m0(torch.ones(M, K, device="cuda", dtype=torch.bfloat16), (1, 128))
+    wq, ws = G.quant_fp8_e4m3_scale_e8m0(torch.ones(N, K, device="cuda", dtype=torch.bfloat16))
+    print("[case]", (M, N, K), native, flush=True)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = G.gemm_fp8_block_scaling_impl(xq, xs, wq, ws)
+    assert torch.cuda.max_memory_allocated() - before == out.numel() * 2

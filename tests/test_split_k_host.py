@@ -41,3 +41,16 @@ def test_shapes_the_decode_kernels_are_faster_at_are_not_cut(M, N, K):
 def test_shapes_the_ranges_are_faster_at_are_cut(M, N, K):
     from gcore_lowp import _abi
     assert _abi.lib().lp_gemm_split_workspace_bytes(M, N, K) > 0
+
+
+def test_scratch_by_type_of_scales():
+    """Decode shapes ask for none with e8m0 scales, which keep the decode kernels; elsewhere both types take the same plan, of at most 256 pieces."""
+    from gcore_lowp import _abi
+    L = _abi.lib()
+    for M, N, K in ((64, 5120, 6144), (48, 8192, 9216), (24, 5120, 9216), (70, 4096, 7168), (512, 1024, 7168), (64, 6144, 14336)):
+        assert L.lp_gemm_split_workspace_bytes(M, N, K) > 0 == L.lp_gemm_block_workspace_bytes(_abi.E8M0, M, N, K), (M, N, K)
+    r256 = lambda x: (x + 255) // 256 * 256
+    for M, N, K in ((2048, 256, 8192), (4096, 128, 8192), (129, 128, 7168), (145, 2176, 12416), (1899, 3072, 13696)):
+        copies = r256(M * (K // 128) * 4) + r256((N // 128) * (K // 128) * 4) if K % 512 == 0 else 0
+        need = L.lp_gemm_split_workspace_bytes(M, N, K)
+        assert 0 < need - copies <= 16 << 20 and need == L.lp_gemm_block_workspace_bytes(_abi.E8M0, M, N, K), (M, N, K)
