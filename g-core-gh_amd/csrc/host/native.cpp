@@ -280,8 +280,14 @@ PyObject *gemm(PyObject *, PyObject *const *args, Py_ssize_t n)
             at::Tensor ws;
             c = make({M, N}, out_code == LP_BF16 ? at::kBFloat16 : at::kFloat, dev);
             const int scales = scale_code(sa->scalar_type());
-            const int64_t need = p_gemm_ws(scales, M, N, K);
-            if (need > 0) ws = make({need}, at::kByte, dev);
+            int64_t need = p_gemm_ws(scales, M, N, K);
+            if (need > 0) {
+                try {
+                    ws = make({need}, at::kByte, dev);
+                } catch (const c10::OutOfMemoryError &) {
+                    need = 0;                                // the kernels that need none are slower, not fewer
+                }
+            }
             rc = p_gemm(a->const_data_ptr(), sa->const_data_ptr(), b->const_data_ptr(), sb->const_data_ptr(), scales, M, N, K,
                         c.data_ptr(), (int)out_code, need > 0 ? ws.data_ptr() : nullptr, need, stream(dev));
         }

@@ -17,10 +17,14 @@ __all__ = ["gemm_fp8_block_scaling_impl", "gemm_impl"]
 def _get_workspace(dev: torch.device, nbytes: int) -> torch.Tensor | None:
     """Scratch for the K-split kernels: a fresh tensor per call.  The caching allocator hands the block back to
     the stream that used it last, so two GEMMs on different streams never share partial sums (a cached buffer
-    per device would) and a block that is still being read is not given to another stream."""
+    per device would) and a block that is still being read is not given to another stream.
+    None where there is no room for it: the call runs without."""
     if nbytes <= 0:
         return None
-    return torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def _scale_arg(s: torch.Tensor, dev) -> tuple[torch.Tensor, int]:
@@ -66,7 +70,7 @@ def gemm_fp8_block_scaling_impl(Aq, As, Bq, Bs, BLK_M=64, BLK_N=128, BLK_K=128, 
         A.check(A.lib().lp_gemm_fp8_block(
             a.data_ptr(), sa.data_ptr(), b.data_ptr(), sb.data_ptr(), ca, M, N, K, C.data_ptr(),
             A.BF16 if out_dtype == torch.bfloat16 else A.F32,
-            ws.data_ptr() if ws is not None else None, nws, A.stream_ptr()))
+            ws.data_ptr() if ws is not None else None, nws if ws is not None else 0, A.stream_ptr()))
     return C.to(home)
 
 

@@ -139,3 +139,34 @@ def test_decode_kernels_get_no_scratch(monkeypatch, native):
     before = torch.cuda.memory_allocated()
     out = G.gemm_fp8_block_scaling_impl(xq, xs, wq, ws)
     assert torch.cuda.max_memory_allocated() - before == out.numel() * 2
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_no_room_for_scratch_is_no_error(monkeypatch, native):
+    """Memory for the result and not for the partial sums: the call runs as one without scratch does."""
+    import gcore_lowp as G
+    from gcore_lowp import _abi as A, mygemm_fp8
+    if not native:
+        class Nothing:
+            gemm = staticmethod(lambda *a: None)
+        monkeypatch.setattr(mygemm_fp8, "fast", Nothing)
+    L, (M, N, K) = A.lib(), (96, 5120, 14720)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    xq, xs = G.quant_1d(torch.randn(M, K, generator=g, device="cuda", dtype=torch.bfloat16))
+    wq, ws = G.quant_2d(torch.randn(N, K, generator=g, device="cuda", dtype=torch.bfloat16))
+    want = _call(L, A, (xq, xs, wq, ws), A.F32, M, N, K, torch.bfloat16, 0)
+    need = L.lp_gemm_split_workspace_bytes(M, N, K)
+    print("[case]", (M, N, K), native, flush=True)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    taken = []
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (6 << 20)) / total)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):          # what the cached segments still have room for goes first
+            while True:
+                taken.append(torch.empty(need, dtype=torch.uint8, device="cuda"))
+        got = G.gemm_fp8_block_scaling_impl(xq, xs, wq, ws)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(got, want)
