@@ -52,6 +52,20 @@ __device__ __forceinline__ bool tile_coords(uint32_t b, int64_t tiles_m, int64_t
     return true;
 }
 
+// Partial sums of a range of K (gemm_asm_split, splitk_reduce): M rows of 128 columns per tile column, a tile's rows behind those of the tile
+// above it.  In a tile, a wave's 64 rows x 64 columns in the order it stores them: blocks of 16 columns, in those blocks of 16 rows, 4 columns
+// of a row per lane.  With the 16-row blocks of both waves side by side a wave's stores jump by 8 KB: 1024 x 512 x 7168 14.6 -> 18.0 us.  The last
+// rows of M take no room beyond them, and go by blocks of rows first, so that only the last block's lines are not whole.  In floats, which 32
+// bits number (at most 32 MiB); `rows`: from the tile's first row to M.
+__device__ __forceinline__ uint32_t partial_tile(uint32_t tm, uint32_t tn, uint32_t M) { return (tn * M + tm * 128) * 128; }
+
+__device__ __forceinline__ int partial_offset(int wm, int wn, int nb, int mb, int lane, int rows)
+{
+    const int left = (rows < 128 ? rows : 128) - wm * 64, own = left < 64 ? left : 64, high = own - mb * 16 < 16 ? own - mb * 16 : 16;
+    const int block = own == 64 ? nb * (16 * 64) + mb * (16 * 16) : mb * (16 * 64) + nb * (16 * high);
+    return wm * (64 * 128) + wn * (64 * own) + block + ((lane >> 4) * (4 * high) + (lane & 15) * 4);
+}
+
 // The tiles of G problems of one shape, numbered problem by problem: pieces of 2^shift consecutive ones are dealt to the XCDs in
 // turn, forwards and backwards: in a list sorted by length the XCD with the longest of one turn has the shortest of the next.  (With every problem dealt from XCD 0 on as above, a problem of few tiles ran on few XCDs: 20 weight gradients of 1024 x
 // 1408 with three K blocks, 24 tiles each, on one of eight: 131 us, dealt in turn 30.  With pieces that end with their problem, the

@@ -97,6 +97,22 @@ def test_workspace_of_the_promised_size_and_the_built_in_buffer_agree(M, N, K):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 128, 12544), (129, 128, 7168), (65, 1152, 12544), (200, 256, 5120), (1041, 128, 16384), (100, 3072, 9216), (700, 128, 4736)], ids=str)
+def test_promised_workspace_holds_the_best_plan(M, N, K):
+    """Few tiles: partial sums take no room for rows beyond M, so lp_gemm_workspace_bytes holds as many ranges as a larger workspace would be used for."""
+    from gcore_lowp import _abi as A
+    L = A.lib()
+    A.require_gpu()
+    print("[case]", (M, N, K), flush=True)
+    (xq, xs), (wq, ws) = (T.quant_block_fp32_scale(t, b) for t, b in ((I.act_like(M, K, 1), (1, 128)), (I.weight_like(N, K, 2, outliers=False), (128, 128))))
+    ops = [t.cuda().contiguous() for t in (xq, xs, wq, ws)]
+    promised, best = L.lp_gemm_workspace_bytes(M, N, K), L.lp_gemm_split_workspace_bytes(M, N, K)
+    assert promised > 0 and best > 0
+    got = _call(L, A, ops, A.F32, M, N, K, torch.float32, promised)
+    assert torch.equal(got, _call(L, A, ops, A.F32, M, N, K, torch.float32, best))
+    assert not torch.equal(got, _call(L, A, ops, A.F32, M, N, K, torch.float32, 0))            # it is cut at all
+
+
 def test_ranges_in_a_graph():
     """Captured with its scratch and replayed: every replay is the eager call's result."""
     import gcore_lowp as G

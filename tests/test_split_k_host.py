@@ -54,3 +54,23 @@ def test_scratch_by_type_of_scales():
         copies = r256(M * (K // 128) * 4) + r256((N // 128) * (K // 128) * 4) if K % 512 == 0 else 0
         need = L.lp_gemm_split_workspace_bytes(M, N, K)
         assert 0 < need - copies <= 16 << 20 and need == L.lp_gemm_block_workspace_bytes(_abi.E8M0, M, N, K), (M, N, K)
+
+
+def test_promised_scratch_holds_every_plan():
+    """Problems of at most 32 tiles: the partial sums of the best plan, M rows per range, fit what lp_gemm_workspace_bytes promises."""
+    from gcore_lowp import _abi
+    L = _abi.lib()
+    rng = random.Random(8)
+    r256 = lambda x: (x + 255) // 256 * 256
+    seen = 0
+    for _ in range(4000):
+        M, N, K = rng.randint(65, 4096), 128 * rng.randint(1, 32), 128 * rng.randint(32, 160)
+        tiles_m = (M + 127) // 128
+        best, promised = L.lp_gemm_split_workspace_bytes(M, N, K), L.lp_gemm_workspace_bytes(M, N, K)
+        copies = r256(M * (K // 128) * 4) + r256((N // 128) * (K // 128) * 4) if K % 512 == 0 else 0
+        if tiles_m * (N // 128) > 32 or promised == copies:
+            continue
+        ranges, left = divmod(best - copies, tiles_m * 128 * N * 4)
+        assert left == 0 and ranges * M * N * 4 <= promised - copies, (M, N, K)
+        seen += 1
+    assert seen > 200
