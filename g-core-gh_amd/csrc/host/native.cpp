@@ -389,9 +389,11 @@ PyObject *grouped_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
             };
             const auto result = [&] { return make({rows, N}, out_code == LP_BF16 ? at::kBFloat16 : at::kFloat, dev); };
             rc = LP_ERR_UNSUPPORTED;
+            bool quantised = false;
             if (!train && !backward) {
-                // nobody else wants the offsets: they go with the GEMM's arguments
+                // nobody else wants the offsets: they go with the GEMM's arguments, unless it refuses (more than 512 experts, 4 GiB)
                 rc = quantise();
+                quantised = !rc;
                 if (!rc) {
                     out = result();
                     rc = p_grouped_rows(q.data_ptr(), s.data_ptr(), wq->const_data_ptr(), ws->const_data_ptr(), LP_E8M0, ex.offsets.data(), (int)E, rows, N,
@@ -414,11 +416,11 @@ PyObject *grouped_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
                     qt = make({K * ex.blocks * 128}, at::kByte, dev), st = make({K * ex.blocks}, at::kByte, dev);
                     rc = p_quant_both(x->const_data_ptr(), in_code, rows, K, offs.data_ptr<int32_t>(), (int)E, ex.blocks, 128, q.data_ptr(), s.data_ptr(),
                                       qt.data_ptr(), st.data_ptr(), LP_E8M0, s_);
-                } else if (!rc) {
+                } else if (!rc && !quantised) {
                     rc = quantise();
                 }
                 if (!rc) {
-                    out = result();
+                    if (!out.defined()) out = result();
                     rc = p_grouped(q.data_ptr(), s.data_ptr(), wq->const_data_ptr(), ws->const_data_ptr(), LP_E8M0, offs.data_ptr<int32_t>(), (int)E, rows,
                                    N, K, out.data_ptr(), (int)out_code, s_);
                 }

@@ -109,6 +109,31 @@ def test_front_end_in_a_graph(G):
             assert torch.equal(out, layer(x, w, splits)), i
 
 
+def test_more_experts_than_the_arguments_hold_are_quantised_once(G):
+    """The launch that takes the offsets by value refuses; the activations are quantised and the result is allocated once all the same."""
+    import ctypes
+    from gcore_lowp import _abi as A, _native
+    mod, L, calls = _native._load(), A.lib(), []
+    restype, argtypes = A.PROTOTYPES["lp_quant_fp8_block"]
+    counting = ctypes.CFUNCTYPE(restype, *argtypes)(lambda *a: calls.append(1) or L.lp_quant_fp8_block(*a))
+    real = [ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in _native._BOUND]
+    at = _native._BOUND.index("lp_quant_fp8_block")
+    splits, (k, n) = SPLITS["513 experts"], (256, 128)
+    x = torch.randn(sum(splits), k, device="cuda", dtype=torch.bfloat16)
+    q = torch.zeros(len(splits), n, k, device="cuda").to(torch.float8_e4m3fn)
+    s = torch.ones(len(splits), n // 128, k // 128, device="cuda").to(torch.float8_e8m0fnu)
+    print("[case]", len(splits), "experts", flush=True)
+    mod.bind(*real[:at], ctypes.cast(counting, ctypes.c_void_p).value, *real[at + 1:])
+    try:
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        out = mod.grouped_forward(x, q, s, splits, A.BF16, False, False)
+        made = torch.cuda.memory_stats()["allocation.all.allocated"] - before
+    finally:
+        mod.bind(*real)
+    assert out is not None and len(calls) == 1
+    assert made == 4                                     # codes, scales, result, the table with the offsets
+
+
 def test_row_counts_the_front_end_refuses(G):
     from gcore_lowp import _abi as A, _native
     x = torch.zeros(4, 128, device="cuda", dtype=torch.bfloat16)
