@@ -18,16 +18,18 @@ CASES = [
     (640, 1920, 11392),
     (1000, 4992, 6016),     # 312 tiles: 32 columns of them whole, seven cut
     (1537, 2688, 9344),     # the last row tile of one row
-    (64, 6144, 6144), (33, 4224, 7168), (49, 4224, 7168), (17, 5120, 7296),       # ahead of the decode kernels
+    (64, 5120, 6144), (56, 4224, 7168), (33, 5120, 7296), (24, 5120, 8192), (17, 5376, 14464), (70, 4096, 7168),      # ahead of the decode kernels
     (47, 2432, 15232),      # up to 64 rows without a decode kernel for this K
 ]
 
 
-def _call(L, A, ops, sdt, M, N, K, dtype, scratch):
+def _call(L, A, ops, sdt, M, N, K, dtype, scratch, cut=None):
+    """`cut`: whether the call must have written partial sums to its scratch"""
     out = torch.full((M, N), float("nan"), dtype=dtype, device="cuda")
     ws = torch.full((max(scratch, 16) // 4,), float("nan"), device="cuda")
     A.check(L.lp_gemm_fp8_block(*(t.data_ptr() for t in ops), sdt, M, N, K, out.data_ptr(), A.BF16 if dtype == torch.bfloat16 else A.F32,
                                 ws.data_ptr() if scratch else None, scratch, A.stream_ptr()))
+    assert cut is None or bool((~ws.isnan()).any()) == cut
     return out
 
 
@@ -39,7 +41,10 @@ def test_ranges_against_whole_tiles(M, N, K, pow2):
     A.require_gpu()
     need = L.lp_gemm_split_workspace_bytes(M, N, K)
     print("[case]", (M, N, K), "e8m0" if pow2 else "f32", need, flush=True)
-    assert 0 < need <= 36 << 20 or M <= 64
+    assert 0 < need <= 20 << 20
+    # with e8m0 scales the decode kernels keep their shapes, whatever the scratch
+    cuts = not pow2 or L.lp_gemm_block_workspace_bytes(A.E8M0, M, N, K) > 0
+    assert cuts or M <= 128
     x, w = I.act_like(M, K, M + K), I.weight_like(N, K, N, outliers=False)
     quant = T.quant_fp8_e4m3_scale_e8m0 if pow2 else T.quant_block_fp32_scale
     (xq, xs), (wq, ws) = quant(x, (1, 128)), quant(w, (128, 128))
@@ -50,18 +55,19 @@ def test_ranges_against_whole_tiles(M, N, K, pow2):
         b = slice(k, k + 128)
         part = ops[0][:, b].double() @ ops[2][:, b].double().t()
         exact += part * ops[1][:, k // 128].double()[:, None] * ops[3][:, k // 128].double().repeat_interleave(128)[None, :]
-    whole, cut = (_call(L, A, ops, sdt, M, N, K, torch.float32, n) for n in (0, need))
+    whole, cut = (_call(L, A, ops, sdt, M, N, K, torch.float32, n, n > 0 and cuts) for n in (0, need))
+    assert cuts or torch.equal(whole, cut)
     err = [((o.double() - exact).norm() / exact.norm()).item() for o in (whole, cut)]
-    # the matrix instruction's own error, 1.5e-5 over one K block and over many (up to 2.5e-5 with loud channels); the ranges are
-    # added in fp32 (half an ulp, 6e-8 each)
-    assert err[1] <= max(err[0], 1e-6) * 1.02 and err[1] < 4e-5, err
-    narrow = _call(L, A, ops, sdt, M, N, K, torch.bfloat16, need)
+    # the matrix instruction's own error, 1.5e-5 over one K block and over many (up to 2.5e-5 with loud channels); up to 16 ranges are
+    # added in fp32 (half an ulp, 6e-8 each: 3e-4 of that error)
+    assert err[1] <= max(err[0], 1e-6) * 1.002 and err[1] < 4e-5, err
+    narrow = _call(L, A, ops, sdt, M, N, K, torch.bfloat16, need, cuts)
     assert torch.equal(narrow, cut.to(torch.bfloat16))                   # the same sums, rounded once
     assert torch.equal(cut, _call(L, A, ops, sdt, M, N, K, torch.float32, need))
     # less scratch than the plan's: fewer ranges or none, same result within the same error
     for n in (need // 2, need // 16 & ~15):
         less = _call(L, A, ops, sdt, M, N, K, torch.float32, n)
-        assert ((less.double() - exact).norm() / exact.norm()).item() <= max(err[0], 1e-6) * 1.02
+        assert ((less.double() - exact).norm() / exact.norm()).item() <= max(err[0], 1e-6) * 1.002
 
 
 @pytest.mark.parametrize("M,N,K", [(100, 2048, 16384), (64, 1024, 18432), (65, 1152, 12544), (129, 128, 7168), (512, 512, 7168), (200, 256, 5120), (927, 128, 4096)], ids=str)
@@ -77,12 +83,11 @@ def test_e8m0_ranges_of_few_tiles_fold_every_block(M, N, K):
     xs, ws = (torch.randint(120, 126, s, generator=g, device="cuda", dtype=torch.uint8) for s in ((M, K // 128), (N // 128, K // 128)))
     f32 = [torch.pow(2.0, t.float() - 127) for t in (xs, ws)]
     need = L.lp_gemm_split_workspace_bytes(M, N, K)
-    assert need > 0
-    folded = _call(L, A, (xq, f32[0], wq, f32[1]), A.F32, M, N, K, torch.float32, need)
-    assert torch.equal(_call(L, A, (xq, xs, wq, ws), A.E8M0, M, N, K, torch.float32, need), folded)
+    folded = _call(L, A, (xq, f32[0], wq, f32[1]), A.F32, M, N, K, torch.float32, need, True)
+    assert torch.equal(_call(L, A, (xq, xs, wq, ws), A.E8M0, M, N, K, torch.float32, need, True), folded)
 
 
-@pytest.mark.parametrize("M,N,K", [(384, 512, 7168), (65, 1152, 7168), (4000, 128, 7168), (1000, 512, 4608), (33, 4224, 7168)], ids=str)
+@pytest.mark.parametrize("M,N,K", [(384, 512, 7168), (65, 1152, 7168), (4000, 128, 7168), (1000, 512, 4608), (33, 5120, 7296)], ids=str)
 def test_workspace_of_the_promised_size_and_the_built_in_buffer_agree(M, N, K):
     """lp_gemm_fp8_block with lp_gemm_workspace_bytes and lp_gemm_fp8_block_static: the same plan, whatever room the former has for scale copies."""
     from gcore_lowp import _abi as A
