@@ -231,10 +231,10 @@ int lp_gemm_fp8_block(const void *Aq, const void *As, const void *Bq, const void
 int64_t lp_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /*
- * Scratch bytes with which lp_gemm_fp8_block is fastest on this shape and type of scales: at most 16 MiB and room for scale copies, 0 where
- * a problem is not cut along K, and no less than the K split can use of lp_gemm_workspace_bytes.  With it problems of more than 32
- * tiles are cut along K too where that pays.  No counterpart in the reference (its GEMM is a JIT kernel without scratch,
- * gfused/mygemm_fp8.py:44-97).
+ * Scratch bytes with which lp_gemm_fp8_block is fastest on this shape and type of scales: the partial sums of its K ranges, at most 16 MiB (always
+ * more than lp_gemm_workspace_bytes where that has no room for any, which only counts from K = 52000 on), and 0 where a problem is not cut along K.
+ * With it problems of more than 32 tiles are cut along K too where that pays.  No counterpart in the reference (its GEMM is a
+ * JIT kernel without scratch, gfused/mygemm_fp8.py:44-97).
  */
 int64_t lp_gemm_block_workspace_bytes(int scale_dtype, int64_t M, int64_t N, int64_t K);
 
