@@ -52,12 +52,12 @@ __device__ __forceinline__ bool tile_coords(uint32_t b, int64_t tiles_m, int64_t
     return true;
 }
 
-// Partial sums of a range of K (gemm_asm_split, splitk_reduce): M rows of 128 columns per tile column, a tile's rows behind those of the tile
+// Partial sums of a range of K (gemm_asm_split, splitk_reduce): SplitPlan's rows of 128 columns per tile column, a tile's rows behind those of the tile
 // above it.  In a tile, a wave's 64 rows x 64 columns in the order it stores them: blocks of 16 columns, in those blocks of 16 rows, 4 columns
-// of a row per lane.  With the 16-row blocks of both waves side by side a wave's stores jump by 8 KB: 1024 x 512 x 7168 14.6 -> 18.0 us.  The last
-// rows of M take no room beyond them, and go by blocks of rows first, so that only the last block's lines are not whole.  In floats, which 32
-// bits number (at most 32 MiB); `rows`: from the tile's first row to M.
-__device__ __forceinline__ uint32_t partial_tile(uint32_t tm, uint32_t tn, uint32_t M) { return (tn * M + tm * 128) * 128; }
+// of a row per lane.  With the 16-row blocks of both waves side by side a wave's stores jump by 8 KB: 1024 x 512 x 7168 14.6 -> 18.0 us.  Where there is no
+// room for rows beyond M its last ones go by blocks of rows first, so that only the last block's lines are not whole.  In floats,
+// which 32 bits number (at most 32 MiB); `rows`: from the tile's first row on.
+__device__ __forceinline__ uint32_t partial_tile(uint32_t tm, uint32_t tn, uint32_t rows) { return (tn * rows + tm * 128) * 128; }
 
 __device__ __forceinline__ int partial_offset(int wm, int wn, int nb, int mb, int lane, int rows)
 {
@@ -151,11 +151,12 @@ bool launch_wide(const void *Aq, const void *As, const void *Bq, const void *Bs,
                  void *C, int64_t ldc, int out_dtype, hipStream_t st, int *rc);
 bool launch_mixed(const void *Aq, const void *As, const void *Bq, const void *Bs, int scale_dtype, int64_t M, int64_t N, int64_t K,
                   int64_t n_big, void *C, int64_t ldc, int out_dtype, hipStream_t st, int *rc);
-// A dense problem on 128 x 128 tiles of which those at or behind column n_whole are cut into `splits` ranges of `per` K blocks; fold: e8m0
-// products are added up in fp32 (gemm_asm_split).
+// A dense problem on 128 x 128 tiles of which those at or behind column n_whole are cut into `splits` ranges of `per` K blocks; rows: of
+// partial sums, M or whole tiles; fold: e8m0 products are added up in fp32 (gemm_asm_split).
 struct SplitPlan {
     int64_t n_whole;
     int splits, per;
+    int64_t rows;
     bool fold;
 };
 int launch_split(const void *Aq, const void *As, const void *Bq, const void *Bs, int scale_dtype, int64_t M, int64_t N, int64_t K,

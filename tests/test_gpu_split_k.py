@@ -104,7 +104,7 @@ def test_workspace_of_the_promised_size_and_the_built_in_buffer_agree(M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(65, 128, 12544), (129, 128, 7168), (65, 1152, 12544), (200, 256, 5120), (1041, 128, 16384), (100, 3072, 9216), (700, 128, 4736)], ids=str)
 def test_promised_workspace_holds_the_best_plan(M, N, K):
-    """Few tiles: partial sums take no room for rows beyond M, so lp_gemm_workspace_bytes holds as many ranges as a larger workspace would be used for."""
+    """Few tiles: partial sums need no room for rows beyond M, so lp_gemm_workspace_bytes holds as many ranges as a larger workspace, with whole tiles of rows, is used for."""
     from gcore_lowp import _abi as A
     L = A.lib()
     A.require_gpu()
