@@ -217,17 +217,21 @@ int lp_act_qdq_group(const void *x, int64_t n, int group, int pow2_scale, int th
  * Aq: device e4m3fn [M,K]; As: device [M,K/128]; Bq: device e4m3fn [N,K];
  * Bs: device [N/128,K/128]; scales of scale_dtype (LP_F32 or LP_E8M0);
  * C: device [M,N] LP_BF16 or LP_F32.  K % 128 == 0, N % 128 == 0, any M.
- * workspace: optional device scratch of at least lp_gemm_workspace_bytes(M,N,K)
- * bytes (256-byte aligned); with it, problems with few output tiles split K
- * across workgroups (fixed summation order) and LP_E8M0 scales are expanded to
- * fp32 for the fastest kernels.  NULL / too small = slower paths, same results.
+ * workspace: optional device scratch (256-byte aligned), best of
+ * lp_gemm_block_workspace_bytes(scale_dtype,M,N,K) bytes; with it, problems
+ * whose tiles leave the GPU idle split K across workgroups, as fp32 partial
+ * sums that are added in a fixed order.  NULL / too small = fewer ranges or
+ * none: slower, and fp32 sums in another order (their last bits differ).
  * Replaces gemm_fp8_block_scaling_impl (gfused/mygemm_fp8.py:44-97).
  */
 int lp_gemm_fp8_block(const void *Aq, const void *As, const void *Bq, const void *Bs, int scale_dtype,
                       int64_t M, int64_t N, int64_t K, void *C, int out_dtype,
                       void *workspace, int64_t workspace_bytes, lp_stream_t stream);
 
-/* Scratch bytes lp_gemm_fp8_block can use for this shape (0 = none needed). */
+/*
+ * Scratch bytes with which lp_gemm_fp8_block splits K of at most 32 tiles of 128 x 128, as lp_gemm_fp8_block_static does (0 = it does not;
+ * from 65 rows on with K % 512 == 0 room for fp32 copies of LP_E8M0 scales is in it, which only a tuning aid fills).
+ */
 int64_t lp_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /*
@@ -248,7 +252,7 @@ int64_t lp_gemm_split_workspace_bytes(int64_t M, int64_t N, int64_t K);
  * holds one copy until the process ends).  Same kernels, same summation order and therefore the same bits as
  * lp_gemm_fp8_block with a workspace of lp_gemm_workspace_bytes(M, N, K).  The call allocates and frees nothing.
  * A shape whose K split needed more than the buffer would be rejected with LP_ERR_INVALID and a message naming both
- * sizes; the K split is taken for at most 32 tiles of 128 x 128 in at most 16 K ranges, which is 32 MiB, so no shape
+ * sizes; the K split is taken here for at most 32 tiles of 128 x 128, and 16 ranges of those are 32 MiB, so no shape
  * is turned away today (shapes that need no scratch always pass).  All calls on one GPU share that GPU's buffer: calls that can
  * overlap on one GPU (different streams, or threads) race on it -- serialise them or use lp_gemm_fp8_block.
  * Nothing has to be cleared between calls: every partial tile is written before it is read.
