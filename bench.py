@@ -300,7 +300,7 @@ def main():
                 wss_.append(ws_)
                 del wb
             cq_ = torch.empty(m_q, n_q, dtype=torch.bfloat16, device=dev)
-            nws_q = L.lp_gemm_split_workspace_bytes(m_q, n_q, k_q)
+            nws_q = L.lp_gemm_block_workspace_bytes(A.F32, m_q, n_q, k_q)
             wsp_q = torch.empty(max(nws_q, 16), dtype=torch.uint8, device=dev)
             fns = [(lambda i=i: chk(L.lp_gemm_fp8_block(xq_.data_ptr(), xs_.data_ptr(), wqs_[i].data_ptr(), wss_[i].data_ptr(), A.F32, m_q, n_q, k_q,
                                                         cq_.data_ptr(), A.BF16, wsp_q.data_ptr(), nws_q, stream()))) for i in range(n_sets_q)]
@@ -472,7 +472,7 @@ def main():
                 w3s.append(sc)
                 del w
             c3 = torch.empty(M3, N3, dtype=torch.bfloat16, device=dev)
-            nws = L.lp_gemm_split_workspace_bytes(M3, N3, K3)   # as the Python wrapper passes it
+            nws = L.lp_gemm_block_workspace_bytes(A.F32, M3, N3, K3)   # as the Python wrapper passes it
             ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=dev)
             fns = [(lambda i=i: chk(L.lp_gemm_fp8_block(a3q.data_ptr(), a3s.data_ptr(), w3q[i].data_ptr(), w3s[i].data_ptr(), A.F32,
                                                         M3, N3, K3, c3.data_ptr(), A.BF16, ws.data_ptr(), nws, stream())))
