@@ -46,7 +46,7 @@ def short(name):
         parts = name.split("_")
         keep = [p for p in parts if p.startswith(("MT", "MI", "SK", "shortname")) or p in ("F8BS", "BH", "NTD")]
         return "hipBLASLt " + "_".join(keep)
-    name = name.replace("(anonymous namespace)::", "").replace("void ", "")
+    name = name.replace("(anonymous namespace)::", "").replace("void ", "").replace(", NoTable>", ">")
     return name.split("(")[0]
 
 
