@@ -20,26 +20,32 @@ namespace {
 
 // ---------------------------------------------------------------- 128 x 128
 
+// Bound by HBM.  A large matrix: eight waves a tile and runs of RUN = 4 neighbouring tiles of a row on one XCD, so that what an XCD's workgroups read
+// together are pieces of 1 KB of a row and not 256 bytes of every eighth tile (us, power-of-two scales, 256 threads and tiles dealt one by one ->
+// 512 and runs of four: 131072 x 4096 276 -> 243 = 6.6 TB/s, where a plain copy of the same 2 : 1 mix takes 252; 18432 x 7168 66.4 -> 63.3,
+// 36864 x 1536 29.7 -> 29.3; runs of two 262, of eight 246; 256 threads in runs of four 256; 1024 threads 262).  Below kRunTiles a launch is few rounds
+// of workgroups and its tail counts: 4096 x 7168 16.4 <- 16.9, divided scales 17.9 <- 18.4.
+constexpr int64_t kRunTiles = 3072;
+
 // amax bits are compared as integers: for non-NaN values the ordering of |x|
 // equals the ordering of the sign-cleared bit patterns, and any NaN sorts
 // above +inf, so one integer max finds both amax and NaN/inf presence.
-template <bool IS_BF16, int MODE>
-__global__ __launch_bounds__(256) void quant_tile128(const void *__restrict__ xin, int64_t cols, int64_t tiles_c,
-                                                     uint8_t *__restrict__ q, void *__restrict__ scale_out,
-                                                     int scale_dtype, float amax_floor, int zero_rule,
-                                                     int32_t *nan_count)
+template <bool IS_BF16, int MODE, int NT, int RUN>
+__global__ __launch_bounds__(NT) void quant_tile128(const void *__restrict__ xin, int64_t cols, uint32_t tiles_c, uint32_t tiles,
+                                                    uint8_t *__restrict__ q, void *__restrict__ scale_out,
+                                                    int scale_dtype, float amax_floor, int zero_rule,
+                                                    int32_t *nan_count)
 {
-    __shared__ uint32_t wave_amax[4];
-    const int64_t tile = blockIdx.x;
-    const int64_t tr = tile / tiles_c, tc = tile - tr * tiles_c;
+    __shared__ uint32_t wave_amax[NT / 64];
+    const uint32_t tile = RUN == 1 ? blockIdx.x : ((blockIdx.x >> 3) / RUN * 8 + (blockIdx.x & 7)) * RUN + (blockIdx.x >> 3) % RUN;
+    if (RUN > 1 && tile >= tiles) return;
+    const uint32_t tr = tile / tiles_c, tc = tile - tr * tiles_c;
     const int t = threadIdx.x;
 
-    constexpr int NV = IS_BF16 ? 8 : 16;        // 128-bit vectors per thread
+    constexpr int PER_ROW = IS_BF16 ? 16 : 32;                        // lanes that cover a row of the tile, 16 bytes each
+    constexpr int row_step = NT / PER_ROW, NV = 128 / row_step;       // 128-bit vectors per thread
     u32x4 w[NV];
-    int64_t row0, col0;
-    int row_step;
-    if (IS_BF16) { row0 = tr * 128 + (t >> 4); col0 = tc * 128 + (t & 15) * 8; row_step = 16; }
-    else         { row0 = tr * 128 + (t >> 5); col0 = tc * 128 + (t & 31) * 4; row_step = 8; }
+    const int64_t row0 = (int64_t)tr * 128 + t / PER_ROW, col0 = (int64_t)tc * 128 + (t % PER_ROW) * (128 / PER_ROW);
 
     const char *xb = (const char *)xin;
     const int esz = IS_BF16 ? 2 : 4;
@@ -73,10 +79,9 @@ __global__ __launch_bounds__(256) void quant_tile128(const void *__restrict__ xi
     mbits = wave_max_u32(mbits);
     if ((t & 63) == 0) wave_amax[t >> 6] = mbits;
     __syncthreads();
-    {
-        uint32_t a = wave_amax[0], b = wave_amax[1], c = wave_amax[2], d = wave_amax[3];
-        a = a > b ? a : b; c = c > d ? c : d; mbits = a > c ? a : c;
-    }
+    mbits = wave_amax[0];
+#pragma unroll
+    for (int i = 1; i < NT / 64; ++i) mbits = wave_amax[i] > mbits ? wave_amax[i] : mbits;
     const bool special = mbits >= 0x7F800000u;       // inf or NaN somewhere in the block
     const bool has_nan = mbits > 0x7F800000u;
     const float amax = u2f(has_nan ? 0x7FC00000u : mbits);
@@ -98,6 +103,12 @@ __global__ __launch_bounds__(256) void quant_tile128(const void *__restrict__ xi
         return;
     }
     if (IS_BF16) {
+        if (MODE == LP_SCALE_POW2 && pow2_convert_ok(bs.exp2)) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+                __builtin_nontemporal_store(bf16_codes8(w[i], bs.stored), (u32x2 *)(q + (row0 + (int64_t)i * row_step) * cols + col0));
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             float v[8];
@@ -268,12 +279,14 @@ int launch_mode(const void *x, bool is_bf16, int64_t rows, int64_t cols, int bm,
     if (bm == 128 && bn == 128 && aligned16) {
         int64_t tiles_c = cols / 128, tiles = (rows / 128) * tiles_c;
         if (tiles > 0x7FFFFFFF) return fail(LP_ERR_UNSUPPORTED, "lp_quant_fp8_block: too many tiles");
-        if (is_bf16)
-            hipLaunchKernelGGL((quant_tile128<true, MODE>), dim3((unsigned)tiles), dim3(256), 0, st, x, cols, tiles_c,
-                               q, scale_out, scale_dtype, amax_floor, zero_rule, nan_count);
-        else
-            hipLaunchKernelGGL((quant_tile128<false, MODE>), dim3((unsigned)tiles), dim3(256), 0, st, x, cols, tiles_c,
-                               q, scale_out, scale_dtype, amax_floor, zero_rule, nan_count);
+        auto go = [&](auto kernel, int threads, int64_t grid) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(threads), 0, st, x, cols, (uint32_t)tiles_c, (uint32_t)tiles, q, scale_out, scale_dtype,
+                               amax_floor, zero_rule, nan_count);
+        };
+        // 512 threads and runs of four tiles per XCD from kRunTiles on (see quant_tile128)
+        if (!is_bf16) go(quant_tile128<false, MODE, 256, 1>, 256, tiles);
+        else if (tiles >= kRunTiles && tiles <= 0x7FFFFFFF - 31) go(quant_tile128<true, MODE, 512, 4>, 512, (tiles + 31) / 32 * 32);
+        else go(quant_tile128<true, MODE, 256, 1>, 256, tiles);
     } else if (bm == 1 && bn == 128 && aligned16) {
         // Passes per workgroup: one up to 2^17 groups, where a launch has few workgroups per CU and what counts is that all
         // of it is on its way at once (us with one / four passes: 1 x 7168 2.1 / 3.4, 64 x 7168 2.5 / 3.7, 1000 x 2944 4.0 / 4.9,

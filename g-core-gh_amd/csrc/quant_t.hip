@@ -63,6 +63,8 @@ __device__ __forceinline__ BlockScale block_scale(uint32_t m, bool special)
 
 // 8 finite values over the scale, as codes: |x| <= amax <= 448 * 2^e and x * 2^-e is exact, no quotient leaves the e4m3
 // range, nothing to clamp.  2^-e is no normal float at the ends of the range: rare, and exact either way.
+// (bf16 within pow2_convert_ok takes bf16_codes8 instead, a column's values side by side by a permute: us, rows and columns, 16384 x 4096 54.8 ->
+// 53.8, 65536 x 4096 193 -> 187.5, 1754 x 2048 12.1 -> 11.7.)
 template <class F>
 __device__ __forceinline__ u32x2 codes8(F value, int exp2)
 {
@@ -197,8 +199,10 @@ __global__ __launch_bounds__(256) void quant_colwise_t(const void *__restrict__ 
             const bool special = rmax[i] >= 0x7F800000u;
             const BlockScale bs = block_scale<IS_BF16>(rmax[i], special);
             if (cc == 0) store_scale(s, scale_dtype, r * (cols >> 7) + (c0 >> 7), bs.stored);
+            u32x2 *dst = (u32x2 *)(q + r * cols + c0 + cc * 8);
             if (special) literal_rows |= 1u << i;
-            else __builtin_nontemporal_store(codes8([&](int j) { return elem(i, j); }, bs.exp2), (u32x2 *)(q + r * cols + c0 + cc * 8));
+            else if (IS_BF16 && pow2_convert_ok(bs.exp2)) __builtin_nontemporal_store(bf16_codes8(u32x4{rw[i][0], rw[i][1], rw[i][2], rw[i][3]}, bs.stored), dst);
+            else __builtin_nontemporal_store(codes8([&](int j) { return elem(i, j); }, bs.exp2), dst);
             // one row after the other, and nothing unpacked is kept for the columns: registers for the workgroups of a CU
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -288,6 +292,11 @@ __global__ __launch_bounds__(256) void quant_colwise_t(const void *__restrict__ 
                 lo |= (uint32_t)quant_slow<LP_SCALE_POW2>(elem(i, j), bs) << (8 * i);
                 hi |= (uint32_t)quant_slow<LP_SCALE_POW2>(elem(4 + i, j), bs) << (8 * i);
             }
+        } else if (IS_BF16 && pow2_convert_ok(bs.exp2)) {
+            // a column's values of two rows, side by side
+            auto two = [&](int i) { return __builtin_amdgcn_perm(rw[i + 1][(j >> 1) & 3], rw[i][(j >> 1) & 3], (j & 1) ? 0x07060302u : 0x05040100u); };
+            const u32x2 c8 = bf16_codes8(u32x4{two(0), two(2), two(4), two(6)}, bs.stored);
+            lo = c8.x; hi = c8.y;
         } else {
             const u32x2 c8 = codes8([&](int i) { return elem(i, j); }, bs.exp2);
             lo = c8.x; hi = c8.y;
