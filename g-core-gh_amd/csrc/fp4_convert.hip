@@ -8,13 +8,14 @@
 //                (scale from amax); the bf16 tensor is written only on request.
 //
 // One workgroup (256 or 512 threads) owns a 128-row x 256-column "super tile" (two scale
-// tiles side by side) so that every row segment it touches is a full 128-byte
+// tiles side by side; the fused kernel has a form with four) so that every row segment it touches is a full 128-byte
 // line of packed input and 256 bytes of output.  Lane l of a 32-lane half wave
 // owns 4 packed bytes (8 elements); lanes 0-15 belong to the left tile, 16-31
 // to the right one (the fused kernel has a form with twice that per lane, 16 lanes
 // to a row).  The packed tile lives in 16 (8) VGPRs per lane, so HBM is
 // read exactly once.
 #include <type_traits>
+#include <utility>
 
 #include "lowp_device.h"
 
@@ -28,61 +29,54 @@ namespace {
 // more when a lane has fewer passes; with 1024 threads both lose 10-20 %).
 constexpr int kRebaseThreads = 512;
 constexpr int kAmaxThreads = 256;
-// The fused kernel, up to this many super tiles: a lane owns two packed words of a row (one scale byte still covers both), which halves its memory
-// instructions and the table work per element.  What counts while a launch is a round or two of workgroups (us a launch, back to back, one word
-// -> two: 512 x 1024 4.20 -> 3.92, 2048 x 7168 6.17 -> 5.95, 7168 x 2048 5.91 -> 5.66, 4096 x 7168 10.68 -> 10.35); level from 8192 x 7168 on, and
-// 1 % behind at 32768 x 7168 (7168 super tiles).
-constexpr int64_t kTwoWordSupers = 4096;
+// The fused kernel where the buffers' alignment lets a lane own two packed words of a row (one scale byte still covers both), which halves its memory
+// instructions and the table work per element (us a launch, back to back, one word -> two: 2048 x 7168 6.13 -> 5.41, 7168 x 2048 5.98 -> 5.25, 512 x
+// 1024 level, 32768 x 1152 15.4 -> 13.8, 65536 x 7168 132.7 -> 131.9).  One word a lane is left to other alignments and to the form that writes bf16 too.
+// From more than kNarrowSupers super tiles (two on every CU) on, four tiles side by side on 512 threads: rows of 256 packed bytes and 512 of output
+// (two -> four tiles: 2560 x 7168 7.81 -> 7.10, 4096 x 7168 11.5 -> 8.3, 16384 x 7168 37.6 -> 34.8, 65536 x 7168 131.9 -> 124.4 = 5.8 TB/s), if
+// that adds no more than a sixteenth of empty tiles at the rows' ends (five tiles a row, 65536 x 640, 15.7 <- 17.3; nine, 32768 x 1152, 13.8 <- 14.5).
+// Below, it leaves CUs without a workgroup: 2048 x 7168 5.41 <- 5.64, 7168 x 2304 5.48 <- 6.84.
+constexpr int kWideThreads = 512;
+constexpr int64_t kNarrowSupers = 512;
 
-// Maxima over the two 128 x 128 tiles of the super tile: every lane gets its own tile's and the other tile's,
-// from one barrier.  The 16 lanes of a DPP row all belong to one tile and the rows of a wave alternate between
-// the tiles, so a wave reduces to one value per tile (DPP within rows, one cross-lane exchange between rows r and
-// r + 2), the workgroup's waves meet in `lds`, and a second DPP reduction over one entry per lane finishes.
+// Maximum over the lane's own 128 x 128 tile, from one barrier.  One word a lane (W = 1, two tiles side by side): the 16 lanes of a DPP row belong to
+// one tile and the rows of a wave alternate between the tiles, so a wave reduces to one value per tile (DPP within rows, one cross-lane
+// exchange between rows r and r + 2).  Two words a lane: 8 lanes of a row belong to a tile, and each of the workgroup's 16 rows of lanes
+// leaves an entry per tile.  They meet in `lds`, and a second DPP reduction finishes.
 // The caller must put a barrier before it uses `lds` again.
-template <int NT>
-__device__ __forceinline__ void tile_max_both_u32(uint32_t m, uint32_t (*lds)[16], int t, uint32_t &own, uint32_t &other)
-{
-    m = row16_max_u32(m);
-    const uint32_t o = (uint32_t)__shfl_xor((int)m, 32);
-    m = o > m ? o : m;
-    const int half = (t >> 4) & 1;
-    if ((t & 47) == 0) lds[half][t >> 6] = m;          // lanes 0 and 16 of every wave
-    __syncthreads();
-    const int e = t & 15;
-    const uint32_t a = e < NT / 64 ? lds[half][e] : 0u, b = e < NT / 64 ? lds[half ^ 1][e] : 0u;
-    own = row16_max_u32(a);
-    other = row16_max_u32(b);
-}
-
-// The same where a lane owns two words of a row (fp4_amax with W = 2): 8 lanes of a DPP row belong to the left tile and 8 to the
-// right one, and each of the workgroup's 16 rows of lanes leaves an entry per tile.
-__device__ __forceinline__ void tile_max_both_half_rows_u32(uint32_t m, uint32_t (*lds)[16], int t, uint32_t &own, uint32_t &other)
-{
-    auto fold = [&](auto ctrl) {
-        const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, decltype(ctrl)::value, 0xF, 0xF, true);
-        m = o > m ? o : m;
-    };
-    fold(std::integral_constant<int, 0xB1>());          // quad_perm: lane ^ 1
-    fold(std::integral_constant<int, 0x4E>());          // quad_perm: lane ^ 2
-    fold(std::integral_constant<int, 0x141>());         // row_half_mirror: the other quad of the 8 lanes
-    const int half = (t >> 3) & 1;
-    if ((t & 7) == 0) lds[half][t >> 4] = m;
-    __syncthreads();
-    // a DPP row holds lanes of both tiles: each tile's entries are reduced by all of them
-    const uint32_t left = row16_max_u32(lds[0][t & 15]), right = row16_max_u32(lds[1][t & 15]);
-    own = half ? right : left;
-    other = half ? left : right;
-}
-
-// Max over the lane's own tile; leaves `lds` free for the next use.
-template <int NT, int W = 1>
+template <int NT, int W, int TILES>
 __device__ __forceinline__ uint32_t tile_max_u32(uint32_t m, uint32_t (*lds)[16], int t)
 {
-    uint32_t own, other;
-    if constexpr (W == 1) tile_max_both_u32<NT>(m, lds, t, own, other);
-    else tile_max_both_half_rows_u32(m, lds, t, own, other);
-    __syncthreads();
-    return own;
+    if constexpr (W == 1) {
+        static_assert(TILES == 2);
+        m = row16_max_u32(m);
+        const uint32_t o = (uint32_t)__shfl_xor((int)m, 32);
+        m = o > m ? o : m;
+        const int half = (t >> 4) & 1;
+        if ((t & 47) == 0) lds[half][t >> 6] = m;          // lanes 0 and 16 of every wave
+        __syncthreads();
+        const int e = t & 15;
+        return row16_max_u32(e < NT / 64 ? lds[half][e] : 0u);
+    } else {
+        static_assert(W == 2 && NT == 128 * TILES);
+        auto fold = [&](auto ctrl) {
+            const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, decltype(ctrl)::value, 0xF, 0xF, true);
+            m = o > m ? o : m;
+        };
+        auto eight = [&] {
+            fold(std::integral_constant<int, 0xB1>());      // quad_perm: lane ^ 1
+            fold(std::integral_constant<int, 0x4E>());      // quad_perm: lane ^ 2
+            fold(std::integral_constant<int, 0x141>());     // row_half_mirror: the other quad of the 8 lanes
+        };
+        eight();
+        const int tile = (t >> 3) & (TILES - 1);
+        if ((t & 7) == 0) lds[tile][t / (8 * TILES)] = m;
+        __syncthreads();
+        const u32x2 e = *(const u32x2 *)&lds[tile][(t & 7) * 2];
+        m = e.x > e.y ? e.x : e.y;
+        eight();
+        return m;
+    }
 }
 
 struct Geometry {
@@ -90,18 +84,18 @@ struct Geometry {
     int64_t colb;        // byte column of this lane's 4 W packed bytes
     int64_t scol;        // scale column of this lane
     int64_t tile;        // index of this lane's tile in the [rows/128, cols/128] grid
-    bool active;         // lane's tile exists (odd number of tiles per row)
+    bool active;         // lane's tile exists (the last super tile of a row may have fewer)
 };
 
-template <int W = 1>
+template <int W = 1, int TILES = 2>
 __device__ __forceinline__ Geometry geometry(int64_t super, int64_t supers_c, int64_t cols, int t)
 {
     Geometry g;
     // the launchers keep the number of super tiles below 2^31: a 32-bit division instead of the
     // ~150 scalar instructions of a 64-bit one
     const int64_t sr = (uint32_t)super / (uint32_t)supers_c, sc = super - sr * supers_c;
-    constexpr int LANES = 32 / W;                   // of a row
-    const int64_t col = sc * 256 + (t & (LANES - 1)) * (8 * W);      // logical column of the lane's first element
+    constexpr int LANES = 16 * TILES / W;           // of a row
+    const int64_t col = sc * (128 * TILES) + (t & (LANES - 1)) * (8 * W);      // logical column of the lane's first element
     g.row0 = sr * 128 + t / LANES;
     g.colb = col >> 1;
     g.scol = col >> 5;
@@ -165,7 +159,7 @@ __global__ __launch_bounds__(NT) void fp4_rebase(const uint8_t *__restrict__ pac
     const int64_t super = xcd_remap(blockIdx.x, per_xcd);
     if (super >= n_supers) return;
     const int t = threadIdx.x;
-    const Geometry g = geometry(super, supers_c, cols, t);
+    const Geometry g = geometry<>(super, supers_c, cols, t);
     const int64_t pcols = cols >> 1, scols = cols >> 5;
 
     uint32_t w[kPasses];
@@ -183,7 +177,7 @@ __global__ __launch_bounds__(NT) void fp4_rebase(const uint8_t *__restrict__ pac
     uint32_t S = 0;
 #pragma unroll
     for (int p = 0; p < kPasses; ++p) S = sb[p] > S ? sb[p] : S;
-    S = tile_max_u32<NT>(S, lds, t);
+    S = tile_max_u32<NT, 1, 2>(S, lds, t);
 
     const bool nan_tile = S == 0xFFu;
     if (g.active && (t & 15) == 0 && (t >> 5) == 0) {
@@ -223,6 +217,12 @@ __global__ __launch_bounds__(NT) void fp4_rebase(const uint8_t *__restrict__ pac
 // is 38 with one conversion for the maximum and the moved code table (W = 1).  us a launch, back to back: 2048 x 7168 6.96 -> 5.85, 512 x
 // 1024 4.3 -> 3.8, 65536 x 7168 137.6 -> 135.3 (256 threads; 512 level with it, 1024 behind: 6.6 and 149).
 
+template <class F, int... I>
+__device__ __forceinline__ void each(F &&f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>()), ...);
+}
+
 template <int W>
 __device__ __forceinline__ void store_codes(const u32x2 *out, uint8_t *dst)
 {
@@ -230,38 +230,55 @@ __device__ __forceinline__ void store_codes(const u32x2 *out, uint8_t *dst)
     else __builtin_nontemporal_store(out[0], (u32x2 *)dst);
 }
 
-template <int MODE, bool WRITE_BF16, int NT, int W>
+template <int MODE, bool WRITE_BF16, int NT, int W, int TILES = 2>
 __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packed, const uint8_t *__restrict__ scale,
                                                 int64_t cols, int64_t supers_c, int64_t n_supers, int64_t per_xcd,
                                                 float amax_floor, int zero_rule, uint8_t *__restrict__ q,
                                                 void *__restrict__ scale_out, int scale_dtype, uint16_t *__restrict__ bf16_out)
 {
-    constexpr int LANES = 32 / W, kRowsPerPass = NT / LANES, kPasses = 128 / kRowsPerPass;
-    static_assert(W == 1 || (W == 2 && NT == 256 && !WRITE_BF16));
-    __shared__ uint32_t lds[2][16];
+    constexpr int LANES = 16 * TILES / W, kRowsPerPass = NT / LANES, kPasses = 128 / kRowsPerPass;
+    static_assert(W == 1 || !WRITE_BF16);
+    __shared__ __attribute__((aligned(8))) uint32_t lds[TILES][16];
     asm volatile("" ::"s"(packed), "s"(scale));              // fetched with the other arguments, not behind the test below
     const int64_t super = xcd_remap(blockIdx.x, per_xcd);
     if (super >= n_supers) return;
     const int t = threadIdx.x;
-    const Geometry g = geometry<W>(super, supers_c, cols, t);
+    const Geometry g = geometry<W, TILES>(super, supers_c, cols, t);
     const int64_t pcols = cols >> 1, scols = cols >> 5;
 
-    // Lanes of a half that lies past the last tile (odd tile count per row) read the left half's
-    // columns instead, so the loads need no branches; their results are never stored.
-    const int64_t ld_colb = g.active ? g.colb : g.colb - 64, ld_scol = g.active ? g.scol : g.scol - 4;
+    // Lanes of a tile past the last one read the super tile's first tile instead, so the loads need no branches; their results
+    // are never stored.
+    const int place = g.active ? 0 : (t & (LANES - 1)) / (16 / W);
+    const int64_t ld_colb = g.colb - place * 64, ld_scol = g.scol - place * 4;
     uint32_t w[kPasses][W];
     uint32_t sb[kPasses];
+    uint32_t four = 0;
+    if constexpr (W == 2) four = *(const uint32_t *)(scale + (g.row0 + (t & 7) * kRowsPerPass) * scols + (ld_scol & ~3));
 #pragma unroll
     for (int p = 0; p < kPasses; ++p) {
         const int64_t r = g.row0 + p * kRowsPerPass;
         if constexpr (W == 2) {
             const u32x2 v = __builtin_nontemporal_load((const u32x2 *)(packed + r * pcols + ld_colb));
-            w[p][0] = fp4_pos_zero(v.x);
-            w[p][W - 1] = fp4_pos_zero(v.y);
+            w[p][0] = v.x;
+            w[p][W - 1] = v.y;
         } else {
             w[p][0] = fp4_pos_zero(__builtin_nontemporal_load((const uint32_t *)(packed + r * pcols + ld_colb)));
+            sb[p] = scale[r * scols + ld_scol];
         }
-        sb[p] = scale[r * scols + ld_scol];
+    }
+    if constexpr (W == 2) {
+        // Each of the 8 lanes that share a row of a tile has loaded the row's four scale bytes of one pass; they hand them round.
+        static_assert(kPasses == 8);
+        const uint32_t shift = (t & 6) * 4;
+        auto pass = [&](auto pc) {
+            constexpr int p = decltype(pc)::value;
+            w[p][0] = fp4_pos_zero(w[p][0]);
+            w[p][W - 1] = fp4_pos_zero(w[p][W - 1]);
+            int d = __builtin_amdgcn_update_dpp(0, (int)four, 0x150 + p, 0xF, 0x3, false);      // row_newbcast to lanes 0 .. 7 of the row
+            d = __builtin_amdgcn_update_dpp(d, (int)four, 0x158 + p, 0xF, 0xC, false);          // ... 8 .. 15
+            sb[p] = ((uint32_t)d >> shift) & 0xFFu;
+        };
+        each(pass, std::make_integer_sequence<int, kPasses>());
     }
 
     // amax of |table(code)| * 2^(sb-127).  The product is exact in fp32 (and
@@ -287,15 +304,11 @@ __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packe
     }
     const uint32_t mbits = f2u(amax_lane);
     const bool edge = sb_min < 2u || sb_max > 252u;
-    // Every thread of the workgroup must take the same number of barriers, so both slow decisions
-    // (edge scale bytes, tile scale outside the fast range) are made for the super tile as a whole -- by
-    // every lane for both tiles, from one reduction: an edge byte travels as the key 0xFFFFFFFF (products
-    // are finite positive floats, so that pattern is free), and the scale of the other tile is derived
-    // redundantly instead of being voted on.
-    uint32_t key, key_other;
-    if constexpr (W == 1) tile_max_both_u32<NT>(edge ? 0xFFFFFFFFu : mbits, lds, t, key, key_other);
-    else tile_max_both_half_rows_u32(edge ? 0xFFFFFFFFu : mbits, lds, t, key, key_other);
-    bool slow_tile = key == 0xFFFFFFFFu || key_other == 0xFFFFFFFFu;
+    // Every thread of the workgroup must take the same number of barriers, so both slow decisions (edge scale bytes, tile scale outside the
+    // fast range) are made for the super tile as a whole: an edge byte travels as the key 0xFFFFFFFF (products are finite
+    // positive floats, so that pattern is free), and a wave, which holds lanes of every tile, asks whether any of its lanes has a slow one.
+    const uint32_t key = tile_max_u32<NT, W, TILES>(edge ? 0xFFFFFFFFu : mbits, lds, t);
+    bool slow_tile = __any(key == 0xFFFFFFFFu);
     BlockScale bs;
     // Each element is +-{0, .5, 1, 2, 4} * 2^e (even codes and 0.5) or +-{1, 2, 4} * 1.5 * 2^e (codes
     // 1.5, 3, 6), so its quotient by the tile scale is a power-of-two multiple of one of two numbers,
@@ -310,7 +323,7 @@ __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packe
             return !(b.div >= 0x1p-100f && b.div <= 0x1p100f);
         };
         bs = derive_scale<MODE>(u2f(key), amax_floor, zero_rule);
-        slow_tile = out_of_range(bs) || out_of_range(derive_scale<MODE>(u2f(key_other), amax_floor, zero_rule));
+        slow_tile = __any(out_of_range(bs));
         if (MODE == LP_SCALE_POW2) {
             c1 = ldexpf(1.0f, -bs.exp2);
             c3 = ldexpf(1.5f, -bs.exp2);
@@ -406,7 +419,7 @@ __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packe
             }
         }
     }
-    m2 = tile_max_u32<NT, W>(m2, lds, t);
+    m2 = tile_max_u32<NT, W, TILES>(m2, lds, t);
     const bool has_nan = m2 > 0x7F800000u;
     const float amax = u2f(has_nan ? 0x7FC00000u : m2);
     bs = derive_scale<MODE>(amax, amax_floor, zero_rule);
@@ -473,30 +486,24 @@ extern "C" int lp_fp4_to_fp8_amax(const void *packed, const void *scale, int64_t
     int rc = check_fp4_args("lp_fp4_to_fp8_amax", packed, scale, rows, cols, q_out, scale_out);
     if (rc) return rc > 0 ? LP_OK : rc;
     LP_REQUIRE(!bf16_out || (uintptr_t)bf16_out % 16 == 0, "lp_fp4_to_fp8_amax: bf16_out must be 16-byte aligned");
-    const int64_t supers_c = (cols + 255) / 256, n_supers = (rows / 128) * supers_c;
-    const int64_t per_xcd = (n_supers + 7) / 8;
-    LP_REQUIRE(per_xcd * 8 <= 0x7FFFFFFF, "lp_fp4_to_fp8_amax: too many tiles");
-    dim3 grid((unsigned)(per_xcd * 8)), block(kAmaxThreads);
-    const bool two = n_supers <= kTwoWordSupers && (uintptr_t)packed % 8 == 0 && (uintptr_t)q_out % 16 == 0;
     hipStream_t st = (hipStream_t)stream;
+    auto go = [&](auto kernel, int threads, int tiles) -> int {
+        const int64_t supers_c = (cols / 128 + tiles - 1) / tiles, n_supers = (rows / 128) * supers_c, per_xcd = (n_supers + 7) / 8;
+        LP_REQUIRE(per_xcd * 8 <= 0x7FFFFFFF, "lp_fp4_to_fp8_amax: too many tiles");
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(per_xcd * 8)), dim3(threads), 0, st, (const uint8_t *)packed, (const uint8_t *)scale, cols, supers_c,
+                           n_supers, per_xcd, amax_floor, zero_rule, (uint8_t *)q_out, scale_out, scale_dtype, (uint16_t *)bf16_out);
+        return check_launch("lp_fp4_to_fp8_amax");
+    };
+    const bool aligned = (uintptr_t)packed % 8 == 0 && (uintptr_t)q_out % 16 == 0 && (uintptr_t)scale % 4 == 0;
+    const int64_t per_row = cols / 128, two = (per_row + 1) / 2 * 2, four = (per_row + 3) / 4 * 4;
+    const bool wide = rows / 128 * (two / 2) > kNarrowSupers && four * 16 <= two * 17;
 #define LAUNCH(MODE)                                                                                                   \
-    do {                                                                                                               \
-        if (bf16_out)                                                                                                  \
-            hipLaunchKernelGGL((fp4_amax<MODE, true, kAmaxThreads, 1>), grid, block, 0, st, (const uint8_t *)packed, (const uint8_t *)scale, \
-                               cols, supers_c, n_supers, per_xcd, amax_floor, zero_rule, (uint8_t *)q_out, scale_out,   \
-                               scale_dtype, (uint16_t *)bf16_out);                                                      \
-        else if (two)                                                                                                  \
-            hipLaunchKernelGGL((fp4_amax<MODE, false, kAmaxThreads, 2>), grid, block, 0, st, (const uint8_t *)packed, (const uint8_t *)scale, \
-                               cols, supers_c, n_supers, per_xcd, amax_floor, zero_rule, (uint8_t *)q_out, scale_out,   \
-                               scale_dtype, (uint16_t *)bf16_out);                                                      \
-        else                                                                                                           \
-            hipLaunchKernelGGL((fp4_amax<MODE, false, kAmaxThreads, 1>), grid, block, 0, st, (const uint8_t *)packed, (const uint8_t *)scale, \
-                               cols, supers_c, n_supers, per_xcd, amax_floor, zero_rule, (uint8_t *)q_out, scale_out,   \
-                               scale_dtype, (uint16_t *)bf16_out);                                                      \
-    } while (0)
+    return bf16_out ? go(fp4_amax<MODE, true, kAmaxThreads, 1>, kAmaxThreads, 2)                                        \
+         : !aligned ? go(fp4_amax<MODE, false, kAmaxThreads, 1>, kAmaxThreads, 2)                                       \
+         : wide ? go(fp4_amax<MODE, false, kWideThreads, 2, 4>, kWideThreads, 4)                                        \
+                : go(fp4_amax<MODE, false, kAmaxThreads, 2>, kAmaxThreads, 2)
     if (scale_mode == LP_SCALE_POW2) LAUNCH(LP_SCALE_POW2);
-    else if (scale_mode == LP_SCALE_DIV) LAUNCH(LP_SCALE_DIV);
-    else LAUNCH(LP_SCALE_MUL);
+    if (scale_mode == LP_SCALE_DIV) LAUNCH(LP_SCALE_DIV);
+    LAUNCH(LP_SCALE_MUL);
 #undef LAUNCH
-    return check_launch("lp_fp4_to_fp8_amax");
 }
