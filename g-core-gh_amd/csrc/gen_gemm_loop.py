@@ -42,7 +42,7 @@ def configure(tm, tn, waves_m, waves_n, ksub, hw=False, nstage=2, brow=False, ea
     for problems of about one tile per CU whose time is the chain of K steps)."""
     global A_BYTES, B_BYTES, SCL_LDS, SCL_HALF, NB, WAVES, KSUB, SPLIT, HW, NSTAGE, BROW, EARLY, WIDE, lines
     global ACC, P, AF, SC, SC2, SAN, WFB, RA0, RA1, RB0, RB1, SRD0, SRD, WS1, WS2, WSCUR, HALFSPLIT, ROT, WITH_IDLE, IDLE, PINGPONG, GRP, SPREAD, NN, BF, RBN
-    global WIDE_GROUP, WIDE_PART, BF16, RAG, WSC, FOLD
+    global WIDE_GROUP, WIDE_PART, WIDE_FIRST, BF16, RAG, WSC, FOLD
     # rag: any number of K blocks (the other loops need a multiple of four: their scale groups).  Three things differ.  The
     # operand bases stop at the last K block (s93 / s94 = their low halves there), so the requests of a last trip of fewer than
     # four blocks re-read that block instead of running past the matrices, and every counted wait stays as it is.  The last trip
@@ -53,7 +53,7 @@ def configure(tm, tn, waves_m, waves_n, ksub, hw=False, nstage=2, brow=False, ea
     # nn: the scale bytes of the stored weight lie a table row apart, four byte loads per group, whatever that row's length.
     RAG = rag
     # brow: the weight scales take the activation scales' way, loaded (rag) or copied by the other half of the waves.
-    assert not rag or (early and not wide and not bf16)
+    assert not rag or (early and not bf16 and (not wide or tm == 128))
     # fold: the hardware-scaled loop in which every matrix instruction starts from zero and its result (RES) goes to the accumulator by plain
     # fp32 additions, as in the fp32 loops: the instruction cuts the bits of a product that lie below its accumulator instead of
     # rounding them, which on operands of one sign costs 0.02 % of the error against float64 over four K blocks, 0.1 % over 23, 3 % over 143.
@@ -109,10 +109,21 @@ def configure(tm, tn, waves_m, waves_n, ksub, hw=False, nstage=2, brow=False, ea
     # addresses and the scale buffer base are used straight from the asm operands, and the weight copies share one
     # per-lane offset (the tile's weight rows are never clamped: N is a multiple of the tile width) with one scalar
     # base per copy.
-    WIDE = wide
+    # The 128 x 160 tile (rag only): four waves of 64 x 80 columns, five blocks each, two workgroups on a CU.  Its tiles need not
+    # divide N: a copy whose group of weight rows lies past the end moves the tile's first groups again (%[glim] = groups
+    # there are, less the wave's number).  80 accumulators leave room, so it keeps the register plan of the tiles below 288 and 224.
+    WIDE, WIDE_FIRST = wide, 4
     if wide:
-        assert tm == 256 and tn in WIDE_PLANS and waves_m == 4 and waves_n == 2 and ksub == 1 and nstage == 2 and not brow
         WIDE_GROUP, WIDE_PART = WIDE_PLANS[tn]
+    if wide and tm == 128:
+        assert tn == 160 and rag and waves_m == 2 and waves_n == 2 and ksub == 1 and nstage == 2 and not brow and not idle and not pingpong
+        WIDE_FIRST = 2
+        ACC, P, AF, WFB = 128, 96, 64, (48, 56)
+        SAN, SC, SC2, SRD = 40, 44, 208, "v35"
+        WS1, WS2, WSCUR = "v212", "v213", "v36"
+        RA0, RA1, RB0, RB1, SRD0 = "v30", "v31", "v32", "v33", "v34"
+    elif wide:
+        assert tm == 256 and tn in WIDE_PLANS and waves_m == 4 and waves_n == 2 and ksub == 1 and nstage == 2 and not brow
         ACC, P, AF, WFB = 112, 80, 48, (32, 40)
         SAN, SC, SC2, SRD = 24, 28, 20, "v19"
         WS1, WS2, WSCUR = "v20", "v21", "v22"            # hardware-scaled variant: weight-scale bytes of row 1, row 2, in use
@@ -182,9 +193,13 @@ WB_EXTRA = ("s[42:43]", "s[78:79]", "s[80:81]", "s[82:83]", "s[84:85]")     # wi
 # 224 columns: 28 groups, wave columns of 14.  Mid-step: groups 0..7 and 14..21 (blocks 0..3 of both wave columns); at
 # the end of the step the third copy moves groups 8..13 (waves 0..5) and 22, 23 (waves 6, 7) -- the set-up code's group --
 # and the fourth, of waves 0..3 only, groups 24..27.
-WIDE_PLANS = {288: ((0, 18, 8, 26, None), ("mid", "mid", "end", "end", "end")),
+# 160 columns on four waves: 20 groups, wave columns of ten, every wave five copies.  Mid-step: groups 0..3 and 10..13 (blocks 0, 1 of both
+# wave columns); at the end of the step groups 4..7, 14..17, and 8, 9 (waves 0, 1) and 18, 19 (waves 2, 3).
+WIDE_PLANS = {160: ((0, 10, 4, 14, None), ("mid", "mid", "end", "end", "end")),
+              288: ((0, 18, 8, 26, None), ("mid", "mid", "end", "end", "end")),
               224: ((0, 14, None, 24), ("mid", "mid", "end", "end"))}
 WIDE_GROUP, WIDE_PART = WIDE_PLANS[288]
+WIDE_FIRST = 4      # blocks of a wave column whose weight rows are handed back half way through a step
 
 _uid = 0
 
@@ -276,7 +291,7 @@ def dma(stage, part="all"):
         if part in ("all", "end"):
             for i in range(ncopies if WIDE else 1):
                 lo = int(WB_EXTRA[i][2:4])
-                if RAG:
+                if RAG and i == 0:                        # (the copies' bases move on together)
                     emit("s_cmp_eq_u32 s42, s94")
                     emit(f"s_cselect_b32 s96, 0, {'s66' if NN else 128}")
                 emit(f"s_add_u32 s{lo}, s{lo}, {'s96' if RAG else 's66' if NN else 128}")      # nn: 128 rows of the stored weight further on
@@ -379,6 +394,7 @@ def wait_copies(c, at_end, extra=""):
 
 
 RSA, RSB, RZERO = 112, 116, 120     # rag, e8m0: activation / weight scales of the next group on their way, a zero offset
+RSB2 = 214                          # ... of the second weight-scale row of a wave column that straddles two
 RSA_F32 = 36                        # rag, fp32: the lane's four activation scales of the next group
 
 
@@ -436,6 +452,8 @@ def rag_scale_load(tag):
     if HW:
         for i in range(1, 4):
             emit(f"v_mov_b32 v{RSB + i}, 0")
+            if WIDE:
+                emit(f"v_mov_b32 v{RSB2 + i}, 0")
     if NN:
         # four bytes a table row (s64 bytes) apart; a short last group has s95 of them
         for i in range(4):
@@ -450,28 +468,31 @@ def rag_scale_load(tag):
             emit("s_addc_u32 s47, s47, 0")
         emit(f"Lrb{tag}%=:")
         return
-    rag_short(f"Lrg{tag}%=")
-    if HW:
-        rag_elements(RSB, "global_load_ubyte", f"v{RZERO}", "s[46:47]", 1, f"Lrb{tag}%=")
-    else:
-        emit("s_cmp_eq_u32 s95, 1")
-        emit(f"s_cbranch_scc0 Lrh{tag}%=")
-        emit("s_load_dword s60, s[46:47], 0x0")
+    # (row, its place, base, tag): the second row for a wave column that straddles two scale blocks
+    rows = [(RSB, 60, 46, tag)] + ([(RSB2, 68, 72, "2" + tag)] if WIDE else [])
+    for reg, sreg, base, tag in rows:
+        rag_short(f"Lrg{tag}%=")
+        if HW:
+            rag_elements(reg, "global_load_ubyte", f"v{RZERO}", f"s[{base}:{base + 1}]", 1, f"Lrb{tag}%=")
+        else:
+            emit("s_cmp_eq_u32 s95, 1")
+            emit(f"s_cbranch_scc0 Lrh{tag}%=")
+            emit(f"s_load_dword s{sreg}, s[{base}:{base + 1}], 0x0")
+            emit(f"s_branch Lrb{tag}%=")
+            emit(f"Lrh{tag}%=:")
+            emit(f"s_load_dwordx2 s[{sreg}:{sreg + 1}], s[{base}:{base + 1}], 0x0")
+            emit("s_cmp_eq_u32 s95, 2")
+            emit(f"s_cbranch_scc1 Lrb{tag}%=")
+            emit(f"s_load_dword s{sreg + 2}, s[{base}:{base + 1}], 0x8")
         emit(f"s_branch Lrb{tag}%=")
-        emit(f"Lrh{tag}%=:")
-        emit("s_load_dwordx2 s[60:61], s[46:47], 0x0")
-        emit("s_cmp_eq_u32 s95, 2")
-        emit(f"s_cbranch_scc1 Lrb{tag}%=")
-        emit("s_load_dword s62, s[46:47], 0x8")
-    emit(f"s_branch Lrb{tag}%=")
-    emit(f"Lrg{tag}%=:")
-    if HW:
-        emit(f"global_load_dword v{RSB}, v{RZERO}, s[46:47]")
-    else:
-        emit("s_load_dwordx4 s[60:63], s[46:47], 0x0")
-    emit(f"Lrb{tag}%=:")
-    emit(f"s_add_u32 s46, s46, {4 if HW else 16}")
-    emit("s_addc_u32 s47, s47, 0")
+        emit(f"Lrg{tag}%=:")
+        if HW:
+            emit(f"global_load_dword v{reg}, v{RZERO}, s[{base}:{base + 1}]")
+        else:
+            emit(f"s_load_dwordx4 s[{sreg}:{sreg + 3}], s[{base}:{base + 1}], 0x0")
+        emit(f"Lrb{tag}%=:")
+        emit(f"s_add_u32 s{base}, s{base}, {4 if HW else 16}")
+        emit(f"s_addc_u32 s{base + 1}, s{base + 1}, 0")
 
 
 @staging
@@ -481,7 +502,7 @@ def rag_scale_write(tag):
     if HW:
         if not NN:
             rag_short(f"Lrc{tag}%=")
-        for base in (RSB,) if NN else (RSA,) if BROW else (RSA, RSB):
+        for base in (RSB,) if NN else (RSA,) if BROW else (RSA, RSB, RSB2) if WIDE else (RSA, RSB):
             for i in range(1, 4 if NN else 3):
                 emit(f"v_lshl_or_b32 v{base}, v{base + i}, {8 * i}, v{base}")
         if NN:
@@ -690,7 +711,7 @@ def step(c):
         # Early hand-back: the barrier sits in front of the first read of the second weight half (block NB / 2, read
         # one block ahead), so that half is known to have landed before anyone reads it, and behind every wave's
         # last read of the first half, so those rows and the activation rows can be requested again right after it.
-        handback = EARLY and nb == (3 if WIDE else NB // 2 - 1)      # wide: blocks 0..3 are the first part whatever NB
+        handback = EARLY and nb == (WIDE_FIRST if WIDE else NB // 2) - 1
         if handback:
             assert nb + 1 < NB and not pieces
             wait_copies(c, False, " lgkmcnt(0)")
@@ -808,6 +829,8 @@ def loop_body():
                 emit(f"v_mov_b32 v{WSN + nb}, v{WSC + nb}")
         elif RAG:
             emit(f"v_mov_b32 {WS1}, v{RSB}")
+            if WIDE:
+                emit(f"v_mov_b32 {WS2}, v{RSB2}")
         elif NN:
             # byte (address & 3) of each of the four dwords -> the four scale bytes of this group in one register
             for i in range(4):
@@ -861,16 +884,22 @@ def generate():
     if WIDE:
         emit("s_mov_b64 s[72:73], %[bsptr2]")
         emit("s_mov_b32 s74, %[splitnb]")
-        emit("s_mov_b32 s86, %[bextra]")
+        if not RAG:
+            emit("s_mov_b32 s86, %[bextra]")
         # weight base of copy i: WIDE_GROUP[i] groups of 8 rows further on (%[bstride] = bytes per group); the fifth
         # copy's group comes from the set-up code (%[g4])
         for i in range(1, len(WIDE_GROUP)):
             lo = int(WB_EXTRA[i][2:4])
-            if WIDE_GROUP[i] is None:
-                emit("s_mul_i32 s87, %[bstride], %[g4]")
-                emit("s_lshl_b32 s88, %[g4], 10")
+            group = "%[g4]" if WIDE_GROUP[i] is None else WIDE_GROUP[i]
+            if RAG:
+                # rows past the end of N: the tile's first groups again
+                emit(f"s_cmp_lt_i32 {group}, %[glim]" if WIDE_GROUP[i] is None else f"s_cmp_gt_i32 %[glim], {group}")
+                emit(f"s_cselect_b32 s87, {group}, 0")
+                emit("s_mul_i32 s87, %[bstride], s87")
             else:
-                emit(f"s_mul_i32 s87, %[bstride], {WIDE_GROUP[i]}")
+                emit(f"s_mul_i32 s87, %[bstride], {group}")
+            if WIDE_GROUP[i] is None:
+                emit("s_lshl_b32 s88, %[g4], 10")
             emit(f"s_add_u32 s{lo}, s42, s87")
             emit(f"s_addc_u32 s{lo + 1}, s43, 0")
     if RAG:
@@ -1016,6 +1045,8 @@ def main():
                       ("gemm_mid_hwrow_rag_loop.inc", (128, 128, 2, 2, 1, True, 2, True, True, False, False, False, False, False, True)),
                       ("gemm_big_hwrow_rag_loop.inc", (256, 256, 4, 2, 1, True, 2, True, True, False, True, PP, False, False, True)),
                       ("gemm_big_hw_nn_rag_loop.inc", (256, 256, 4, 2, 1, True, 2, False, True, False, True, PP, True, False, True)),
+                      ("gemm_mid160_rag_loop.inc", (128, 160, 2, 2, 1, False, 2, False, True, True, False, False, False, False, True)),
+                      ("gemm_mid160_hw_rag_loop.inc", (128, 160, 2, 2, 1, True, 2, False, True, True, False, False, False, False, True)),
                       ("gemm_flat_hw_nn_rag_loop.inc", (128, 256, 2, 4, 1, True, 3, False, True, False, True, False, True, False, True))):
         configure(*cfg)
         generate()
