@@ -388,17 +388,19 @@ PyObject *grouped_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
                                    nullptr, s_);
             };
             const auto result = [&] { return make({rows, N}, out_code == LP_BF16 ? at::kBFloat16 : at::kFloat, dev); };
+            // The row counts go with the GEMM's arguments, by which it also chooses its tiles, unless it refuses (more than 512 experts, 4 GiB)
+            const auto multiply = [&] {
+                out = result();
+                return p_grouped_rows(q.data_ptr(), s.data_ptr(), wq->const_data_ptr(), ws->const_data_ptr(), LP_E8M0, ex.offsets.data(), (int)E, rows, N, K,
+                                      out.data_ptr(), (int)out_code, s_);
+            };
             rc = LP_ERR_UNSUPPORTED;
             bool quantised = false;
             if (!train && !backward) {
-                // nobody else wants the offsets: they go with the GEMM's arguments, unless it refuses (more than 512 experts, 4 GiB)
+                // nobody else wants the offsets
                 rc = quantise();
                 quantised = !rc;
-                if (!rc) {
-                    out = result();
-                    rc = p_grouped_rows(q.data_ptr(), s.data_ptr(), wq->const_data_ptr(), ws->const_data_ptr(), LP_E8M0, ex.offsets.data(), (int)E, rows, N,
-                                        K, out.data_ptr(), (int)out_code, s_);
-                }
+                if (!rc) rc = multiply();
             }
             if (rc == LP_ERR_UNSUPPORTED) {
                 std::vector<int32_t> words = ex.offsets;
@@ -420,9 +422,10 @@ PyObject *grouped_forward(PyObject *, PyObject *const *args, Py_ssize_t n)
                     rc = quantise();
                 }
                 if (!rc) {
-                    if (!out.defined()) out = result();
-                    rc = p_grouped(q.data_ptr(), s.data_ptr(), wq->const_data_ptr(), ws->const_data_ptr(), LP_E8M0, offs.data_ptr<int32_t>(), (int)E, rows,
-                                   N, K, out.data_ptr(), (int)out_code, s_);
+                    rc = out.defined() ? LP_ERR_UNSUPPORTED : multiply();          // defined: refused above
+                    if (rc == LP_ERR_UNSUPPORTED)
+                        rc = p_grouped(q.data_ptr(), s.data_ptr(), wq->const_data_ptr(), ws->const_data_ptr(), LP_E8M0, offs.data_ptr<int32_t>(), (int)E, rows,
+                                       N, K, out.data_ptr(), (int)out_code, s_);
                 }
             }
         }
