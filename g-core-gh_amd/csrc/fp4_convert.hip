@@ -253,7 +253,8 @@ __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packe
     uint32_t w[kPasses][W];
     uint32_t sb[kPasses];
     uint32_t four = 0;
-    if constexpr (W == 2) four = *(const uint32_t *)(scale + (g.row0 + (t & 7) * kRowsPerPass) * scols + (ld_scol & ~3));
+    // (a load at any address: the scales need not start on a word)
+    if constexpr (W == 2) __builtin_memcpy(&four, scale + (g.row0 + (t & 7) * kRowsPerPass) * scols + (ld_scol & ~3), 4);
 #pragma unroll
     for (int p = 0; p < kPasses; ++p) {
         const int64_t r = g.row0 + p * kRowsPerPass;
@@ -494,7 +495,7 @@ extern "C" int lp_fp4_to_fp8_amax(const void *packed, const void *scale, int64_t
                            n_supers, per_xcd, amax_floor, zero_rule, (uint8_t *)q_out, scale_out, scale_dtype, (uint16_t *)bf16_out);
         return check_launch("lp_fp4_to_fp8_amax");
     };
-    const bool aligned = (uintptr_t)packed % 8 == 0 && (uintptr_t)q_out % 16 == 0 && (uintptr_t)scale % 4 == 0;
+    const bool aligned = (uintptr_t)packed % 8 == 0 && (uintptr_t)q_out % 16 == 0;
     const int64_t per_row = cols / 128, two = (per_row + 1) / 2 * 2, four = (per_row + 3) / 4 * 4;
     const bool wide = rows / 128 * (two / 2) > kNarrowSupers && four * 16 <= two * 17;
 #define LAUNCH(MODE)                                                                                                   \

@@ -4,6 +4,7 @@ form changes, and with edge scale bytes in any of the four tiles."""
 import pytest
 import torch
 
+from tests._routes import kernels
 from tests.test_gpu_fp4_words import convert
 
 pytestmark = pytest.mark.gpu
@@ -29,13 +30,21 @@ def test_four_tiles_a_workgroup(rows, tiles, edge):
         assert torch.equal(a, b) and torch.equal(sa.view(torch.uint8), sb.view(torch.uint8))
 
 
-def test_scales_off_their_alignment():
-    """Scale bytes that start anywhere: one byte load per row, the same result."""
+@pytest.mark.parametrize("offset", [1, 2, 3])
+@pytest.mark.parametrize("rows,tiles,kernel", [(384, 5, "ELb0ELi256ELi2ELi2E"), (128 * 31, 34, "ELb0ELi512ELi2ELi4E")], ids=["two tiles", "four tiles"])
+def test_scales_off_their_alignment(rows, tiles, kernel, offset):
+    """Scale bytes that start anywhere: the same kernel, the same result."""
     from gcore_lowp import _abi as A
     g = torch.Generator(device="cuda").manual_seed(3)
-    packed = torch.randint(0, 256, (384, 320), generator=g, device="cuda", dtype=torch.uint8)
-    flat = torch.randint(117, 128, (384 * 20 + 4,), generator=g, device="cuda", dtype=torch.uint8)
-    print("[case] scale offset", flush=True)
-    a, sa = convert(packed, flat[1:384 * 20 + 1].view(384, 20), A.SCALE_DIV, A.F32, 0)
-    b, sb = convert(packed, flat[1:384 * 20 + 1].clone().view(384, 20), A.SCALE_DIV, A.F32, 0)
-    assert torch.equal(a, b) and torch.equal(sa, sb)
+    cols = 128 * tiles
+    packed = torch.randint(0, 256, (rows, cols // 2), generator=g, device="cuda", dtype=torch.uint8)
+    flat = torch.randint(117, 128, (rows * cols // 32 + 4,), generator=g, device="cuda", dtype=torch.uint8)
+    scale = flat[offset:offset + rows * cols // 32].view(rows, cols // 32)
+    assert scale.data_ptr() % 4 == offset
+    print("[case] scale offset", offset, rows, cols, flush=True)
+    a, sa = convert(packed, scale, A.SCALE_DIV, A.F32, 0)
+    b, sb = convert(packed, scale.clone(), A.SCALE_DIV, A.F32, 0)
+    c, sc = convert(packed, scale, A.SCALE_DIV, A.F32, 1)
+    assert torch.equal(a, b) and torch.equal(sa, sb) and torch.equal(a, c) and torch.equal(sa, sc)
+    ran = kernels(lambda: convert(packed, scale, A.SCALE_DIV, A.F32, 0, guarded=False))
+    assert [kernel in n for n in ran if "fp4_amax" in n] == [True], ran

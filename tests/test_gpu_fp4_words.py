@@ -6,7 +6,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def convert(packed, scale, mode, dtype, shift):
+def convert(packed, scale, mode, dtype, shift, guarded=True):
     """lp_fp4_to_fp8_amax with the codes and the packed input `shift` times 4 / 8 bytes off their alignment"""
     from gcore_lowp import _abi as A
     rows, cols = packed.shape[0], packed.shape[1] * 2
@@ -18,7 +18,7 @@ def convert(packed, scale, mode, dtype, shift):
     s = torch.empty(rows // 128, cols // 128, dtype=torch.float32 if dtype == A.F32 else torch.uint8, device="cuda")
     A.check(A.lib().lp_fp4_to_fp8_amax(src.data_ptr(), scale.data_ptr(), rows, cols, mode, 1e-12 if mode == A.SCALE_DIV else 0.0, 0, out.data_ptr(),
                                        s.data_ptr(), dtype, None, A.stream_ptr()))
-    assert bool((q[:16 + 8 * shift] == 77).all()) and bool((q[16 + 8 * shift + rows * cols:] == 77).all())
+    assert not guarded or bool((q[:16 + 8 * shift] == 77).all()) and bool((q[16 + 8 * shift + rows * cols:] == 77).all())
     return out, s
 
 
