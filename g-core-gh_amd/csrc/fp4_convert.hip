@@ -32,12 +32,18 @@ constexpr int kAmaxThreads = 256;
 // The fused kernel where the buffers' alignment lets a lane own two packed words of a row (one scale byte still covers both), which halves its memory
 // instructions and the table work per element (us a launch, back to back, one word -> two: 2048 x 7168 6.13 -> 5.41, 7168 x 2048 5.98 -> 5.25, 512 x
 // 1024 level, 32768 x 1152 15.4 -> 13.8, 65536 x 7168 132.7 -> 131.9).  One word a lane is left to other alignments and to the form that writes bf16 too.
-// From more than kNarrowSupers super tiles (two on every CU) on, four tiles side by side on 512 threads: rows of 256 packed bytes and 512 of output
-// (two -> four tiles: 2560 x 7168 7.81 -> 7.10, 4096 x 7168 11.5 -> 8.3, 16384 x 7168 37.6 -> 34.8, 65536 x 7168 131.9 -> 124.4 = 5.8 TB/s), if
-// that adds no more than a sixteenth of empty tiles at the rows' ends (five tiles a row, 65536 x 640, 15.7 <- 17.3; nine, 32768 x 1152, 13.8 <- 14.5).
-// Below, it leaves CUs without a workgroup: 2048 x 7168 5.41 <- 5.64, 7168 x 2304 5.48 <- 6.84.
+// Three forms of it, by the super tiles of 128 x 256 there are for the 256 CUs and by the tiles in a row (lp_fp4_to_fp8_amax).  In brackets super tiles; us,
+// two tiles a workgroup with the scale bytes handed round / two with a byte load for each / four with the bytes handed round:
+// - up to three on every CU the first is ahead for short rows: 33024 x 512 [516] 6.16 / 6.32 / 6.65, 24576 x 1024 [768] 6.92 / 7.63 / 7.45.  From 16 tiles a row on only
+//   up to two: 8960 x 2048 [560] 6.76 / 6.52 / 6.81, 5888 x 3584 [644] 7.40 / 6.73 / 7.02; and from 32 on, four tiles have what they need from there:
+//   4480 x 4096 [560] 7.83 / 7.12 / 7.05, 2944 x 7168 [644] 8.25 / 7.05 / 7.22, 4224 x 7168 [924] 11.63 / 10.84 / 8.41.
+// - beyond, four tiles: 57600 x 512 [900] 9.27 / 8.44 / 7.93, 14464 x 2048 [904] 10.64 / 10.37 / 8.11, 12288 x 2048 [768] 7.65 / 7.53 / 7.24, 65536 x 7168 131.1 / 136.2 / 123.4 =
+//   5.8 TB/s; with rows of 1024 columns, whose pieces of a workgroup lie a power of two apart, only past nine halves: 32768 x 1024 [1024] 10.72 / 9.48 / 11.68, 35200 x 1024
+//   [1100] 12.48 / 11.93 / 13.05, 41600 x 1024 [1300] 14.85 / 14.40 / 14.38 (28800 x 896 [900] 9.10 with byte loads, 7.41 in fours).
+// - where four tiles would leave more than a sixteenth empty at the rows' ends, byte loads up to five on every CU: 38400 x 768 [900] 9.70 / 8.52, 23040 x 1280 [900]
+//   10.36 / 8.68, 55552 x 768 [1302] 14.49 / 14.20; and handed round again beyond, 174848 x 768 [4098] 39.3 / 40.6.
 constexpr int kWideThreads = 512;
-constexpr int64_t kNarrowSupers = 512;
+constexpr int64_t kCUs = 256;
 
 // Maximum over the lane's own 128 x 128 tile, from one barrier.  One word a lane (W = 1, two tiles side by side): the 16 lanes of a DPP row belong to
 // one tile and the rows of a wave alternate between the tiles, so a wave reduces to one value per tile (DPP within rows, one cross-lane
@@ -230,7 +236,7 @@ __device__ __forceinline__ void store_codes(const u32x2 *out, uint8_t *dst)
     else __builtin_nontemporal_store(out[0], (u32x2 *)dst);
 }
 
-template <int MODE, bool WRITE_BF16, int NT, int W, int TILES = 2>
+template <int MODE, bool WRITE_BF16, int NT, int W, int TILES = 2, bool BYTES = W == 1>
 __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packed, const uint8_t *__restrict__ scale,
                                                 int64_t cols, int64_t supers_c, int64_t n_supers, int64_t per_xcd,
                                                 float amax_floor, int zero_rule, uint8_t *__restrict__ q,
@@ -254,7 +260,7 @@ __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packe
     uint32_t sb[kPasses];
     uint32_t four = 0;
     // (a load at any address: the scales need not start on a word)
-    if constexpr (W == 2) __builtin_memcpy(&four, scale + (g.row0 + (t & 7) * kRowsPerPass) * scols + (ld_scol & ~3), 4);
+    if constexpr (!BYTES) __builtin_memcpy(&four, scale + (g.row0 + (t & 7) * kRowsPerPass) * scols + (ld_scol & ~3), 4);
 #pragma unroll
     for (int p = 0; p < kPasses; ++p) {
         const int64_t r = g.row0 + p * kRowsPerPass;
@@ -264,10 +270,14 @@ __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packe
             w[p][W - 1] = v.y;
         } else {
             w[p][0] = fp4_pos_zero(__builtin_nontemporal_load((const uint32_t *)(packed + r * pcols + ld_colb)));
-            sb[p] = scale[r * scols + ld_scol];
+        }
+        if constexpr (BYTES) sb[p] = scale[r * scols + ld_scol];
+        if constexpr (BYTES && W == 2) {
+            w[p][0] = fp4_pos_zero(w[p][0]);
+            w[p][W - 1] = fp4_pos_zero(w[p][W - 1]);
         }
     }
-    if constexpr (W == 2) {
+    if constexpr (!BYTES) {
         // Each of the 8 lanes that share a row of a tile has loaded the row's four scale bytes of one pass; they hand them round.
         static_assert(kPasses == 8);
         const uint32_t shift = (t & 6) * 4;
@@ -337,7 +347,11 @@ __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packe
         }
     }
 
-    if (!slow_tile) {
+    // Behind a branch that it knows to be uniform the compiler keeps 30 registers more, which takes two to three of eight waves of a SIMD.  Two words
+    // with a byte load each, which are for launches of few rounds, are better off with the waves; large launches are not (65536 x 4096 in fours 74.9 <- 80.3).
+    uint32_t slow = slow_tile;
+    if constexpr (BYTES && W == 2) asm volatile("" : "+v"(slow));
+    if (!slow) {
         if (g.active && (t & (16 / W - 1)) == 0 && t < LANES) store_scale(scale_out, scale_dtype, g.tile, bs.stored);
         if (!g.active) return;
         // All 8 elements of a pass share one scale byte sb, so their codes are eight numbers per pass:
@@ -495,14 +509,17 @@ extern "C" int lp_fp4_to_fp8_amax(const void *packed, const void *scale, int64_t
                            n_supers, per_xcd, amax_floor, zero_rule, (uint8_t *)q_out, scale_out, scale_dtype, (uint16_t *)bf16_out);
         return check_launch("lp_fp4_to_fp8_amax");
     };
-    const bool aligned = (uintptr_t)packed % 8 == 0 && (uintptr_t)q_out % 16 == 0;
-    const int64_t per_row = cols / 128, two = (per_row + 1) / 2 * 2, four = (per_row + 3) / 4 * 4;
-    const bool wide = rows / 128 * (two / 2) > kNarrowSupers && four * 16 <= two * 17;
+    const bool two_words = (uintptr_t)packed % 8 == 0 && (uintptr_t)q_out % 16 == 0;
+    // see kCUs
+    const int64_t per_row = cols / 128, two = (per_row + 1) / 2 * 2, four = (per_row + 3) / 4 * 4, supers = rows / 128 * (two / 2);
+    const bool wide = four * 16 <= two * 17 && supers * 4 > kCUs * (per_row >= 32 ? 8 : per_row >= 16 ? 11 : per_row == 8 ? 18 : 12);
+    const bool handed = supers <= kCUs * (per_row < 16 ? 3 : 2) || supers > kCUs * 5;
 #define LAUNCH(MODE)                                                                                                   \
     return bf16_out ? go(fp4_amax<MODE, true, kAmaxThreads, 1>, kAmaxThreads, 2)                                        \
-         : !aligned ? go(fp4_amax<MODE, false, kAmaxThreads, 1>, kAmaxThreads, 2)                                       \
+         : !two_words ? go(fp4_amax<MODE, false, kAmaxThreads, 1>, kAmaxThreads, 2)                                     \
          : wide ? go(fp4_amax<MODE, false, kWideThreads, 2, 4>, kWideThreads, 4)                                        \
-                : go(fp4_amax<MODE, false, kAmaxThreads, 2>, kAmaxThreads, 2)
+         : handed ? go(fp4_amax<MODE, false, kAmaxThreads, 2>, kAmaxThreads, 2)                                         \
+                  : go(fp4_amax<MODE, false, kAmaxThreads, 2, 2, true>, kAmaxThreads, 2)
     if (scale_mode == LP_SCALE_POW2) LAUNCH(LP_SCALE_POW2);
     if (scale_mode == LP_SCALE_DIV) LAUNCH(LP_SCALE_DIV);
     LAUNCH(LP_SCALE_MUL);

@@ -1,5 +1,5 @@
-"""The fused FP4 -> FP8 conversion with two packed words per lane (aligned buffers, up to 4096 super tiles of 128 x 256) against the form with one
-(buffers off 8 and 16 bytes): the same bytes, for odd numbers of tiles per row, edge scale bytes and the first size beyond."""
+"""The fused FP4 -> FP8 conversion with two packed words per lane (aligned buffers) against the form with one (buffers off 8 and 16 bytes): the same
+bytes, for odd numbers of tiles per row and edge scale bytes, from one tile to 4160 workgroups of two."""
 import pytest
 import torch
 
