@@ -1,22 +1,33 @@
 """Short-K products just past a round of 256 x 256 tiles, which run on 128 x 128 ones where those fill whole rounds: against float64, with cases on
-both sides of every line of the rule."""
+both sides of every line of the rule.  Each case names the tiles it is for, and the kernels that ran are checked."""
 import pytest
 import torch
 
+from tests._routes import kernels
+
 pytestmark = pytest.mark.gpu
 
+TILES = {"128": "gemm_asmILi128ELi128E", "256": "gemm_asmILi256ELi256E", "wide": "gemm_asm_wide"}
 CASES = [
-    (2409, 6528, 1152), (1665, 9216, 2688), (2305, 6912, 128), (2817, 5888, 2688), (4097, 7936, 2048),      # 128 x 128: 969, 1008, 1026 > 1024, 1058, 2046 tiles
-    (1665, 9216, 2816), (4097, 7936, 2176),                                                              # K one block longer: 256-row tiles
+    # (M, N, K), tiles of 128 x 128, of 256 x 256, the ones that run
+    ((2409, 6528, 1152), 969, 260, "128"),
+    ((2665, 6144, 2688), 1008, 264, "128"), ((2665, 6144, 2816), 1008, 264, "256"),        # 21 K blocks, 22
+    ((3963, 4224, 1920), 1023, 272, "128"), ((2305, 6912, 128), 1026, 270, "256"), ((2817, 5888, 2688), 1058, 276, "256"),
+    ((1665, 9216, 2688), 1008, 252, "256"),                                                # one round
+    ((4097, 7936, 2048), 2046, 527, "128"), ((4097, 7936, 2176), 2046, 527, "256"), ((4097, 8064, 1152), 2079, 544, "256"),
+    ((896, 18432, 1024), 1008, 288, "128"), ((896, 18432, 1536), 1008, 288, "wide"), ((1408, 11520, 1536), 990, 270, "128"), ((1408, 11520, 2048), 990, 270, "wide"),      # 256 x 288 tiles in one round
+    ((2176, 14976, 1536), 1989, 531, "128"),                                               # ... in two
 ]
 
 
 @pytest.mark.parametrize("pow2", [False, True], ids=["f32scale", "e8m0scale"])
-@pytest.mark.parametrize("M,N,K", CASES, ids=str)
-def test_products_past_a_round(M, N, K, pow2):
+@pytest.mark.parametrize("shape,small,big,tiles", CASES, ids=str)
+def test_products_past_a_round(shape, small, big, tiles, pow2):
     from gcore_lowp import _abi as A
     L = A.lib()
     A.require_gpu()
+    M, N, K = shape
+    assert -(-M // 128) * (N // 128) == small and -(-M // 256) * -(-N // 256) == big
     print("[case]", (M, N, K), pow2, flush=True)
     g = torch.Generator(device="cuda").manual_seed(M + K)
     xq, wq = (torch.randn(r, K, generator=g, device="cuda").to(torch.float8_e4m3fn) for r in (M, N))
@@ -25,8 +36,15 @@ def test_products_past_a_round(M, N, K, pow2):
         xs, ws = (torch.pow(2.0, t.float() - 127) * 1.25 for t in (xs, ws))
     guard = 4096
     room = torch.full((M * N + guard,), float("nan"), device="cuda")
-    A.check(L.lp_gemm_fp8_block(xq.data_ptr(), xs.data_ptr(), wq.data_ptr(), ws.data_ptr(), A.E8M0 if pow2 else A.F32, M, N, K, room.data_ptr(), A.F32,
-                                None, 0, A.stream_ptr()))
+
+    def product():
+        A.check(L.lp_gemm_fp8_block(xq.data_ptr(), xs.data_ptr(), wq.data_ptr(), ws.data_ptr(), A.E8M0 if pow2 else A.F32, M, N, K, room.data_ptr(), A.F32,
+                                    None, 0, A.stream_ptr()))
+
+    product()
+    ran = kernels(product)
+    # (the columns past the last whole round of 256-row tiles may be a second launch, of 128 x 128 tiles)
+    assert TILES[tiles] in ran[0] and (len(ran) == 1 or tiles == "256" and len(ran) == 2 and TILES["128"] in ran[1]), ran
     out = room[:-guard].view(M, N)
     assert bool(room[-guard:].isnan().all()) and not bool(out.isnan().any())
     sx, sw = (torch.pow(2.0, t.double() - 127) if pow2 else t.double() for t in (xs, ws))
