@@ -7,7 +7,7 @@ from tests._routes import kernels
 
 pytestmark = pytest.mark.gpu
 
-TILES = {"128": "gemm_asmILi128ELi128E", "256": "gemm_asmILi256ELi256E", "wide": "gemm_asm_wide"}
+TILES = {"128": "gemm_asmILi128ELi128E", "256": "gemm_asmILi256ELi256E", "wide": "gemm_asm_wide", "both in one": "gemm_asm_mixed"}
 CASES = [
     # (M, N, K), tiles of 128 x 128, of 256 x 256, the ones that run
     ((2409, 6528, 1152), 969, 260, "128"),
@@ -17,6 +17,9 @@ CASES = [
     ((4097, 7936, 2048), 2046, 527, "128"), ((4097, 7936, 2176), 2046, 527, "256"), ((4097, 8064, 1152), 2079, 544, "256"),
     ((896, 18432, 1024), 1008, 288, "128"), ((896, 18432, 1536), 1008, 288, "wide"), ((1408, 11520, 1536), 990, 270, "128"), ((1408, 11520, 2048), 990, 270, "wide"),      # 256 x 288 tiles in one round
     ((2176, 14976, 1536), 1989, 531, "128"),                                               # ... in two
+    # few row tiles: tiles with fp32 scales, with e8m0 scales
+    ((1152, 13952, 1792), 981, 275, "128"), ((1152, 13952, 1920), 981, 275, ("128", "256")), ((1153, 12928, 1920), 1010, 255, "256"), ((1281, 11904, 1920), 1023, 282, "128"),
+    ((1664, 9984, 2048), 1014, 273, ("128", "both in one")), ((1664, 9984, 2560), 1014, 273, ("128", "256")), ((1664, 9984, 2176), 1014, 273, "128"), ((1665, 9344, 2048), 1022, 259, "128"),
 ]
 
 
@@ -43,6 +46,7 @@ def test_products_past_a_round(shape, small, big, tiles, pow2):
 
     product()
     ran = kernels(product)
+    tiles = tiles if isinstance(tiles, str) else tiles[pow2]
     # (the columns past the last whole round of 256-row tiles may be a second launch, of 128 x 128 tiles)
     assert TILES[tiles] in ran[0] and (len(ran) == 1 or tiles == "256" and len(ran) == 2 and TILES["128"] in ran[1]), ran
     out = room[:-guard].view(M, N)
