@@ -98,3 +98,25 @@ def test_lines_of_the_rule(shape, narrow, wide, with_f32, with_e8m0, pow2):
     if not pow2:
         xs, ws = (torch.pow(2.0, t.float() - 127) * 1.25 for t in (xs, ws))
     same_as_columns_apart(M, N, K, (xq, xs, wq, ws), pow2, torch.float32, with_e8m0 if pow2 else with_f32)
+
+
+@pytest.mark.parametrize("knob", ["LP_GEMM_MID_DUAL=0", "LP_GEMM_MID_STAGES=4", "LP_GEMM_MID_KSUB=1"])
+def test_knobs_of_the_128_wide_loops_hold(knob):
+    """The knobs force a loop of 128 x 128 tiles (they are read once per process, hence the child); a shape that takes 128 x 160 tiles without them."""
+    import os
+    import subprocess
+    import sys
+    code = (
+        "import torch\n"
+        "from gcore_lowp import _abi as A\n"
+        "from tests._routes import kernels\n"
+        "M, N, K = 1000, 5120, 2560\n"
+        "t = [torch.zeros(n, dtype=torch.uint8, device='cuda') for n in (M * K, M * K // 32, N * K, N * K // 4096, 2 * M * N)]\n"
+        "print('kernels', *kernels(lambda: A.check(A.lib().lp_gemm_fp8_block(*[x.data_ptr() for x in t[:4]], A.F32, M, N, K, t[4].data_ptr(), A.BF16, None, 0, A.stream_ptr()))))\n")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    print("[case]", knob, flush=True)
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([root] + [p for p in sys.path if p]), **dict([knob.split("=")]))
+    r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=110)
+    assert r.returncode == 0, (r.stdout[-1500:], r.stderr[-1500:])
+    ran = [line.split()[1:] for line in r.stdout.splitlines() if line.startswith("kernels")]
+    assert len(ran) == 1 and len(ran[0]) == 1 and "gemm_asmILi128ELi128E" in ran[0][0], ran
