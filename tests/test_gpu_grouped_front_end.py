@@ -46,11 +46,11 @@ def step(G, splits, form, dtype, want_x, want_w, k=256, n=384):
     return [out.detach(), *grads]
 
 
-CASES = [(s, "plain", torch.bfloat16, True, True) for s in SPLITS if s != "513 experts"] + [
+CASES = [(s, "plain", torch.bfloat16, True, True) for s in SPLITS] + [
     ("ragged", f, torch.bfloat16, True, True) for f in ("three dims", "strided", "off 16 bytes")] + [
     ("ragged", "plain", torch.float32, True, True), ("ragged", "plain", torch.bfloat16, False, True), ("ragged", "plain", torch.bfloat16, True, False),
     ("ragged", "plain", torch.bfloat16, False, False), ("ragged", "strided", torch.bfloat16, False, False), ("many", "plain", torch.bfloat16, False, False),
-    ("513 experts", "plain", torch.bfloat16, False, False), ("long", "plain", torch.bfloat16, False, False), ("long", "off 16 bytes", torch.bfloat16, True, False)]
+    ("513 experts", "plain", torch.bfloat16, False, False), ("513 experts", "plain", torch.bfloat16, True, False), ("long", "plain", torch.bfloat16, False, False), ("long", "off 16 bytes", torch.bfloat16, True, False)]
 
 
 @pytest.mark.parametrize("splits,form,dtype,want_x,want_w", CASES, ids=str)
@@ -64,7 +64,9 @@ def test_front_end_and_wrappers_give_the_same_bits(G, monkeypatch, splits, form,
         monkeypatch.setattr(_native.fast, name, lambda *a, real=real, name=name: [r for r in [real(*a)] if taken.append((name, r is not None)) is None][0])
     got = step(G, *args)
     if form == "plain" and dtype == torch.bfloat16:
-        assert ("grouped_forward", True) in taken and (not want_x or ("grouped_backward", True) in taken), taken
+        # (the backward leaves more than 512 experts to the wrappers)
+        backward = ("grouped_backward", splits != "513 experts")
+        assert ("grouped_forward", True) in taken and (not want_x or backward in taken), taken
     for name in ("grouped_forward", "grouped_backward"):
         monkeypatch.setattr(_native.fast, name, lambda *a: None)
     want = step(G, *args)
@@ -73,16 +75,34 @@ def test_front_end_and_wrappers_give_the_same_bits(G, monkeypatch, splits, form,
         assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
 
 
-@pytest.mark.parametrize("splits,k,n", [([3] * 40, 2560, 1024), ([3] * 40, 2432, 1024), ([0, 64, 1] * 30, 1280, 1152), ([64] * 11 + [65], 1280, 1152),
-                                           ([1] * 440, 256, 256), ([1] * 439 + [129] + [0] * 5, 256, 256), ([0] * 9 + [257, 0, 128], 1152, 640)],
-                         ids=["weights streamed", "K of 19 blocks", "short K", "short K, more rows", "440 row tiles", "441 row tiles", "row tiles of an expert"])
-def test_kernel_chosen_by_the_row_counts(G, monkeypatch, splits, k, n):
+@pytest.mark.parametrize("train", [False, True], ids=["inference", "training"])
+@pytest.mark.parametrize("splits,k,n,host,device", [
+    ([3] * 40, 3328, 1024, "two", "128"), ([3] * 40, 2432, 1024, "128", "128"), ([0, 64, 1] * 30, 1280, 1152, "128", "two"), ([64] * 11 + [65], 1280, 1152, "128", "128"),
+    ([1] * 440, 256, 256, "128", "128"), ([1] * 439 + [129] + [0] * 5, 256, 256, "128", "128"), ([0] * 9 + [257, 0, 128], 1152, 640, "128", "128"),
+    ([3, 0, 0] * 46, 3456, 1408, "128", "two"), ([200] * 3 + [56] * 9, 2816, 4608, "two", "128")],
+    ids=["weights streamed", "K of 19 blocks", "short K", "short K, more rows", "440 row tiles", "441 row tiles", "row tiles of an expert", "a few in a second round", "one round"])
+def test_kernel_chosen_by_the_row_counts(G, monkeypatch, splits, k, n, host, device, train):
     """The launch that knows the counts may take tiles of another size than the one that does not: the same sums."""
     from gcore_lowp import _native
-    args = (splits, "plain", torch.bfloat16, False, False, k, n)
-    got = step(G, *args)[0]
+    from tests._routes import kernels
+    args = (splits, "plain", torch.bfloat16, train, False, k, n)
+    names = {"128": "gemm_asm_groupedILi128ELi128E", "two": "gemm_asm_grouped_mixedILb1ELb0E"}      # (the backward's product is grouped_mixed<true, true, ..>)
+    print("[case]", len(splits), sum(splits), k, n, train, flush=True)
+
+    def run(wanted):
+        layer, x, weight = G.MyTeGroupedLinearFp8(len(splits)), *operands
+        forward = [m for m in kernels(lambda: layer(x, weight, splits)) if "gemm_asm_grouped" in m]
+        assert len(forward) == 1 and names[wanted] in forward[0], (wanted, forward)
+        return step(G, *args)
+
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q, s = G.quant_fp8_e4m3_scale_e8m0(torch.randn(len(splits) * n, k, generator=g, device="cuda", dtype=torch.bfloat16))
+    operands = (torch.randn(sum(splits), k, generator=g, device="cuda", dtype=torch.bfloat16).requires_grad_(train),
+                (q.view(len(splits), n, k), s.view(len(splits), n // 128, k // 128)))
+    got = run(host)
     monkeypatch.setattr(_native.fast, "grouped_forward", lambda *a: None)
-    assert torch.equal(got, step(G, *args)[0])
+    want = run(device)
+    assert len(got) == len(want) == 1 + train and all(torch.equal(a, b) for a, b in zip(got, want))
 
 
 def test_front_end_in_a_graph(G):
