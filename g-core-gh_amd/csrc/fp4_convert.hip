@@ -43,7 +43,6 @@ constexpr int kAmaxThreads = 256;
 // - where four tiles would leave more than a sixteenth empty at the rows' ends, byte loads up to five on every CU: 38400 x 768 [900] 9.70 / 8.52, 23040 x 1280 [900]
 //   10.36 / 8.68, 55552 x 768 [1302] 14.49 / 14.20; and handed round again beyond, 174848 x 768 [4098] 39.3 / 40.6.
 constexpr int kWideThreads = 512;
-constexpr int64_t kCUs = 256;
 
 // Maximum over the lane's own 128 x 128 tile, from one barrier.  One word a lane (W = 1, two tiles side by side): the 16 lanes of a DPP row belong to
 // one tile and the rows of a wave alternate between the tiles, so a wave reduces to one value per tile (DPP within rows, one cross-lane
@@ -510,7 +509,7 @@ extern "C" int lp_fp4_to_fp8_amax(const void *packed, const void *scale, int64_t
         return check_launch("lp_fp4_to_fp8_amax");
     };
     const bool two_words = (uintptr_t)packed % 8 == 0 && (uintptr_t)q_out % 16 == 0;
-    // see kCUs
+    // see kWideThreads
     const int64_t per_row = cols / 128, two = (per_row + 1) / 2 * 2, four = (per_row + 3) / 4 * 4, supers = rows / 128 * (two / 2);
     const bool wide = four * 16 <= two * 17 && supers * 4 > kCUs * (per_row >= 32 ? 8 : per_row >= 16 ? 11 : per_row == 8 ? 18 : 12);
     const bool handed = supers <= kCUs * (per_row < 16 ? 3 : 2) || supers > kCUs * 5;

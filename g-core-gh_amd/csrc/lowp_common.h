@@ -9,6 +9,10 @@
 
 namespace lowp {
 
+// Compute units of an MI355X.  The lines of the rules that choose a kernel are in tiles for all of them, which is how they were measured; a persistent launch
+// asks the device how many it has.
+constexpr int64_t kCUs = 256;
+
 // thread-local message buffer behind lp_last_error()
 char *error_buffer();
 constexpr int kErrorBufferSize = 512;
