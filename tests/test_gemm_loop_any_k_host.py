@@ -26,15 +26,19 @@ LOOPS = {          # name -> configure arguments
     "big [K, N]": (256, 256, 4, 2, 1, True, 2, False, True, False, True, True, True, False, True),
     "mid row scales": (128, 128, 2, 2, 1, True, 2, True, True, False, False, False, False, False, True),
     "big row scales": (256, 256, 4, 2, 1, True, 2, True, True, False, True, True, False, False, True),
+    "160 columns": (128, 160, 2, 2, 1, False, 2, False, True, True, False, False, False, False, True),
+    "160 columns e8m0": (128, 160, 2, 2, 1, True, 2, False, True, True, False, False, False, False, True),
     "flat [K, N]": (128, 256, 2, 4, 1, True, 3, False, True, False, True, False, True, False, True),
 }
 ABASE, BBASE, SBASE, BSBASE = 0x1_0000_0000 - 256, 0x3_0000_0000 - 384, 0x5_0000_0001, 0x7_0000_0003     # low halves that carry
+BSBASE2 = 0x9_0000_0005                                      # the second row of weight scales of a wave column that straddles two
 NPITCH = 1408                                                # [K, N]: columns of the stored weight
 
 
 class Wave:
-    def __init__(self, lines, kblocks, copies, idle, second):
+    def __init__(self, lines, kblocks, copies, idle, second, wave=0, groups=20):
         g = gen
+        self.wave, self.row_groups = wave, groups                # (160 columns: the groups of eight weight rows there are of the tile's 20)
         self.kblocks, self.copies, self.idle = kblocks, copies, idle
         self.code, self.labels = [], {}
         for ln in lines:
@@ -47,8 +51,11 @@ class Wave:
                    ard0=0, ard1=0, brd0=g.NSTAGE * g.A_BYTES, brd1=g.NSTAGE * g.A_BYTES)
         for i in range(8):
             ops[f"brdn{i}"] = ops["brd0"]
+        if g.WIDE:
+            ops.update(bstride=8 * 128 * kblocks, g4=8 if wave < 2 else 16, glim=groups - wave, splitnb=3)
         self.ops = ops
-        self.pairs = dict(abase=ABASE, bbase=BBASE, sbase=SBASE, bsptr=BSBASE)
+        self.pairs = dict(abase=ABASE, bbase=BBASE, sbase=SBASE, bsptr=BSBASE, bsptr2=BSBASE2)
+        self.moved = {}                                          # 160 columns: group of LDS rows -> the groups of weight rows copied there
         self.s, self.v, self.scc, self.m0 = {}, {}, 0, 0
         self.queue, self.landed, self.scales_on_way = [], {}, None
         self.step, self.mfma, self.groups = 0, 0, []
@@ -100,7 +107,7 @@ class Wave:
         off = re.search(r"offset:(\d+)", rest)
         off = int(off.group(1)) if off else int(rest.split(",")[-1], 0) if op.startswith("s_load") else 0
         ss = 1 if g.HW else 4
-        for name, start, pitch in (("a", SBASE, 1), ("b", BSBASE, NPITCH // 128 if g.NN else 1)):
+        for name, start, pitch in (("a", SBASE, 1), ("b", BSBASE, NPITCH // 128 if g.NN else 1), ("b2", BSBASE2, 1)):
             rel = base + off - start
             if 0 <= rel < 1 << 20:
                 if name == "b" and g.NN:
@@ -138,9 +145,9 @@ class Wave:
                 x = self.val(a[1]) + self.val(a[2]) + self.scc if op == "s_addc_u32" else self.val(a[1]) + (self.val(a[2]) if op == "s_add_u32" else -self.val(a[2]))
                 self.put(a[0], x)
                 self.scc = int(x >> 32 != 0)
-            elif op in ("s_and_b32", "s_xor_b32", "s_lshr_b32", "s_mul_i32"):
+            elif op in ("s_and_b32", "s_xor_b32", "s_lshr_b32", "s_lshl_b32", "s_mul_i32"):
                 x, y = self.val(a[1]), self.val(a[2])
-                self.put(a[0], {"s_and_b32": x & y, "s_xor_b32": x ^ y, "s_lshr_b32": x >> y, "s_mul_i32": x * y}[op])
+                self.put(a[0], x << y if op == "s_lshl_b32" else {"s_and_b32": x & y, "s_xor_b32": x ^ y, "s_lshr_b32": x >> y, "s_mul_i32": x * y}[op])
             elif op == "s_bfe_u32":
                 x, y = self.val(a[1]), self.val(a[2])
                 self.put(a[0], x >> (y & 31) & (1 << (y >> 16)) - 1)
@@ -160,6 +167,14 @@ class Wave:
                     rel = self.pair(a[1]) - ABASE
                     assert rel % 128 == 0 and 0 <= rel // 128 < self.kblocks, (ln, rel)
                     block = rel // 128
+                elif g.WIDE:
+                    rel = self.pair(a[1].split()[0]) - BBASE
+                    group, block = rel // self.ops["bstride"], rel % self.ops["bstride"] // 128
+                    # this wave's rows of the group lie inside the weight matrix; and the copy's place in LDS is that group's, or that of one past its end
+                    assert rel % 128 == 0 and 0 <= group and group + self.wave < self.row_groups, (ln, group, block)
+                    place = (self.m0 - g.NSTAGE * g.A_BYTES) % g.B_BYTES // 1024
+                    assert place == group if place + self.wave < self.row_groups else group == 0, (ln, place, group)
+                    self.moved.setdefault(place + self.wave, set()).add(block)
                 else:
                     rel, unit = self.pair(a[1].split()[0]) - BBASE, 128 * NPITCH if g.NN else 128
                     assert rel % unit == 0 and 0 <= rel // unit < self.kblocks, (ln, rel)
@@ -229,5 +244,19 @@ def test_requests_stay_inside_and_every_block_is_multiplied_once(name):
                         got = set(w.groups)
                         assert {x for x in got if x[0] == "b"} == (set() if gen.BROW else ss_total(kblocks)), (kblocks, sorted(got))
                         assert {x for x in got if x[0] == "a"} == ({("a", k) for k in range(kblocks)} if copies else set())
+    if gen.WIDE:
+        # all waves together: every group of weight rows there is at every block, wherever the matrix ends in the tile; the second row of scales like the first
+        for kblocks in (1, 2, 5, 8, 23):
+            for groups in (4, 8, 12, 16, 20):
+                moved = {}
+                for wave in range(4):
+                    w = Wave(lines, kblocks, int(wave < 2), 0, int(wave >= 2), wave, groups)
+                    w.run()
+                    assert w.step == kblocks
+                    assert {x for x in w.groups if x[0] == "b2"} == {("b2", k) for k in range(kblocks)}
+                    for place, blocks in w.moved.items():
+                        assert place not in moved, (place, wave)
+                        moved[place] = blocks
+                assert all(moved[i] == set(range(kblocks)) for i in range(groups)) and sorted(moved) == list(range(20)), (kblocks, groups, moved)
     for key, ways in staging.items():
         assert all(x == ways[0] for x in ways), ("an idle wave handles the scales it stages otherwise than a live one", key)
