@@ -27,7 +27,7 @@ CASES = {
     "streams_of_a_long_k": ([3] * 43 + [0] * 30, 1, 1536, 5504, 516, 258, "two", "128"),
     "streams_of_a_short_k": ([300] * 6 + [10] * 38 + [0] * 56, 1, 1280, 1024, 560, 250, "128", "two"),
     "by_rows": ([150] * 60, 1, 1024, 1024, 960, 240, "two", "two"),
-    # the order of the XCDs: few tall tiles, few flat ones, both, and few at 33 K blocks
+    # the order of the XCDs: few tall tiles, few flat ones, both, and few with a long K
     "few_tall": ([8] * 296 + [300] * 4, 1, 512, 1024, 1232, 608, "128", "two"),
     "few_flat": ([256] * 140 + [50] * 8, 1, 512, 1024, 1152, 296, "128", "two"),
     "both": ([40, 200] * 70, 1, 512, 1024, 840, 280, "128", "two"),
