@@ -15,14 +15,27 @@ CASES = {
     # rows per expert, N, K, tiles of 128 x 128 and of both heights, what the host's rule takes, what the device's
     "one_tile_a_cu": ([2] + [0] * 9, 15, 1280, 3840, 150, 75, "128", "two"),
     "second_round": ([3, 0, 0], 46, 1408, 3456, 506, 276, "128", "two"),
-    "tall_experts": ([40] * 21 + [176] * 2 + [0] * 60, 1, 1408, 3200, 275, 138, "128", "two"),
-    "two_a_cu_short_k": ([9, 0, 0], 46, 1280, 2944, 460, 230, "128", "two"),
+    "tall_experts": ([100] * 10 + [200] * 10 + [0] * 64, 1, 1408, 3200, 330, 120, "128", "two"),
+    "tall_experts_beside_streams": ([40] * 21 + [176] * 2, 1, 1408, 3200, 275, 138, "two", "128"),
+    "tall_and_short_of_one_expert": ([40] * 21 + [300] * 2 + [0] * 60, 1, 1408, 3200, 297, 150, "128", "two"),
+    "two_a_cu_short_k": ([9, 0, 0], 46, 1280, 2432, 460, 230, "128", "two"),
+    "two_a_cu_20_blocks": ([9] * 33, 1, 1536, 2560, 396, 198, "two", "128"),
     "two_a_cu_streams": ([6] * 35 + [0] * 3, 1, 1408, 3840, 385, 210, "two", "128"),
     "one_round": ([200] * 3 + [56] * 9, 1, 4608, 2816, 540, 216, "two", "128"),
     "half_a_second_round": ([7, 0], 64, 1408, 3200, 704, 384, "128", "two"),
+    "half_a_second_round_36_blocks": ([24], 42, 2048, 4608, 672, 336, "128", "128"),
+    "half_a_second_round_37_blocks": ([24], 42, 2048, 4736, 672, 336, "two", "128"),
+    "more_of_a_second_round_32_blocks": ([24] * 48 + [0] * 16, 1, 2048, 4096, 768, 384, "128", "two"),
+    "more_of_a_second_round_33_blocks": ([24], 48, 2048, 4224, 768, 384, "two", "128"),
     "short_k": ([300] * 10 + [80] * 10, 1, 3328, 1664, 1040, 390, "128", "two"),
     "short_k_of_20_blocks": ([5] * 193 + [0] * 107, 1, 512, 2560, 772, 386, "128", "two"),
     "short_k_two_full_rounds": ([64] * 12 + [200] * 3 + [300] * 3, 1, 6144, 1536, 1296, 504, "two", "two"),
+    "short_k_two_rounds_14_blocks": ([38], 28, 3840, 1792, 840, 420, "two", "two"),
+    "short_k_two_rounds_13_blocks": ([38], 28, 3840, 1664, 840, 420, "128", "two"),
+    "short_k_400_tiles": ([64], 50, 2048, 2048, 800, 400, "128", "two"),
+    "short_k_408_tiles": ([64], 51, 2048, 2048, 816, 408, "two", "two"),
+    "short_k_two_rounds_for_four": ([254], 74, 1408, 1280, 1628, 444, "two", "two"),
+    "short_k_two_rounds_for_three": ([254], 69, 1408, 1280, 1518, 414, "128", "two"),
     "more_than_three_a_cu": ([300] * 5 + [640] * 8, 1, 2048, 4224, 880, 272, "two", "128"),
     "streams_of_a_long_k": ([3] * 43 + [0] * 30, 1, 1536, 5504, 516, 258, "two", "128"),
     "streams_of_a_short_k": ([300] * 6 + [10] * 38 + [0] * 56, 1, 1280, 1024, 560, 250, "128", "two"),
