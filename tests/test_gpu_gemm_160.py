@@ -70,8 +70,8 @@ def same_as_columns_apart(M, N, K, ops, pow2, dtype, wide):
 LINES = [
     # two workgroups a CU
     ((1024, 8704, 2176), 544, 440, True, True), ((1000, 8576, 2176), 536, 432, True, False), ((1000, 8704, 1920), 544, 440, True, False),
-    ((1024, 8704, 2048), 544, 440, True, True), ((1100, 7808, 2048), 549, 441, True, False),
-    ((1200, 7040, 2560), 550, 440, True, True), ((1300, 6400, 2560), 550, 440, True, False), ((1300, 6400, 3072), 550, 440, True, True),
+    ((1024, 8704, 2048), 544, 440, True, True), ((1100, 7808, 2048), 549, 441, True, True),
+    ((1200, 7040, 2560), 550, 440, True, True), ((1300, 6400, 2560), 550, 440, True, True), ((1300, 6400, 3072), 550, 440, True, True),
     ((400, 17408, 1024), 544, 436, True, False), ((1000, 8704, 1024), 544, 440, True, False), ((640, 15104, 1024), 590, 475, True, False),
     ((400, 17408, 1152), 544, 436, True, False), ((1000, 8704, 896), 544, 440, False, False), ((1000, 8320, 1152), 520, 416, False, False), ((1000, 8320, 2048), 520, 416, True, False),
     ((1000, 10496, 2176), 656, 528, False, False),                                          # three a CU either way
