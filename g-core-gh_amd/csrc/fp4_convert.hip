@@ -34,12 +34,11 @@ constexpr int kAmaxThreads = 256;
 // 1024 level, 32768 x 1152 15.4 -> 13.8, 65536 x 7168 132.7 -> 131.9).  One word a lane is left to other alignments and to the form that writes bf16 too.
 // Three forms of it, by the super tiles of 128 x 256 there are for the 256 CUs and by the tiles in a row (lp_fp4_to_fp8_amax).  In brackets super tiles; us,
 // two tiles a workgroup with the scale bytes handed round / two with a byte load for each / four with the bytes handed round:
-// - up to three on every CU the first is ahead for short rows: 33024 x 512 [516] 6.16 / 6.32 / 6.65, 24576 x 1024 [768] 6.92 / 7.63 / 7.45.  From 16 tiles a row on only
-//   up to two: 8960 x 2048 [560] 6.76 / 6.52 / 6.81, 5888 x 3584 [644] 7.40 / 6.73 / 7.02; and from 32 on, four tiles have what they need from there:
-//   4480 x 4096 [560] 7.83 / 7.12 / 7.05, 2944 x 7168 [644] 8.25 / 7.05 / 7.22, 4224 x 7168 [924] 11.63 / 10.84 / 8.41.
-// - beyond, four tiles: 57600 x 512 [900] 9.27 / 8.44 / 7.93, 14464 x 2048 [904] 10.64 / 10.37 / 8.11, 12288 x 2048 [768] 7.65 / 7.53 / 7.24, 65536 x 7168 131.1 / 136.2 / 123.4 =
-//   5.8 TB/s; with rows of 1024 columns, whose pieces of a workgroup lie a power of two apart, only past nine halves: 32768 x 1024 [1024] 10.72 / 9.48 / 11.68, 35200 x 1024
-//   [1100] 12.48 / 11.93 / 13.05, 41600 x 1024 [1300] 14.85 / 14.40 / 14.38 (28800 x 896 [900] 9.10 with byte loads, 7.41 in fours).
+// - up to two on every CU, and three with rows of fewer than 16 tiles, the first: 33024 x 512 [516] 6.16 / 6.32 / 6.65, 24576 x 1024 [768] 6.92 / 7.63 / 7.45; longer rows up to three
+//   the second: 8960 x 2048 [560] 6.76 / 6.52 / 6.81, 5888 x 3584 [644] 7.40 / 6.73 / 7.02, 2944 x 7168 [644] 8.25 / 7.05 / 7.22, 70 such sizes drawn 0.96 of the time in fours.
+// - beyond, four tiles: 57600 x 512 [900] 9.27 / 8.44 / 7.93, 14464 x 2048 [904] 10.64 / 10.37 / 8.11, 4224 x 7168 [924] 11.63 / 10.84 / 8.41, 65536 x 7168 131.1 / 136.2 / 123.4 =
+//   5.8 TB/s.  Not with rows of 1024 columns, whose pieces of a workgroup lie a power of two apart, from seven halves to five on every CU: 25600 x 1024 [800] - / 8.35 / 7.73, 28672 x
+//   1024 [896] - / 9.15 / 8.41, 30464 x 1024 [952] - / 9.00 / 9.24, 32768 x 1024 [1024] 10.72 / 9.48 / 11.68, 38400 x 1024 [1200] - / 13.4 / 14.2, 41600 x 1024 [1300] 14.85 / 14.40 / 14.38.
 // - where four tiles would leave more than a sixteenth empty at the rows' ends, byte loads up to five on every CU: 38400 x 768 [900] 9.70 / 8.52, 23040 x 1280 [900]
 //   10.36 / 8.68, 55552 x 768 [1302] 14.49 / 14.20; and handed round again beyond, 174848 x 768 [4098] 39.3 / 40.6.
 constexpr int kWideThreads = 512;
@@ -235,7 +234,7 @@ __device__ __forceinline__ void store_codes(const u32x2 *out, uint8_t *dst)
     else __builtin_nontemporal_store(out[0], (u32x2 *)dst);
 }
 
-template <int MODE, bool WRITE_BF16, int NT, int W, int TILES = 2, bool BYTES = W == 1>
+template <int MODE, bool WRITE_BF16, int NT, int W, int TILES = 2, bool BYTES = W == 1, bool WAVES = BYTES && W == 2>
 __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packed, const uint8_t *__restrict__ scale,
                                                 int64_t cols, int64_t supers_c, int64_t n_supers, int64_t per_xcd,
                                                 float amax_floor, int zero_rule, uint8_t *__restrict__ q,
@@ -346,10 +345,11 @@ __global__ __launch_bounds__(NT) void fp4_amax(const uint8_t *__restrict__ packe
         }
     }
 
-    // Behind a branch that it knows to be uniform the compiler keeps 30 registers more, which takes two to three of eight waves of a SIMD.  Two words
-    // with a byte load each, which are for launches of few rounds, are better off with the waves; large launches are not (65536 x 4096 in fours 74.9 <- 80.3).
+    // Behind a branch that it knows to be uniform the compiler keeps 30 registers more, which takes two to three of eight waves of a SIMD.  WAVES: the waves
+    // instead, for launches of few rounds -- two words with a byte load each, and one word up to five super tiles on every CU (0.95 of the time up to two); larger
+    // ones are better off with the registers (one word from 1280 super tiles on 1.03 <- 1; 65536 x 4096 in fours 74.9 <- 80.3).
     uint32_t slow = slow_tile;
-    if constexpr (BYTES && W == 2) asm volatile("" : "+v"(slow));
+    if constexpr (WAVES) asm volatile("" : "+v"(slow));
     if (!slow) {
         if (g.active && (t & (16 / W - 1)) == 0 && t < LANES) store_scale(scale_out, scale_dtype, g.tile, bs.stored);
         if (!g.active) return;
@@ -511,11 +511,13 @@ extern "C" int lp_fp4_to_fp8_amax(const void *packed, const void *scale, int64_t
     const bool two_words = (uintptr_t)packed % 8 == 0 && (uintptr_t)q_out % 16 == 0;
     // see kWideThreads
     const int64_t per_row = cols / 128, two = (per_row + 1) / 2 * 2, four = (per_row + 3) / 4 * 4, supers = rows / 128 * (two / 2);
-    const bool wide = four * 16 <= two * 17 && supers * 4 > kCUs * (per_row >= 32 ? 8 : per_row >= 16 ? 11 : per_row == 8 ? 18 : 12);
-    const bool handed = supers <= kCUs * (per_row < 16 ? 3 : 2) || supers > kCUs * 5;
+    const bool apart = per_row == 8 && 2 * supers > 7 * kCUs && supers <= 5 * kCUs;
+    const bool wide = four * 16 <= two * 17 && supers > 3 * kCUs && !apart;
+    const bool many = supers > 5 * kCUs, handed = many || supers <= kCUs * (per_row < 16 ? 3 : 2);
 #define LAUNCH(MODE)                                                                                                   \
     return bf16_out ? go(fp4_amax<MODE, true, kAmaxThreads, 1>, kAmaxThreads, 2)                                        \
-         : !two_words ? go(fp4_amax<MODE, false, kAmaxThreads, 1>, kAmaxThreads, 2)                                     \
+         : !two_words && many ? go(fp4_amax<MODE, false, kAmaxThreads, 1>, kAmaxThreads, 2)                             \
+         : !two_words ? go(fp4_amax<MODE, false, kAmaxThreads, 1, 2, true, true>, kAmaxThreads, 2)                      \
          : wide ? go(fp4_amax<MODE, false, kWideThreads, 2, 4>, kWideThreads, 4)                                        \
          : handed ? go(fp4_amax<MODE, false, kAmaxThreads, 2>, kAmaxThreads, 2)                                         \
                   : go(fp4_amax<MODE, false, kAmaxThreads, 2, 2, true>, kAmaxThreads, 2)

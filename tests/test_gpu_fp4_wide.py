@@ -9,15 +9,16 @@ from tests.test_gpu_fp4_words import convert
 
 pytestmark = pytest.mark.gpu
 
-FORMS = {"handed": "ELb0ELi256ELi2ELi2ELb0E", "bytes": "ELb0ELi256ELi2ELi2ELb1E", "four": "ELb0ELi512ELi2ELi4ELb0E", "one word": "ELb0ELi256ELi1ELi2ELb1E"}
+FORMS = {"handed": "ELb0ELi256ELi2ELi2ELb0E", "bytes": "ELb0ELi256ELi2ELi2ELb1E", "four": "ELb0ELi512ELi2ELi4ELb0E",
+         "one word": "ELb0ELi256ELi1ELi2ELb1ELb1E", "one word, many": "ELb0ELi256ELi1ELi2ELb1ELb0E"}
 CASES = [
     # (rows of tiles, tiles a row), form
     ((768, 2), "handed"), ((769, 2), "bytes"), ((1280, 2), "bytes"), ((1281, 2), "handed"), ((600, 1), "handed"),      # four tiles would leave half of them empty
     ((384, 3), "handed"), ((385, 3), "four"), ((384, 4), "handed"), ((385, 4), "four"),
     ((300, 5), "bytes"),                                                                                              # a quarter empty
-    ((192, 7), "handed"), ((193, 7), "four"), ((192, 8), "handed"), ((193, 8), "bytes"), ((288, 8), "bytes"), ((289, 8), "four"),
-    ((64, 16), "handed"), ((65, 16), "bytes"), ((88, 16), "bytes"), ((89, 16), "four"), ((89, 18), "bytes"),
-    ((30, 33), "handed"), ((31, 33), "four"), ((30, 34), "handed"), ((31, 34), "four"), ((30, 35), "four"),
+    ((192, 7), "handed"), ((193, 7), "four"), ((192, 8), "handed"), ((193, 8), "four"), ((224, 8), "four"), ((225, 8), "bytes"), ((320, 8), "bytes"), ((321, 8), "four"),
+    ((64, 16), "handed"), ((65, 16), "bytes"), ((96, 16), "bytes"), ((97, 16), "four"), ((89, 18), "bytes"),
+    ((30, 33), "handed"), ((31, 33), "bytes"), ((45, 33), "bytes"), ((46, 33), "four"), ((30, 34), "handed"), ((45, 34), "bytes"), ((46, 34), "four"), ((43, 35), "four"),
 ]
 
 
@@ -25,7 +26,8 @@ def check(packed, scale, modes, form):
     for mode, dtype in modes:
         (a, sa), (b, sb) = (convert(packed, scale, mode, dtype, shift) for shift in (0, 1))
         assert torch.equal(a, b) and torch.equal(sa.view(torch.uint8), sb.view(torch.uint8))
-    for shift, wanted in ((0, form), (1, "one word")):
+    pairs = packed.shape[0] // 128 * -(-packed.shape[1] // 128)
+    for shift, wanted in ((0, form), (1, "one word, many" if pairs > 1280 else "one word")):
         ran = kernels(lambda: convert(packed, scale, *modes[0], shift, False))
         assert [FORMS[wanted] in n for n in ran if "fp4_amax" in n] == [True], (wanted, ran)
 
@@ -50,7 +52,7 @@ def test_forms_give_the_same_bytes(size, form, edge):
 
 
 @pytest.mark.parametrize("offset", [1, 2, 3])
-@pytest.mark.parametrize("size,form", [((3, 5), "handed"), ((65, 16), "bytes"), ((31, 34), "four")], ids=str)
+@pytest.mark.parametrize("size,form", [((3, 5), "handed"), ((65, 16), "bytes"), ((46, 34), "four")], ids=str)
 def test_scales_off_their_alignment(size, form, offset):
     """Scale bytes that start anywhere: the same kernels, the same result."""
     from gcore_lowp import _abi as A
